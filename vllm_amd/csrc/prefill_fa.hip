@@ -62,10 +62,11 @@ constexpr int KR128 = 8, VR128 = 4;   // fragment reads in flight: K reads, V^T 
 constexpr int KR256 = FA_KRW, VR256 = FA_VRW;
 constexpr float THR = 8.f;        // lazy rescale threshold (log2 domain)
 
+// One v_maximum3_f32.  (fmaxf on MFMA results makes hipcc canonicalise every input first; inline asm must not read them
+// at all: the wait states between an MFMA and a VALU read of its result are the compiler's to insert, it inserts none in
+// front of an asm block, and the hardware does not wait -- the row maximum then came from a sum still being accumulated.)
 __device__ __forceinline__ float max3(float a, float b, float c) {
-  float r;   // (fmaxf on MFMA results makes hipcc canonicalise every input first)
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
 // own value and the value of lane ^ 32, in some order.  v_permlane32_swap vdst, src exchanges lanes 32-63 of vdst
 // with lanes 0-31 of src; inline asm (with the two wait states a VALU write of an operand needs in front of it),
