@@ -469,7 +469,7 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*   "pa_order":   0 = unpartitioned decode launches keep the hardware's workgroup     */
 /*                 order (default 1: sequences handed out longest first, the two       */
 /*                 workgroups of a CU paired long + short; same output bits)          */
-/*   "mm_kernel":  scaled_mm kernel for M > 32: 0 = heuristic, 1 = register-   */
+/*   "mm_kernel":  scaled_mm kernel: 0 = heuristic,             1 = register-   */
 /*                 staged 128x128 tile, 2..10 = direct-to-LDS tile shapes       */
 /*                 (256x256, 128x128, 128x64, 64x64, 64x32; even ids 4..10      */
 /*                 take 2 or 4 K blocks per barrier; scaled_mm_large.hip),      */
@@ -484,7 +484,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 block; 21 = what the heuristic ships for MFMA-bound shapes),     */
 /*                 26..28 = 64x64 / 128x64 tiles with deeper rings (no gain),       */
 /*                 29..36 = 18..25 with 256 x 192 tiles (the heuristic takes them  */
-/*                 where they save a round of workgroups: N 6144)                  */
+/*                 where they save a round of workgroups: N 6144),                 */
+/*                 37 = scaled_mm_stream.hip (M <= 64, K a multiple of 128)         */
 /*   "mm_patch":   tile columns per super-column of the scaled_mm_pp tile order    */
 /*                 (default 8; <= 1 = column-major)                                  */
 /*   "mm_store":   scaled_mm_pp measurement: 3 = no output stores (garbage)         */

@@ -347,3 +347,34 @@ def test_scaled_mm_split_k_graph_capture(ops, force_kernel):
     assert torch.equal(out, ref)          # captured = unsplit
     assert torch.equal(again, eager)
     torch.testing.assert_close(eager.float(), ref.float(), rtol=1.6e-2, atol=5e-3)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 49, 64])
+@pytest.mark.parametrize("NK", [(16, 256), (24, 384), (971, 1152), (1280, 2048), (5136, 1024), (5126, 4096), (16400, 256),
+                                (8232, 1280), (8232, 4224)])
+def test_scaled_mm_stream_edges(ops, force_kernel, M, NK):
+    """The weight-streaming kernel for M <= 64 (scaled_mm_stream.hip): row blocks of 16 and their remainders; 16- and
+    32-column tiles (the rule turns at 160 of the latter), one and several tiles per workgroup, ragged N (scalar stores),
+    fewer K blocks than waves, K blocks that do not divide among them, resident and streamed activations.  Small-integer
+    operands and power-of-two scales: the fp32 product is exact, whatever the order of the sums."""
+    N, K = NK
+    force_kernel(37)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-3, 4, (M, K), generator=g).float()
+    w = torch.randint(-2, 3, (N, K), generator=g).float()
+    a[:, 0] = torch.arange(M).float() % 7
+    w[:, 1] = torch.arange(N).float() % 5
+    a8, w8 = a.to(torch.float8_e4m3fn).cuda(), w.to(torch.float8_e4m3fn).cuda()
+    prod = (a.double() @ w.double().t()).float().cuda()
+    sa = (2.0 ** -(torch.arange(M) % 5).float()).reshape(M, 1).cuda()
+    sb = (2.0 ** -(torch.arange(N) % 3).float()).reshape(N, 1).cuda()
+    bias = (torch.arange(N) % 9).to(torch.float16).cuda()
+    out = ops.cutlass_scaled_mm(a8, w8.t(), sa, sb, torch.float16, bias)
+    ref = (prod * sa * sb.t()).to(torch.float16)
+    assert torch.equal(out, (ref.float() + bias.float()).to(torch.float16))
+    one = torch.ones((1, 1), device="cuda")
+    # rows of the output 4 bytes off the 8-byte grid, guard columns on both sides untouched
+    buf = torch.full((M, N + 6), 7.0, dtype=torch.bfloat16, device="cuda")
+    torch.ops._C.cutlass_scaled_mm(buf[:, 2:2 + N], a8, w8.t(), one, one, None)
+    assert torch.equal(buf[:, 2:2 + N], prod.to(torch.bfloat16))
+    assert (buf[:, :2] == 7).all() and (buf[:, 2 + N:] == 7).all()

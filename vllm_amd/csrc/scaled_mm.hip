@@ -171,7 +171,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void scaled_mm_kernel(
 
 
 // ---------------------------------------------------------------------------
-// Skinny GEMM, M <= 64 (decode): weight-bandwidth bound.  A workgroup of 8 waves
+// Skinny GEMM, M <= 32 and K not a multiple of 128 (scaled_mm_stream.hip takes the others).  A workgroup of 8 waves
 // owns 16 weight rows (output columns) and ALL M rows; the waves split K.  W is
 // streamed once, straight into VGPRs in MFMA operand order (no LDS round trip:
 // each byte is used by one wave only); the contraction index inside a 128-byte
@@ -272,11 +272,16 @@ int launch_scaled_mm_large(int shape, void* out, const void* a, const void* b,
                            int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
                            int out_dtype, bool vec, int splits, int ws_mode, hipStream_t st);
 bool scaled_mm_large_fits(int M, int N, int K, int64_t lda, int64_t ldb);
+// scaled_mm_stream.hip
+bool scaled_mm_stream_pays(int M, int N, int K);
+int launch_scaled_mm_stream(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
+                            const void* bias, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
+                            int out_dtype, hipStream_t st);
 // scaled_mm_pp.hip
 int launch_scaled_mm_pp(int variant, void* out, const void* a, const void* b, const float* a_scales,
                         const float* b_scales, const void* bias, int M, int N, int K, int64_t lda,
                         int64_t ldb, int64_t ldc, int asn, int bsn, int out_dtype, hipStream_t st);
-int g_mm_kernel = 0;   // tuning: 0 auto, 1 = register-staged 128x128, 2..10, 12, 13 = glds tile shapes
+int g_mm_kernel = 0;   // tuning: 0 auto, 1 = register-staged 128x128, 2..10, 12, 13 = glds tile shapes, 37 = the stream kernel
 int g_mm_splitk = 0;   // tuning: 0 auto, n >= 1 = n K slices (1 = never split)
 int g_mm_tail = 0;     // tuning key kept for old scripts; the tail split went away with the persistent kernel
 }  // namespace va
@@ -300,13 +305,16 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
   VA_REQUIRE((a_scale_numel == 1 || a_scale_numel == M) && (b_scale_numel == 1 || b_scale_numel == N),
              VLLM_AMD_EINVAL, "%s: scales must be per-tensor or per-row/per-column", op);
   const bool glds_ok = K % 128 == 0 && K >= 256 && scaled_mm_large_fits(M, N, K, lda, ldb);
-  // M <= 32: the weight-streaming kernel (one workgroup per 16 output columns) wins while
-  // its grid is a single wave of workgroups and M fits one MFMA tile; beyond that the
-  // 64x32 direct-to-LDS tile is flat in M and faster (profiles/r01_gemm_sweep_small.csv).
-  // "mm_kernel" 11 forces it.
-  const bool skinny = g_mm_kernel == 11 ||
-                      (g_mm_kernel == 0 &&
-                       (!glds_ok || (M <= 16 && ceil_div(N, 16) <= 256)));   // (round 3, HBM-served weights: 14336 x 4096 at M 16 18.9 vs 20.3 us)
+  const int want_splits = req_splits > 0 ? req_splits : g_mm_splitk;   // 0 = heuristic
+  // M <= 64: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it)
+  if (glds_ok && M <= 64 &&
+      (g_mm_kernel == 37 || (g_mm_kernel == 0 && want_splits == 0 && scaled_mm_stream_pays(M, N, K)))) {
+    launch_scaled_mm_stream(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel, out_dtype, st);
+    VA_LAUNCH_CHECK(op);
+    return VLLM_AMD_OK;
+  }
+  // K not a multiple of 128: the register-streaming kernel.  "mm_kernel" 11 forces it.
+  const bool skinny = g_mm_kernel == 11 || (g_mm_kernel == 0 && !glds_ok);
   if (M <= 32 && skinny) {
     const int mt = ceil_div(M, 16);
 #define SK(T, MT)                                                                              \
@@ -316,8 +324,7 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
                      b_scale_numel)
 #define SKT(T)                                       \
   do {                                               \
-    if (mt == 1) SK(T, 1); else if (mt == 2) SK(T, 2); \
-    else if (mt == 3) SK(T, 3); else SK(T, 4);       \
+    if (mt == 1) SK(T, 1); else SK(T, 2);            \
   } while (0)
     if (out_dtype == VLLM_AMD_BF16) SKT(bf16_t); else SKT(f16_t);
 #undef SKT
@@ -329,7 +336,6 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
   const bool vec = (ldc % 4 == 0) && ((((uintptr_t)out) & 7) == 0);
   if (glds_ok) {
     int sel = g_mm_kernel;
-    const int want_splits = req_splits > 0 ? req_splits : g_mm_splitk;   // 0 = heuristic
     int splits = want_splits > 0 ? want_splits : 1;
     if (sel >= 29 && sel <= 36) sel = -(sel - 29 + 8) - 100;   // 29 .. 36: the same variants with 256 x 192 tiles
     if ((sel >= 18 && sel <= 25) || sel <= -100) {
