@@ -362,6 +362,28 @@ int vllm_amd_context_attention_fwd(
     int64_t vc_block_stride, int64_t vc_head_stride, float sm_scale, int sliding_window,
     int skip_decode, int num_tokens, int dtype, int kv_cache_dtype, void* stream);
 
+/* The same, split over the keys where few row blocks would each walk a long key range alone:
+ * segm_output float[num_tokens][num_heads][num_segments][head_size] (16-byte aligned), segm_max /
+ * segm_expsum float[num_tokens][num_heads][num_segments], caller-owned scratch; num_segments =
+ * what vllm_amd_context_attention_fwd_segments answers (1: no scratch needed), max_seq_len = the
+ * longest sequence or an upper bound of it. */
+int vllm_amd_context_attention_fwd_split(
+    void* o, const void* q, const void* k, const void* v, const void* k_cache,
+    const void* v_cache, const int* b_loc, const int* b_start_loc,
+    const int* b_seq_len, const float* k_scale, const float* v_scale,
+    const float* alibi_slopes, const float* fp8_out_scale, int batch, int num_heads,
+    int num_kv_heads, int head_size, int block_size, int max_input_len,
+    int64_t b_loc_stride, int64_t q_stride_t, int64_t q_stride_h, int64_t k_stride_t,
+    int64_t k_stride_h, int64_t v_stride_t, int64_t v_stride_h, int64_t o_stride_t,
+    int64_t o_stride_h, int64_t kc_block_stride, int64_t kc_head_stride,
+    int64_t vc_block_stride, int64_t vc_head_stride, float sm_scale, int sliding_window,
+    int skip_decode, int num_tokens, float* segm_output, float* segm_max, float* segm_expsum,
+    int num_segments, int max_seq_len, int dtype, int kv_cache_dtype, void* stream);
+int vllm_amd_context_attention_fwd_segments(int batch, int num_heads, int num_kv_heads,
+                                            int head_size, int max_input_len, int max_seq_len,
+                                            int num_tokens, int has_alibi, int sliding_window,
+                                            int skip_decode);
+
 /* Replaces unified_attention (vllm/attention/ops/triton_unified_attention.py:588-700; Triton
  * kernels kernel_unified_attention_2d :52-272 / _3d :276-586): the V1 engine's attention over
  * the FLASH-layout cache.  For sequence b the query tokens q[cu_seqlens_q[b] :
@@ -405,6 +427,10 @@ int vllm_amd_unified_attention(
     int64_t vc_stride_slot, int64_t vc_stride_head, float softmax_scale, int sliding_window,
     float softcap, int num_tokens, int max_seqlen_k, float* segm_output, float* segm_max,
     float* segm_expsum, int num_segments, int dtype, int kv_cache_dtype, void* stream);
+/* num_segments a launch of these sizes can use (1: no scratch needed) */
+int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, int num_kv_heads,
+                                        int head_size, int max_seqlen_q, int max_seqlen_k,
+                                        int num_tokens, int has_alibi);
 
 /* ------------------------------------------------------------------------- */
 /* Peer-to-peer all-reduce over xGMI                         */
@@ -469,6 +495,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*   "pa_order":   0 = unpartitioned decode launches keep the hardware's workgroup     */
 /*                 order (default 1: sequences handed out longest first, the two       */
 /*                 workgroups of a CU paired long + short; same output bits)          */
+/*   "pf_segs":    key segments of the 256-row prefill kernel (0 = heuristic; at most the  */
+/*                 num_segments the caller brings scratch for)                            */
 /*   "mm_kernel":  scaled_mm kernel: 0 = heuristic,             1 = register-   */
 /*                 staged 128x128 tile, 2..10 = direct-to-LDS tile shapes       */
 /*                 (256x256, 128x128, 128x64, 64x64, 64x32; even ids 4..10      */

@@ -298,3 +298,37 @@ def test_prefill_long_chunk_repeats_bit_for_bit(dtype, kv, ctx):
     first = run(c, kv)
     for _ in range(6):
         assert torch.equal(run(c, kv), first)
+
+
+@pytest.fixture
+def tuning():
+    from vllm_amd import _lib
+    used = []
+
+    def set_(key, value):
+        used.append(key)
+        _lib.set_tuning(key, value)
+    yield set_
+    for key in used:
+        _lib.set_tuning(key, 0)
+
+
+@pytest.mark.parametrize("segs", [2, 5, 32])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("head_size,gqa", [(128, 4), (64, 1), (96, 8), (256, 2)])
+def test_prefill_key_segments(oracle, tuning, segs, kv, head_size, gqa):
+    """Few row blocks: the keys split over workgroups (segments that end inside the context, inside the new tokens and on
+    the boundary; more segments than tiles; a one-token and a context-free sequence; rows past a block)."""
+    tuning("pf_segs", segs)
+    dtype = torch.bfloat16 if segs == 5 else torch.float16
+    c = make_prefill_case([70, 1, 150, 33], [500, 130, 0, 64], 8, 8 // gqa, head_size, 16, dtype, kv, seed=segs + head_size,
+                          kv_scale=0.02)
+    out = run(c, kv)
+    assert not out.isnan().any()
+    torch.testing.assert_close(out.float(), run_oracle(oracle, c, kv).float(), atol=tol(dtype), rtol=0)
+    assert torch.equal(run(c, kv), out)
+    scale = torch.tensor([0.01], device="cuda")
+    o8 = run(c, kv, fp8_out_scale=scale)
+    ref = (out.float() / 0.01).clamp(-448, 448).to(torch.float8_e4m3fn).float()
+    # the partial sums are the same; out is rounded to 16 bits before the division here: one code apart
+    assert ((o8.view(torch.float8_e4m3fn).float() - ref).abs() <= 0.13 * ref.abs() + 2 ** -9).all()

@@ -500,3 +500,25 @@ def test_unified_fa_kernel_softcap(oracle, force_fa, soft_cap, D, fp8, window):
         c = make_unified_case([(300, 700), (129, 463), (1, 90), (70, 70)], 8, 2, D, 16, dtype, fp8=fp8,
                               seed=int(soft_cap) + D, kv_scale=0.5)
         run(oracle, c, dtype, fp8=fp8, softcap=soft_cap, window=window)
+
+
+@pytest.mark.parametrize("segs", [2, 5, 32])
+@pytest.mark.parametrize("num_heads,head_size", [((8, 2), 128), ((8, 8), 64), ((8, 1), 80), ((4, 2), 256)])
+@pytest.mark.parametrize("mode", ["plain", "fp8", "window", "softcap", "fp8_out", "mixed"])
+def test_unified_prefill_key_segments(oracle, segs, num_heads, head_size, mode):
+    """Few row blocks over long key ranges: the 256-row kernel split over the keys.  Segments that end inside a sequence,
+    more segments than tiles, rows that see nothing of a segment (the causal edge, the window), a one-token sequence;
+    "mixed": 16 sequences, whose one-token ones the decode kernel takes and the merge must leave alone."""
+    from vllm_amd import _lib
+    lens = [(70, 700), (1, 300), (150, 150), (33, 97)]
+    if mode == "mixed":
+        lens += [(1, 20 + 40 * i) for i in range(12)]
+    fp8 = mode in ("fp8", "fp8_out", "mixed")
+    c = make_unified_case(lens, num_heads[0], num_heads[1], head_size, 16, torch.bfloat16, fp8=fp8, seed=segs + head_size,
+                          kv_scale=0.5)
+    _lib.set_tuning("pf_segs", segs)
+    try:
+        run(oracle, c, torch.bfloat16, window=100 if mode == "window" else None, softcap=20.0 if mode == "softcap" else 0.0,
+            out_scale=torch.tensor([0.02]) if mode == "fp8_out" else None, fp8=fp8)
+    finally:
+        _lib.set_tuning("pf_segs", 0)

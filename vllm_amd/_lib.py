@@ -66,6 +66,12 @@ SIGNATURES = {
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i,
         _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f, _i, _f, _i, _i, _vp,
         _vp, _vp, _i, _i, _i, _vp],
+    "vllm_amd_context_attention_fwd_split": [
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i,
+        _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f, _i, _i,
+        _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
+    "vllm_amd_context_attention_fwd_segments": [_i] * 10,
+    "vllm_amd_unified_attention_segments": [_i] * 8,
     "vllm_amd_set_tuning": [C.c_char_p, _i],
     "vllm_amd_get_tuning": [C.c_char_p, C.POINTER(_i)],
     "vllm_amd_ar_init": [C.POINTER(_vp), C.POINTER(_vp), _i64, _vp, _i64, _i, _i, _i],

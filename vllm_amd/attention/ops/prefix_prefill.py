@@ -66,12 +66,27 @@ def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_l
     assert k_cache.stride(4) == 1 and k_cache.stride(3) == k_cache.shape[4] \
         and k_cache.stride(2) == k_cache.shape[3] * k_cache.shape[4]
     assert v_cache.stride(3) == 1 and v_cache.stride(2) == block_size
+    # scratch for launches that split the keys (few row blocks over long prefixes)
+    num_tokens = q.shape[0]
+    max_k = int(max_seq_len) if max_seq_len else b_loc.shape[1] * block_size
+    nseg = lib.vllm_amd_context_attention_fwd_segments(batch, head, k.shape[1], Lq, int(max_input_len), max_k, num_tokens,
+                                                       int(alibi_slopes is not None), int(sliding_window), int(bool(skip_decode)))
+    segm_out = segm_max = segm_sum = None
+    if nseg > 1 and q.dtype != torch.float32:
+        rows = num_tokens * head * nseg
+        segm = torch.empty(rows * (Lq + 2), dtype=torch.float32, device=q.device)
+        segm_out = segm.data_ptr()
+        segm_max = segm_out + 4 * rows * Lq
+        segm_sum = segm_max + 4 * rows
+    else:
+        nseg = 1
     with _dev(q):
-        check(lib.vllm_amd_context_attention_fwd(
+        check(lib.vllm_amd_context_attention_fwd_split(
             _ptr(o), _ptr(q), _ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), _ptr(b_loc),
             _ptr(b_start_loc), _ptr(b_seq_len), _ptr(k_scale), _ptr(v_scale),
             _ptr(alibi_slopes), _ptr(fp8_out_scale), batch, head, k.shape[1], Lq, block_size,
             int(max_input_len), b_loc.stride(0), q.stride(0), q.stride(1), k.stride(0),
             k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), k_cache.stride(0),
             k_cache.stride(1), v_cache.stride(0), v_cache.stride(1), float(sm_scale),
-            int(sliding_window), int(bool(skip_decode)), q.shape[0], _DT[q.dtype], kvd, _stream(q)))
+            int(sliding_window), int(bool(skip_decode)), num_tokens,
+            segm_out, segm_max, segm_sum, nseg, max_k, _DT[q.dtype], kvd, _stream(q)))

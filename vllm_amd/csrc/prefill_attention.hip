@@ -30,6 +30,7 @@ int g_pf_rows = 0;   // tuning "pf_rows": query rows per workgroup (0 = default)
 int g_uni_decode = 1;   // tuning "uni_decode": 0 = decode-only launches take the packed tile kernel
 extern int g_pf_fa_stagger;   // prefill_fa.hip
 int g_pf_fa_abl = 0;    // tuning "pf_fa_abl": measurement only, see prefill_fa.cuh
+int g_pf_segs = 0;      // tuning "pf_segs": key segments of the 256-row kernel (0 = heuristic; needs the caller's scratch)
 int g_pf_fa = 0;        // tuning "pf_fa": 1 = unified_attention never takes the 256-row kernel (prefill_fa.hip), 2 = whenever it can
 
 struct PrefillParams {
@@ -753,6 +754,37 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
   else if constexpr (!UNI)
     hipLaunchKernelGGL((prefill_kernel<T, FP8, D, 32, MT, NW, UNI, PACK>), grid, dim3(64 * NW), 0, st, p);
 }
+// Whether a launch of query chunks takes the 256-row kernel (prefill_fa.hip; 128 rows above head size 128), and into how
+// many key segments it is split.  max_k: longest key range (an upper bound will do), ptok: query tokens of the chunks,
+// nchunk: sequences among them (a lower bound will do), cap: segments the caller has scratch for.
+//   * >= 128 row blocks, chunks of at least one: unsplit.
+//   * fewer: the 64-row kernel's four times as many workgroups finished sooner than that (chunk 256 over 4096 cached tokens
+//     among 255 decodes: 32 blocks, 82 against 150 us) and still left the chip idle behind one serial walk over the keys
+//     (2.1 us per 64-key tile).  Split, the blocks give at least 256 workgroups; a segment is worth its start-up from three
+//     tiles on, the merge its launch from 16 tiles on (400 keys: 26.7 us unsplit, 32.6 split).  us, 64-row kernel -> split:
+//     35 tokens over 3723, 8 q / 1 kv head 123 -> 32; 512 over 8000, 32 / 8 208 -> 87; 1024 over 4000 139 -> 102; head 64,
+//     300 over 3000 87 -> 33; head 256, 2 x 300 over 3000 159 -> 60; x-layout prefix, 300 over 3000 106 -> 44.
+struct FaPlan { bool use; int nseg; };
+static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap) {
+  const int gqa = num_heads / num_kv_heads;
+  const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
+  const int tpb = (head_size > 128 ? 128 : 256) / pack;
+  const int y = pack > 1 ? num_kv_heads : num_heads;
+  if (g_pf_fa == 1 || g_pf_rows != 0 || (max_q <= 1 && g_pf_fa != 2) || head_size > 256) return {false, 1};
+  const bool whole = head_size > 64 && (g_pf_fa == 2 || (max_q >= tpb && ptok / tpb * y >= 128));
+  int64_t blocks = (ptok + tpb - 1) / tpb;
+  if (blocks < nchunk) blocks = nchunk;
+  blocks *= y;
+  int nseg = blocks > 0 && blocks <= 128 && max_k >= 16 * PF_BN ? (int)(256 / blocks) : 1;
+  const int by_len = max_k / (3 * PF_BN);
+  if (nseg > by_len) nseg = by_len;
+  if (nseg > cap) nseg = cap;
+  if (nseg > FA_MAX_SEGMENTS) nseg = FA_MAX_SEGMENTS;
+  if (g_pf_segs > 0) nseg = g_pf_segs < cap ? g_pf_segs : cap;
+  if (nseg < 2) return {whole, 1};
+  return {true, nseg};
+}
+
 // unified_attention: padded head sizes 64 and 128 (one configuration each)
 template <typename T, bool FP8>
 static int launch_unified(PrefillParams p, int head_size, int block_size, int max_q, int max_k,
@@ -814,19 +846,14 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       p.skip_decode = 1;
     }
   }
-  // Long query chunks at head size 128 with only the causal mask: the 256-row kernel (prefill_fa.hip; rows =
-  // (token, q head of the group) pairs when the group divides into 256 rows).  "Long" = the longest chunk
-  // fills at least one of its row blocks.
+  // Query chunks with only the causal mask (+ window, softcap): the 256-row kernel (prefill_fa.hip; rows = (token, q head of
+  // the group) pairs when the group divides into 256 rows), where fa_plan takes it
   {
     const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
-    const int fa_rows = head_size > 128 ? 128 : 256;   // rows of a workgroup: four waves at head sizes above 128
-    const bool can = head_size > 64 && head_size <= 256 && p.alibi_slopes == nullptr &&
-                     p.flat_batch > 0 && p.sm_scale > 0.f && g_pf_rows == 0;
-    // ... and the launch has enough 256-row blocks for the chip: below ~128 of them the 64-row kernel's four times as
-    // many workgroups finish sooner (chunk 256 over 4096 cached tokens among 255 decodes: 32 blocks, 82 vs 150 us)
+    const bool can = p.alibi_slopes == nullptr && p.flat_batch > 0 && p.sm_scale > 0.f;
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
-    const int64_t fa_blocks = ptok / (fa_rows / pack) * (pack > 1 ? p.num_kv_heads : p.num_heads);
-    if (can && g_pf_fa != 1 && (g_pf_fa == 2 || (max_q >= fa_rows / pack && fa_blocks >= 128))) {
+    const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments);
+    if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
       f.block_table = p.b_loc; f.cu_seqlens_q = p.b_start_loc; f.seq_lens = p.b_seq_len;
@@ -841,6 +868,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       f.window = p.sliding_window; f.softcap = p.softcap;
       f.prefix = 0; f.k_new = f.v_new = nullptr; f.k_stride_t = f.k_stride_h = f.v_stride_t = f.v_stride_h = 0;
       f.blocks_per_seq = 0;
+      f.num_segments = plan.nseg; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
       f.abl = g_pf_fa_abl;
       f.stagger = g_pf_fa_stagger;
       return launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
@@ -892,18 +920,18 @@ static void launch_bs(const PrefillParams& p, int block_size, int max_input_len,
   }
 }
 template <typename T, bool FP8>
-static void launch_d(const PrefillParams& p, int head_size, int block_size, int max_input_len,
+static void launch_d(const PrefillParams& p, int head_size, int block_size, int max_input_len, int max_k,
                      int num_heads, int batch, hipStream_t st) {
-  // Long chunks at head size 128 with only the causal mask: the 256-row kernel (prefill_fa.hip, PREFIX form)
+  // Chunks with only the causal mask: the 256-row kernel (prefill_fa.hip, PREFIX form) where fa_plan takes it
   {
     const int gqa = p.num_heads / p.num_kv_heads;
     const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
-    const int fa_rows = head_size > 128 ? 128 : 256;
-    const bool can = head_size > 64 && head_size <= 256 && p.alibi_slopes == nullptr && p.sliding_window == 0 && p.sm_scale > 0.f &&
-                     g_pf_rows == 0 && (block_size & (block_size - 1)) == 0;
+    const bool can = p.alibi_slopes == nullptr && p.sliding_window == 0 && p.sm_scale > 0.f &&
+                     (block_size & (block_size - 1)) == 0;
     const int64_t ptok = p.flat_batch > 0 ? (int64_t)p.flat_tokens : (int64_t)max_input_len * batch;
-    const int64_t fa_blocks = ptok / (fa_rows / pack) * (pack > 1 ? p.num_kv_heads : p.num_heads);   // (see launch_unified)
-    if (can && g_pf_fa != 1 && (g_pf_fa == 2 || (max_input_len >= fa_rows / pack && fa_blocks >= 128))) {
+    const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
+                                p.flat_batch > 0 ? p.num_segments : 1);
+    if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
       f.block_table = p.b_loc; f.cu_seqlens_q = p.b_start_loc; f.seq_lens = p.b_seq_len;
@@ -920,8 +948,9 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
       f.window = 0; f.softcap = 0.f;
       f.prefix = 1; f.k_new = p.k; f.v_new = p.v;
       f.k_stride_t = p.k_stride_t; f.k_stride_h = p.k_stride_h; f.v_stride_t = p.v_stride_t; f.v_stride_h = p.v_stride_h;
-      const int tpb = fa_rows / pack;
+      const int tpb = (head_size > 128 ? 128 : 256) / pack;
       f.blocks_per_seq = p.flat_batch > 0 ? 0 : (max_input_len + tpb - 1) / tpb;
+      f.num_segments = plan.nseg; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
       f.abl = 0; f.stagger = g_pf_fa_stagger;
       launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
       return;
@@ -1071,7 +1100,7 @@ __global__ __launch_bounds__(256) void prefix_f32_kernel(PrefillParams p, int ba
   }
 }
 
-extern "C" int vllm_amd_context_attention_fwd(
+static int context_attention(
     void* o, const void* q, const void* k, const void* v, const void* k_cache, const void* v_cache,
     const int* b_loc, const int* b_start_loc, const int* b_seq_len, const float* k_scale,
     const float* v_scale, const float* alibi_slopes, const float* fp8_out_scale, int batch,
@@ -1080,10 +1109,12 @@ extern "C" int vllm_amd_context_attention_fwd(
     int64_t k_stride_h, int64_t v_stride_t, int64_t v_stride_h, int64_t o_stride_t,
     int64_t o_stride_h, int64_t kc_block_stride, int64_t kc_head_stride, int64_t vc_block_stride,
     int64_t vc_head_stride, float sm_scale, int sliding_window, int skip_decode, int num_tokens,
-    int dtype, int kv_cache_dtype, void* stream) {
+    int dtype, int kv_cache_dtype, void* stream, float* segm_out, float* segm_max, float* segm_sum, int num_segments, int max_k) {
   const char* op = "context_attention_fwd";
   VA_REQUIRE(batch >= 0 && max_input_len >= 0, VLLM_AMD_EINVAL, "%s: negative size", op);
   if (batch == 0 || max_input_len == 0 || num_heads == 0) return VLLM_AMD_OK;
+  VA_REQUIRE(num_segments <= 1 || (segm_out && segm_max && segm_sum && num_tokens > 0 && (((uintptr_t)segm_out) & 15) == 0),
+             VLLM_AMD_EINVAL, "%s: num_segments > 1 needs the three segment buffers (16-byte aligned) and num_tokens", op);
   VA_REQUIRE(o && q && k && v && k_cache && v_cache && b_loc && b_start_loc && b_seq_len,
              VLLM_AMD_EINVAL, "%s: null pointer", op);
   VA_REQUIRE(dtype == VLLM_AMD_F16 || dtype == VLLM_AMD_BF16 || dtype == VLLM_AMD_F32,
@@ -1176,21 +1207,68 @@ extern "C" int vllm_amd_context_attention_fwd(
   p.skip_decode = skip_decode;
   p.kc_page_bytes = p.vc_page_bytes = 0;
   p.softcap = 0.f;
-  p.segm_out = p.segm_max = p.segm_sum = nullptr;
-  p.num_segments = p.segm_stride = 1;
+  p.segm_out = segm_out; p.segm_max = segm_max; p.segm_sum = segm_sum;
+  p.num_segments = p.segm_stride = num_segments > 1 ? num_segments : 1;
   p.bs_shift = 0;
   p.flat_batch = num_tokens > 0 ? batch : 0;
   p.flat_tokens = num_tokens;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == VLLM_AMD_BF16) {
-    if (es == 2) launch_d<bf16_t, false>(p, head_size, block_size, max_input_len, num_heads, batch, st);
-    else launch_d<bf16_t, true>(p, head_size, block_size, max_input_len, num_heads, batch, st);
+    if (es == 2) launch_d<bf16_t, false>(p, head_size, block_size, max_input_len, max_k, num_heads, batch, st);
+    else launch_d<bf16_t, true>(p, head_size, block_size, max_input_len, max_k, num_heads, batch, st);
   } else {
-    if (es == 2) launch_d<f16_t, false>(p, head_size, block_size, max_input_len, num_heads, batch, st);
-    else launch_d<f16_t, true>(p, head_size, block_size, max_input_len, num_heads, batch, st);
+    if (es == 2) launch_d<f16_t, false>(p, head_size, block_size, max_input_len, max_k, num_heads, batch, st);
+    else launch_d<f16_t, true>(p, head_size, block_size, max_input_len, max_k, num_heads, batch, st);
   }
   VA_LAUNCH_CHECK(op);
   return VLLM_AMD_OK;
+}
+
+extern "C" int vllm_amd_context_attention_fwd(
+    void* o, const void* q, const void* k, const void* v, const void* k_cache, const void* v_cache,
+    const int* b_loc, const int* b_start_loc, const int* b_seq_len, const float* k_scale,
+    const float* v_scale, const float* alibi_slopes, const float* fp8_out_scale, int batch,
+    int num_heads, int num_kv_heads, int head_size, int block_size, int max_input_len,
+    int64_t b_loc_stride, int64_t q_stride_t, int64_t q_stride_h, int64_t k_stride_t,
+    int64_t k_stride_h, int64_t v_stride_t, int64_t v_stride_h, int64_t o_stride_t,
+    int64_t o_stride_h, int64_t kc_block_stride, int64_t kc_head_stride, int64_t vc_block_stride,
+    int64_t vc_head_stride, float sm_scale, int sliding_window, int skip_decode, int num_tokens,
+    int dtype, int kv_cache_dtype, void* stream) {
+  return context_attention(o, q, k, v, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, k_scale, v_scale, alibi_slopes, fp8_out_scale, batch, num_heads, num_kv_heads, head_size, block_size, max_input_len, b_loc_stride, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h, kc_block_stride, kc_head_stride, vc_block_stride, vc_head_stride, sm_scale, sliding_window, skip_decode, num_tokens, dtype, kv_cache_dtype, stream, nullptr, nullptr, nullptr, 1, 0);
+}
+
+extern "C" int vllm_amd_context_attention_fwd_split(
+    void* o, const void* q, const void* k, const void* v, const void* k_cache, const void* v_cache,
+    const int* b_loc, const int* b_start_loc, const int* b_seq_len, const float* k_scale,
+    const float* v_scale, const float* alibi_slopes, const float* fp8_out_scale, int batch,
+    int num_heads, int num_kv_heads, int head_size, int block_size, int max_input_len,
+    int64_t b_loc_stride, int64_t q_stride_t, int64_t q_stride_h, int64_t k_stride_t,
+    int64_t k_stride_h, int64_t v_stride_t, int64_t v_stride_h, int64_t o_stride_t,
+    int64_t o_stride_h, int64_t kc_block_stride, int64_t kc_head_stride, int64_t vc_block_stride,
+    int64_t vc_head_stride, float sm_scale, int sliding_window, int skip_decode, int num_tokens,
+    float* segm_output,
+    float* segm_max, float* segm_expsum, int num_segments, int max_seq_len, int dtype, int kv_cache_dtype, void* stream) {
+  return context_attention(o, q, k, v, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, k_scale, v_scale, alibi_slopes, fp8_out_scale, batch, num_heads, num_kv_heads, head_size, block_size, max_input_len, b_loc_stride, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h, kc_block_stride, kc_head_stride, vc_block_stride, vc_head_stride, sm_scale, sliding_window, skip_decode, num_tokens, dtype, kv_cache_dtype, stream, segm_output, segm_max, segm_expsum, num_segments, max_seq_len);
+}
+
+// Key segments that a launch of these sizes can use (1 = none; the caller then brings no scratch)
+extern "C" int vllm_amd_context_attention_fwd_segments(int batch, int num_heads, int num_kv_heads, int head_size, int max_input_len,
+                                                       int max_seq_len, int num_tokens, int has_alibi, int sliding_window,
+                                                       int skip_decode) {
+  if (batch <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || num_tokens <= 0 || has_alibi || sliding_window > 0) return 1;
+  return fa_plan(head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch, FA_MAX_SEGMENTS).nseg;
+}
+
+extern "C" int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, int num_kv_heads, int head_size, int max_seqlen_q,
+                                                   int max_seqlen_k, int num_tokens, int has_alibi) {
+  if (num_seqs <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || num_tokens <= 0) return 1;
+  // decode batches of less than two rounds of workgroups: up to 16 segments (the reference's NUM_SEGMENTS,
+  // triton_unified_attention.py:659-683)
+  if (max_seqlen_q == 1) return num_seqs * num_kv_heads * ((num_heads / num_kv_heads + 15) / 16) < 1024 ? 16 : 1;
+  if (has_alibi) return 1;
+  const bool mixed = num_seqs >= 16 && (int64_t)num_tokens < (int64_t)num_seqs * max_seqlen_q;   // (launch_unified)
+  return fa_plan(head_size, num_heads, num_kv_heads, max_seqlen_q, max_seqlen_k, mixed ? num_tokens - num_seqs : num_tokens,
+                 mixed ? 1 : num_seqs, FA_MAX_SEGMENTS).nseg;
 }
 
 // unified_attention (vllm/attention/ops/triton_unified_attention.py:588-700): q over the new

@@ -1,5 +1,5 @@
-// unified_attention, long query chunks at head size 128: the 256-row tile kernel of prefill_fa.hip
-// (launched from prefill_attention.hip's launch_unified when its conditions hold).
+// unified_attention / context_attention_fwd, query chunks of more than one token: the 256-row tile kernel of prefill_fa.hip
+// (launched from prefill_attention.hip when fa_plan says so).
 #pragma once
 #include "common.cuh"
 
@@ -12,7 +12,7 @@ struct FaParams {
   const float* k_scale; const float* v_scale;             // fp8 cache only
   const float* out_scale;                                  // != null: e4m3 output
   int num_heads, num_kv_heads, num_seqs, num_tokens;
-  int head_size;       // 72 .. 256 (padded to 128, above 128 to 256, inside the kernel)
+  int head_size;       // up to 256 (padded to 128, above 128 to 256, inside the kernel)
   int bs_shift;        // log2(block size)
   int skip_decode;     // sequences of query length 1 were taken by the decode kernel
   int pack;            // q heads per tile-row group: the GQA group (rows = (token, head) pairs) or 1
@@ -28,11 +28,17 @@ struct FaParams {
   int64_t k_stride_t, k_stride_h, v_stride_t, v_stride_h;   // elements
   int blocks_per_seq;  // > 0: num_tokens unknown, grid.x = blocks_per_seq * num_seqs (ceil(max query length / tokens per block))
   int stagger;         // 1 = waves 4-7 stage at the top of the interval (tuning "pf_fa_stagger", default 1)
+  // Split over the keys: num_segments workgroups per row block, each over its share of the block's tiles; they leave
+  // unnormalised fp32 partials [token][q head][segment] that fa_reduce_kernel merges.  1 = no split (buffers unused).
+  int num_segments;
+  float* segm_out; float* segm_max; float* segm_sum;
   int abl;             // (unused; the kernel's ablations are compile-time: -DVA_FA_ABL=bits, garbage results: 1 no exp2,
                        // 2 no staging after the first tiles, 4 no S^T MFMAs, 8 no PV MFMAs, 16 no barrier)
 };
 
 // dtype: VLLM_AMD_F16 / VLLM_AMD_BF16 (queries, output, and the cache unless fp8)
 int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st);
+// largest num_segments
+constexpr int FA_MAX_SEGMENTS = 32;
 
 }  // namespace va

@@ -152,8 +152,11 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     const int q8 = nwg / 8, r8 = nwg % 8, xcd = wg % 8, idx = wg / 8;
     wg = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + idx;
   }
-  const int g = gridDim.x - 1 - wg % gridDim.x;
-  const int y = wg / gridDim.x;
+  // (split launches: the row blocks of one key segment are adjacent, they read the same K / V)
+  const int nseg = p.num_segments, gx = nseg > 1 ? gridDim.x / nseg : gridDim.x;
+  const int y = wg / gridDim.x, gs = wg % gridDim.x;
+  const int seg = nseg > 1 ? gs / gx : 0;
+  const int g = gx - 1 - (gs - seg * gx);
   const int pack = p.pack, tpb = BM / pack;   // tokens per workgroup
   // grid.x enumerates the row blocks of ALL sequences (num_tokens / tpb + num_seqs is an upper bound); the
   // sequence is the last one whose first block cu[i] / tpb + i is <= g (find_seq_idx, :33-48)
@@ -536,12 +539,16 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // and the loads of tile t + 2 are issued.  One barrier per tile.
   // (sliding window: the tiles left of the window of the workgroup's first row are not even staged)
   const int t_start = window > 0 ? max(ctx + tok_base - window + 1, 0) / BN : 0;
-  Blk blk = load_blk(t_start);
-  issue_loads(t_start, blk);
-  blk = load_blk(t_start + 1);
-  write_tile(t_start);
-  if (t_start + 1 < ntiles) issue_loads(t_start + 1, blk);
-  blk = load_blk(t_start + 2);
+  // (split: this segment's share [t0, t1) of the block's tiles, possibly none)
+  const int per = nseg > 1 ? (ntiles - t_start + nseg - 1) / nseg : ntiles - t_start;
+  const int t0 = t_start + seg * per, t1 = min(t0 + per, ntiles);
+  if (t0 < t1) {
+  Blk blk = load_blk(t0);
+  issue_loads(t0, blk);
+  blk = load_blk(t0 + 1);
+  write_tile(t0);
+  if (t0 + 1 < t1) issue_loads(t0 + 1, blk);
+  blk = load_blk(t0 + 2);
   __syncthreads();
 #ifdef VA_PROBES
   last__ = __builtin_readcyclecounter();
@@ -559,14 +566,15 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   if ((p.stagger & 4) && wave < NW / 2) __builtin_amdgcn_s_setprio(1);
   auto stage = [&](int t) __attribute__((always_inline)) {
     if (!(abl & 2)) {
-      if (t + 1 < ntiles) write_tile(t + 1);
-      if (t + 2 < ntiles) issue_loads(t + 2, blk);
+      if (t + 1 < t1) write_tile(t + 1);
+      if (t + 2 < t1) issue_loads(t + 2, blk);
       blk = load_blk(t + 3);
     }
   };
   auto tile_loop = [&](int t_begin, int t_end, auto mode_c, auto vt_c) __attribute__((always_inline)) {
     constexpr int MODE = decltype(mode_c)::value;
-    for (int t = t_begin; t < t_end; ++t) {
+    t_end = min(t_end, t1);
+    for (int t = max(t_begin, t0); t < t_end; ++t) {
       if (stage_first) stage(t);
       FA_T(1);
       if constexpr (MODE < 2) {
@@ -613,6 +621,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     tile_loop(b2, e2, MASKED_, std::false_type{});
     tile_loop(e2, ntiles, SKIP, std::false_type{});
   }
+  }   // t0 < t1
 
 #ifdef VA_PROBES
   if (lane == 0 && blockIdx.y == 0 && blockIdx.x < 2048) {
@@ -623,6 +632,23 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // ---- O^T / l -> out ------------------------------------------------------------------------------------------
   if (!rok) return;
   const float l = xsum(l_run);
+  if (nseg > 1) {   // this segment's partial: O unnormalised, running maximum (log2 domain; -inf: nothing visible), sum
+    const int64_t row = ((int64_t)(tok0 + rtok) * p.num_heads + rhead) * nseg + seg;
+    if (hi == 0) {
+      p.segm_max[row] = m_run;
+      p.segm_sum[row] = l;
+    }
+    if (t0 < t1) {
+      float* so = p.segm_out + row * dr + 4 * hi;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq)
+          if (32 * db + 8 * rq + 4 * hi < dr)
+            *reinterpret_cast<float4*>(so + 32 * db + 8 * rq) = make_float4(o[db][4 * rq], o[db][4 * rq + 1], o[db][4 * rq + 2], o[db][4 * rq + 3]);
+    }
+    return;
+  }
   const float inv = l > 0.f ? 1.0f / l : 0.f;
   if (p.out_scale == nullptr) {
     T* op = (T*)p.o + (int64_t)(tok0 + rtok) * p.o_stride_t + (int64_t)rhead * p.o_stride_h + 4 * hi;
@@ -650,6 +676,70 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   }
 }
 
+// Merge of a split launch: one wave per (token, q head).  Lane s holds segment s's maximum and sum; a half wave (D <= 128;
+// the whole wave above) reads one partial row per step, four rows in flight.  Segments that saw nothing were not written
+// and are not read.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
+  constexpr int LPR = D / 4, PAR = 64 / LPR;      // lanes per row, rows per step
+  const int lane = threadIdx.x & 63;
+  const int pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tok = pair / p.num_heads, head = pair % p.num_heads;
+  if (tok >= p.num_tokens || tok >= p.cu_seqlens_q[p.num_seqs]) return;
+  if (p.skip_decode) {
+    int lo = 0, hi = p.num_seqs;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (p.cu_seqlens_q[mid] <= tok) lo = mid; else hi = mid;
+    }
+    if (p.cu_seqlens_q[lo + 1] - p.cu_seqlens_q[lo] == 1) return;   // the decode kernel's token
+  }
+  const int nseg = p.num_segments, dr = p.head_size;
+  const int64_t row = ((int64_t)tok * p.num_heads + head) * nseg;
+  const float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
+  const float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
+  const float mx = wave_max(ms);
+  const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);
+  const float l = wave_sum(ls * w);
+  const int d = 4 * (lane % LPR), sub = lane / LPR;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  const float* base = p.segm_out + row * dr + (d < dr ? d : 0);
+  for (int s0 = 0; s0 < nseg; s0 += 4 * PAR) {
+    float4 part[4];
+    float ws[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + u * PAR + sub;
+      ws[u] = __shfl(w, s < nseg ? s : 0, 64);
+      if (s >= nseg) ws[u] = 0.f;
+      part[u] = ws[u] > 0.f ? *reinterpret_cast<const float4*>(base + (int64_t)s * dr) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      acc.x = fmaf(part[u].x, ws[u], acc.x);
+      acc.y = fmaf(part[u].y, ws[u], acc.y);
+      acc.z = fmaf(part[u].z, ws[u], acc.z);
+      acc.w = fmaf(part[u].w, ws[u], acc.w);
+    }
+  }
+  if constexpr (PAR == 2) {
+    acc.x += __shfl_xor(acc.x, 32, 64);
+    acc.y += __shfl_xor(acc.y, 32, 64);
+    acc.z += __shfl_xor(acc.z, 32, 64);
+    acc.w += __shfl_xor(acc.w, 32, 64);
+  }
+  if (sub != 0 || d >= dr) return;
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  const int64_t oi = (int64_t)tok * p.o_stride_t + (int64_t)head * p.o_stride_h + d;
+  if (p.out_scale == nullptr) {
+    *reinterpret_cast<u32x2*>((T*)p.o + oi) = (u32x2){Mma<T>::pack2(acc.x * inv, acc.y * inv), Mma<T>::pack2(acc.z * inv, acc.w * inv)};
+  } else {
+    const float oinv = inv / *p.out_scale;
+    auto cl = [](float y) { return fmaxf(-448.0f, fminf(y, 448.0f)); };
+    *reinterpret_cast<uint32_t*>((uint8_t*)p.o + oi) = f32x4_to_fp8x4(cl(acc.x * oinv), cl(acc.y * oinv), cl(acc.z * oinv), cl(acc.w * oinv));
+  }
+}
+
 }  // namespace fa
 
 int g_pf_fa_stagger = 1;   // tuning "pf_fa_stagger": 0 = all eight waves stage at the bottom of the interval
@@ -657,7 +747,7 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st) {
   const bool wide = p.head_size > 128;                 // 128-row workgroups of four waves
   const int tpb = (wide ? 128 : 256) / p.pack;
   const unsigned gx = p.blocks_per_seq > 0 ? (unsigned)(p.blocks_per_seq * p.num_seqs) : (unsigned)(p.num_tokens / tpb + p.num_seqs);
-  const dim3 grid(gx, (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads));
+  const dim3 grid(gx * (unsigned)p.num_segments, (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads));
 #define FA_LAUNCH___(T_, F_, P_, D_, NW_, S_) \
   hipLaunchKernelGGL((fa::fa_fwd_kernel<T_, F_, P_, D_, NW_, S_>), grid, dim3(64 * NW_), 0, st, p)
 #define FA_LAUNCH__(T_, F_, P_, D_, NW_)                                                           \
@@ -675,6 +765,16 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st) {
   } while (0)
   if (dtype == VLLM_AMD_BF16) { if (fp8) FA_LAUNCH(bf16_t, true); else FA_LAUNCH(bf16_t, false); }
   else { if (fp8) FA_LAUNCH(f16_t, true); else FA_LAUNCH(f16_t, false); }
+  if (p.num_segments > 1) {
+    const dim3 rgrid((unsigned)(((int64_t)p.num_tokens * p.num_heads + 3) / 4));
+#define FA_REDUCE(T_)                                                                          \
+  do {                                                                                         \
+    if (wide) hipLaunchKernelGGL((fa::fa_reduce_kernel<T_, 256>), rgrid, dim3(256), 0, st, p); \
+    else hipLaunchKernelGGL((fa::fa_reduce_kernel<T_, 128>), rgrid, dim3(256), 0, st, p);      \
+  } while (0)
+    if (dtype == VLLM_AMD_BF16) FA_REDUCE(bf16_t); else FA_REDUCE(f16_t);
+#undef FA_REDUCE
+  }
 #undef FA_LAUNCH
 #undef FA_LAUNCH_
 #undef FA_LAUNCH__
