@@ -167,3 +167,27 @@ def test_opcheck_fused_quant():
     opcheck(torch.ops._C.rms_norm_dynamic_per_token_quant, (q, x, wgt, st, 1e-6, None, res))
     gate = torch.randn((T, 2 * Hd), device="cuda", dtype=torch.bfloat16)
     opcheck(torch.ops._C.silu_and_mul_quant, (q, gate, sc))
+
+
+def test_opcheck_call_operators():
+    """The operators that stand for a whole Python call (torch.ops._vllm_amd_C)."""
+    g = torch.Generator().manual_seed(0)
+    r = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).cuda()
+    x, w = r(5, 256), r(64, 256)
+    wq = torch.empty((64, 256), dtype=torch.float8_e4m3fn, device="cuda")
+    ws = torch.empty((64, 1), device="cuda")
+    torch.ops._C.dynamic_per_token_scaled_fp8_quant(wq, w, ws, None)
+    out = torch.empty((5, 64), dtype=torch.bfloat16, device="cuda")
+    for per_token in (True, False):
+        opcheck(torch.ops._vllm_amd_C.fp8_linear, (out, x, wq.t(), ws, None, r(64), per_token))
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    # 70 new tokens over 1100 (split over the keys: scratch inside) and a one-token sequence
+    q, o = r(71, 4, 128), torch.empty((71, 4, 128), dtype=torch.bfloat16, device="cuda")
+    table = torch.arange(160, dtype=torch.int32, device="cuda").view(2, 80)
+    kc, vc = r(160, 16, 2, 128), r(160, 16, 2, 128)
+    opcheck(torch.ops._vllm_amd_C.unified_attention, (q, kc, vc, o, i32(0, 70, 71), 70, i32(1170, 40), 1170, 0.09, 0, table,
+                                                      0.0, None, None, None, None))
+    kx, vx, k = r(160, 2, 16, 16, 8), r(160, 2, 128, 16), r(71, 2, 128)
+    one = torch.ones(1, device="cuda")
+    opcheck(torch.ops._vllm_amd_C.context_attention_fwd, (q, k, k, o, kx, vx, table, i32(0, 70, 71), i32(1170, 40), 1280, 70,
+                                                          one, one, None, 0, 0.09, False, None))

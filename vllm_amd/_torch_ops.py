@@ -7,7 +7,8 @@ The operators of
 are implemented and registered IN C++ by ``csrc/torch_shim.cpp`` (libvllm_amd_torch.so), with the
 reference's exact schema strings, for the CUDA(=HIP) dispatch key: each one unpacks tensors into
 raw device pointers / shapes / strides and calls libvllm_amd.so on torch's current stream -- no
-allocation, no synchronisation, HIP-graph capturable.  This module only loads that library,
+allocation, no synchronisation, HIP-graph capturable (torch.ops._vllm_amd_C.*, which are no
+operators of the reference, allocate their scratch).  This module only loads that library,
 calls its registration entry point, and keeps Python names for the same operators (they forward
 to ``torch.ops``) plus the small helpers the ctypes callers of the non-operator entry points
 (context_attention_fwd, unified_attention) use.  There is no Python implementation to fall back
@@ -111,3 +112,7 @@ silu_and_mul_quant = torch.ops._C.silu_and_mul_quant
 #: device-side BlockTable.compute_slot_mapping (vllm/v1/worker/block_table.py:84-99); not a
 #: reference op -- the reference does this with numpy on the host
 compute_slot_mapping = torch.ops._vllm_amd_C.compute_slot_mapping
+#: dynamic activation quantisation + cutlass_scaled_mm; the attention calls behind attention/ops
+fp8_linear = torch.ops._vllm_amd_C.fp8_linear.default
+unified_attention = torch.ops._vllm_amd_C.unified_attention.default
+context_attention_fwd = torch.ops._vllm_amd_C.context_attention_fwd.default

@@ -8,11 +8,9 @@ from typing import Optional
 
 import torch
 
-from ... import _lib
-from ..._lib import check, lib
-from ..._torch_ops import _dev, _ptr, _stream
+from ... import _torch_ops
 
-_DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
+_DT = (torch.float16, torch.bfloat16, torch.float32)
 _FP8 = (torch.uint8, torch.float8_e4m3fn)
 
 
@@ -20,7 +18,6 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.int32 else t.to(torch.int32)
 
 
-@torch.inference_mode()
 def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_loc, b_start_loc,
                           b_seq_len, max_seq_len, max_input_len, k_scale: torch.Tensor,
                           v_scale: torch.Tensor, alibi_slopes=None, sliding_window=None,
@@ -30,11 +27,9 @@ def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_l
         assert k_cache.dtype in _FP8 and v_cache.dtype in _FP8
         if kv_cache_dtype not in ("fp8", "fp8_e4m3"):
             raise ValueError("Unsupported FP8 dtype:", kv_cache_dtype)
-        kvd = _lib.KV_FP8_E4M3
     else:
         if k_cache.dtype == torch.uint8 or v_cache.dtype == torch.uint8:
             raise ValueError("kv_cache_dtype='auto' unsupported for FP8 KV Cache prefill kernel")
-        kvd = _lib.KV_AUTO
         assert k_cache.dtype == q.dtype and v_cache.dtype == q.dtype
     if q.dtype not in _DT:
         raise RuntimeError(f"context_attention_fwd: unsupported query dtype {q.dtype}")
@@ -42,8 +37,7 @@ def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_l
     assert Lq == Lk and Lk == Lv
     if sm_scale is None:
         sm_scale = 1.0 / (Lq ** 0.5)
-    batch, head = b_seq_len.shape[0], q.shape[1]
-    assert batch + 1 == len(b_start_loc)
+    assert b_seq_len.shape[0] + 1 == b_start_loc.shape[0]
     if sliding_window is None or sliding_window <= 0:
         sliding_window = 0
     for t in (q, k, v, o):
@@ -66,27 +60,8 @@ def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_l
     assert k_cache.stride(4) == 1 and k_cache.stride(3) == k_cache.shape[4] \
         and k_cache.stride(2) == k_cache.shape[3] * k_cache.shape[4]
     assert v_cache.stride(3) == 1 and v_cache.stride(2) == block_size
-    # scratch for launches that split the keys (few row blocks over long prefixes)
-    num_tokens = q.shape[0]
-    max_k = int(max_seq_len) if max_seq_len else b_loc.shape[1] * block_size
-    nseg = lib.vllm_amd_context_attention_fwd_segments(batch, head, k.shape[1], Lq, int(max_input_len), max_k, num_tokens,
-                                                       int(alibi_slopes is not None), int(sliding_window), int(bool(skip_decode)))
-    segm_out = segm_max = segm_sum = None
-    if nseg > 1 and q.dtype != torch.float32:
-        rows = num_tokens * head * nseg
-        segm = torch.empty(rows * (Lq + 2), dtype=torch.float32, device=q.device)
-        segm_out = segm.data_ptr()
-        segm_max = segm_out + 4 * rows * Lq
-        segm_sum = segm_max + 4 * rows
-    else:
-        nseg = 1
-    with _dev(q):
-        check(lib.vllm_amd_context_attention_fwd_split(
-            _ptr(o), _ptr(q), _ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), _ptr(b_loc),
-            _ptr(b_start_loc), _ptr(b_seq_len), _ptr(k_scale), _ptr(v_scale),
-            _ptr(alibi_slopes), _ptr(fp8_out_scale), batch, head, k.shape[1], Lq, block_size,
-            int(max_input_len), b_loc.stride(0), q.stride(0), q.stride(1), k.stride(0),
-            k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), k_cache.stride(0),
-            k_cache.stride(1), v_cache.stride(0), v_cache.stride(1), float(sm_scale),
-            int(sliding_window), int(bool(skip_decode)), num_tokens,
-            segm_out, segm_max, segm_sum, nseg, max_k, _DT[q.dtype], kvd, _stream(q)))
+    # (scratch for launches that split the keys -- few row blocks over long prefixes -- is allocated in there)
+    max_k = max_seq_len if max_seq_len else b_loc.shape[1] * block_size
+    _torch_ops.context_attention_fwd(q, k, v, o, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, int(max_k), int(max_input_len),
+                                     k_scale, v_scale, alibi_slopes, int(sliding_window), float(sm_scale), bool(skip_decode),
+                                     fp8_out_scale)

@@ -3,8 +3,9 @@
 // schema strings (csrc/torch_bindings.cpp:45-69, 117-120, 188-211, 422-427, 575-593, 676-708;
 // csrc/rocm/torch_bindings.cpp:34-56).  Every implementation unpacks data_ptr / sizes /
 // strides, takes torch's current HIP stream and calls libvllm_amd.so; a non-zero status
-// becomes the c10::Error (RuntimeError) the reference's TORCH_CHECK raises.  No tensor is
-// allocated inside an op, except the one-time per-device workspace (ensure_workspace).
+// becomes the c10::Error (RuntimeError) the reference's TORCH_CHECK raises.  The reference's operators
+// allocate nothing here, except the one-time per-device workspace (ensure_workspace); those of
+// _vllm_amd_C that stand for a whole Python call allocate its scratch.
 //
 // Registration is a function (vllm_amd_torch_register), not a static TORCH_LIBRARY block:
 // when the real vLLM extension was imported first its schemas already exist, and a static
@@ -421,6 +422,96 @@ void compute_slot_mapping(Tensor& slot_mapping, const Tensor& block_table, const
                                       n, (int)block_table.size(1), (int)block_size, stream_of(block_table)));
 }
 
+// ---- calls that are one operator here and several steps of Python in the reference ----------
+// Scratch that such a call needs is allocated inside it, on the current stream, and released when it returns: later
+// allocations on that stream are ordered behind its kernels.  The result is always the caller's `out`.
+
+// Dynamic activation quantisation (per token, or per tensor) + scaled_mm: vllm/model_executor/layers/quantization/utils/
+// w8a8_utils.py:297-377.  As two operators with three allocations from Python a call cost 18 us of host time, whatever
+// the GEMM took (17 tokens, 4096 -> 6144: 10 us on the GPU).
+void fp8_linear(Tensor& out, const Tensor& input, const Tensor& weight, const Tensor& weight_scale, const OptTensor& scale_ub,
+                const OptTensor& bias, bool per_token) {
+  need_devs(out, input, weight, weight_scale, scale_ub, bias);
+  TORCH_CHECK(input.dim() == 2, "input.ndim == 2");
+  const Tensor x = input.contiguous();
+  const int64_t m = x.size(0), k = x.size(1);
+  const Tensor q = at::empty({m, k}, x.options().dtype(at::kFloat8_e4m3fn));
+  Tensor scale = at::empty({per_token ? m : 1}, x.options().dtype(at::kFloat));
+  {
+    DevGuard g(x.device());
+    if (per_token) {
+      check(vllm_amd_dynamic_per_token_scaled_fp8_quant(q.data_ptr(), x.data_ptr(), (float*)scale.data_ptr(), fptr(scale_ub),
+                                                        m, (int)k, dt(x), stream_of(x)));
+    } else {
+      scale.zero_();   // the kernel's atomic maximum starts there
+      check(vllm_amd_dynamic_scaled_fp8_quant(q.data_ptr(), x.data_ptr(), (float*)scale.data_ptr(), m, (int)k, dt(x),
+                                              stream_of(x)));
+    }
+  }
+  cutlass_scaled_mm(out, q, weight, scale, weight_scale, bias);
+}
+
+// One buffer for the partial outputs, maxima and sums of `nseg` key segments.
+struct Segments {
+  Tensor buf;
+  float *out = nullptr, *max = nullptr, *sum = nullptr;
+  int n = 1;
+  Segments(int nseg, const Tensor& q) {
+    if (nseg <= 1) return;
+    const int64_t rows = q.size(0) * q.size(1) * nseg, d = q.size(2);
+    buf = at::empty({rows * (d + 2)}, q.options().dtype(at::kFloat));
+    out = (float*)buf.data_ptr();
+    max = out + rows * d;
+    sum = max + rows;
+    n = nseg;
+  }
+};
+
+inline int kv_of_cache(const Tensor& k) { return is_fp8(k) ? VLLM_AMD_KV_FP8_E4M3 : VLLM_AMD_KV_AUTO; }
+
+// vllm/attention/ops/triton_unified_attention.py:588-700 (the arguments are checked in the Python mirror)
+void unified_attention(const Tensor& q, const Tensor& k, const Tensor& v, Tensor& out, const Tensor& cu_seqlens_q,
+                       int64_t max_seqlen_q, const Tensor& seqused_k, int64_t max_seqlen_k, double softmax_scale,
+                       int64_t sliding_window, const Tensor& block_table, double softcap, const OptTensor& k_descale,
+                       const OptTensor& v_descale, const OptTensor& alibi_slopes, const OptTensor& output_scale) {
+  need_devs(q, k, v, out, cu_seqlens_q, seqused_k, block_table, k_descale, v_descale, alibi_slopes, output_scale);
+  const int num_seqs = (int)seqused_k.size(0), num_tokens = (int)q.size(0), heads = (int)q.size(1), kv_heads = (int)k.size(2);
+  const int d = (int)q.size(2);
+  const Segments sg(vllm_amd_unified_attention_segments(num_seqs, heads, kv_heads, d, (int)max_seqlen_q, (int)max_seqlen_k,
+                                                        num_tokens, alibi_slopes.has_value()), q);
+  DevGuard g(q.device());
+  check(vllm_amd_unified_attention(
+      out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), (const int*)cu_seqlens_q.data_ptr(),
+      (const int*)seqused_k.data_ptr(), (const int*)block_table.data_ptr(), fptr(k_descale), fptr(v_descale), fptr(alibi_slopes),
+      fptr(output_scale), num_seqs, heads, kv_heads, d, (int)v.size(1), (int)max_seqlen_q, block_table.stride(0), q.stride(0),
+      q.stride(1), out.stride(0), out.stride(1), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
+      (float)softmax_scale, (int)sliding_window, (float)softcap, num_tokens, (int)max_seqlen_k, sg.out, sg.max, sg.sum, sg.n,
+      dt(q), kv_of_cache(k), stream_of(q)));
+}
+
+// vllm/attention/ops/prefix_prefill.py:726-913 (checked in the Python mirror); max_k: longest sequence or a bound of it
+void context_attention_fwd(const Tensor& q, const Tensor& k, const Tensor& v, Tensor& o, const Tensor& k_cache,
+                           const Tensor& v_cache, const Tensor& b_loc, const Tensor& b_start_loc, const Tensor& b_seq_len,
+                           int64_t max_k, int64_t max_input_len, const OptTensor& k_scale, const OptTensor& v_scale,
+                           const OptTensor& alibi_slopes, int64_t sliding_window, double sm_scale, bool skip_decode,
+                           const OptTensor& fp8_out_scale) {
+  need_devs(q, k, v, o, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, k_scale, v_scale, alibi_slopes, fp8_out_scale);
+  const int batch = (int)b_seq_len.size(0), num_tokens = (int)q.size(0), heads = (int)q.size(1), kv_heads = (int)k.size(1);
+  const int d = (int)q.size(2);
+  const Segments sg(q.scalar_type() == at::kFloat
+                        ? 1
+                        : vllm_amd_context_attention_fwd_segments(batch, heads, kv_heads, d, (int)max_input_len, (int)max_k, num_tokens,
+                                                                  alibi_slopes.has_value(), (int)sliding_window, skip_decode), q);
+  DevGuard g(q.device());
+  check(vllm_amd_context_attention_fwd_split(
+      o.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), (const int*)b_loc.data_ptr(),
+      (const int*)b_start_loc.data_ptr(), (const int*)b_seq_len.data_ptr(), fptr(k_scale), fptr(v_scale), fptr(alibi_slopes),
+      fptr(fp8_out_scale), batch, heads, kv_heads, d, (int)v_cache.size(3), (int)max_input_len, b_loc.stride(0), q.stride(0),
+      q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), k_cache.stride(0),
+      k_cache.stride(1), v_cache.stride(0), v_cache.stride(1), (float)sm_scale, (int)sliding_window, skip_decode, num_tokens,
+      sg.out, sg.max, sg.sum, sg.n, (int)max_k, dt(q), kv_of_cache(k_cache), stream_of(q)));
+}
+
 // ---- registration ------------------------------------------------------------------------
 #define PA_TAIL                                                                                               \
   " int num_kv_heads, float scale, Tensor block_tables, Tensor seq_lens, int block_size,"                   \
@@ -436,6 +527,7 @@ struct Registrar {
   torch::Library* frag;
   torch::Library* impl;
   torch::Library* impl_any;
+  torch::Library* impl_grad;
   template <class F>
   void op(const char* name, const char* schema, F* fn, bool any_device = false) {
     try {
@@ -444,6 +536,11 @@ struct Registrar {
       // already defined (the real vLLM extension was imported first): override the kernel only
     }
     (any_device ? impl_any : impl)->impl(name, fn);
+  }
+  template <class F>
+  void op_no_grad(const char* name, const char* schema, F* fn) {
+    op(name, schema, fn);
+    impl_grad->impl(name, torch::CppFunction::makeFallthrough());
   }
 };
 
@@ -454,7 +551,8 @@ Registrar open_ns(const char* ns) {
   };
   return Registrar{ns, mk(torch::Library::FRAGMENT, std::nullopt),
                    mk(torch::Library::IMPL, c10::DispatchKey::CUDA),
-                   mk(torch::Library::IMPL, c10::DispatchKey::CompositeExplicitAutograd)};
+                   mk(torch::Library::IMPL, c10::DispatchKey::CompositeExplicitAutograd),
+                   mk(torch::Library::IMPL, c10::DispatchKey::AutogradCUDA)};
 }
 
 void register_all() {
@@ -530,6 +628,21 @@ void register_all() {
        "compute_slot_mapping(Tensor! slot_mapping, Tensor block_table, Tensor req_indices,"
        " Tensor positions, int block_size) -> ()",
        &compute_slot_mapping);
+  x.op("fp8_linear",
+       "fp8_linear(Tensor! out, Tensor input, Tensor weight, Tensor weight_scale, Tensor? scale_ub, Tensor? bias,"
+       " bool per_token) -> ()",
+       &fp8_linear);
+  // (no gradient passes through these two, as under the inference mode the reference runs them in)
+  x.op_no_grad("unified_attention",
+       "unified_attention(Tensor q, Tensor k, Tensor v, Tensor! out, Tensor cu_seqlens_q, int max_seqlen_q,"
+       " Tensor seqused_k, int max_seqlen_k, float softmax_scale, int sliding_window, Tensor block_table,"
+       " float softcap, Tensor? k_descale, Tensor? v_descale, Tensor? alibi_slopes, Tensor? output_scale) -> ()",
+       &unified_attention);
+  x.op_no_grad("context_attention_fwd",
+       "context_attention_fwd(Tensor q, Tensor k, Tensor v, Tensor! o, Tensor k_cache, Tensor v_cache, Tensor b_loc,"
+       " Tensor b_start_loc, Tensor b_seq_len, int max_k, int max_input_len, Tensor? k_scale, Tensor? v_scale,"
+       " Tensor? alibi_slopes, int sliding_window, float sm_scale, bool skip_decode, Tensor? fp8_out_scale) -> ()",
+       &context_attention_fwd);
 }
 
 std::string g_reg_error;

@@ -60,6 +60,12 @@ class Fp8LinearOp:
         output_shape = [*input.shape[:-1], weight.shape[1]]
         if out_dtype is None:
             out_dtype = input.dtype
+        if (input_scale is None and input.dtype != ops.FP8_DTYPE and not self.act_quant_static
+                and self.quant_fp8.num_token_padding is None):
+            # dynamic quantisation (QuantFP8) and the GEMM as one operator
+            assert input_scale_ub is None or (self.quant_fp8.per_token and input_scale_ub.numel() == 1)
+            return ops.fp8_linear(input_2d, weight, weight_scale, out_dtype, input_scale_ub, bias,
+                                  self.quant_fp8.per_token).view(*output_shape)
         if input.dtype != ops.FP8_DTYPE:
             qinput, x_scale = self.quant_fp8(input_2d, input_scale, input_scale_ub)
         else:
