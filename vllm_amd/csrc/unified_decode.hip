@@ -23,6 +23,10 @@
 //      page) and transposes in registers: v_perm_b32 interleaves the bytes of a token pair, the
 //      fp8 -> 16-bit widening (exact) then yields the packed (token, token + 1) operand dwords.
 //      MFMA j produces rows d = DT i + j (i = A row): a permutation of d undone in the merge.
+//   The loop waits for exactly the loads it consumes (K in front of the LDS image, V in front of P V): every load is
+//   unconditional, a wave's last step is peeled, block-table entries are scalar loads.  With loads behind branches and
+//   block ids through vector loads a step drained everything in flight: whole engine steps (us, fp8, 32q / 8kv) 61 ragged
+//   sequences up to 3000 tokens 49.3 -> 39.6, 64 x 4096 90.6 -> 85.5, 16 ragged up to 16384 77.8 -> 65.2; head 64 37.5 -> 24.5.
 //   Addresses are a wave-uniform 64-bit base per (tile, row) plus one 32-bit lane offset per
 //   operand that never changes (SGPR base + VGPR offset loads); no workgroup barrier in the loop.
 #include "unified_decode.cuh"
@@ -54,7 +58,9 @@ __device__ __forceinline__ typename DwVec<N>::type nt_load(const uint8_t* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const typename DwVec<N>::type*>(p));
 }
 
-template <typename T, bool FP8, int D, int NW>
+// GEN: soft cap, sliding window or ALiBi; without them the scores need no pass of their own, and only a wave's last step a
+// mask.
+template <typename T, bool FP8, int D, int NW, bool GEN>
 __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decode_kernel(const UniDecodeParams p, int sub_shift, int xcd_group, int order) {
   constexpr int ES = FP8 ? 1 : 2;             // cache element bytes
   constexpr int TILES = (FP8 && D <= 128) ? 4 : 2;   // 16-token tiles per step (the 256-wide form: 32-token steps -- 223 registers, two workgroups per CU)
@@ -115,7 +121,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
   if (qend - qtok != 1) return;   // not a decode token: the tile kernel's (or nobody's) business
   const int ctx = seq_len - 1;                       // position of the query
   const bool split = p.num_segments > 1;
-  const int kv_lo = p.window > 0 ? max(0, seq_len - p.window) : 0;   // first visible key
+  const int kv_lo = GEN && p.window > 0 ? max(0, seq_len - p.window) : 0;   // first visible key
   int start_tok = 0, end_tok = seq_len;
   if (split) {
     const int ntiles = (seq_len + 63) >> 6;
@@ -128,15 +134,18 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
   const int nsteps = end_tok > start_tok ? (end_tok - start_tok + STEP_TOK - 1) / STEP_TOK : 0;
   const int last_page = seq_len > 0 ? (seq_len - 1) >> (4 + sub_shift) : 0;
   const int sub_mask = (1 << sub_shift) - 1;
-  const int* bt = p.block_table + (int64_t)seq * p.bt_stride;
+  // (constant address space: scalar loads.  Through the struct's plain pointer they were vector loads behind vmcnt(0) -- the
+  // whole refill -- at the end of every step, since the kernel also stores)
+  typedef const __attribute__((address_space(4))) int cint;
+  cint* const bt = (cint*)(uintptr_t)(p.block_table + (int64_t)seq * p.bt_stride);
 
   float kscale = 1.f, vscale = 1.f;
   if constexpr (FP8) { kscale = *p.k_scale; vscale = *p.v_scale; }
   const float sc2 = p.sm_scale * kscale * kLog2e;
   const bool col_ok = c16 < G;
-  const bool alibi = p.alibi_slopes != nullptr;
+  const bool alibi = GEN && p.alibi_slopes != nullptr;
   const float slope2 = (alibi && col_ok) ? p.alibi_slopes[head0 + c16] * kLog2e : 0.f;
-  const float softcap = p.softcap;
+  const float softcap = GEN ? p.softcap : 0.f;
   const float cap_inv = softcap > 0.f ? 1.0f / (kLog2e * softcap) : 0.f, cap2 = softcap * kLog2e;
 
   constexpr int K_LDS = TILES * 16 * D * ES;   // one step of K per wave
@@ -149,14 +158,16 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
   // fp8 : K load i gives d = 16 (g4 + 4 i) + [0,16) -> two k-steps (lo / hi 8); 16 bit: d = 8 (g4 + 4 i) + [0,8)
   uint4 qf[QF];
   {
-    const int dlo = hp > 1 ? (c16 / Gq) * dsub : 0;   // the column's head starts at row d = dlo
-    const T* qp = (const T*)p.q + (int64_t)qtok * p.q_stride_t + (int64_t)(head0 + c16) * p.q_stride_h - dlo;
+    const int dlo = hp > 1 && col_ok ? (c16 / Gq) * dsub : 0;   // the column's head starts at row d = dlo
+    const T* qp = (const T*)p.q + (int64_t)qtok * p.q_stride_t + (int64_t)(head0 + (col_ok ? c16 : 0)) * p.q_stride_h - dlo;
 #pragma unroll
     for (int s = 0; s < QF; ++s) {
       int d;
       if constexpr (FP8) d = 16 * (g4 + 4 * (s >> 1)) + 8 * (s & 1);
       else d = 8 * (g4 + 4 * s);
-      qf[s] = (col_ok && d >= dlo && d < dlo + dsub) ? *reinterpret_cast<const uint4*>(qp + d) : make_uint4(0, 0, 0, 0);
+const bool ok = col_ok && d >= dlo && d < dlo + dsub;
+      const uint4 v = *reinterpret_cast<const uint4*>(qp + (ok ? d : dlo));
+      qf[s] = ok ? v : make_uint4(0, 0, 0, 0);
     }
   }
 
@@ -176,29 +187,28 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
   // (lane order = [row][position]) is read back conflict-free in the MFMA order
   constexpr int RB = D * ES, CPR = RB / 16, RPI = 64 / CPR;   // row bytes, chunks per row, rows per instruction
   auto kswz = [](int row) { return (row * CPR / 16) & (CPR - 1); };
+  // (head sizes below the padded D: a lane whose chunk does not exist fetches the row's first one -- its Q^T rows are zero,
+  // and a V column past the head is never stored.  No load sits behind a branch: the compiler then counts the loads in
+  // flight and waits for K alone where K is needed, instead of for everything)
   uint32_t koff[KL], krd[KL];
-  bool kval[KL];   // the chunk this lane fetches exists (head sizes below the padded D)
 #pragma unroll
   for (int i = 0; i < KL; ++i) {
     const int row = i * RPI + lane / CPR;
     const int chunk = (lane % CPR) ^ kswz(row);
-    kval[i] = chunk * 16 < dr * ES;
-    koff[i] = (uint32_t)(row * p.kc_slot_bytes + (chunk << 4));
+    koff[i] = (uint32_t)(row * p.kc_slot_bytes + (chunk * 16 < dr * ES ? chunk << 4 : 0));
     krd[i] = (uint32_t)(c16 * RB + (((g4 + 4 * i) ^ kswz(c16)) << 4));
   }
   uint32_t voff[4];   // row r of the lane's four tokens of a tile
 #pragma unroll
-  for (int r = 0; r < 4; ++r) voff[r] = (uint32_t)((4 * g4 + r) * p.vc_slot_bytes + c16 * (DT * ES));
-  const bool vval = c16 * DT < dr;   // this lane's d elements exist
+  for (int r = 0; r < 4; ++r) voff[r] = (uint32_t)((4 * g4 + r) * p.vc_slot_bytes + (c16 * DT < dr ? c16 * (DT * ES) : 0));
   const uint8_t* const k_head = p.k_cache + (int64_t)kvh * hp * p.kc_head_bytes;
   const uint8_t* const v_head = p.v_cache + (int64_t)kvh * hp * p.vc_head_bytes;
 
-  auto load_pb = [&](int step) {
-    if (step >= nsteps) return;
+  auto load_pb = [&](int step) {   // (past the last step: entries of the last page, not used)
     const int tile0 = (start_tok >> 4) + step * TILES;
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
-      pb[t] = __builtin_amdgcn_readfirstlane(bt[min((tile0 + t) >> sub_shift, last_page)]);
+      pb[t] = bt[min((tile0 + t) >> sub_shift, last_page)];
   };
   // (the empty asm keeps the 32-bit offsets from being widened to 64 bits outside the loop,
   // which would turn every load into a 64-bit VGPR address + add instead of SGPR base + offset)
@@ -215,7 +225,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
       const uint8_t* base = k_head + (int64_t)pb[t] * p.kc_block_bytes +
                             (int64_t)(((tile0 + t) & sub_mask) * 16) * p.kc_slot_bytes;
 #pragma unroll
-      for (int i = 0; i < KL; ++i) kreg[t * KL + i] = kval[i] ? nt_load<4>(base + ko[i]) : (u32x4)(0);
+      for (int i = 0; i < KL; ++i) kreg[t * KL + i] = nt_load<4>(base + ko[i]);
     }
   };
   auto issue_v = [&](int step) {
@@ -231,19 +241,20 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
       const uint8_t* base = v_head + (int64_t)pb[t] * p.vc_block_bytes +
                             (int64_t)(((tile0 + t) & sub_mask) * 16) * p.vc_slot_bytes;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) vreg[t * 4 + r] = vval ? nt_load<VDW>(base + vo[r]) : (vrow_t)(0);
+      for (int r = 0; r < 4; ++r) vreg[t * 4 + r] = nt_load<VDW>(base + vo[r]);
     }
   };
 
-  auto do_step = [&](int step) {
+  // MORE: the wave has another step behind this one -- refills unconditionally, and every token of this one exists
+  auto do_step = [&](int step, auto more_c) __attribute__((always_inline)) {
+    constexpr bool MORE = decltype(more_c)::value;
     const int tok0 = start_tok + step * STEP_TOK;
     const int pf = step + NW;
     // ---------------- K: registers -> wave-private LDS image -> MFMA order ----------------
 #pragma unroll
     for (int n = 0; n < TILES * KL; ++n)
       *reinterpret_cast<u32x4*>(k_lds + n * 1024 + lane * 16) = kreg[n];
-    const bool more = pf < nsteps;
-    if (more) issue_k(pf);
+    if constexpr (MORE) issue_k(pf);
     // ---------------- S^T = K Q^T ----------------------------------------------------
     f32x4 s[TILES];
 #pragma unroll
@@ -274,13 +285,13 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
         // triton_unified_attention.py:219-238: softcap, causal / padding mask, window, ALiBi
         const int tok = tok0 + 16 * t + 4 * g4 + r;
         float x = s[t][r] * sc2;
-        if (softcap > 0.f) {   // softcap * tanh(S / softcap) from one exp2 (log2 domain throughout)
+        if (GEN && softcap > 0.f) {   // softcap * tanh(S / softcap) from one exp2 (log2 domain throughout)
           const float y = x * cap_inv;
           const float e2 = fast_exp2(-2.0f * kLog2e * fabsf(y));
           x = copysignf(cap2 * (1.0f - e2) * __builtin_amdgcn_rcpf(1.0f + e2), y);
         }
-        x += slope2 * (float)(tok - ctx);
-        x = (tok >= kv_lo && tok < end_tok) ? x : -FLT_MAX;
+        if constexpr (GEN) x += slope2 * (float)(tok - ctx);
+        if constexpr (GEN || !MORE) x = (tok >= kv_lo && tok < end_tok) ? x : -FLT_MAX;
         s[t][r] = x;
         mx = fmaxf(mx, x);
       }
@@ -298,7 +309,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
       for (int r = 0; r < 4; ++r) {
         const int tok = tok0 + 16 * t + 4 * g4 + r;
         e[r] = fast_exp2(s[t][r] - m_new);
-        e[r] = (tok >= kv_lo && tok < end_tok) ? e[r] : 0.f;
+        if constexpr (GEN || !MORE) e[r] = (tok >= kv_lo && tok < end_tok) ? e[r] : 0.f;
         psum += e[r];
       }
       pk[t][0] = Mma<T>::pack2(e[0], e[1]);
@@ -311,7 +322,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
     }
 
     // ---------------- O^T += V^T P^T ----------------------------------------------------
-    if (tok0 + STEP_TOK > end_tok) {
+    if (!MORE && tok0 + STEP_TOK > end_tok) {
       // never-written slots past the sequence may hold NaN patterns: 0 * NaN
 #pragma unroll
       for (int t = 0; t < TILES; ++t)
@@ -343,7 +354,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
         o[j] = Mma<T>::mfma(make_uint4(a[0], a[1], a[2], a[3]), pfrag, o[j]);
       }
     }
-    if (more) {
+    if constexpr (MORE) {
       issue_v(pf);
       load_pb(pf + NW);
     }
@@ -355,9 +366,13 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
     issue_v(wave);
     load_pb(wave + NW);
   }
-  for (int step = wave; step < nsteps; step += NW) {
-    do_step(step);
-  }
+  // q, older than K and V, is waited for here (behind the join of both paths): pending at the loop's head it would be
+  // waited for -- and with it the refill -- in front of the first MFMA of every step
+#pragma unroll
+  for (int s = 0; s < QF; ++s) asm volatile("" ::"v"(qf[s].x), "v"(qf[s].y), "v"(qf[s].z), "v"(qf[s].w));
+  int step = wave;
+  for (; step + NW < nsteps; step += NW) do_step(step, std::true_type{});
+  if (step < nsteps) do_step(step, std::false_type{});
 
   // ---------------- merge the NW waves ----------------------------------------------------
   l_run += __shfl_xor(l_run, 16, 64);
@@ -506,8 +521,10 @@ int launch(const UniDecodeParams& p) {
     order = 1;
     while (order < 30 && (ml >> order) != 0) ++order;
   }
-  hipLaunchKernelGGL((ua_decode_kernel<T, FP8, D, NW>), grid, dim3(NW * 64), 0, p.stream, p, sub_shift,
-                     xcd_group, order);
+  if (p.softcap > 0.f || p.window > 0 || p.alibi_slopes != nullptr)
+    hipLaunchKernelGGL((ua_decode_kernel<T, FP8, D, NW, true>), grid, dim3(NW * 64), 0, p.stream, p, sub_shift, xcd_group, order);
+  else
+    hipLaunchKernelGGL((ua_decode_kernel<T, FP8, D, NW, false>), grid, dim3(NW * 64), 0, p.stream, p, sub_shift, xcd_group, order);
   VA_LAUNCH_CHECK("unified_attention decode launch");
   if (p.num_segments > 1) {
     hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D>), dim3((unsigned)((p.num_seqs * p.num_heads + 3) / 4)),
