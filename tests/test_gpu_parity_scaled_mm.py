@@ -378,3 +378,32 @@ def test_scaled_mm_stream_edges(ops, force_kernel, M, NK):
     torch.ops._C.cutlass_scaled_mm(buf[:, 2:2 + N], a8, w8.t(), one, one, None)
     assert torch.equal(buf[:, 2:2 + N], prod.to(torch.bfloat16))
     assert (buf[:, :2] == 7).all() and (buf[:, 2 + N:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 256), (65, 72, 256), (127, 64, 384), (128, 128, 512), (129, 136, 640),
+                                   (200, 264, 768), (256, 1096, 896), (383, 200, 1024), (509, 520, 3712)])
+def test_scaled_mm_kgroup_edges(ops, force_kernel, M, N, K):
+    """The two-K-group kernel (scaled_mm_kgroup.hip): rows and columns past the edge of a tile, fewer K blocks than ring
+    slots, odd and even numbers of them (one group has a block more), a ring that wraps.  Small-integer operands and
+    power-of-two scales: the fp32 product is exact, whatever the order of the sums.  Outputs without 16-byte rows stay
+    with the kernels that take them."""
+    force_kernel(38)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-3, 4, (M, K), generator=g).float()
+    w = torch.randint(-2, 3, (N, K), generator=g).float()
+    a[:, 0] = torch.arange(M).float() % 7
+    w[:, 1] = torch.arange(N).float() % 5
+    a8, w8 = a.to(torch.float8_e4m3fn).cuda(), w.to(torch.float8_e4m3fn).cuda()
+    prod = (a.double() @ w.double().t()).float().cuda()
+    sa = (2.0 ** -(torch.arange(M) % 5).float()).reshape(M, 1).cuda()
+    sb = (2.0 ** -(torch.arange(N) % 3).float()).reshape(N, 1).cuda()
+    bias = (torch.arange(N) % 9).to(torch.float16).cuda()
+    out = ops.cutlass_scaled_mm(a8, w8.t(), sa, sb, torch.float16, bias)
+    ref = (prod * sa * sb.t()).to(torch.float16)
+    assert torch.equal(out, (ref.float() + bias.float()).to(torch.float16))
+    one = torch.ones((1, 1), device="cuda")
+    for pad in (8, 1):   # guard columns on both sides: 16-byte rows, and 2 bytes off
+        buf = torch.full((M, N + 2 * pad), 7.0, dtype=torch.bfloat16, device="cuda")
+        torch.ops._C.cutlass_scaled_mm(buf[:, pad:pad + N], a8, w8.t(), one, one, None)
+        assert torch.equal(buf[:, pad:pad + N], prod.to(torch.bfloat16))
+        assert (buf[:, :pad] == 7).all() and (buf[:, pad + N:] == 7).all()

@@ -277,11 +277,16 @@ bool scaled_mm_stream_pays(int M, int N, int K);
 int launch_scaled_mm_stream(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
                             const void* bias, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
                             int out_dtype, hipStream_t st);
+// scaled_mm_kgroup.hip
+bool scaled_mm_kgroup_pays(int M, int N, int K);
+int launch_scaled_mm_kgroup(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
+                            const void* bias, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
+                            int out_dtype, hipStream_t st);
 // scaled_mm_pp.hip
 int launch_scaled_mm_pp(int variant, void* out, const void* a, const void* b, const float* a_scales,
                         const float* b_scales, const void* bias, int M, int N, int K, int64_t lda,
                         int64_t ldb, int64_t ldc, int asn, int bsn, int out_dtype, hipStream_t st);
-int g_mm_kernel = 0;   // tuning: 0 auto, 1 = register-staged 128x128, 2..10, 12, 13 = glds tile shapes, 37 = the stream kernel
+int g_mm_kernel = 0;   // tuning: 0 auto, 1 = register-staged 128x128, 2..10, 12, 13 = glds tile shapes, 37 = the stream kernel, 38 = two K groups
 int g_mm_splitk = 0;   // tuning: 0 auto, n >= 1 = n K slices (1 = never split)
 int g_mm_tail = 0;     // tuning key kept for old scripts; the tail split went away with the persistent kernel
 }  // namespace va
@@ -350,6 +355,14 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
       }
       sel = 2;
     }
+    // a single round of 128 x 128 tiles: scaled_mm_kgroup.hip ("mm_kernel" 38 forces it)
+    if ((sel == 38 || (sel == 0 && want_splits == 0 && scaled_mm_kgroup_pays(M, N, K))) && ldc % 8 == 0 && N % 8 == 0 &&
+        (((uintptr_t)out) & 15) == 0) {
+      launch_scaled_mm_kgroup(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel,
+                              out_dtype, st);
+      VA_LAUNCH_CHECK(op);
+      return VLLM_AMD_OK;
+    }
     if (sel == 0 || sel == 11 || sel > 36) {
       // Largest tile that still yields ~3/4 of a full wave of workgroups (256 CUs); rows of
       // a tile beyond M are wasted MFMA work, so BM <= 2 M.  With more than one wave of tiles the
@@ -363,7 +376,10 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
         const GldsTile& t = tiles_tab[i];
         if (i < 4 && t.bm > 64 && M <= t.bm / 2) continue;
         const int nt = ceil_div(M, t.bm) * ceil_div(N, t.bn);
-        if (nt >= 190 || i == 4) {
+        // (128 x 64 tiles of few rows already from 160 on: 4096 x 10240 at M 96 19.8 -> 17.7 us, 8192 x 5120 at M 256 36.0 ->
+        // 29.5; not where a quarter of the rows is padding, M 160 12.3 -> 13.7, nor above, 8192 x 2048 at M 640 25.2 -> 26.1)
+        const int enough = i == 2 && M <= 256 && (M <= 128 || M > 192) ? 160 : 190;
+        if (nt >= enough || i == 4) {
           // (the 64 x 64 tile with 4 K blocks per barrier loses on long K loops: 14336 x 4096 at
           // M 192 / 256 31.1 vs 25.3 / 27.5 us, 8192 x 4096 18.2 / 19.0 vs 16.0 / 16.6 us; at K 4096
           // it wins, 8.5 vs 9.1 us -- profiles/r02_gemm_sweep_mid.csv)
