@@ -850,7 +850,9 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
   // the group) pairs when the group divides into 256 rows), where fa_plan takes it
   {
     const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
-    const bool can = p.alibi_slopes == nullptr && p.flat_batch > 0 && p.sm_scale > 0.f;
+    // (its lanes add 32-bit multiples of the slot stride)
+    const bool can = p.alibi_slopes == nullptr && p.flat_batch > 0 && p.sm_scale > 0.f &&
+                     p.kc_page_bytes < (1 << 27) && p.vc_page_bytes < (1 << 27);
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments);
     if (can && plan.use) {

@@ -235,6 +235,26 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // PREFIX, context V^T: item -> (d = item % D, tokens 16 vq .. of the tile with vq = item / D)
   auto vd_of = [&](int i) __attribute__((always_inline)) { return (tid + NTHR * i) % D; };
   auto vq_of = [&](int i) __attribute__((always_inline)) { return (tid + NTHR * i) / D; };
+  // A wave's items are 64 / PPK = 8 (D = 256: 4) neighbouring keys and, for the context V^T, one group of 16 tokens: inside
+  // one block of the cache (16 slots or more), so block ids and base addresses are wave-uniform -- scalar arithmetic -- and
+  // a lane adds a 32-bit constant.  (Per-lane 64-bit products cost ~400 of the ~4100 cycles of a tile on every SIMD.)
+  constexpr int WK = 64 / PPK;
+  const int wkey = WK * wave, lkey = lane / PPK;                   // skey = wkey + lkey
+  auto wvq_of = [&](int i) __attribute__((always_inline)) { return (64 * wave + NTHR * i) / D; };
+  uint32_t koff, koff1 = 0, voff, voff1 = 0;                       // context / paged part: first and second 16 bytes
+  uint32_t vtoff[IPT];
+  if constexpr (PREFIX) {
+    koff = (uint32_t)((((FP8 ? spl : 2 * spl) << p.bs_shift) + lkey) << 4);
+    koff1 = FP8 ? 0 : (uint32_t)((((2 * spl + (pv1 ? 1 : 0)) << p.bs_shift) + lkey) << 4);
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) vtoff[i] = (uint32_t)((min(vd_of(i), dr - 1) << p.bs_shift) * (FP8 ? 1 : 2));
+    voff = 0;
+  } else {
+    koff = (uint32_t)lkey * (uint32_t)p.kc_slot_bytes + 16 * NST * spl;
+    voff = (uint32_t)lkey * (uint32_t)p.vc_slot_bytes + 16 * NST * spl;
+    koff1 = koff + 2 * o1;
+    voff1 = voff + 2 * o1;
+  }
   struct Blk { int k[IPT], v[IPT]; };
   auto load_blk = [&](int t) __attribute__((always_inline)) {
     Blk b;
@@ -243,53 +263,45 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
       b.k[i] = 0; b.v[i] = 0;
       if constexpr (PREFIX) {
         if (t < ctx_tiles) {
-          b.k[i] = bt[min((t * BN + skey + KSTEP * i) >> p.bs_shift, last_page)];
-          b.v[i] = bt[min((t * BN + 16 * vq_of(i)) >> p.bs_shift, last_page)];
+          b.k[i] = bt[min((t * BN + wkey + KSTEP * i) >> p.bs_shift, last_page)];
+          b.v[i] = bt[min((t * BN + 16 * wvq_of(i)) >> p.bs_shift, last_page)];
         }
       } else {
-        if (t < ntiles) b.k[i] = bt[min((t * BN + skey + KSTEP * i) >> p.bs_shift, last_page)];
+        if (t < ntiles) b.k[i] = bt[min((t * BN + wkey + KSTEP * i) >> p.bs_shift, last_page)];
       }
     }
     return b;
   };
   auto ld16 = [](const void* ptr) __attribute__((always_inline)) { return *reinterpret_cast<const u32x4*>(ptr); };
   auto issue_loads = [&](int t, const Blk& blk) __attribute__((always_inline)) {
+    const int bsm = (1 << p.bs_shift) - 1;
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
-      const int key = skey + KSTEP * i;
+      const int slot = (t * BN + wkey + KSTEP * i) & bsm;
       if constexpr (PREFIX) {
         if (t < ctx_tiles) {
-          const int bsm = (1 << p.bs_shift) - 1;
-          const int slot = (t * BN + key) & bsm;
-          const uint8_t* kb = p.k_cache + (int64_t)blk.k[i] * p.kc_block_bytes + (int64_t)kvh * p.kc_head_bytes;
-          if constexpr (FP8) {
-            kst[i][0] = ld16(kb + (((spl << p.bs_shift) + slot) << 4));
-          } else {
-            kst[i][0] = ld16(kb + ((((2 * spl) << p.bs_shift) + slot) << 4));
-            kst[i][1] = ld16(kb + ((((2 * spl + (pv1 ? 1 : 0)) << p.bs_shift) + slot) << 4));
-          }
-          const int slot0 = (t * BN + 16 * vq_of(i)) & bsm;
-          const uint8_t* vb = p.v_cache + (int64_t)blk.v[i] * p.vc_block_bytes + (int64_t)kvh * p.vc_head_bytes +
-                              ((min(vd_of(i), dr - 1) << p.bs_shift) + slot0) * (FP8 ? 1 : 2);
-          vst[i][0] = ld16(vb);
-          if constexpr (!FP8) vst[i][1] = ld16(vb + 16);
+          const uint8_t* kb = p.k_cache + (int64_t)__builtin_amdgcn_readfirstlane(blk.k[i]) * p.kc_block_bytes + (int64_t)kvh * p.kc_head_bytes + (slot << 4);
+          kst[i][0] = ld16(kb + koff);
+          if constexpr (!FP8) kst[i][1] = ld16(kb + koff1);
+          const int slot0 = (t * BN + 16 * wvq_of(i)) & bsm;
+          const uint8_t* vb = p.v_cache + (int64_t)__builtin_amdgcn_readfirstlane(blk.v[i]) * p.vc_block_bytes + (int64_t)kvh * p.vc_head_bytes + slot0 * (FP8 ? 1 : 2);
+          vst[i][0] = ld16(vb + vtoff[i]);
+          if constexpr (!FP8) vst[i][1] = ld16(vb + vtoff[i] + 16);
         } else {
-          const int64_t row = tok0 + min((t - ctx_tiles) * BN + key, qlen - 1);
+          const int64_t row = tok0 + min((t - ctx_tiles) * BN + skey + KSTEP * i, qlen - 1);
           const T* kr = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h + 16 * spl;
           const T* vr = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h + 16 * spl;
           kst[i][0] = ld16(kr); kst[i][1] = ld16(kr + o1);
           vst[i][0] = ld16(vr); vst[i][1] = ld16(vr + o1);
         }
       } else {
-        const int slot = (t * BN + key) & ((1 << p.bs_shift) - 1);
-        const uint8_t* kr = p.k_cache + (int64_t)blk.k[i] * p.kc_block_bytes + (int64_t)slot * p.kc_slot_bytes +
-                            (int64_t)kvh * p.kc_head_bytes + 16 * NST * spl;
-        const uint8_t* vr = p.v_cache + (int64_t)blk.k[i] * p.vc_block_bytes + (int64_t)slot * p.vc_slot_bytes +
-                            (int64_t)kvh * p.vc_head_bytes + 16 * NST * spl;
+        const int64_t bid = __builtin_amdgcn_readfirstlane(blk.k[i]);
+        const uint8_t* kr = p.k_cache + bid * p.kc_block_bytes + (int64_t)slot * p.kc_slot_bytes + (int64_t)kvh * p.kc_head_bytes;
+        const uint8_t* vr = p.v_cache + bid * p.vc_block_bytes + (int64_t)slot * p.vc_slot_bytes + (int64_t)kvh * p.vc_head_bytes;
 #pragma unroll
         for (int j = 0; j < NST; ++j) {
-          kst[i][j] = ld16(kr + (j ? 2 * o1 : 0));   // (fp8: one load; 16-bit: the second chunk 16 bytes on, if it exists)
-          vst[i][j] = ld16(vr + (j ? 2 * o1 : 0));
+          kst[i][j] = ld16(kr + (j ? koff1 : koff));   // (fp8: one load; 16-bit: the second chunk 16 bytes on, if it exists)
+          vst[i][j] = ld16(vr + (j ? voff1 : voff));
         }
       }
     }
@@ -307,6 +319,8 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
     const bool is_ctx = PREFIX && t < ctx_tiles;
     const bool conv = FP8 && (!PREFIX || is_ctx);   // this tile's registers hold e4m3
+    // (wave-uniform) every key of the tile exists and no column is padding: nothing to zero
+    const bool whole = dr == D && (PREFIX ? (is_ctx ? (t + 1) * BN <= ctx : (t - ctx_tiles + 1) * BN <= qlen) : (t + 1) * BN <= seq_len);
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
       const int key = skey + KSTEP * i;
@@ -323,8 +337,10 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
       } else {
         k0 = kst[i][0]; k1 = kst[i][NST - 1];
       }
-      if (!live || !pv0) k0 = (u32x4){0, 0, 0, 0};
-      if (!live || !pv1) k1 = (u32x4){0, 0, 0, 0};
+      if (!whole) {
+        if (!live || !pv0) k0 = (u32x4){0, 0, 0, 0};
+        if (!live || !pv1) k1 = (u32x4){0, 0, 0, 0};
+      }
       *reinterpret_cast<u32x4*>(k_wr + kb_ + KSTEP * i * ROWB + kc0) = k0;
       *reinterpret_cast<u32x4*>(k_wr + kb_ + KSTEP * i * ROWB + kc1) = k1;
       if (is_ctx) {
@@ -333,10 +349,16 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
         const int valid = vd < dr ? ctx - (t * BN + 16 * vq) : 0;
         uint4 lo, hi4;
         if constexpr (FP8) {
-          widen16<T>(mask_bytes(u4(vst[i][0]), valid), lo, hi4);
+          uint4 raw = u4(vst[i][0]);
+          if (!whole) raw = mask_bytes(raw, valid);
+          widen16<T>(raw, lo, hi4);
         } else {
-          lo = mask_halfs(u4(vst[i][0]), valid);
-          hi4 = mask_halfs(u4(vst[i][NST - 1]), valid - 8);
+          lo = u4(vst[i][0]);
+          hi4 = u4(vst[i][NST - 1]);
+          if (!whole) {
+            lo = mask_halfs(lo, valid);
+            hi4 = mask_halfs(hi4, valid - 8);
+          }
         }
         uint8_t* row = lds + V_OFF + vb_ + vd * 128;
         const int f = (vd >> 1) & 15;
@@ -353,8 +375,10 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
         } else {
           v0 = vst[i][0]; v1 = vst[i][NST - 1];
         }
-        if (!live || !pv0) v0 = (u32x4){0, 0, 0, 0};
-        if (!live || !pv1) v1 = (u32x4){0, 0, 0, 0};
+        if (!whole) {
+          if (!live || !pv0) v0 = (u32x4){0, 0, 0, 0};
+          if (!live || !pv1) v1 = (u32x4){0, 0, 0, 0};
+        }
         *reinterpret_cast<u32x4*>(v_wr + vb_ + KSTEP * i * ROWB + vc0) = v0;
         *reinterpret_cast<u32x4*>(v_wr + vb_ + KSTEP * i * ROWB + vc1) = v1;
       }
