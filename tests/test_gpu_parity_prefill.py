@@ -300,6 +300,22 @@ def test_prefill_long_chunk_repeats_bit_for_bit(dtype, kv, ctx):
         assert torch.equal(run(c, kv), first)
 
 
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("block_size", [16, 32])
+@pytest.mark.parametrize("head_size", [128, 112, 256])
+def test_prefill_fa_kernel_whole_tiles(oracle, force_fa, head_size, block_size, kv):
+    """Runs of whole 64-key tiles are staged without checks while two more whole tiles of the same kind follow: contexts and
+    chunks of 0 .. 5 whole tiles, ending on a tile, one key before and one behind; a head size
+    with padding columns, which has no such run."""
+    qls = [320, 64, 129, 255, 192, 65, 257, 128]
+    ctxs = [0, 64, 128, 191, 192, 193, 256, 321]
+    c = make_prefill_case(qls, ctxs, 4, 2, head_size, block_size, torch.bfloat16, kv, seed=head_size + block_size, kv_scale=0.02)
+    out = run(c, kv)
+    assert not out.isnan().any()
+    torch.testing.assert_close(out.float(), run_oracle(oracle, c, kv).float(), atol=tol(torch.bfloat16), rtol=0)
+    torch.testing.assert_close(out.float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)
+
+
 @pytest.fixture
 def tuning():
     from vllm_amd import _lib

@@ -502,6 +502,18 @@ def test_unified_fa_kernel_softcap(oracle, force_fa, soft_cap, D, fp8, window):
         run(oracle, c, dtype, fp8=fp8, softcap=soft_cap, window=window)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D", [128, 112, 256])
+@pytest.mark.parametrize("window", [None, 130])
+def test_unified_fa_kernel_whole_tiles(oracle, force_fa, window, D, fp8):
+    """Runs of whole 64-key tiles are staged without checks while two more follow: sequences of 1 .. 8 whole tiles, ending
+    on a tile, one key before and one behind, with and without keys before the chunk; a head size with padding columns,
+    which has no such run."""
+    lens = [(320, 320), (64, 128), (129, 257), (255, 446), (192, 384), (65, 258), (257, 513), (128, 449)]
+    c = make_unified_case(lens, 4, 2, D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
+    run(oracle, c, torch.bfloat16, fp8=fp8, window=window)
+
+
 @pytest.mark.parametrize("segs", [2, 5, 32])
 @pytest.mark.parametrize("num_heads,head_size", [((8, 2), 128), ((8, 8), 64), ((8, 1), 80), ((4, 2), 256)])
 @pytest.mark.parametrize("mode", ["plain", "fp8", "window", "softcap", "fp8_out", "mixed"])

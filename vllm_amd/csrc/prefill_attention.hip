@@ -928,8 +928,9 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
   {
     const int gqa = p.num_heads / p.num_kv_heads;
     const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
+    // (its lanes add 32-bit multiples of the token stride)
     const bool can = p.alibi_slopes == nullptr && p.sliding_window == 0 && p.sm_scale > 0.f &&
-                     (block_size & (block_size - 1)) == 0;
+                     (block_size & (block_size - 1)) == 0 && p.k_stride_t < (1 << 27) && p.v_stride_t < (1 << 27);
     const int64_t ptok = p.flat_batch > 0 ? (int64_t)p.flat_tokens : (int64_t)max_input_len * batch;
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
                                 p.flat_batch > 0 ? p.num_segments : 1);

@@ -273,38 +273,63 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     return b;
   };
   auto ld16 = [](const void* ptr) __attribute__((always_inline)) { return *reinterpret_cast<const u32x4*>(ptr); };
-  auto issue_loads = [&](int t, const Blk& blk) __attribute__((always_inline)) {
+  // (one branch per tile, not per item: hipcc copies the loaded registers at every join)
+  auto issue_ctx = [&](int t, const Blk& blk) __attribute__((always_inline)) {
+    const int bsm = (1 << p.bs_shift) - 1;
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) {
+      const int slot = (t * BN + wkey + KSTEP * i) & bsm, slot0 = (t * BN + 16 * wvq_of(i)) & bsm;
+      const uint8_t* kb = p.k_cache + (int64_t)__builtin_amdgcn_readfirstlane(blk.k[i]) * p.kc_block_bytes + (int64_t)kvh * p.kc_head_bytes + (slot << 4);
+      kst[i][0] = ld16(kb + koff);
+      if constexpr (!FP8) kst[i][1] = ld16(kb + koff1);
+      const uint8_t* vb = p.v_cache + (int64_t)__builtin_amdgcn_readfirstlane(blk.v[i]) * p.vc_block_bytes + (int64_t)kvh * p.vc_head_bytes + slot0 * (FP8 ? 1 : 2);
+      vst[i][0] = ld16(vb + vtoff[i]);
+      if constexpr (!FP8) vst[i][1] = ld16(vb + vtoff[i] + 16);
+      // (dead until a tile of new tokens: said so, hipcc does not carry -- copy, wait for -- them around the loop)
+      if constexpr (FP8) {
+        kst[i][NST - 1] = __builtin_nondeterministic_value(kst[i][NST - 1]);
+        vst[i][NST - 1] = __builtin_nondeterministic_value(vst[i][NST - 1]);
+      }
+    }
+  };
+  auto issue_new = [&](int t, auto fast_c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) {
+      if constexpr (decltype(fast_c)::value) {   // every row exists: a scalar base and a lane constant
+        const int64_t row = tok0 + (t - ctx_tiles) * BN + wkey + KSTEP * i;
+        const T* kb = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h;
+        const T* vb = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h;
+        const uint32_t ko = (uint32_t)lkey * (uint32_t)p.k_stride_t + 16 * spl, vo = (uint32_t)lkey * (uint32_t)p.v_stride_t + 16 * spl;
+        kst[i][0] = ld16(kb + ko); kst[i][NST - 1] = ld16(kb + ko + 8);
+        vst[i][0] = ld16(vb + vo); vst[i][NST - 1] = ld16(vb + vo + 8);
+        continue;
+      }
+      const int64_t row = tok0 + min((t - ctx_tiles) * BN + skey + KSTEP * i, qlen - 1);
+      const T* kr = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h + 16 * spl;
+      const T* vr = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h + 16 * spl;
+      kst[i][0] = ld16(kr); kst[i][NST - 1] = ld16(kr + o1);
+      vst[i][0] = ld16(vr); vst[i][NST - 1] = ld16(vr + o1);
+    }
+  };
+  auto issue_paged = [&](int t, const Blk& blk) __attribute__((always_inline)) {
     const int bsm = (1 << p.bs_shift) - 1;
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
       const int slot = (t * BN + wkey + KSTEP * i) & bsm;
-      if constexpr (PREFIX) {
-        if (t < ctx_tiles) {
-          const uint8_t* kb = p.k_cache + (int64_t)__builtin_amdgcn_readfirstlane(blk.k[i]) * p.kc_block_bytes + (int64_t)kvh * p.kc_head_bytes + (slot << 4);
-          kst[i][0] = ld16(kb + koff);
-          if constexpr (!FP8) kst[i][1] = ld16(kb + koff1);
-          const int slot0 = (t * BN + 16 * wvq_of(i)) & bsm;
-          const uint8_t* vb = p.v_cache + (int64_t)__builtin_amdgcn_readfirstlane(blk.v[i]) * p.vc_block_bytes + (int64_t)kvh * p.vc_head_bytes + slot0 * (FP8 ? 1 : 2);
-          vst[i][0] = ld16(vb + vtoff[i]);
-          if constexpr (!FP8) vst[i][1] = ld16(vb + vtoff[i] + 16);
-        } else {
-          const int64_t row = tok0 + min((t - ctx_tiles) * BN + skey + KSTEP * i, qlen - 1);
-          const T* kr = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h + 16 * spl;
-          const T* vr = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h + 16 * spl;
-          kst[i][0] = ld16(kr); kst[i][1] = ld16(kr + o1);
-          vst[i][0] = ld16(vr); vst[i][1] = ld16(vr + o1);
-        }
-      } else {
-        const int64_t bid = __builtin_amdgcn_readfirstlane(blk.k[i]);
-        const uint8_t* kr = p.k_cache + bid * p.kc_block_bytes + (int64_t)slot * p.kc_slot_bytes + (int64_t)kvh * p.kc_head_bytes;
-        const uint8_t* vr = p.v_cache + bid * p.vc_block_bytes + (int64_t)slot * p.vc_slot_bytes + (int64_t)kvh * p.vc_head_bytes;
+      const int64_t bid = __builtin_amdgcn_readfirstlane(blk.k[i]);
+      const uint8_t* kr = p.k_cache + bid * p.kc_block_bytes + (int64_t)slot * p.kc_slot_bytes + (int64_t)kvh * p.kc_head_bytes;
+      const uint8_t* vr = p.v_cache + bid * p.vc_block_bytes + (int64_t)slot * p.vc_slot_bytes + (int64_t)kvh * p.vc_head_bytes;
 #pragma unroll
-        for (int j = 0; j < NST; ++j) {
-          kst[i][j] = ld16(kr + (j ? koff1 : koff));   // (fp8: one load; 16-bit: the second chunk 16 bytes on, if it exists)
-          vst[i][j] = ld16(vr + (j ? voff1 : voff));
-        }
+      for (int j = 0; j < NST; ++j) {
+        kst[i][j] = ld16(kr + (j ? koff1 : koff));   // (fp8: one load; 16-bit: the second chunk 16 bytes on, if it exists)
+        vst[i][j] = ld16(vr + (j ? voff1 : voff));
       }
     }
+  };
+  auto issue_loads = [&](int t, const Blk& blk) __attribute__((always_inline)) {
+    if constexpr (!PREFIX) issue_paged(t, blk);
+    else if (t < ctx_tiles) issue_ctx(t, blk);
+    else issue_new(t, std::false_type{});
   };
   // K image: chunk ^= key & 15 (conflict-free ds_read_b128 of 32 keys x one chunk); V image: chunk ^= (key & 3) << 2
   // (the four keys of a transposing read land in four different 64-byte bank ranges); context V^T image (PREFIX):
@@ -315,74 +340,69 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   const int kc0 = ((2 * spiece) ^ (skey & 15)) << 4, kc1 = ((2 * spiece + 1) ^ (skey & 15)) << 4;
   const int vc0 = ((2 * spiece) ^ ((skey & 3) << 2)) << 4, vc1 = ((2 * spiece + 1) ^ ((skey & 3) << 2)) << 4;
   auto u4 = [](u32x4 v) __attribute__((always_inline)) { return make_uint4(v[0], v[1], v[2], v[3]); };
-  auto write_tile = [&](int t) __attribute__((always_inline)) {
+  // Slots past the sequence hold stale bytes (possibly NaN): K and V rows of such keys are zeroed (their scores are 0 + the
+  // mask's -inf, their probabilities 0, and 0 * NaN = NaN), and so are the padding columns.  whole: every key of the tile
+  // exists and no column is padding, nothing to zero.  conv: the registers hold e4m3.
+  auto write_row = [&](uint8_t* row, int c0, int c1, const u32x4 (&st)[NST], bool live, auto whole, auto conv_c) __attribute__((always_inline)) {
+    u32x4 x0, x1;
+    if constexpr (decltype(conv_c)::value) {
+      uint4 lo, hi4;
+      widen16<T>(u4(st[0]), lo, hi4);
+      x0 = (u32x4){lo.x, lo.y, lo.z, lo.w};
+      x1 = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
+    } else {
+      x0 = st[0]; x1 = st[NST - 1];
+    }
+    if (!whole) {
+      if (!live || !pv0) x0 = (u32x4){0, 0, 0, 0};
+      if (!live || !pv1) x1 = (u32x4){0, 0, 0, 0};
+    }
+    *reinterpret_cast<u32x4*>(row + c0) = x0;
+    *reinterpret_cast<u32x4*>(row + c1) = x1;
+  };
+  // rows of keys base + (0..63) of `keys` keys, K and V
+  auto write_rows = [&](int t, int base, int keys, auto conv_c, auto whole) __attribute__((always_inline)) {
     const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
-    const bool is_ctx = PREFIX && t < ctx_tiles;
-    const bool conv = FP8 && (!PREFIX || is_ctx);   // this tile's registers hold e4m3
-    // (wave-uniform) every key of the tile exists and no column is padding: nothing to zero
-    const bool whole = dr == D && (PREFIX ? (is_ctx ? (t + 1) * BN <= ctx : (t - ctx_tiles + 1) * BN <= qlen) : (t + 1) * BN <= seq_len);
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
-      const int key = skey + KSTEP * i;
-      // slots past the sequence hold stale bytes (possibly NaN): K and V rows of such keys are zeroed (their
-      // scores are 0 + the mask's -inf, their probabilities 0, and 0 * NaN = NaN)
-      const bool live = PREFIX ? (is_ctx ? t * BN + key < ctx : (t - ctx_tiles) * BN + key < qlen)
-                               : t * BN + key < seq_len;
-      u32x4 k0, k1, v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-      if (conv) {
-        uint4 lo, hi4;
-        widen16<T>(u4(kst[i][0]), lo, hi4);
-        k0 = (u32x4){lo.x, lo.y, lo.z, lo.w};
-        k1 = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
-      } else {
-        k0 = kst[i][0]; k1 = kst[i][NST - 1];
-      }
-      if (!whole) {
-        if (!live || !pv0) k0 = (u32x4){0, 0, 0, 0};
-        if (!live || !pv1) k1 = (u32x4){0, 0, 0, 0};
-      }
-      *reinterpret_cast<u32x4*>(k_wr + kb_ + KSTEP * i * ROWB + kc0) = k0;
-      *reinterpret_cast<u32x4*>(k_wr + kb_ + KSTEP * i * ROWB + kc1) = k1;
-      if (is_ctx) {
-        // V^T: the item's 16 tokens of row vd = four 8-byte units
-        const int vd = vd_of(i), vq = vq_of(i);
-        const int valid = vd < dr ? ctx - (t * BN + 16 * vq) : 0;
-        uint4 lo, hi4;
-        if constexpr (FP8) {
-          uint4 raw = u4(vst[i][0]);
-          if (!whole) raw = mask_bytes(raw, valid);
-          widen16<T>(raw, lo, hi4);
-        } else {
-          lo = u4(vst[i][0]);
-          hi4 = u4(vst[i][NST - 1]);
-          if (!whole) {
-            lo = mask_halfs(lo, valid);
-            hi4 = mask_halfs(hi4, valid - 8);
-          }
-        }
-        uint8_t* row = lds + V_OFF + vb_ + vd * 128;
-        const int f = (vd >> 1) & 15;
-        *reinterpret_cast<u32x2*>(row + (((4 * vq + 0) ^ f) << 3)) = (u32x2){lo.x, lo.y};
-        *reinterpret_cast<u32x2*>(row + (((4 * vq + 1) ^ f) << 3)) = (u32x2){lo.z, lo.w};
-        *reinterpret_cast<u32x2*>(row + (((4 * vq + 2) ^ f) << 3)) = (u32x2){hi4.x, hi4.y};
-        *reinterpret_cast<u32x2*>(row + (((4 * vq + 3) ^ f) << 3)) = (u32x2){hi4.z, hi4.w};
-      } else {
-        if (conv) {
-          uint4 lo, hi4;
-          widen16<T>(u4(vst[i][0]), lo, hi4);
-          v0 = (u32x4){lo.x, lo.y, lo.z, lo.w};
-          v1 = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
-        } else {
-          v0 = vst[i][0]; v1 = vst[i][NST - 1];
-        }
-        if (!whole) {
-          if (!live || !pv0) v0 = (u32x4){0, 0, 0, 0};
-          if (!live || !pv1) v1 = (u32x4){0, 0, 0, 0};
-        }
-        *reinterpret_cast<u32x4*>(v_wr + vb_ + KSTEP * i * ROWB + vc0) = v0;
-        *reinterpret_cast<u32x4*>(v_wr + vb_ + KSTEP * i * ROWB + vc1) = v1;
-      }
+      const bool live = base + skey + KSTEP * i < keys;
+      write_row(k_wr + kb_ + KSTEP * i * ROWB, kc0, kc1, kst[i], live, whole, conv_c);
+      write_row(v_wr + vb_ + KSTEP * i * ROWB, vc0, vc1, vst[i], live, whole, conv_c);
     }
+  };
+  auto write_ctx = [&](int t, auto whole) __attribute__((always_inline)) {
+    const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
+#pragma unroll
+    for (int i = 0; i < IPT; ++i) {
+      write_row(k_wr + kb_ + KSTEP * i * ROWB, kc0, kc1, kst[i], t * BN + skey + KSTEP * i < ctx, whole, std::integral_constant<bool, FP8>{});
+      // V^T: the item's 16 tokens of row vd = four 8-byte units
+      const int vd = vd_of(i), vq = vq_of(i);
+      const int valid = vd < dr ? ctx - (t * BN + 16 * vq) : 0;
+      uint4 lo, hi4;
+      if constexpr (FP8) {
+        uint4 raw = u4(vst[i][0]);
+        if (!whole) raw = mask_bytes(raw, valid);
+        widen16<T>(raw, lo, hi4);
+      } else {
+        lo = u4(vst[i][0]);
+        hi4 = u4(vst[i][NST - 1]);
+        if (!whole) {
+          lo = mask_halfs(lo, valid);
+          hi4 = mask_halfs(hi4, valid - 8);
+        }
+      }
+      uint8_t* row = lds + V_OFF + vb_ + vd * 128;
+      const int f = (vd >> 1) & 15;
+      *reinterpret_cast<u32x2*>(row + (((4 * vq + 0) ^ f) << 3)) = (u32x2){lo.x, lo.y};
+      *reinterpret_cast<u32x2*>(row + (((4 * vq + 1) ^ f) << 3)) = (u32x2){lo.z, lo.w};
+      *reinterpret_cast<u32x2*>(row + (((4 * vq + 2) ^ f) << 3)) = (u32x2){hi4.x, hi4.y};
+      *reinterpret_cast<u32x2*>(row + (((4 * vq + 3) ^ f) << 3)) = (u32x2){hi4.z, hi4.w};
+    }
+  };
+  auto write_tile = [&](int t) __attribute__((always_inline)) {
+    if constexpr (!PREFIX) write_rows(t, t * BN, seq_len, std::integral_constant<bool, FP8>{}, false);
+    else if (t < ctx_tiles) write_ctx(t, false);
+    else write_rows(t, (t - ctx_tiles) * BN, qlen, std::false_type{}, false);
   };
 
   // ---- fragment read addresses (lane constants; buffer, key block and key group are immediates) ---------
@@ -588,18 +608,34 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // ("pf_fa_stagger" bits 1 / 2, measurement: a static priority for waves 4-7 / 0-3)
   if ((p.stagger & 2) && wave >= NW / 2) __builtin_amdgcn_s_setprio(1);
   if ((p.stagger & 4) && wave < NW / 2) __builtin_amdgcn_s_setprio(1);
-  auto stage = [&](int t) __attribute__((always_inline)) {
-    if (!(abl & 2)) {
+  // FAST: tiles t + 1 and t + 2 exist, are whole and belong to the run's domain: no branch in the staging.  (us with the
+  // checks -> without: unified bf16 1 x 8192 521 -> 507, head 256 bf16 4 x 2048 + 2048 1297 -> 1139, fp8 64 x 128 + 4096
+  // 1695 -> 1392; context_attention fp8 64 x 128 + 4096 738 -> 653, head 256 2170 instead of 3218: behind the checks hipcc
+  // copied the loaded registers at every join, which waited for the loads just issued.)
+  auto stage = [&](int t, auto fast_c, auto vt_c) __attribute__((always_inline)) {
+    if (abl & 2) return;
+    if constexpr (decltype(fast_c)::value) {
+      if constexpr (!PREFIX) {
+        write_rows(t + 1, 0, 0, std::integral_constant<bool, FP8>{}, std::true_type{});
+        issue_paged(t + 2, blk);
+      } else if constexpr (decltype(vt_c)::value) {
+        write_ctx(t + 1, std::true_type{});
+        issue_ctx(t + 2, blk);
+      } else {
+        write_rows(t + 1, 0, 0, std::false_type{}, std::true_type{});
+        issue_new(t + 2, std::true_type{});
+      }
+    } else {
       if (t + 1 < t1) write_tile(t + 1);
       if (t + 2 < t1) issue_loads(t + 2, blk);
-      blk = load_blk(t + 3);
     }
+    blk = load_blk(t + 3);
   };
-  auto tile_loop = [&](int t_begin, int t_end, auto mode_c, auto vt_c) __attribute__((always_inline)) {
+  auto tile_loop = [&](int t_begin, int t_end, auto mode_c, auto vt_c, auto fast_c) __attribute__((always_inline)) {
     constexpr int MODE = decltype(mode_c)::value;
     t_end = min(t_end, t1);
     for (int t = max(t_begin, t0); t < t_end; ++t) {
-      if (stage_first) stage(t);
+      if (stage_first) stage(t, fast_c, vt_c);
       FA_T(1);
       if constexpr (MODE < 2) {
         compute(t, std::integral_constant<bool, MODE == 1>{}, vt_c);
@@ -609,7 +645,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
 #endif
       }
       // (behind the compute the fragment rings are dead: room for the conversion temporaries)
-      if (!stage_first) stage(t);
+      if (!stage_first) stage(t, fast_c, vt_c);
       FA_T(0);
       if (!(abl & 16)) __syncthreads();
       FA_T(5);
@@ -621,17 +657,23 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // new-domain tiles u = t - ctx_tiles: interior while 64 u + 63 <= w_lo, computed while 64 u <= w_hi
   const int n2 = w_rows ? min(w_hi / BN + 1, new_tiles) : 0;
   const int n1 = w_rows ? min((w_lo + 1) / BN, n2) : 0;
+  // interior tiles whose staging has nothing to check (stage()) run in loops of their own: [begin, fast_end), the tiles t with
+  // t + 2 below `wholes`, the end of the whole tiles of the domain
+  auto fast_end = [&](int begin, int end, int wholes) __attribute__((always_inline)) {
+    return dr == D ? max(min(min(wholes, t1) - 2, end), begin) : begin;
+  };
   if constexpr (PREFIX) {
     // context: whole tiles are interior, the last one (ctx % 64 tokens) is masked
-    const int c2 = w_rows ? ctx_tiles : 0, c1 = w_rows ? ctx / BN : 0;
-    tile_loop(0, c1, INTERIOR, std::true_type{});
-    tile_loop(c1, c2, MASKED_, std::true_type{});
-    tile_loop(c2, ctx_tiles, SKIP, std::true_type{});
-  }
-  if constexpr (PREFIX) {
-    tile_loop(ctx_tiles, ctx_tiles + n1, INTERIOR, std::false_type{});
-    tile_loop(ctx_tiles + n1, ctx_tiles + n2, MASKED_, std::false_type{});
-    tile_loop(ctx_tiles + n2, ntiles, SKIP, std::false_type{});
+    const int c2 = w_rows ? ctx_tiles : 0, c1 = w_rows ? ctx / BN : 0, cf = fast_end(0, c1, ctx / BN);
+    tile_loop(0, cf, INTERIOR, std::true_type{}, std::true_type{});
+    tile_loop(cf, c1, INTERIOR, std::true_type{}, std::false_type{});
+    tile_loop(c1, c2, MASKED_, std::true_type{}, std::false_type{});
+    tile_loop(c2, ctx_tiles, SKIP, std::true_type{}, std::false_type{});
+    const int nf = fast_end(ctx_tiles, ctx_tiles + n1, ctx_tiles + qlen / BN);
+    tile_loop(ctx_tiles, nf, INTERIOR, std::false_type{}, std::true_type{});
+    tile_loop(nf, ctx_tiles + n1, INTERIOR, std::false_type{}, std::false_type{});
+    tile_loop(ctx_tiles + n1, ctx_tiles + n2, MASKED_, std::false_type{}, std::false_type{});
+    tile_loop(ctx_tiles + n2, ntiles, SKIP, std::false_type{}, std::false_type{});
   } else {
     // sliding window: tiles wholly left of every row's window are skipped (64 t + 63 <= w_lo - window), tiles that
     // some row sees only in part (64 t <= w_hi - window) are masked
@@ -639,11 +681,13 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     const int l0 = (window > 0 && w_rows) ? max(w_lo - window + 1, 0) / BN : 0;
     const int l1 = (window > 0 && w_rows && w_hi >= window) ? (w_hi - window) / BN + 1 : 0;
     const int b0 = min(max(l0, t_start), e2), b1 = min(max(l1, b0), e2), b2 = min(max(n1, b1), e2);
-    tile_loop(t_start, b0, SKIP, std::false_type{});
-    tile_loop(b0, b1, MASKED_, std::false_type{});
-    tile_loop(b1, b2, INTERIOR, std::false_type{});
-    tile_loop(b2, e2, MASKED_, std::false_type{});
-    tile_loop(e2, ntiles, SKIP, std::false_type{});
+    const int bf = fast_end(b1, b2, seq_len / BN);
+    tile_loop(t_start, b0, SKIP, std::false_type{}, std::false_type{});
+    tile_loop(b0, b1, MASKED_, std::false_type{}, std::false_type{});
+    tile_loop(b1, bf, INTERIOR, std::false_type{}, std::true_type{});
+    tile_loop(bf, b2, INTERIOR, std::false_type{}, std::false_type{});
+    tile_loop(b2, e2, MASKED_, std::false_type{}, std::false_type{});
+    tile_loop(e2, ntiles, SKIP, std::false_type{}, std::false_type{});
   }
   }   // t0 < t1
 
