@@ -108,7 +108,7 @@ __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];
 // PREFIX = context_attention_fwd (vllm/attention/ops/prefix_prefill.py:36-288, 726-913): the keys are the sequence's
 // cached context -- K [block][kv head][D / x][BS][x] (x = 16 bytes), V [block][kv head][D][BS], every cached token
 // visible -- followed by the new tokens' dense k / v (causal).  Context V is already V^T: its tile is staged as
-// [d][token] (8-byte units XOR-swizzled by d >> 1) and the PV MFMA's A operand is two plain 8-byte reads; the new
+// [d][token] (16-byte units XOR-swizzled by d >> 1) and the PV MFMA's A operand is one plain 16-byte read; the new
 // tokens take the unified path's row-major image and transposing reads.  Dense k / v are never fp8.
 //
 // D_ = 128, NW_ = 8: head sizes 72 .. 128, eight waves = 256 rows, two waves per SIMD.
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   };
   // K image: chunk ^= key & 15 (conflict-free ds_read_b128 of 32 keys x one chunk); V image: chunk ^= (key & 3) << 2
   // (the four keys of a transposing read land in four different 64-byte bank ranges); context V^T image (PREFIX):
-  // rows of 128 bytes = 64 tokens of one d, 8-byte unit ^= (d >> 1) & 15 (32 rows x one unit: every bank once).
+  // rows of 128 bytes = 64 tokens of one d, 16-byte unit ^= (d >> 1) & 7 (16 rows x one unit: every bank once).
   // (the keys of a thread's items are KSTEP apart, a multiple of 16: one pair of swizzled chunk offsets for all)
   uint8_t* k_wr = lds + K_OFF + skey * ROWB;
   uint8_t* v_wr = lds + V_OFF + skey * ROWB;
@@ -370,12 +370,18 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
       write_row(v_wr + vb_ + KSTEP * i * ROWB, vc0, vc1, vst[i], live, whole, conv_c);
     }
   };
+  // Context tiles: LDS row i of K is key i with bits 2 and 3 swapped.  S^T row (r & 3) + 8 (r >> 2) + 4 hi, which lane half hi
+  // holds in register r, is then key 16 (r >> 3) + 8 hi + (r & 7): eight keys in a row per register group, so that a fragment
+  // of V^T is one 16-byte read (two 8-byte ones before: head 128 2 .. 5 %, head 256 5 .. 23 % slower).
+  const int kperm = (skey & ~12) | ((skey & 4) << 1) | ((skey & 8) >> 1);
+  uint8_t* k_wr_ctx = lds + K_OFF + kperm * ROWB;
+  const int kc0_ctx = ((2 * spiece) ^ (kperm & 15)) << 4, kc1_ctx = ((2 * spiece + 1) ^ (kperm & 15)) << 4;
   auto write_ctx = [&](int t, auto whole) __attribute__((always_inline)) {
     const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
-      write_row(k_wr + kb_ + KSTEP * i * ROWB, kc0, kc1, kst[i], t * BN + skey + KSTEP * i < ctx, whole, std::integral_constant<bool, FP8>{});
-      // V^T: the item's 16 tokens of row vd = four 8-byte units
+      write_row(k_wr_ctx + kb_ + KSTEP * i * ROWB, kc0_ctx, kc1_ctx, kst[i], t * BN + skey + KSTEP * i < ctx, whole, std::integral_constant<bool, FP8>{});
+      // V^T: the item's 16 tokens of row vd = two 16-byte units
       const int vd = vd_of(i), vq = vq_of(i);
       const int valid = vd < dr ? ctx - (t * BN + 16 * vq) : 0;
       uint4 lo, hi4;
@@ -392,11 +398,9 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
         }
       }
       uint8_t* row = lds + V_OFF + vb_ + vd * 128;
-      const int f = (vd >> 1) & 15;
-      *reinterpret_cast<u32x2*>(row + (((4 * vq + 0) ^ f) << 3)) = (u32x2){lo.x, lo.y};
-      *reinterpret_cast<u32x2*>(row + (((4 * vq + 1) ^ f) << 3)) = (u32x2){lo.z, lo.w};
-      *reinterpret_cast<u32x2*>(row + (((4 * vq + 2) ^ f) << 3)) = (u32x2){hi4.x, hi4.y};
-      *reinterpret_cast<u32x2*>(row + (((4 * vq + 3) ^ f) << 3)) = (u32x2){hi4.z, hi4.w};
+      const int f = (vd >> 1) & 7;
+      *reinterpret_cast<u32x4*>(row + (((2 * vq + 0) ^ f) << 4)) = (u32x4){lo.x, lo.y, lo.z, lo.w};
+      *reinterpret_cast<u32x4*>(row + (((2 * vq + 1) ^ f) << 4)) = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
     }
   };
   auto write_tile = [&](int t) __attribute__((always_inline)) {
@@ -424,10 +428,10 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   const int k_off0 = K_OFF + l32 * ROWB + ((hi ^ (l32 & 15)) << 4);
   const int v_off0 = V_OFF + (4 * hi + ((lane & 15) >> 2)) * ROWB + ((4 * ((lane & 15) >> 2) + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) << 4) +
                      8 * (lane & 1);
-  // context V^T (PREFIX): row d = 32 db + l32, unit 4 g16 + 2 e + hi = tokens 16 g16 + 8 e + 4 hi .. + 3
-  int vt_o[8];
+  // context V^T (PREFIX): row d = 32 db + l32, unit 2 g16 + hi = tokens 16 g16 + 8 hi .. + 7
+  int vt_o[4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) vt_o[i] = V_OFF + l32 * 128 + (((2 * i + hi) ^ ((l32 >> 1) & 15)) << 3);
+  for (int i = 0; i < 4; ++i) vt_o[i] = V_OFF + l32 * 128 + (((2 * i + hi) ^ ((l32 >> 1) & 7)) << 4);
 
   float m_run = -INFINITY, l_run = 0.f;
   f32x16 o[DB];   // O^T[d = 32 db + (r & 3) + 8 (r >> 2) + 4 hi][this row]
@@ -457,7 +461,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   const float sct = SOFTCAP ? 1.f : sct0;                // (soft-capped scores are rewritten in the log2 domain)
   const int bound0 = VT ? bound_ctx - t * BN : bound_new - (t - ctx_tiles) * BN;
   f32x16 s[2];
-  u32x4 pb[4];   // P^T fragments of key groups 16 g16 ..: slots 0-3 = keys 4 hi + (0..3), 4-7 = 8 + 4 hi + (0..3)
+  u32x4 pb[4];   // P^T fragments of key groups 16 g16 ..: slots 0-3 = keys 4 hi + (0..3), 4-7 = 8 + 4 hi + (0..3) (VT: 8 hi + (0..7))
   u32x4 kf[KR];
   const int kofs = (t & (KN - 1)) * TILE;
   const int vofs = (t & (VN - 1)) * TILE;
@@ -480,11 +484,11 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
         // the accumulator starts at 0, or at -inf where the key is invisible to this row: the mask rides in the
         // MFMA's C operand (K rows past the sequence are staged as zeros, so nothing there is NaN or inf)
         f32x16 z;
-        const int lim = bound0 - 32 * kb - 4 * hi;
+        const int lim = bound0 - 32 * kb - (VT ? 8 : 4) * hi;
         const int lim_lo = window > 0 ? lim - window + 1 : -(1 << 30);   // sliding window: keys (bound - window, bound]
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int c = (r & 3) + 8 * (r >> 2);
+          const int c = VT ? 16 * (r >> 3) + (r & 7) : (r & 3) + 8 * (r >> 2);
           z[r] = (!MASKED || (c <= lim && c >= lim_lo)) ? 0.f : -INFINITY;
         }
         s[kb] = Mma32<T>::mfma(f, qf[0], z);
@@ -503,11 +507,8 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   auto v_read = [&](auto ic, int vofs) __attribute__((always_inline)) {
     constexpr int i = decltype(ic)::value;   // MFMA i -> (key group i / DB, d block i % DB)
     if constexpr (VT) {
-      const int oa = D > 128 ? (vt_o[0] ^ ((2 * (i / DB)) << 4)) : vt_o[2 * (i / DB)];
-      const int ob = D > 128 ? (vt_o[0] ^ ((2 * (i / DB) + 1) << 4)) : vt_o[2 * (i / DB) + 1];
-      const u32x2 va = *reinterpret_cast<const u32x2*>(lds + oa + vofs + 4096 * (i % DB));
-      const u32x2 vb = *reinterpret_cast<const u32x2*>(lds + ob + vofs + 4096 * (i % DB));
-      return (u32x4){va[0], va[1], vb[0], vb[1]};
+      const int oa = D > 128 ? (vt_o[0] ^ ((i / DB) << 5)) : vt_o[i / DB];
+      return *reinterpret_cast<const u32x4*>(lds + oa + vofs + 4096 * (i % DB));
     } else {
       const uint8_t* vp = D > 128 ? lds + ((v_off0 ^ ((i % DB) << 6)) + vofs) : v_rd[i % DB] + vofs;
       const u32x2 va = lds_tr16(vp + (16 * (i / DB)) * ROWB);
@@ -518,7 +519,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   {
     static_for<VR>([&](auto ic) { vf[decltype(ic)::value] = v_read(ic, vofs); });
     __builtin_amdgcn_sched_barrier(0);
-    // lane holds S^T[key = 64 t + 32 kb + (r & 3) + 8 (r >> 2) + 4 hi][this row]
+    // lane holds S^T[key = 64 t + 32 kb + (r & 3) + 8 (r >> 2) + 4 hi][this row] (context tiles: 16 (r >> 3) + 8 hi + (r & 7))
     if constexpr (SOFTCAP) {
       // x = cap2 tanh(y), y = score / softcap, cap2 = softcap log2 e; tanh from one exp2 of -2 |y| and one rcp.  A
       // masked score (-inf) would come out as -cap2: kept at -inf.
