@@ -425,3 +425,44 @@ def test_v1_longest_first_order(ops, oracle, shape, kv):
         torch.cuda.synchronize()
         assert not outs[0].isnan().any(), name
         assert torch.equal(outs[0], outs[1]), name
+
+
+@pytest.mark.parametrize("version", ["v2", "rocm"])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("head_size,max_len", [(64, 1290), (128, 600), (80, 513), (256, 520)])
+def test_one_piece_per_sequence(ops, oracle, version, kv, head_size, max_len):
+    """Short sequences are not cut: one workgroup per (sequence, kv head) writes the output itself.  Lengths on both sides of
+    the partitions, one of 0 (zeros); the result is that of the cut launch up to its rounding of the partial outputs to 16 bits."""
+    from vllm_amd import _lib
+    lens = [max_len, 1, 64, 255, 256, 257, 511, 512] * 4
+    c = make_attn_case(len(lens), 8, 2, head_size, 16, torch.bfloat16, kv, lens, seed=head_size, kv_scale=1.0 if kv == "auto" else 0.5)
+    _lib.set_tuning("pa_sp", 1000)   # (every partition in one piece, whatever the rule says)
+    try:
+        run_case(ops, oracle, c, version)
+    finally:
+        _lib.set_tuning("pa_sp", 0)
+    run_case(ops, oracle, c, version)
+    q, kc, vc, bt = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt"))
+    sl = c["sl"].clone()
+    sl[1] = 0
+    P = -(-max_len // (512 if version == "v2" else 256))
+    es = torch.full((len(lens), 8, P), float("nan"), device="cuda")
+    tmp = torch.full((len(lens), 8, P, head_size), float("nan"), dtype=torch.bfloat16, device="cuda")
+    sc = torch.tensor([c["kv_scale"]], device="cuda")
+    outs = []
+    for sp in (1000, 1):
+        _lib.set_tuning("pa_sp", sp)
+        out = torch.full_like(q, float("nan"))
+        try:
+            if version == "v2":
+                ops.paged_attention_v2(out, es, es.clone(), tmp, q, kc, vc, 2, c["scale"], bt, sl.cuda(), 16, max_len, None, kv, sc, sc)
+            else:
+                ops.paged_attention_rocm(out, es, es.clone(), tmp, q, kc, vc, 2, c["scale"], bt, sl.cuda(), None, 16, max_len, None,
+                                         kv, sc, sc)
+        finally:
+            _lib.set_tuning("pa_sp", 0)
+        assert (out[1] == 0).all()
+        outs.append(out.float())
+    # the cut launch rounds every partial output (|o| <= max |v|) and the merged one to bf16: 2^-8 each
+    bound = 2 * 2.0 ** -8 * outs[0].abs().max()
+    assert (outs[0] - outs[1]).abs().max() <= bound

@@ -158,7 +158,7 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
 
   // ---- LDS: per-wave P tile, then (aliased) the cross-wave merge buffers ------
   constexpr int P_BYTES = 16 * kPRowBytes;                       // 2304
-  constexpr int MERGE_BYTES = NW * HEAD_SIZE * 16 * 4 + NW * 16 * 8;
+  constexpr int MERGE_BYTES = NW * 16 * (HEAD_SIZE + 4) * 4 + NW * 16 * 8;
   constexpr int LDS_BYTES = (NW * P_BYTES > MERGE_BYTES) ? NW * P_BYTES : MERGE_BYTES;
   char* p_tile = lds + wave * P_BYTES;
 
@@ -245,6 +245,8 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
                                             : make_uint4(0, 0, 0, 0);
   };
 
+  // steps with a successor are whole: they need the mask only where the window begins, the bias only with ALiBi
+  const bool masked = alibi_slopes != nullptr || P.first_tok > start_tok;
   // one step of the online-softmax recurrence on the registers of (kreg, vreg);
   // `pf` = the step whose K/V are loaded into the same registers once they are free
   auto do_step = [&](KRegs& kreg, VRegs& vreg, int step, int pf, auto more_c) {
@@ -298,11 +300,13 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
     for (int t = 0; t < TILES; ++t) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int tok = tok0 + 16 * t + 4 * g4 + r;
-        float v = s[t][r] * sc2 + slope2 * (float)(tok - seq_len + 1);
-        v = (unsigned)(tokr0 + 16 * t + 4 * g4 + r) < span ? v : -FLT_MAX;
-        s[t][r] = v;
-        mx = fmaxf(mx, v);
+        s[t][r] *= sc2;
+        if (!more || masked) {
+          const int tok = tok0 + 16 * t + 4 * g4 + r;
+          s[t][r] += slope2 * (float)(tok - seq_len + 1);
+          s[t][r] = (unsigned)(tokr0 + 16 * t + 4 * g4 + r) < span ? s[t][r] : -FLT_MAX;
+        }
+        mx = fmaxf(mx, s[t][r]);
       }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -318,7 +322,7 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float e = fast_exp2(s[t][r] - m_new);
-        e = (unsigned)(tokr0 + 16 * t + 4 * g4 + r) < span ? e : 0.f;
+        if (!more || masked) e = (unsigned)(tokr0 + 16 * t + 4 * g4 + r) < span ? e : 0.f;
         p[r] = e;
         psum += e;
       }
@@ -353,7 +357,7 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
     // tail: zero V of tokens >= end_tok (their P is 0, but stale bytes may be NaN)
     const int vt0 = FP8 ? tok0 + 16 * g4 : tok0 + 8 * g4;   // first token of this lane's V vector
     const int vvalid = end_tok - vt0;                        // may be <= 0 or >= 16
-    const bool tail = tok0 + STEP_TOK > end_tok;             // wave-uniform
+    const bool tail = !more && tok0 + STEP_TOK > end_tok;    // wave-uniform (a step with a successor is whole)
 #pragma unroll
     for (int m = 0; m < DT; ++m) {
       uint4 raw = vreg[m];
@@ -403,22 +407,18 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
   __syncthreads();   // P tiles are dead; LDS becomes the merge buffer
-  float* om = reinterpret_cast<float*>(lds);                         // [NW][HEAD_SIZE][16]
-  float* ml = om + NW * HEAD_SIZE * 16;                               // [NW][16][2]
+  // [NW][16 q heads][HEAD_SIZE + 4]: four consecutive d per 16-byte access, rows 16 bytes further along the banks than a
+  // multiple of them.  (As [NW][HEAD_SIZE][16], 4 bytes at a time, the threads of a row read the same bank: 32-way conflicts
+  // at head 256, 3 us a workgroup.)  Unscaled: the reader has every wave's maximum anyway.
+  constexpr int OM = HEAD_SIZE + 4;
+  float* om = reinterpret_cast<float*>(lds);
+  float* ml = om + NW * 16 * OM;                                      // [NW][16][2]
   if (g4 == 0) {
-    ml[(wave * 16 + c16) * 2 + 0] = m_run;
+    ml[(wave * 16 + c16) * 2 + 0] = m_run;                            // (waves with no step: -FLT_MAX, factor 0 below)
     ml[(wave * 16 + c16) * 2 + 1] = l_run;
   }
-  __syncthreads();
-  float m_tot = -FLT_MAX;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) m_tot = fmaxf(m_tot, ml[(w * 16 + c16) * 2]);
-  const float f_w = fast_exp2(m_run - m_tot);   // waves with no step: m_run = -FLT_MAX -> 0
-#pragma unroll
-  for (int m = 0; m < DT; ++m)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      om[(wave * HEAD_SIZE + 16 * m + 4 * g4 + r) * 16 + c16] = o[m][r] * f_w;
+  for (int m = 0; m < DT; ++m) *reinterpret_cast<f32x4*>(om + (wave * 16 + c16) * OM + 16 * m + 4 * g4) = o[m];
   __syncthreads();
 
   // thread -> (q head qh, 8 consecutive d)
@@ -432,16 +432,15 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
 #pragma unroll
     for (int w = 0; w < NW; ++w) mt = fmaxf(mt, ml[(w * 16 + qh) * 2]);
     float lt = 0.f;
+    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < NW; ++w) lt += ml[(w * 16 + qh) * 2 + 1] * fast_exp2(ml[(w * 16 + qh) * 2] - mt);
-    float acc[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float a = 0.f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) a += om[(w * HEAD_SIZE + d0 + j) * 16 + qh];
-      acc[j] = a;
+    for (int w = 0; w < NW; ++w) {
+      const float f = fast_exp2(ml[(w * 16 + qh) * 2] - mt);
+      lt += ml[(w * 16 + qh) * 2 + 1] * f;
+      lo += *reinterpret_cast<const f32x4*>(om + (w * 16 + qh) * OM + d0) * f;
+      hi += *reinterpret_cast<const f32x4*>(om + (w * 16 + qh) * OM + d0 + 4) * f;
     }
+    const float acc[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     if (P.mode == 2) {
       // unnormalised partial (relative to mt) -> this piece's workspace slot, written through
       float* so = P.slot + qh * HEAD_SIZE + d0;
@@ -556,7 +555,7 @@ __global__ __launch_bounds__(NW * 64, (HEAD_SIZE > 128 ? 1 : 2)) void pa_mfma_ke
                         max_parts, gqa_chunks, slot_stride_arg, dr_arg, bal_ws, bal_ctr, num_seqs, window, order};
   constexpr int STEP_TOK = (FP8 ? 4 : 2) * 16;
   constexpr int P_BYTES = 16 * kPRowBytes;
-  constexpr int MERGE_BYTES = NW * HEAD_SIZE * 16 * 4 + NW * 16 * 8;
+  constexpr int MERGE_BYTES = NW * 16 * (HEAD_SIZE + 4) * 4 + NW * 16 * 8;
   constexpr int LDS_BYTES = (NW * P_BYTES > MERGE_BYTES) ? NW * P_BYTES : MERGE_BYTES;
   __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES + 16];   // + the "last ticket" flag
   const int lane = threadIdx.x & 63;
@@ -598,16 +597,17 @@ __global__ __launch_bounds__(NW * 64, (HEAD_SIZE > 128 ? 1 : 2)) void pa_mfma_ke
     P.seq_len = A.order > 0 ? lpt_len : A.seq_lens[seq];
     const bool partitioned = A.partition_size > 0;
     P.start_tok = partitioned ? part * A.partition_size : 0;
-    if (partitioned && P.start_tok >= P.seq_len) return;
+    const bool direct = A.max_parts == 0;   // one piece per sequence, straight into out: no reduce kernel behind it
+    if (partitioned && !direct && P.start_tok >= P.seq_len) return;
     P.end_tok = partitioned ? min(P.start_tok + A.partition_size, P.seq_len) : P.seq_len;
     if (A.window > 0) {
       // sliding window: pieces in front of it write nothing (the reduce kernel starts at the
       // window's first partition), the piece it starts in begins at the window's step
       P.first_tok = max(0, P.seq_len - A.window);
-      if (partitioned && P.end_tok <= P.first_tok) return;
+      if (partitioned && !direct && P.end_tok <= P.first_tok) return;
       P.start_tok = max(P.start_tok, P.first_tok / STEP_TOK * STEP_TOK);
     }
-    P.mode = partitioned ? 1 : 0;
+    P.mode = partitioned && !direct ? 1 : 0;
     P.part = part;
     PaK<scalar_t> B = A;
     B.slot_stride = slot_stride < 0 ? -slot_stride : slot_stride;
@@ -754,7 +754,9 @@ static int launch_mfma_v(const PagedAttnParams& p) {
   const int sp = part ? p.sp_parts : 1;   // reference partitions per super-partition
   dim3 grid((unsigned)(p.num_seqs * p.num_kv_heads * chunks),
             part ? ceil_div(p.max_num_partitions, sp) : 1);
-  void* out = part ? p.tmp_out : p.out;
+  // one piece per sequence: it writes the output itself
+  const bool direct = part && grid.y == 1 && p.fp8_out_scale == nullptr;
+  void* out = part && !direct ? p.tmp_out : p.out;
   // "pa_group": 0 = heuristic, 1 = always, 2 = never
   const bool group = g_pa_group == 1 || (g_pa_group == 0 && p.num_kv_heads >= 2 && grid.x >= 1024);
   PaK<scalar_t> A;
@@ -766,7 +768,7 @@ static int launch_mfma_v(const PagedAttnParams& p) {
   A.max_num_blocks_per_seq = p.max_num_blocks_per_seq; A.alibi_slopes = p.alibi_slopes;
   A.q_stride = p.q_stride; A.kv_block_bytes = p.kv_block_stride * es;
   A.kv_head_bytes = p.kv_head_stride * es; A.k_scale_p = p.k_scale; A.v_scale_p = p.v_scale;
-  A.partition_size = p.partition_size * sp; A.max_parts = p.max_num_partitions;
+  A.partition_size = p.partition_size * sp; A.max_parts = direct ? 0 : p.max_num_partitions;
   A.gqa_chunks = chunks; A.slot_stride = group ? -sp : sp; A.dr_arg = p.head_size;
   A.bal_ws = nullptr; A.bal_ctr = nullptr; A.num_seqs = p.num_seqs; A.window = p.window;
   // longest-first order (pa_lpt_wg): launches of one piece per sequence (v1, or v2 / rocm when one
@@ -815,7 +817,7 @@ static int launch_mfma_v(const PagedAttnParams& p) {
   hipLaunchKernelGGL((pa_mfma_kernel<scalar_t, FP8, HS, BS, NW, VARIANT, PAD, false>), grid, dim3(NW * 64), 0,
                      p.stream, PA_ARGS(A));
   VA_LAUNCH_CHECK("paged_attention mfma launch");
-  if (part) return paged_attention_reduce(p);
+  if (part && !direct) return paged_attention_reduce(p);
   return VLLM_AMD_OK;
 }
 
@@ -881,6 +883,18 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       const int64_t sp_min = p.partition_size >= 2048 ? 1 : 2048 / p.partition_size;
       sp = sp_fill < sp_min ? sp_fill : sp_min;
       if (sp < sp_bal) sp = sp_bal;
+      // Short sequences: one piece each, which writes the output itself -- no reduce kernel (~4.3 us with the gap in front
+      // of it) -- where that costs less than the longest piece gains.  A workgroup alone takes 3.5 ns + 1 ns per 82 bytes for
+      // a token (us, 1500 tokens: head 64 fp8 7.5, head 128 fp8 9.9, 16-bit 14.6), the chip 1 us per 6.2 MB; the batch is
+      // taken to be 0.6 full.  Up to 10 us only: a long sequence among short ones has to be cut.  Measured, cut -> one piece:
+      // 1 x 600 fp8 10.5 -> 8.7, 1 x 1000 11.6 -> 10.4, 32 x 1000 17.8 -> 13.8, 32 x 1500 23.1 -> 18.7, 16 x 600 16-bit
+      // 14.5 -> 11.1; kept cut: 1 x 1000 16-bit 12.0 (one piece 12.9), 1 x 1500 fp8 11.4 (13.2), head 256 1 x 1000 15.2 (15.8).
+      if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
+        const double tb = 2.0 * p.head_size * (p.kv_dtype == VLLM_AMD_KV_AUTO ? 2 : 1), t = 3.5e-3 + tb * 12.2e-6;
+        const double alone = p.max_seq_len * t, stream = 0.6 * (double)base * p.max_seq_len * tb / 6.2e6;
+        const double one = 1.05 * (alone > stream ? alone : stream), piece = (double)sp * p.partition_size * t;
+        if (alone <= 10.0 && (4.5 + one) * 1.03 < 4.5 + (piece > stream ? piece : stream) + 4.3) sp = P;
+      }
     } else {
       // Enough pairs to fill the chip: few long pieces stream best (256 x 16k tokens: one piece per
       // sequence 81.3 % of peak, sp 16 80.3 %, sp 8 78.5 %, sp 4 76.0 %) and a ragged batch is

@@ -149,7 +149,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
   const float cap_inv = softcap > 0.f ? 1.0f / (kLog2e * softcap) : 0.f, cap2 = softcap * kLog2e;
 
   constexpr int K_LDS = TILES * 16 * D * ES;   // one step of K per wave
-  constexpr int MERGE_BYTES = NW * D * 16 * 4 + NW * 16 * 8;
+  constexpr int MERGE_BYTES = NW * 16 * (D + 4) * 4 + NW * 16 * 8;
   constexpr int LDS_BYTES = NW * K_LDS > MERGE_BYTES ? NW * K_LDS : MERGE_BYTES;
   __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
   char* const k_lds = lds + wave * K_LDS;
@@ -378,22 +378,21 @@ const bool ok = col_ok && d >= dlo && d < dlo + dsub;
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
   __syncthreads();   // the K images are dead; LDS becomes the merge buffer
-  float* om = reinterpret_cast<float*>(lds);   // [NW][D][16]
-  float* ml = om + NW * D * 16;                 // [NW][16][2]
+  // [NW][16 q heads][D + 4], in 16-byte accesses, the rows 16 bytes further along the banks than a multiple of them (as
+  // [NW][D][16] the threads of a row read the same bank).  Unscaled: the reader has every wave's maximum anyway.
+  constexpr int OM = D + 4;
+  float* om = reinterpret_cast<float*>(lds);
+  float* ml = om + NW * 16 * OM;                // [NW][16][2]
   if (g4 == 0) {
-    ml[(wave * 16 + c16) * 2 + 0] = m_run;
+    ml[(wave * 16 + c16) * 2 + 0] = m_run;      // (waves with no step: -FLT_MAX, o = 0)
     ml[(wave * 16 + c16) * 2 + 1] = l_run;
   }
-  __syncthreads();
-  float m_tot = -FLT_MAX;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) m_tot = fmaxf(m_tot, ml[(w * 16 + c16) * 2]);
-  const float f_w = fast_exp2(m_run - m_tot) * vscale;   // waves with no step: m_run = -FLT_MAX, o = 0
   // lane holds O^T[row 4 g4 + r of MFMA j][q head c16] = d = DT (4 g4 + r) + j
 #pragma unroll
-  for (int j = 0; j < DT; ++j)
+  for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) om[(wave * D + DT * (4 * g4 + r) + j) * 16 + c16] = o[j][r] * f_w;
+    for (int j = 0; j < DT; j += 4)
+      *reinterpret_cast<f32x4*>(om + (wave * 16 + c16) * OM + DT * (4 * g4 + r) + j) = (f32x4){o[j][r], o[j + 1][r], o[j + 2][r], o[j + 3][r]};
   __syncthreads();
 
   // thread -> (q head qh, 8 consecutive d); head 256: 32 threads per q head, two passes over the 16 heads
@@ -407,16 +406,15 @@ const bool ok = col_ok && d >= dlo && d < dlo + dsub;
 #pragma unroll
     for (int w = 0; w < NW; ++w) mt = fmaxf(mt, ml[(w * 16 + qh) * 2]);
     float lt = 0.f;
+    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < NW; ++w) lt += ml[(w * 16 + qh) * 2 + 1] * fast_exp2(ml[(w * 16 + qh) * 2] - mt);
-    float acc[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float a = 0.f;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) a += om[(w * D + d0 + j) * 16 + qh];
-      acc[j] = a;
+    for (int w = 0; w < NW; ++w) {
+      const float f = fast_exp2(ml[(w * 16 + qh) * 2] - mt), fv = f * vscale;
+      lt += ml[(w * 16 + qh) * 2 + 1] * f;
+      lo += *reinterpret_cast<const f32x4*>(om + (w * 16 + qh) * OM + d0) * fv;
+      hi += *reinterpret_cast<const f32x4*>(om + (w * 16 + qh) * OM + d0 + 4) * fv;
     }
+    const float acc[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     const int head = head0 + qh;
     if (split) {
       // unnormalised partial (v_scale applied), running max in the log2 domain, sum
