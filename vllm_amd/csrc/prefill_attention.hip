@@ -765,7 +765,8 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 //     35 tokens over 3723, 8 q / 1 kv head 123 -> 32; 512 over 8000, 32 / 8 208 -> 87; 1024 over 4000 139 -> 102; head 64,
 //     300 over 3000 87 -> 33; head 256, 2 x 300 over 3000 159 -> 60; x-layout prefix, 300 over 3000 106 -> 44.
 struct FaPlan { bool use; int nseg; };
-static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap) {
+static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap,
+                      int64_t num_tokens, int num_seqs) {
   const int gqa = num_heads / num_kv_heads;
   const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
   const int tpb = (head_size > 128 ? 128 : 256) / pack;
@@ -780,6 +781,14 @@ static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q,
   if (nseg > by_len) nseg = by_len;
   if (nseg > cap) nseg = cap;
   if (nseg > FA_MAX_SEGMENTS) nseg = FA_MAX_SEGMENTS;
+  // The grid has a row block for every sequence, also for those the decode kernel takes: an empty workgroup costs ~4.5 ns, the
+  // merge ~4 us, and max_k may belong to a decode.  So only where the walk over max_k keys (1.9 us per tile) would shrink by
+  // 2.8 times that overhead.  Whole steps in us, 64-row kernel / split: 300 over 3000 among 63 decodes 137 / 100, among 120
+  // 166 / 135, 256 over 4096 among 255 222 / 180, 8 q / 1 kv head 300 over 2000 among 100 87 / 48; left unsplit: 512 fresh
+  // tokens among 100 decodes of up to 2000 keys 74 / 79, 100 among 63 of 1500 39.4 / 41.0, 213 among 185 of 1056 74 / 112.
+  const int64_t launched = (num_tokens / tpb + num_seqs) * y;
+  if ((int64_t)nseg * launched > 4400) nseg = (int)(4400 / launched);
+  if (nseg > 1 && max_k / PF_BN * 1.9 * (1.0 - 1.0 / nseg) < 2.8 * (4.0 + (double)nseg * (double)launched * 4.5e-3)) nseg = 1;
   if (g_pf_segs > 0) nseg = g_pf_segs < cap ? g_pf_segs : cap;
   if (nseg < 2) return {whole, 1};
   return {true, nseg};
@@ -854,7 +863,8 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     const bool can = p.alibi_slopes == nullptr && p.flat_batch > 0 && p.sm_scale > 0.f &&
                      p.kc_page_bytes < (1 << 27) && p.vc_page_bytes < (1 << 27);
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
-    const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments);
+    const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
+                                num_tokens, batch);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -933,7 +943,7 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
                      (block_size & (block_size - 1)) == 0 && p.k_stride_t < (1 << 27) && p.v_stride_t < (1 << 27);
     const int64_t ptok = p.flat_batch > 0 ? (int64_t)p.flat_tokens : (int64_t)max_input_len * batch;
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
-                                p.flat_batch > 0 ? p.num_segments : 1);
+                                p.flat_batch > 0 ? p.num_segments : 1, ptok, batch);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -1259,7 +1269,8 @@ extern "C" int vllm_amd_context_attention_fwd_segments(int batch, int num_heads,
                                                        int max_seq_len, int num_tokens, int has_alibi, int sliding_window,
                                                        int skip_decode) {
   if (batch <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || num_tokens <= 0 || has_alibi || sliding_window > 0) return 1;
-  return fa_plan(head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch, FA_MAX_SEGMENTS).nseg;
+  return fa_plan(head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch, FA_MAX_SEGMENTS,
+                 num_tokens, batch).nseg;
 }
 
 extern "C" int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, int num_kv_heads, int head_size, int max_seqlen_q,
@@ -1271,7 +1282,7 @@ extern "C" int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, 
   if (has_alibi) return 1;
   const bool mixed = num_seqs >= 16 && (int64_t)num_tokens < (int64_t)num_seqs * max_seqlen_q;   // (launch_unified)
   return fa_plan(head_size, num_heads, num_kv_heads, max_seqlen_q, max_seqlen_k, mixed ? num_tokens - num_seqs : num_tokens,
-                 mixed ? 1 : num_seqs, FA_MAX_SEGMENTS).nseg;
+                 mixed ? 1 : num_seqs, FA_MAX_SEGMENTS, num_tokens, num_seqs).nseg;
 }
 
 // unified_attention (vllm/attention/ops/triton_unified_attention.py:588-700): q over the new

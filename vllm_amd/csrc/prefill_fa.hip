@@ -90,6 +90,20 @@ __device__ __forceinline__ u32x2 lds_tr16(const uint8_t* p) {
   return __builtin_bit_cast(u32x2, v);
 }
 
+// The last i of [0, n) for which le(i) holds (it holds for 0, and for all i up to that one): 64 candidates per step, so that
+// 64 sequences take one load and 4096 two, where a binary search chains 6 and 12.
+template <typename F>
+__device__ __forceinline__ int wave_last(int n, int lane, F&& le) {
+  int lo = 0;
+  while (n > 1) {
+    const int step = (n + 63) >> 6, i = lane * step;
+    const int c = __popcll(__ballot(i < n && le(lo + (i < n ? i : 0)))) - 1;
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
 // -DVA_PROBES (tools/fa_stamps.py): shader-clock time per wave spent in each part of the tile loop, summed over
 // the wave's tiles: 0 K ring fill + staging (LDS writes of tile t + 1, loads of t + 2), 2 S^T, 4 softmax + PV,
 // 5 barrier, 6 tiles computed, 7 whole kernel
@@ -165,12 +179,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   if (p.blocks_per_seq > 0) {
     seq = g / p.blocks_per_seq;
   } else {
-    int lo = 0, hi2 = p.num_seqs;
-    while (hi2 - lo > 1) {
-      const int mid = (lo + hi2) >> 1;
-      if (p.cu_seqlens_q[mid] / tpb + mid <= g) lo = mid; else hi2 = mid;
-    }
-    seq = lo;
+    seq = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] / tpb + i <= g; });
   }
   const int tok0 = p.cu_seqlens_q[seq];
   const int qlen = p.cu_seqlens_q[seq + 1] - tok0;
@@ -756,11 +765,7 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
   const int tok = pair / p.num_heads, head = pair % p.num_heads;
   if (tok >= p.num_tokens || tok >= p.cu_seqlens_q[p.num_seqs]) return;
   if (p.skip_decode) {
-    int lo = 0, hi = p.num_seqs;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (p.cu_seqlens_q[mid] <= tok) lo = mid; else hi = mid;
-    }
+    const int lo = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] <= tok; });
     if (p.cu_seqlens_q[lo + 1] - p.cu_seqlens_q[lo] == 1) return;   // the decode kernel's token
   }
   const int nseg = p.num_segments, dr = p.head_size;
