@@ -1,6 +1,6 @@
 // How fast does the chip get through workgroups that exit at once?  (Partitioned decode launches
 // of ragged batches hold many: grid = sequences x max partitions.)
-// hipcc --offload-arch=gfx950 -O3 tools/empty_wg_bench.hip -o tools/empty_wg_bench
+// hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/empty_wg_bench.hip -o tools/empty_wg_bench
 // Measured (MI355X): 16384 workgroups 4.6 us per launch = 0.3 ns each, 65536: 15 us = 0.2 ns each
 // (plain or with 32 KB of LDS and 2 workgroups per CU): the ~6000 empty workgroups of a ragged
 // 256 x U[2k, 16k] v2 launch cost about 1.5 us, not the 60 us that launch lacks against a uniform batch.

@@ -4,7 +4,7 @@
 // a barrier per 64 KiB block and therefore measures issue + latency, not the rate of the path.
 // 256 workgroups (one per CU: 128 KiB of LDS each), NW waves; every workgroup walks the K blocks of
 // "its" 256 A rows and 256 W rows of a 4096 x K fp8 operand pair, XCD-grouped like the GEMM's tiles.
-// build: hipcc --offload-arch=gfx950 -O3 tools/fillrate.hip -o tools/fillrate
+// build: hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/fillrate.hip -o tools/fillrate
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>

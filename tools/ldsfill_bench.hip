@@ -2,7 +2,7 @@
 // (global_load_dwordx4 + ds_write_b128) and a half / half mix.  256 workgroups x 512 threads, one
 // per CU; every workgroup streams the GEMM's fill pattern (8 rows x 128 B per wave-instruction,
 // rows 4096 B apart) from a 16 MiB operand that stays in L2 / MALL, into a 128 KiB LDS ring.
-// build: hipcc --offload-arch=gfx950 -O3 tools/ldsfill_bench.hip -o tools/ldsfill_bench
+// build: hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/ldsfill_bench.hip -o tools/ldsfill_bench
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>

@@ -1,7 +1,7 @@
 // Streaming-read rate of 16-byte global loads by cache policy bits (gfx950): plain, nt, sc1, sc0 sc1, sc1 nt,
 // sc0 sc1 nt.  512 workgroups x 256 threads (two per CU, like the decode kernel), 8 loads in flight per lane,
 // two 512 MiB buffers alternated (no Infinity-Cache reuse), steady state (each policy runs ~40 ms first).
-// hipcc --offload-arch=gfx950 -O3 tools/loadpolicy_bench.hip -o tools/loadpolicy_bench
+// hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/loadpolicy_bench.hip -o tools/loadpolicy_bench
 // Measured (MI355X, 512 workgroups): plain 6.21, nt 6.89, sc1 6.20, sc0 sc1 6.19, sc1 nt 6.88, sc0 sc1 nt 6.85, sc0 nt 6.87 TB/s
 // (768 / 2048 workgroups: the same picture, 6.1 vs 6.7-6.9): only the nt bit matters; ~6.9 TB/s = 86 % of the 8 TB/s
 // spec is the streaming-read ceiling, and the decode kernel's steady 6.55 TB/s is 95 % of it.

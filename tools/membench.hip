@@ -1,7 +1,7 @@
 // HBM read ceiling for the paged-attention access pattern (tools only, not in the library).
 //   mode 0: linear streaming read, 16 B/lane
 //   mode 1: random 2 KiB pages (fp8 KV page of one (block, head)), two streams (K and V)
-// build: hipcc --offload-arch=gfx950 -O3 tools/membench.hip -o tools/membench
+// build: hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/membench.hip -o tools/membench
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>

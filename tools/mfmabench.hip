@@ -1,5 +1,5 @@
 // MFMA issue-rate ceiling for v_mfma_scale_f32_16x16x128_f8f6f4 (fp8 operands, unit scales):
-//   hipcc --offload-arch=gfx950 -O3 tools/mfmabench.hip -o tools/mfmabench && tools/mfmabench
+//   hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/mfmabench.hip -o tools/mfmabench && tools/mfmabench
 // 256*k workgroups of W waves, each wave loops over NACC independent accumulators; operands
 // are random bytes (zero operands read high: the chip clocks up).
 #include <hip/hip_runtime.h>

@@ -1,7 +1,7 @@
 // MFMA shape A/B under the power limit: v_mfma_scale_f32_16x16x128_f8f6f4 against v_mfma_scale_f32_32x32x64_f8f6f4
 // (fp8 operands, unit scales; same FLOP per cycle on paper), random operands, 128 accumulator registers per lane,
 // one or two waves per SIMD, ~10 ms per launch, in-kernel clock from s_memtime / s_memrealtime.
-//   hipcc --offload-arch=gfx950 -O3 tools/mfmabench2.hip -o tools/mfmabench2 && tools/mfmabench2
+//   hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 tools/mfmabench2.hip -o tools/mfmabench2 && tools/mfmabench2
 #include <hip/hip_runtime.h>
 #include <cstdio>
 #include <cstdlib>

@@ -2,7 +2,7 @@
 // Compiles the library's own kernel source with -DVA_PROBES: per-workgroup s_memrealtime stamps
 // (entry, first K data consumed, loop end, exit) and two ablations (loads only; no merge), on
 // the configs[1] shape (64 seqs x 4096 tokens, 32q/8kv, fp8, block 16) or any S / ctx / KVH.
-// build: hipcc --offload-arch=gfx950 -O3 -std=c++17 -DVA_PROBES -DNDEBUG tools/pa_probe.hip \
+// build: hipcc --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops -O3 -std=c++17 -DVA_PROBES -DNDEBUG tools/pa_probe.hip \
 //        vllm_amd/csrc/common.hip -o tools/pa_probe
 #include "../vllm_amd/csrc/paged_attention_mfma.hip"
 

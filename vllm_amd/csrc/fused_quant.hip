@@ -1,4 +1,4 @@
-// The ops either side of the fp8 GEMM and of the cache write (SURVEY.md 8f):
+// The ops either side of the fp8 GEMM and of the cache write:
 //   rms_norm_static_fp8_quant, fused_add_rms_norm_static_fp8_quant   (layernorm_quant_kernels.cu)
 //   rms_norm_dynamic_per_token_quant                                 (fused_layernorm_dynamic_per_token_quant.cu)
 //   silu_and_mul_quant                                               (activation_kernels.cu)

@@ -36,7 +36,7 @@
 
 namespace va {
 
-constexpr int kDefaultVariant = 1;   // set from measurements, see DESIGN.md
+constexpr int kDefaultVariant = 1;   // set from measurements
 
 // tools/pa_probe.hip compiles this file with -DVA_PROBES: per-workgroup time stamps (100 MHz
 // s_memrealtime) and two ablations (VARIANT bit 2 = loads only, bit 3 = no cross-wave merge).

@@ -1,4 +1,4 @@
-// Prefill / chunked-prefill attention with a paged prefix (SURVEY.md 8f-4): the MFMA-bound
+// Prefill / chunked-prefill attention with a paged prefix: the MFMA-bound
 // sibling of the decode kernel.  Replaces context_attention_fwd
 // (vllm/attention/ops/prefix_prefill.py:726-913; Triton kernels _fwd_kernel :36-288 and
 // _fwd_kernel_alibi :477-722): every query token of a sequence attends to

@@ -1,7 +1,7 @@
 // unified_attention (vllm/attention/ops/triton_unified_attention.py:52-272, 588-700) and context_attention_fwd
 // (vllm/attention/ops/prefix_prefill.py:36-288, 726-913; the PREFIX instantiation below) for LONG query chunks at head
 // sizes 72 .. 128 with the causal + padding mask (unified: + sliding window): the matrix-core-bound case of prefill_attention.hip,
-// re-built around what bounds that kernel (DESIGN.md 3.7: 16 query rows per wave = one LDS fragment byte per
+// re-built around what bounds that kernel (16 query rows per wave = one LDS fragment byte per
 // 32 flops and ~300 VALU per 32 MFMAs; a 64-row tile restages every K / V tile for 64 rows).
 //
 //   * a workgroup = 8 waves = 256 tile rows; a wave owns 32 rows and computes with v_mfma_f32_32x32x16:

@@ -332,7 +332,7 @@ void wvSplitKQ(const Tensor& in_a, const Tensor& in_b, Tensor& out_c, const Tens
                            stream_of(in_a)));
 }
 
-// ---- fused neighbours -------------------------------------------------------
+// ---- fused neighbours -------------------------------------------------------------------------
 // csrc/layernorm_quant_kernels.cu:172-198
 void rms_norm_static_fp8_quant(Tensor& result, const Tensor& input, const Tensor& weight, const Tensor& scale,
                                double epsilon) {

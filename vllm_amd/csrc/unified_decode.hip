@@ -86,7 +86,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
   }
   // GQA groups of more than 16 q heads (MQA models) take ceil(G / 16) workgroups per kv head,
   // chunk fastest: the chunks re-read the same K / V, through L2 when they run together
-  // hp > 1 (round 3, token-major caches): hp ADJACENT kv heads are taken as one row of hp * head_size elements -- one
+  // hp > 1 (token-major caches): hp ADJACENT kv heads are taken as one row of hp * head_size elements -- one
   // load instruction then fetches 256 contiguous bytes per token instead of 128 (or 64): pieces below 256 bytes cost
   // 10 (128 B) to 40 % (64 B) of the bandwidth, 256-byte pieces nothing (tools/bench_uni_decode_d.py).  The q heads of
   // the hp groups are the columns of ONE Q^T operand, each zero outside its own head's d range, so S^T, the per-column
