@@ -175,18 +175,44 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // grid.x enumerates the row blocks of ALL sequences (num_tokens / tpb + num_seqs is an upper bound); the
   // sequence is the last one whose first block cu[i] / tpb + i is <= g (find_seq_idx, :33-48)
   // (blocks_per_seq > 0: the caller did not say how many query tokens there are; every sequence gets that many blocks)
-  int seq = 0;
+  int seq = 0, blk = -1;   // sequence, row block in it
   if (p.blocks_per_seq > 0) {
     seq = g / p.blocks_per_seq;
-  } else {
+    blk = g % p.blocks_per_seq;
+  } else if (PREFIX && p.num_seqs > 1 && p.num_seqs <= 64 && nseg == 1 && gridDim.y % 8 == 0) {
+    // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD: the row blocks of the
+    // longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24 chunks of
+    // 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us; 19 prompts of 745 .. 1242 without
+    // context, whose blocks differ more than the prompts, 294 -> 302: they keep the order below).
+    int len = -1, nb = 0, before = 0;   // lane i: sequence i, its blocks, the blocks in front of them
+    bool over = false;
+    if (lane < p.num_seqs) {
+      const int ql = p.cu_seqlens_q[lane + 1] - p.cu_seqlens_q[lane];
+      len = p.seq_lens[lane];
+      nb = p.skip_decode && ql == 1 ? 0 : (ql + tpb - 1) / tpb;
+      over = len >= 3 * ql;
+    }
+    if (2 * __popcll(__ballot(nb > 0 && over)) >= __popcll(__ballot(nb > 0))) {
+      for (int j = 0; j < p.num_seqs; ++j) {
+        const int lj = __builtin_amdgcn_readlane(len, j), nj = __builtin_amdgcn_readlane(nb, j);
+        before += (lj > len || (lj == len && j < lane)) ? nj : 0;
+      }
+      const unsigned long long mine = __ballot(before <= gs && gs < before + nb);
+      if (mine == 0) return;            // the grid is an upper bound
+      seq = __builtin_amdgcn_readfirstlane(__ffsll((long long)mine) - 1);
+      blk = __builtin_amdgcn_readlane(nb, seq) - 1 - (gs - __builtin_amdgcn_readlane(before, seq));
+    }
+  }
+  if (blk < 0) {
     seq = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] / tpb + i <= g; });
+    blk = g - (p.cu_seqlens_q[seq] / tpb + seq);
   }
   const int tok0 = p.cu_seqlens_q[seq];
   const int qlen = p.cu_seqlens_q[seq + 1] - tok0;
   const int seq_len = p.seq_lens[seq];
   const int ctx = seq_len - qlen;
   // first query token of this block
-  const int tok_base = (p.blocks_per_seq > 0 ? g % p.blocks_per_seq : g - (tok0 / tpb + seq)) * tpb;
+  const int tok_base = blk * tpb;
   if (tok_base >= qlen) return;
   if (p.skip_decode && qlen == 1) return;
   const int new_end = min(tok_base + tpb, qlen);
@@ -670,7 +696,8 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // interior tiles whose staging has nothing to check (stage()) run in loops of their own: [begin, fast_end), the tiles t with
   // t + 2 below `wholes`, the end of the whole tiles of the domain
   auto fast_end = [&](int begin, int end, int wholes) __attribute__((always_inline)) {
-    return dr == D ? max(min(min(wholes, t1) - 2, end), begin) : begin;
+    const int e = min(min(wholes, t1) - 2, end);
+    return dr == D && e - max(begin, t0) >= 4 ? e : begin;   // (fewer tiles do not pay for another cold copy of the loop)
   };
   if constexpr (PREFIX) {
     // context: whole tiles are interior, the last one (ctx % 64 tokens) is masked
