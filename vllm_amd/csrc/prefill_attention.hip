@@ -757,7 +757,11 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 // Whether a launch of query chunks takes the 256-row kernel (prefill_fa.hip; 128 rows above head size 128), and into how
 // many key segments it is split.  max_k: longest key range (an upper bound will do), ptok: query tokens of the chunks,
 // nchunk: sequences among them (a lower bound will do), cap: segments the caller has scratch for.
-//   * >= 128 row blocks, chunks of at least one: unsplit.
+//   * >= 128 row blocks, chunks of at least one: unsplit.  Without decodes beside the chunks from 64 on, over the
+//     flash-layout fp8 cache at head sizes up to 128 from 96 on and from 512 keys (min_blocks).  us, 64-row kernel -> this one: x-layout fp8 1000 tokens, 32 / 8
+//     heads (120 blocks) 40.7 -> 33.0, 600 over 200 (72) 35.9 -> 31.4, head 256 900 tokens (112) 90.8 -> 46.1; flash layout 16-bit
+//     800 (96) 34.3 -> 28.5, head 256 600 over 300 (72) 76.0 -> 44.7; fp8 1000 (120) 36.6 -> 33.5, but 400 + 300
+//     over 100 (80) 20.5 -> 23.0 and 64 / 8 heads 180 + 300 (120) 16.2 -> 18.8.
 //   * fewer: the 64-row kernel's four times as many workgroups finished sooner than that (chunk 256 over 4096 cached tokens
 //     among 255 decodes: 32 blocks, 82 against 150 us) and still left the chip idle behind one serial walk over the keys
 //     (2.1 us per 64-key tile).  Split, the blocks give at least 256 workgroups; a segment is worth its start-up from three
@@ -766,13 +770,13 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 //     300 over 3000 87 -> 33; head 256, 2 x 300 over 3000 159 -> 60; x-layout prefix, 300 over 3000 106 -> 44.
 struct FaPlan { bool use; int nseg; };
 static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap,
-                      int64_t num_tokens, int num_seqs) {
+                      int64_t num_tokens, int num_seqs, int min_blocks = 128) {
   const int gqa = num_heads / num_kv_heads;
   const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
   const int tpb = (head_size > 128 ? 128 : 256) / pack;
   const int y = pack > 1 ? num_kv_heads : num_heads;
   if (g_pf_fa == 1 || g_pf_rows != 0 || (max_q <= 1 && g_pf_fa != 2) || head_size > 256) return {false, 1};
-  const bool whole = head_size > 64 && (g_pf_fa == 2 || (max_q >= tpb && ptok / tpb * y >= 128));
+  const bool whole = head_size > 64 && (g_pf_fa == 2 || (max_q >= tpb && ptok / tpb * y >= min_blocks));
   int64_t blocks = (ptok + tpb - 1) / tpb;
   if (blocks < nchunk) blocks = nchunk;
   blocks *= y;
@@ -864,7 +868,8 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
                      p.kc_page_bytes < (1 << 27) && p.vc_page_bytes < (1 << 27);
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
-                                num_tokens, batch);
+                                num_tokens, batch,
+                                mixed ? 128 : (!FP8 || head_size > 128) ? 64 : max_k >= 512 ? 96 : 128);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -943,7 +948,7 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
                      (block_size & (block_size - 1)) == 0 && p.k_stride_t < (1 << 27) && p.v_stride_t < (1 << 27);
     const int64_t ptok = p.flat_batch > 0 ? (int64_t)p.flat_tokens : (int64_t)max_input_len * batch;
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
-                                p.flat_batch > 0 ? p.num_segments : 1, ptok, batch);
+                                p.flat_batch > 0 ? p.num_segments : 1, ptok, batch, p.skip_decode ? 128 : 64);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
