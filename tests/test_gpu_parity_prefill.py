@@ -348,3 +348,24 @@ def test_prefill_key_segments(oracle, tuning, segs, kv, head_size, gqa):
     ref = (out.float() / 0.01).clamp(-448, 448).to(torch.float8_e4m3fn).float()
     # the partial sums are the same; out is rounded to 16 bits before the division here: one code apart
     assert ((o8.view(torch.float8_e4m3fn).float() - ref).abs() <= 0.13 * ref.abs() + 2 ** -9).all()
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("head_size", [128, 256])
+def test_prefill_key_segments_nan(tuning, kv, head_size):
+    """A NaN query, and NaN keys in live context slots (a whole tile: the first of a segment, for some of the segment counts),
+    make exactly the rows NaN that see them -- split over the keys as unsplit."""
+    c = make_prefill_case([70, 33, 90], [500, 130, 200], 8, 2, head_size, 16, torch.bfloat16, kv, seed=head_size, kv_scale=0.02)
+    bad = torch.zeros(c["q"].shape[:2], dtype=torch.bool)
+    c["q"][40, 5] = float("nan")
+    bad[40, 5] = True
+    for n in range(128, 192):   # the third sequence's third tile, kv head 1
+        c["k_cache"][int(c["b_loc"][2, n // 16]), 1, :, n % 16] = 0x7f if kv == "fp8" else float("nan")
+    bad[103:, 4:] = True
+    ref = prefill_reference(c)
+    tuning("pf_fa", 2)
+    for segs in (1, 2, 3, 5, 32):
+        tuning("pf_segs", segs)
+        out = run(c, kv)
+        assert torch.equal(out.isnan().any(-1), bad) and torch.equal(out.isnan().all(-1), bad), segs
+        torch.testing.assert_close(out.float()[~bad], ref[~bad], atol=tol(torch.bfloat16), rtol=0)

@@ -534,3 +534,38 @@ def test_unified_prefill_key_segments(oracle, segs, num_heads, head_size, mode):
             out_scale=torch.tensor([0.02]) if mode == "fp8_out" else None, fp8=fp8)
     finally:
         _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D", [128, 256])
+def test_unified_prefill_key_segments_nan(oracle, D, fp8):
+    """A NaN query, and NaN keys that a whole sequence sees (a whole tile: the first of a segment, for some of the segment
+    counts), make exactly the rows NaN that see them -- split over the keys as unsplit."""
+    from vllm_amd import _lib
+    from vllm_amd.attention.ops import unified_attention
+    c = make_unified_case([(70, 700), (33, 97), (90, 350)], 8, 2, D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
+    kd = c["scale"] if fp8 else None
+    ref = torch.zeros_like(c["q"])
+    oracle.unified_attention(c["q"], c["k"], c["v"], ref, c["cu_seqlens_q"], c["max_seqlen_q"], c["seqused_k"],
+                             c["max_seqlen_k"], D ** -0.5, True, (-1, -1), c["block_table"], 0.0, None, kd, kd, None, None)
+    bad = torch.zeros(c["q"].shape[:2], dtype=torch.bool)
+    c["q"][40, 5] = float("nan")
+    bad[40, 5] = True
+    for n in range(128, 192):   # the third sequence's third tile, kv head 1
+        c["k"][int(c["block_table"][2, n // 16]), n % 16, 1] = 0x7f if fp8 else float("nan")
+    bad[103:, 4:] = True
+    d = {k: v.cuda() for k, v in c.items() if torch.is_tensor(v)}
+    kd = d["scale"] if fp8 else None
+    _lib.set_tuning("pf_fa", 2)
+    try:
+        for segs in (1, 2, 3, 5, 32):
+            _lib.set_tuning("pf_segs", segs)
+            out = torch.zeros_like(d["q"])
+            unified_attention(d["q"], d["k"], d["v"], out, d["cu_seqlens_q"], c["max_seqlen_q"], d["seqused_k"], c["max_seqlen_k"], D ** -0.5,
+                              True, (-1, -1), d["block_table"], 0.0, None, kd, kd)
+            out = out.cpu()
+            assert torch.equal(out.isnan().any(-1), bad) and torch.equal(out.isnan().all(-1), bad), segs
+            torch.testing.assert_close(out.float()[~bad], ref.float()[~bad], atol=ATOL, rtol=RTOL)
+    finally:
+        _lib.set_tuning("pf_segs", 0)
+        _lib.set_tuning("pf_fa", 0)

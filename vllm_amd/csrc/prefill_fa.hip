@@ -830,7 +830,8 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
     acc.w += __shfl_xor(acc.w, 32, 64);
   }
   if (sub != 0 || d >= dr) return;
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  // (a row of NaN scores never raises its maximum from -inf: weight 0, but its sum is NaN, and so is the row, as unsplit)
+  const float inv = l == 0.f ? 0.f : 1.0f / l;
   const int64_t oi = (int64_t)tok * p.o_stride_t + (int64_t)head * p.o_stride_h + d;
   if (p.out_scale == nullptr) {
     *reinterpret_cast<u32x2*>((T*)p.o + oi) = (u32x2){Mma<T>::pack2(acc.x * inv, acc.y * inv), Mma<T>::pack2(acc.z * inv, acc.w * inv)};
