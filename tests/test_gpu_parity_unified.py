@@ -569,3 +569,23 @@ def test_unified_prefill_key_segments_nan(oracle, D, fp8):
     finally:
         _lib.set_tuning("pf_segs", 0)
         _lib.set_tuning("pf_fa", 0)
+
+
+@pytest.mark.parametrize("D", [32, 80, 120, 192, 256])
+@pytest.mark.parametrize("nseq", [5, 260])
+@pytest.mark.parametrize("window", [None, 100])
+def test_unified_decode_keys_of_minus_infinity(oracle, D, nseq, window):
+    """A key whose score is -inf has probability 0: the columns that pad the head size inside the decode kernel must not
+    make a NaN of it (0 * inf).  Split and unsplit launches, one kv head per row ("uni_hp" = 1)."""
+    from vllm_amd import _lib
+    lens = [33, 64, 130, 500]
+    c = make_unified_case([(1, lens[i % 4] + i // 4) for i in range(nseq)], 8, 2, D, 16, torch.bfloat16, seed=D + nseq)
+    c["q"][..., 3] = c["q"][..., 3].abs() + 0.5
+    for i, n in enumerate(c["seqused_k"].tolist()):
+        for t in {n // 2, n - 1, 5}:
+            c["k"][int(c["block_table"][i, t // 16]), t % 16, :, 3] = float("-inf")
+    _lib.set_tuning("uni_hp", 1)
+    try:
+        run(oracle, c, torch.bfloat16, window=window)
+    finally:
+        _lib.set_tuning("uni_hp", 0)

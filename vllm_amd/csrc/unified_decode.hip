@@ -165,7 +165,7 @@ __global__ __launch_bounds__(NW * 64, ((D > 128 && !FP8) ? 1 : 2)) void ua_decod
       int d;
       if constexpr (FP8) d = 16 * (g4 + 4 * (s >> 1)) + 8 * (s & 1);
       else d = 8 * (g4 + 4 * s);
-const bool ok = col_ok && d >= dlo && d < dlo + dsub;
+      const bool ok = col_ok && d >= dlo && d < dlo + dsub;
       const uint4 v = *reinterpret_cast<const uint4*>(qp + (ok ? d : dlo));
       qf[s] = ok ? v : make_uint4(0, 0, 0, 0);
     }
@@ -187,15 +187,19 @@ const bool ok = col_ok && d >= dlo && d < dlo + dsub;
   // (lane order = [row][position]) is read back conflict-free in the MFMA order
   constexpr int RB = D * ES, CPR = RB / 16, RPI = 64 / CPR;   // row bytes, chunks per row, rows per instruction
   auto kswz = [](int row) { return (row * CPR / 16) & (CPR - 1); };
-  // (head sizes below the padded D: a lane whose chunk does not exist fetches the row's first one -- its Q^T rows are zero,
-  // and a V column past the head is never stored.  No load sits behind a branch: the compiler then counts the loads in
-  // flight and waits for K alone where K is needed, instead of for everything)
+  // (head sizes below the padded D: a lane whose chunk does not exist fetches the row's first one; K is zeroed in front of the
+  // LDS image -- its Q^T rows are zero, but 0 * inf is NaN -- and a V column past the head is never stored.  No load sits
+  // behind a branch: the compiler then counts the loads in flight and waits for K alone where K is needed, instead of for
+  // everything)
+  const bool padded = dr < D;
+  bool kval[KL];
   uint32_t koff[KL], krd[KL];
 #pragma unroll
   for (int i = 0; i < KL; ++i) {
     const int row = i * RPI + lane / CPR;
     const int chunk = (lane % CPR) ^ kswz(row);
-    koff[i] = (uint32_t)(row * p.kc_slot_bytes + (chunk * 16 < dr * ES ? chunk << 4 : 0));
+    kval[i] = chunk * 16 < dr * ES;
+    koff[i] = (uint32_t)(row * p.kc_slot_bytes + (kval[i] ? chunk << 4 : 0));
     krd[i] = (uint32_t)(c16 * RB + (((g4 + 4 * i) ^ kswz(c16)) << 4));
   }
   uint32_t voff[4];   // row r of the lane's four tokens of a tile
@@ -251,6 +255,10 @@ const bool ok = col_ok && d >= dlo && d < dlo + dsub;
     const int tok0 = start_tok + step * STEP_TOK;
     const int pf = step + NW;
     // ---------------- K: registers -> wave-private LDS image -> MFMA order ----------------
+    if (padded) {
+#pragma unroll
+      for (int n = 0; n < TILES * KL; ++n) kreg[n] = kval[n % KL] ? kreg[n] : (u32x4)(0);
+    }
 #pragma unroll
     for (int n = 0; n < TILES * KL; ++n)
       *reinterpret_cast<u32x4*>(k_lds + n * 1024 + lane * 16) = kreg[n];
