@@ -369,3 +369,23 @@ def test_prefill_key_segments_nan(tuning, kv, head_size):
         out = run(c, kv)
         assert torch.equal(out.isnan().any(-1), bad) and torch.equal(out.isnan().all(-1), bad), segs
         torch.testing.assert_close(out.float()[~bad], ref[~bad], atol=tol(torch.bfloat16), rtol=0)
+
+
+@pytest.mark.parametrize("kernel", ["64 rows", "256 rows", "split"])
+@pytest.mark.parametrize("skip_decode", [False, True])
+def test_prefill_rows_in_front_of_the_first_sequence(tuning, kernel, skip_decode):
+    """b_start_loc that starts above 0 (the last sequences of a longer batch): the others' rows are left alone."""
+    c = make_prefill_case([300, 70, 1, 90], [40, 500, 77, 200], 8, 2, 128, 16, torch.bfloat16, "auto", seed=3)
+    ref = prefill_reference(c)
+    tuning("pf_fa", 1 if kernel == "64 rows" else 2)
+    tuning("pf_segs", 3 if kernel == "split" else 0)
+    for first in (1, 3):
+        d = dict(c, b_loc=c["b_loc"][first:], b_start_loc=c["b_start_loc"][first:], b_seq_len=c["b_seq_len"][first:])
+        out = run(d, "auto", skip_decode=skip_decode)
+        at = c["b_start_loc"].tolist()
+        assert float(out[:at[first]].abs().max()) == 0.0
+        for i in range(first, 4):
+            if skip_decode and c["query_lens"][i] == 1:
+                assert float(out[at[i]:at[i + 1]].abs().max()) == 0.0
+            else:
+                torch.testing.assert_close(out[at[i]:at[i + 1]].float(), ref[at[i]:at[i + 1]], atol=tol(torch.bfloat16), rtol=0)

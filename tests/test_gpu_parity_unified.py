@@ -589,3 +589,28 @@ def test_unified_decode_keys_of_minus_infinity(oracle, D, nseq, window):
         run(oracle, c, torch.bfloat16, window=window)
     finally:
         _lib.set_tuning("uni_hp", 0)
+
+
+@pytest.mark.parametrize("kernel", ["64 rows", "256 rows", "split"])
+def test_unified_rows_in_front_of_the_first_sequence(oracle, kernel):
+    """cu_seqlens_q that starts above 0 (the last sequences of a longer batch): the others' rows are left alone."""
+    from vllm_amd import _lib
+    from vllm_amd.attention.ops import unified_attention
+    c = make_unified_case([(300, 340), (70, 570), (1, 78), (90, 290)], 8, 2, 128, 16, torch.bfloat16, seed=3)
+    ref = torch.zeros_like(c["q"])
+    oracle.unified_attention(c["q"], c["k"], c["v"], ref, c["cu_seqlens_q"], c["max_seqlen_q"], c["seqused_k"],
+                             c["max_seqlen_k"], 128 ** -0.5, True, (-1, -1), c["block_table"], 0.0, None, None, None, None, None)
+    d = {k: v.cuda() for k, v in c.items() if torch.is_tensor(v)}
+    _lib.set_tuning("pf_fa", 1 if kernel == "64 rows" else 2)
+    _lib.set_tuning("pf_segs", 3 if kernel == "split" else 0)
+    try:
+        for first in (1, 3):
+            out = torch.zeros_like(d["q"])
+            unified_attention(d["q"], d["k"], d["v"], out, d["cu_seqlens_q"][first:], c["max_seqlen_q"], d["seqused_k"][first:],
+                              c["max_seqlen_k"], 128 ** -0.5, True, (-1, -1), d["block_table"][first:], 0.0, None, None, None)
+            out, at = out.cpu(), int(c["cu_seqlens_q"][first])
+            assert float(out[:at].abs().max()) == 0.0
+            torch.testing.assert_close(out[at:].float(), ref[at:].float(), atol=ATOL, rtol=RTOL)
+    finally:
+        _lib.set_tuning("pf_segs", 0)
+        _lib.set_tuning("pf_fa", 0)

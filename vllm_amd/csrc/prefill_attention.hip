@@ -143,6 +143,7 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
     }
     seq = lo;
     start_m = g - (p.b_start_loc[seq] / tpb + seq);
+    if (start_m < 0) return;   // rows in front of the first sequence (b_start_loc may start above 0)
   }
   const int kvh = PACK ? head : head / gqa;
   // global row id m = start_m PF_BM + local row -> (query token within the sequence's new

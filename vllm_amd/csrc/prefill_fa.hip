@@ -90,14 +90,15 @@ __device__ __forceinline__ u32x2 lds_tr16(const uint8_t* p) {
   return __builtin_bit_cast(u32x2, v);
 }
 
-// The last i of [0, n) for which le(i) holds (it holds for 0, and for all i up to that one): 64 candidates per step, so that
-// 64 sequences take one load and 4096 two, where a binary search chains 6 and 12.
+// The last i of [0, n) for which le(i) holds (it holds for all i up to that one; 0 if it holds for none): 64 candidates per
+// step, so that 64 sequences take one load and 4096 two, where a binary search chains 6 and 12.
 template <typename F>
 __device__ __forceinline__ int wave_last(int n, int lane, F&& le) {
   int lo = 0;
   while (n > 1) {
     const int step = (n + 63) >> 6, i = lane * step;
-    const int c = __popcll(__ballot(i < n && le(lo + (i < n ? i : 0)))) - 1;
+    const int m = (int)__popcll(__ballot(i < n && le(lo + (i < n ? i : 0))));   // (popcll is unsigned)
+    const int c = m > 0 ? m - 1 : 0;
     lo += c * step;
     n = min(step, n - c * step);
   }
@@ -206,6 +207,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   if (blk < 0) {
     seq = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] / tpb + i <= g; });
     blk = g - (p.cu_seqlens_q[seq] / tpb + seq);
+    if (blk < 0) return;                // rows in front of the first sequence (cu_seqlens_q may start above 0)
   }
   const int tok0 = p.cu_seqlens_q[seq];
   const int qlen = p.cu_seqlens_q[seq + 1] - tok0;
@@ -790,7 +792,7 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
   const int lane = threadIdx.x & 63;
   const int pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tok = pair / p.num_heads, head = pair % p.num_heads;
-  if (tok >= p.num_tokens || tok >= p.cu_seqlens_q[p.num_seqs]) return;
+  if (tok >= p.num_tokens || tok < p.cu_seqlens_q[0] || tok >= p.cu_seqlens_q[p.num_seqs]) return;
   if (p.skip_decode) {
     const int lo = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] <= tok; });
     if (p.cu_seqlens_q[lo + 1] - p.cu_seqlens_q[lo] == 1) return;   // the decode kernel's token
