@@ -389,3 +389,20 @@ def test_prefill_rows_in_front_of_the_first_sequence(tuning, kernel, skip_decode
                 assert float(out[at[i]:at[i + 1]].abs().max()) == 0.0
             else:
                 torch.testing.assert_close(out[at[i]:at[i + 1]].float(), ref[at[i]:at[i + 1]], atol=tol(torch.bfloat16), rtol=0)
+
+
+def test_prefill_scales_of_an_unquantised_cache_are_not_read(oracle):
+    """kv_cache_dtype "auto": k_scale / v_scale may be anywhere (a layer's scales on the host); with an fp8 cache they may not."""
+    from vllm_amd.attention.ops import context_attention_fwd
+    for kv in ("auto", "fp8"):
+        c = make_prefill_case([70, 1], [100, 30], 4, 2, 128, 16, torch.bfloat16, kv, seed=1, kv_scale=0.02)
+        d = {k: v.cuda() for k, v in c.items() if torch.is_tensor(v)}
+        o = torch.zeros_like(d["q"])
+        call = lambda: context_attention_fwd(d["q"], d["k"], d["v"], o, kv, d["k_cache"], d["v_cache"], d["b_loc"], d["b_start_loc"],
+                                             d["b_seq_len"], c["max_seq_len"], c["max_input_len"], c["scale"], c["scale"])
+        if kv == "fp8":
+            with pytest.raises(RuntimeError, match="device tensors"):
+                call()
+        else:
+            call()
+            torch.testing.assert_close(o.cpu().float(), run_oracle(oracle, c, kv).float(), atol=tol(torch.bfloat16), rtol=0)

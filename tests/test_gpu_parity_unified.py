@@ -614,3 +614,25 @@ def test_unified_rows_in_front_of_the_first_sequence(oracle, kernel):
     finally:
         _lib.set_tuning("pf_segs", 0)
         _lib.set_tuning("pf_fa", 0)
+
+
+def test_unified_scales_of_an_unquantised_cache_are_not_read(oracle):
+    """A cache in the query's type: k_descale / v_descale may be anywhere (a layer's scales on the host); with fp8 they may not."""
+    from vllm_amd.attention.ops import unified_attention
+    for fp8 in (False, True):
+        c = make_unified_case([(70, 170), (1, 30)], 4, 2, 128, 16, torch.bfloat16, fp8=fp8, seed=1, kv_scale=0.5)
+        d = {k: v.cuda() for k, v in c.items() if torch.is_tensor(v)}
+        out = torch.zeros_like(d["q"])
+        call = lambda: unified_attention(d["q"], d["k"], d["v"], out, d["cu_seqlens_q"], c["max_seqlen_q"], d["seqused_k"],
+                                         c["max_seqlen_k"], 128 ** -0.5, True, (-1, -1), d["block_table"], 0.0, None, c["scale"],
+                                         c["scale"])
+        if fp8:
+            with pytest.raises(RuntimeError, match="device tensors"):
+                call()
+        else:
+            call()
+            ref = torch.zeros_like(c["q"])
+            oracle.unified_attention(c["q"], c["k"], c["v"], ref, c["cu_seqlens_q"], c["max_seqlen_q"], c["seqused_k"],
+                                     c["max_seqlen_k"], 128 ** -0.5, True, (-1, -1), c["block_table"], 0.0, None, None, None, None,
+                                     None)
+            torch.testing.assert_close(out.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)

@@ -474,7 +474,8 @@ void unified_attention(const Tensor& q, const Tensor& k, const Tensor& v, Tensor
                        int64_t max_seqlen_q, const Tensor& seqused_k, int64_t max_seqlen_k, double softmax_scale,
                        int64_t sliding_window, const Tensor& block_table, double softcap, const OptTensor& k_descale,
                        const OptTensor& v_descale, const OptTensor& alibi_slopes, const OptTensor& output_scale) {
-  need_devs(q, k, v, out, cu_seqlens_q, seqused_k, block_table, k_descale, v_descale, alibi_slopes, output_scale);
+  need_devs(q, k, v, out, cu_seqlens_q, seqused_k, block_table, alibi_slopes, output_scale);
+  if (is_fp8(k)) need_devs(k_descale, v_descale);   // (not read otherwise: a layer's scales may be anywhere)
   const int num_seqs = (int)seqused_k.size(0), num_tokens = (int)q.size(0), heads = (int)q.size(1), kv_heads = (int)k.size(2);
   const int d = (int)q.size(2);
   const Segments sg(vllm_amd_unified_attention_segments(num_seqs, heads, kv_heads, d, (int)max_seqlen_q, (int)max_seqlen_k,
@@ -495,7 +496,8 @@ void context_attention_fwd(const Tensor& q, const Tensor& k, const Tensor& v, Te
                            int64_t max_k, int64_t max_input_len, const OptTensor& k_scale, const OptTensor& v_scale,
                            const OptTensor& alibi_slopes, int64_t sliding_window, double sm_scale, bool skip_decode,
                            const OptTensor& fp8_out_scale) {
-  need_devs(q, k, v, o, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, k_scale, v_scale, alibi_slopes, fp8_out_scale);
+  need_devs(q, k, v, o, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, alibi_slopes, fp8_out_scale);
+  if (is_fp8(k_cache)) need_devs(k_scale, v_scale);   // (not read otherwise: a layer's scales may be anywhere)
   const int batch = (int)b_seq_len.size(0), num_tokens = (int)q.size(0), heads = (int)q.size(1), kv_heads = (int)k.size(1);
   const int d = (int)q.size(2);
   const Segments sg(q.scalar_type() == at::kFloat
