@@ -180,6 +180,8 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
     rtok[mt] = row_tok(m_wave + 16 * mt + c16);
     rok[mt] = row_valid(m_wave + 16 * mt + c16);
   }
+  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+  auto as_u4 = [](u32x4 v) { return make_uint4(v.x, v.y, v.z, v.w); };
   uint4 qf[MT][QK_STEPS];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
@@ -189,8 +191,9 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
 #pragma unroll
     for (int ks = 0; ks < QK_STEPS; ++ks) {
       const int d0 = 32 * ks + 8 * g4;
-      const uint4 v = *reinterpret_cast<const uint4*>(qp + (d0 < dr ? d0 : 0));
-      qf[mt][ks] = (rok[mt] && d0 < dr) ? v : make_uint4(0, 0, 0, 0);
+      // (a select of one vector value: of a uint4 hipcc makes a branch with a wait for the load in it)
+      const u32x4 v = *reinterpret_cast<const u32x4*>(qp + (d0 < dr ? d0 : 0));
+      qf[mt][ks] = as_u4((rok[mt] && d0 < dr) ? v : (u32x4){0, 0, 0, 0});
     }
   }
 
@@ -217,9 +220,7 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
 
   // staging registers of the tile being loaded (native vectors: HIP's uint4 struct arrays were
   // demoted to scratch memory by the compiler, with a wait on every load right behind it)
-  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
   u32x4 kst[NSTG], vst[NSTG];
-  auto as_u4 = [](u32x4 v) { return make_uint4(v.x, v.y, v.z, v.w); };
 
   // Physical block numbers a thread needs for a context tile.  Which page of the tile an item
   // reads is fixed per thread (K: every item of a thread is the same token; V: one page per
@@ -631,6 +632,15 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
   for (int t = t_begin; t < t_end; ++t) {
     __syncthreads();          // everyone is done reading the previous tile
     store_tile(t);
+    // Q, older than the tile, is known to be here from now on.  Pending behind the next tile's loads it would be waited for --
+    // and they with it -- in front of the first MFMAs of every tile: so it was in the build without packed FP32, where hipcc
+    // had made branches of the selects above (us, 1 x 900 tokens, 32 / 8 heads: flash layout fp8 33.3 -> 28.8, 16-bit
+    // 38.0 -> 34.8; x layout 16-bit 39.8 -> 36.1, head 256 97.1 -> 86.4)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int ks = 0; ks < QK_STEPS; ++ks)
+        asm volatile("" ::"v"(qf[mt][ks].x), "v"(qf[mt][ks].y), "v"(qf[mt][ks].z), "v"(qf[mt][ks].w));
     __syncthreads();
     if (t + 1 < t_end) {
       load_tile(t + 1, pages);
@@ -758,11 +768,11 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 // Whether a launch of query chunks takes the 256-row kernel (prefill_fa.hip; 128 rows above head size 128), and into how
 // many key segments it is split.  max_k: longest key range (an upper bound will do), ptok: query tokens of the chunks,
 // nchunk: sequences among them (a lower bound will do), cap: segments the caller has scratch for.
-//   * >= 128 row blocks, chunks of at least one: unsplit.  Without decodes beside the chunks from 64 on, over the
-//     flash-layout fp8 cache at head sizes up to 128 from 96 on and from 512 keys (min_blocks).  us, 64-row kernel -> this one: x-layout fp8 1000 tokens, 32 / 8
-//     heads (120 blocks) 40.7 -> 33.0, 600 over 200 (72) 35.9 -> 31.4, head 256 900 tokens (112) 90.8 -> 46.1; flash layout 16-bit
-//     800 (96) 34.3 -> 28.5, head 256 600 over 300 (72) 76.0 -> 44.7; fp8 1000 (120) 36.6 -> 33.5, but 400 + 300
-//     over 100 (80) 20.5 -> 23.0 and 64 / 8 heads 180 + 300 (120) 16.2 -> 18.8.
+//   * >= 128 row blocks, chunks of at least one: unsplit.  Without decodes beside the chunks from 64 on, over the flash-layout
+//     cache at head sizes up to 128 only in 16 bits and from 512 keys (min_blocks).  us, 64-row kernel -> this one: x-layout fp8
+//     1000 tokens, 32 / 8 heads (120 blocks) 41.3 -> 33.1, 600 over 200 (72) 35.5 -> 31.5, head 256 900 tokens (112) 89.0 ->
+//     46.6; flash layout 16-bit 800 (96) 32.0 -> 28.5, head 256 600 over 200 (72) 58.9 -> 42.4; but fp8 1000 (120) 31.7 ->
+//     33.7, 2 x 500 24.4 -> 27.8, 16-bit 400 + 300 over 100 (80) 21.1 -> 22.8.
 //   * fewer: the 64-row kernel's four times as many workgroups finished sooner than that (chunk 256 over 4096 cached tokens
 //     among 255 decodes: 32 blocks, 82 against 150 us) and still left the chip idle behind one serial walk over the keys
 //     (2.1 us per 64-key tile).  Split, the blocks give at least 256 workgroups; a segment is worth its start-up from three
@@ -870,7 +880,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
                                 num_tokens, batch,
-                                mixed ? 128 : (!FP8 || head_size > 128) ? 64 : max_k >= 512 ? 96 : 128);
+                                !mixed && (head_size > 128 || (!FP8 && max_k >= 512)) ? 64 : 128);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
