@@ -406,3 +406,40 @@ def test_prefill_scales_of_an_unquantised_cache_are_not_read(oracle):
         else:
             call()
             torch.testing.assert_close(o.cpu().float(), run_oracle(oracle, c, kv).float(), atol=tol(torch.bfloat16), rtol=0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("skip_decode", [False, True])
+def test_prefill_key_segments_many_sequences(tuning, n, kv, skip_decode):
+    """A split launch deals its workgroups out to the row blocks there are: sequences without a query, of one token (skipped or
+    not), of several blocks, short ones left whole and long ones beside them, in one, two and three rounds of 64 sequences."""
+    qls = [(100, 0, 1, 40, 7)[i % 5] for i in range(n)]
+    ctxs = [(300, 50, 70, 0, 190)[i % 5] + i // 5 for i in range(n)]
+    c = make_prefill_case(qls, ctxs, 8, 2, 128, 16, torch.bfloat16, kv, seed=n, kv_scale=0.02)
+    ref, at = prefill_reference(c), c["b_start_loc"].tolist()
+    tuning("pf_fa", 2)
+    for segs in (1, 2, 5):
+        tuning("pf_segs", segs)
+        out = run(c, kv, skip_decode=skip_decode)
+        assert not out.isnan().any()
+        for i in range(n):
+            if skip_decode and qls[i] == 1:
+                assert float(out[at[i]].abs().max()) == 0.0
+                ref[at[i]] = 0.0
+        torch.testing.assert_close(out.float(), ref, atol=tol(torch.bfloat16), rtol=0)
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("head_size,heads", [(128, (32, 8)), (64, (8, 1)), (256, (8, 8)), (96, (12, 3))])
+def test_prefill_wide_block_table(tuning, kv, head_size, heads):
+    """A caller that does not say how long its sequences are, under a block table far wider than they are: planned as if they
+    were that long (split), short blocks stay whole, long ones use the segments there are."""
+    from vllm_amd._lib import lib
+    qls, ctxs = [64, 40, 33, 9], [0, 100, 700, 0]
+    c = make_prefill_case(qls, ctxs, *heads, head_size, 16, torch.bfloat16, kv, seed=head_size, kv_scale=0.02)
+    wide = torch.zeros((4, 4096), dtype=torch.int32)
+    wide[:, :c["b_loc"].shape[1]] = c["b_loc"]
+    assert lib.vllm_amd_context_attention_fwd_segments(4, *heads, head_size, 64, 65536, 146, 0, 0, 0) > 1
+    c.update(b_loc=wide, max_seq_len=None)
+    torch.testing.assert_close(run(c, kv).float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)

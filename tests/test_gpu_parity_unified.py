@@ -636,3 +636,20 @@ def test_unified_scales_of_an_unquantised_cache_are_not_read(oracle):
                                      c["max_seqlen_k"], 128 ** -0.5, True, (-1, -1), c["block_table"], 0.0, None, None, None, None,
                                      None)
             torch.testing.assert_close(out.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n", [20, 64, 65, 140])
+def test_unified_prefill_key_segments_among_decodes(oracle, n, fp8):
+    """Chunks anywhere among many decode tokens, split over the keys: workgroups go to the chunks' row blocks only, which are
+    looked for in rounds of 64 sequences; a fresh chunk stays whole."""
+    from vllm_amd import _lib
+    seqs = [(1, 5 + 3 * i) for i in range(n)]
+    seqs[0], seqs[n // 2], seqs[n - 1] = (70, 600), (40, 40), (5, 333)
+    c = make_unified_case(seqs, 8, 2, 128, 16, torch.bfloat16, fp8=fp8, seed=n, kv_scale=0.5)
+    for segs in (2, 4):
+        _lib.set_tuning("pf_segs", segs)
+        try:
+            run(oracle, c, torch.bfloat16, fp8=fp8)
+        finally:
+            _lib.set_tuning("pf_segs", 0)

@@ -248,7 +248,7 @@ class ROCmFlashAttentionImpl:
                 context_attention_fwd(query, key, value, out3[:num_prefill_tokens],
                                       self.kv_cache_dtype, key_cache, value_cache,
                                       prefill_meta.block_tables, prefill_meta.query_start_loc,
-                                      prefill_meta.seq_lens_tensor, None,
+                                      prefill_meta.seq_lens_tensor, prefill_meta.max_prefill_seq_len,
                                       prefill_meta.max_query_len, layer._k_scale, layer._v_scale,
                                       self._slopes(query.device), self.sliding_window[0],
                                       self.scale, fp8_out_scale=output_scale)

@@ -60,7 +60,9 @@ def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_l
     assert k_cache.stride(4) == 1 and k_cache.stride(3) == k_cache.shape[4] \
         and k_cache.stride(2) == k_cache.shape[3] * k_cache.shape[4]
     assert v_cache.stride(3) == 1 and v_cache.stride(2) == block_size
-    # (scratch for launches that split the keys -- few row blocks over long prefixes -- is allocated in there)
+    # (scratch for launches that split the keys -- few row blocks over long prefixes -- is allocated in there.  A caller that
+    # does not know the longest sequence gets the plan for one as long as the table is wide: the kernel leaves the blocks that
+    # turn out short in one piece, but the merge runs behind it)
     max_k = max_seq_len if max_seq_len else b_loc.shape[1] * block_size
     _torch_ops.context_attention_fwd(q, k, v, o, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, int(max_k), int(max_input_len),
                                      k_scale, v_scale, alibi_slopes, int(sliding_window), float(sm_scale), bool(skip_decode),

@@ -127,13 +127,15 @@ class PagedAttention:
     def forward_prefix(query, key, value, kv_cache_dtype: str, key_cache, value_cache,
                        block_tables, query_start_loc, seq_lens_tensor, max_query_len: int,
                        alibi_slopes: Optional[torch.Tensor], sliding_window: Optional[int],
-                       k_scale: torch.Tensor, v_scale: torch.Tensor) -> torch.Tensor:
+                       k_scale: torch.Tensor, v_scale: torch.Tensor,
+                       max_seq_len: Optional[int] = None) -> torch.Tensor:
         """paged_attn.py:196-239: chunked prefill over the cached prefix (HIP kernel instead of
-        the reference's Triton context_attention_fwd)."""
+        the reference's Triton context_attention_fwd).  max_seq_len: the longest sequence, where the
+        caller knows it (else the launch is planned for the width of block_tables)."""
         from .ops.prefix_prefill import context_attention_fwd
         output = torch.empty_like(query)
         context_attention_fwd(query, key, value, output, kv_cache_dtype, key_cache, value_cache,
-                              block_tables, query_start_loc, seq_lens_tensor, None, max_query_len,
+                              block_tables, query_start_loc, seq_lens_tensor, max_seq_len, max_query_len,
                               k_scale, v_scale, alibi_slopes, sliding_window)
         return output
 

@@ -766,27 +766,30 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
     hipLaunchKernelGGL((prefill_kernel<T, FP8, D, 32, MT, NW, UNI, PACK>), grid, dim3(64 * NW), 0, st, p);
 }
 // Whether a launch of query chunks takes the 256-row kernel (prefill_fa.hip; 128 rows above head size 128), and into how
-// many key segments it is split.  max_k: longest key range (an upper bound will do), ptok: query tokens of the chunks,
-// nchunk: sequences among them (a lower bound will do), cap: segments the caller has scratch for.
+// many key segments it is split.  max_k: longest key range as far as the caller knows it (of a decode beside the chunks, or the
+// width of the block table: the kernel leaves short blocks whole, but merge and larger tiles cost 3 .. 6 us against the 64-row
+// kernel: 64 fresh tokens under a table for 8192 7.5 -> 13.3), ptok: query tokens of the chunks, nchunk: sequences among them
+// (a lower bound will do), cap: segments the caller has scratch for.
 //   * >= 128 row blocks, chunks of at least one: unsplit.  Without decodes beside the chunks from 64 on, over the flash-layout
 //     cache at head sizes up to 128 only in 16 bits and from 512 keys (min_blocks).  us, 64-row kernel -> this one: x-layout fp8
 //     1000 tokens, 32 / 8 heads (120 blocks) 41.3 -> 33.1, 600 over 200 (72) 35.5 -> 31.5, head 256 900 tokens (112) 89.0 ->
 //     46.6; flash layout 16-bit 800 (96) 32.0 -> 28.5, head 256 600 over 200 (72) 58.9 -> 42.4; but fp8 1000 (120) 31.7 ->
-//     33.7, 2 x 500 24.4 -> 27.8, 16-bit 400 + 300 over 100 (80) 21.1 -> 22.8.
+//     33.7, 2 x 500 24.4 -> 27.8, 16-bit 400 + 300 over 100 (80) 21.1 -> 22.8.  Windows narrower than half the keys count as
+//     16 bits: this kernel does not stage the tiles left of them (fp8, 900 tokens, window 128: 21.5 -> 15.6).
 //   * fewer: the 64-row kernel's four times as many workgroups finished sooner than that (chunk 256 over 4096 cached tokens
 //     among 255 decodes: 32 blocks, 82 against 150 us) and still left the chip idle behind one serial walk over the keys
-//     (2.1 us per 64-key tile).  Split, the blocks give at least 256 workgroups; a segment is worth its start-up from three
-//     tiles on, the merge its launch from 16 tiles on (400 keys: 26.7 us unsplit, 32.6 split).  us, 64-row kernel -> split:
-//     35 tokens over 3723, 8 q / 1 kv head 123 -> 32; 512 over 8000, 32 / 8 208 -> 87; 1024 over 4000 139 -> 102; head 64,
-//     300 over 3000 87 -> 33; head 256, 2 x 300 over 3000 159 -> 60; x-layout prefix, 300 over 3000 106 -> 44.
-struct FaPlan { bool use; int nseg; };
+//     (2.1 us per 64-key tile).  Split, 256 workgroups are dealt out to the blocks there are; a segment is worth its start-up
+//     from three tiles on, the merge its launch from 16 tiles on (400 keys: 26.7 us unsplit, 32.6 split).  us, 64-row kernel ->
+//     split: 35 tokens over 3723, 8 q / 1 kv head 123 -> 32; 512 over 8000, 32 / 8 208 -> 87; 1024 over 4000 139 -> 102; head
+//     64, 300 over 3000 87 -> 33; head 256, 2 x 300 over 3000 159 -> 60; x-layout prefix, 300 over 3000 106 -> 37.
+struct FaPlan { bool use; int nseg, seg_slots; };
 static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap,
                       int64_t num_tokens, int num_seqs, int min_blocks = 128) {
   const int gqa = num_heads / num_kv_heads;
   const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
   const int tpb = (head_size > 128 ? 128 : 256) / pack;
   const int y = pack > 1 ? num_kv_heads : num_heads;
-  if (g_pf_fa == 1 || g_pf_rows != 0 || (max_q <= 1 && g_pf_fa != 2) || head_size > 256) return {false, 1};
+  if (g_pf_fa == 1 || g_pf_rows != 0 || (max_q <= 1 && g_pf_fa != 2) || head_size > 256) return {false, 1, 0};
   const bool whole = head_size > 64 && (g_pf_fa == 2 || (max_q >= tpb && ptok / tpb * y >= min_blocks));
   int64_t blocks = (ptok + tpb - 1) / tpb;
   if (blocks < nchunk) blocks = nchunk;
@@ -796,17 +799,22 @@ static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q,
   if (nseg > by_len) nseg = by_len;
   if (nseg > cap) nseg = cap;
   if (nseg > FA_MAX_SEGMENTS) nseg = FA_MAX_SEGMENTS;
-  // The grid has a row block for every sequence, also for those the decode kernel takes: an empty workgroup costs ~4.5 ns, the
-  // merge ~4 us, and max_k may belong to a decode.  So only where the walk over max_k keys (1.9 us per tile) would shrink by
-  // 2.8 times that overhead.  Whole steps in us, 64-row kernel / split: 300 over 3000 among 63 decodes 137 / 100, among 120
-  // 166 / 135, 256 over 4096 among 255 222 / 180, 8 q / 1 kv head 300 over 2000 among 100 87 / 48; left unsplit: 512 fresh
-  // tokens among 100 decodes of up to 2000 keys 74 / 79, 100 among 63 of 1500 39.4 / 41.0, 213 among 185 of 1056 74 / 112.
+  // The grid has a workgroup for every row block there may be, also of the sequences the decode kernel takes: an empty one costs
+  // ~4.5 ns, the merge ~4 us, and max_k may belong to a decode.  So only where the walk over the keys (1.9 us per tile) would
+  // shrink by twice that overhead.  Whole steps in us, fp8, 32 / 8 heads, 64-row kernel / split: 300 over 2000 among 20
+  // decodes of 900 keys 78 / 44, 64 over 2936 among 60 of 500 94 / 39, 200 over 3800 among 100 of 700 139 / 66, 256 over 4096
+  // among 200 of 4096 400 / 319; and where max_k is a decode's, 100 fresh tokens among 60 of 3000 76 / 75, 500 over 100 among
+  // 30 of 1500 48 / 45.
   const int64_t launched = (num_tokens / tpb + num_seqs) * y;
-  if ((int64_t)nseg * launched > 4400) nseg = (int)(4400 / launched);
-  if (nseg > 1 && max_k / PF_BN * 1.9 * (1.0 - 1.0 / nseg) < 2.8 * (4.0 + (double)nseg * (double)launched * 4.5e-3)) nseg = 1;
-  if (g_pf_segs > 0) nseg = g_pf_segs < cap ? g_pf_segs : cap;
-  if (nseg < 2) return {whole, 1};
-  return {true, nseg};
+  const double walk = (max_k - 0.5 * (max_q < max_k ? max_q : max_k)) / PF_BN;   // mean over the rows of the longest chunk
+  if (nseg > 1 && walk * 1.9 * (1.0 - 1.0 / nseg) < 2.0 * (4.0 + (double)(launched > 256 ? launched : 256) * 4.5e-3)) nseg = 1;
+  int slots = 256 / y;
+  if (g_pf_segs > 0) {   // every block that many, wherever there are tiles
+    nseg = g_pf_segs < cap ? g_pf_segs : cap;
+    slots = (int)(launched / y) * nseg;
+  }
+  if (nseg < 2) return {whole, 1, 0};
+  return {true, nseg, slots};
 }
 
 // unified_attention: padded head sizes 64 and 128 (one configuration each)
@@ -878,9 +886,10 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     const bool can = p.alibi_slopes == nullptr && p.flat_batch > 0 && p.sm_scale > 0.f &&
                      p.kc_page_bytes < (1 << 27) && p.vc_page_bytes < (1 << 27);
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
+    const bool narrow = p.sliding_window > 0 && 2 * (int64_t)p.sliding_window <= max_k;
     const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
                                 num_tokens, batch,
-                                !mixed && (head_size > 128 || (!FP8 && max_k >= 512)) ? 64 : 128);
+                                !mixed && (head_size > 128 || narrow || (!FP8 && max_k >= 512)) ? 64 : 128);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -896,7 +905,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       f.window = p.sliding_window; f.softcap = p.softcap;
       f.prefix = 0; f.k_new = f.v_new = nullptr; f.k_stride_t = f.k_stride_h = f.v_stride_t = f.v_stride_h = 0;
       f.blocks_per_seq = 0;
-      f.num_segments = plan.nseg; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
+      f.num_segments = plan.nseg; f.seg_slots = plan.seg_slots; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
       f.abl = g_pf_fa_abl;
       f.stagger = g_pf_fa_stagger;
       return launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
@@ -979,7 +988,7 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
       f.k_stride_t = p.k_stride_t; f.k_stride_h = p.k_stride_h; f.v_stride_t = p.v_stride_t; f.v_stride_h = p.v_stride_h;
       const int tpb = (head_size > 128 ? 128 : 256) / pack;
       f.blocks_per_seq = p.flat_batch > 0 ? 0 : (max_input_len + tpb - 1) / tpb;
-      f.num_segments = plan.nseg; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
+      f.num_segments = plan.nseg; f.seg_slots = plan.seg_slots; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
       f.abl = 0; f.stagger = g_pf_fa_stagger;
       launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
       return;

@@ -28,9 +28,10 @@ struct FaParams {
   int64_t k_stride_t, k_stride_h, v_stride_t, v_stride_h;   // elements
   int blocks_per_seq;  // > 0: num_tokens unknown, grid.x = blocks_per_seq * num_seqs (ceil(max query length / tokens per block))
   int stagger;         // 1 = waves 4-7 stage at the top of the interval (tuning "pf_fa_stagger", default 1)
-  // Split over the keys: num_segments workgroups per row block, each over its share of the block's tiles; they leave
+  // Split over the keys: up to num_segments workgroups per row block, each over its share of the block's tiles; they leave
   // unnormalised fp32 partials [token][q head][segment] that fa_reduce_kernel merges.  1 = no split (buffers unused).
-  int num_segments;
+  // seg_slots: workgroups per grid.y to deal out to the row blocks, at least one each.
+  int num_segments, seg_slots;
   float* segm_out; float* segm_max; float* segm_sum;
   int abl;             // (unused; the kernel's ablations are compile-time: -DVA_FA_ABL=bits, garbage results: 1 no exp2,
                        // 2 no staging after the first tiles, 4 no S^T MFMAs, 8 no PV MFMAs, 16 no barrier)

@@ -61,6 +61,7 @@ constexpr int KN = 2, VN = 2;     // K / V tiles in LDS (rings indexed by the ti
 constexpr int KR128 = 8, VR128 = 4;   // fragment reads in flight: K reads, V^T fragments (two transposing reads each)
 constexpr int KR256 = FA_KRW, VR256 = FA_VRW;
 constexpr float THR = 8.f;        // lazy rescale threshold (log2 domain)
+constexpr int ONE_SEG = 3;        // a row block of up to this many tiles is not split
 
 // One v_maximum3_f32.  (fmaxf on MFMA results makes hipcc canonicalise every input first; inline asm must not read them
 // at all: the wait states between an MFMA and a VALU read of its result are the compiler's to insert, it inserts none in
@@ -88,6 +89,17 @@ __device__ __forceinline__ u32x2 lds_tr16(const uint8_t* p) {
   typedef __attribute__((ext_vector_type(4))) short s16x4;
   const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
   return __builtin_bit_cast(u32x2, v);
+}
+
+// Sum of v over the lanes up to and with this one (DPP: rows of 16, then the rows' last lanes)
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2, 3
+  return v;
 }
 
 // The last i of [0, n) for which le(i) holds (it holds for all i up to that one; 0 if it holds for none): 64 candidates per
@@ -131,7 +143,8 @@ __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];
 // whole SIMD's register file: four waves = 128 rows, one per SIMD, 32 KiB tiles (128 KiB of LDS), 32 + 32 MFMAs per tile.
 // SOFTCAP (unified_attention): scores softcap * tanh(score / softcap) (triton_unified_attention.py:219-221): a pass of
 // ~9 VALU per score between S^T and the softmax, in its own instantiation.
-template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP>
+// SPLIT: num_segments > 1, in its own instantiation (the 256-wide forms have no register to spare).
+template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP, bool SPLIT>
 __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   constexpr int NW = NW_, BM = 32 * NW, D = D_;
   constexpr int ROWB = 2 * D;       // bytes per LDS row (one key, D 16-bit values)
@@ -161,53 +174,93 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // ---- workgroup -> (row block of some sequence, head).  Hardware ids go round-robin over the XCDs: the
   // bijective remap gives every XCD a contiguous range of logical ids (row blocks fastest, then heads), so the
   // row blocks and heads that read the same K / V share an L2; later (longer) row blocks first.
-  int wg = blockIdx.x + gridDim.x * blockIdx.y;
-  {
-    const int nwg = gridDim.x * gridDim.y;
-    const int q8 = nwg / 8, r8 = nwg % 8, xcd = wg % 8, idx = wg / 8;
-    wg = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + idx;
-  }
-  // (split launches: the row blocks of one key segment are adjacent, they read the same K / V)
-  const int nseg = p.num_segments, gx = nseg > 1 ? gridDim.x / nseg : gridDim.x;
-  const int y = wg / gridDim.x, gs = wg % gridDim.x;
-  const int seg = nseg > 1 ? gs / gx : 0;
-  const int g = gx - 1 - (gs - seg * gx);
+  auto xcd_order = [](int nwg) __attribute__((always_inline)) {   // -1: more workgroups than work
+    const int hw = blockIdx.x + gridDim.x * blockIdx.y, q8 = nwg / 8, r8 = nwg % 8, xcd = hw % 8, idx = hw / 8;
+    return idx < q8 + (xcd < r8 ? 1 : 0) ? (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + idx : -1;
+  };
+  const int nseg = SPLIT ? p.num_segments : 1;
   const int pack = p.pack, tpb = BM / pack;   // tokens per workgroup
   // grid.x enumerates the row blocks of ALL sequences (num_tokens / tpb + num_seqs is an upper bound); the
   // sequence is the last one whose first block cu[i] / tpb + i is <= g (find_seq_idx, :33-48)
   // (blocks_per_seq > 0: the caller did not say how many query tokens there are; every sequence gets that many blocks)
   int seq = 0, blk = -1;   // sequence, row block in it
-  if (p.blocks_per_seq > 0) {
-    seq = g / p.blocks_per_seq;
-    blk = g % p.blocks_per_seq;
-  } else if (PREFIX && p.num_seqs > 1 && p.num_seqs <= 64 && nseg == 1 && gridDim.y % 8 == 0) {
-    // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD: the row blocks of the
-    // longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24 chunks of
-    // 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us; 19 prompts of 745 .. 1242 without
-    // context, whose blocks differ more than the prompts, 294 -> 302: they keep the order below).
-    int len = -1, nb = 0, before = 0;   // lane i: sequence i, its blocks, the blocks in front of them
-    bool over = false;
-    if (lane < p.num_seqs) {
-      const int ql = p.cu_seqlens_q[lane + 1] - p.cu_seqlens_q[lane];
-      len = p.seq_lens[lane];
-      nb = p.skip_decode && ql == 1 ? 0 : (ql + tpb - 1) / tpb;
-      over = len >= 3 * ql;
-    }
-    if (2 * __popcll(__ballot(nb > 0 && over)) >= __popcll(__ballot(nb > 0))) {
-      for (int j = 0; j < p.num_seqs; ++j) {
-        const int lj = __builtin_amdgcn_readlane(len, j), nj = __builtin_amdgcn_readlane(nb, j);
-        before += (lj > len || (lj == len && j < lane)) ? nj : 0;
+  int seg = 0, segs = 1;   // split launches: key segment, segments of this block
+  int y, gs, g;
+  if constexpr (SPLIT) {
+    // The row blocks there really are, and seg_slots workgroups dealt out to them: as num_segments workgroups for each
+    // block there may be, a launch spent 2.2 ns on each one of a sequence that the decode kernel takes (100 fresh tokens among
+    // 60 decodes of 3000 keys, 32 / 8 heads: 4032 workgroups, whole step 86.7 us, now 75.1; 200 over 3800 among 100 of 700: 91.7
+    // -> 66.0).  The work goes evenly over the XCDs: a few blocks too many on one of them double up on its CUs (512 over 7488,
+    // 8 q / 1 kv head: 60 against 40 us).
+    auto blocks_of = [&](int i) __attribute__((always_inline)) {
+      const int ql = i < p.num_seqs ? p.cu_seqlens_q[i + 1] - p.cu_seqlens_q[i] : 0;
+      return p.skip_decode && ql == 1 ? 0 : (ql + tpb - 1) / tpb;
+    };
+    int n = blocks_of(lane), incl = wave_scan(n);             // the first 64 sequences stay in registers
+    int here = __builtin_amdgcn_readlane(incl, 63), total = here;
+    for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(blocks_of(i + lane)), 63);
+    if (total == 0) return;
+    const int work = max(total, min(p.seg_slots, total * nseg));   // per head
+    const int w = xcd_order(work * (int)gridDim.y);
+    if (w < 0) return;
+    y = w / work;
+    gs = w - y * work;
+    seg = gs / total;
+    int b = gs - seg * total;                                 // (a segment's row blocks are adjacent, they read the same K / V)
+    segs = work / total;
+    segs += b < work - segs * total ? 1 : 0;
+    b = total - 1 - b;                                        // later (longer) row blocks first
+    for (int i = 0; i < p.num_seqs; i += 64) {
+      if (i > 0) {
+        n = blocks_of(i + lane);
+        incl = wave_scan(n);
+        here = __builtin_amdgcn_readlane(incl, 63);
       }
-      const unsigned long long mine = __ballot(before <= gs && gs < before + nb);
-      if (mine == 0) return;            // the grid is an upper bound
-      seq = __builtin_amdgcn_readfirstlane(__ffsll((long long)mine) - 1);
-      blk = __builtin_amdgcn_readlane(nb, seq) - 1 - (gs - __builtin_amdgcn_readlane(before, seq));
+      if (b < here) {
+        const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(b < incl)) - 1);
+        seq = i + l;
+        blk = b - __builtin_amdgcn_readlane(incl - n, l);
+        break;
+      }
+      b -= here;
     }
-  }
-  if (blk < 0) {
-    seq = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] / tpb + i <= g; });
-    blk = g - (p.cu_seqlens_q[seq] / tpb + seq);
-    if (blk < 0) return;                // rows in front of the first sequence (cu_seqlens_q may start above 0)
+  } else {
+    const int w = xcd_order(gridDim.x * gridDim.y);
+    y = w / gridDim.x;
+    gs = w % gridDim.x;
+    g = gridDim.x - 1 - gs;
+    if (p.blocks_per_seq > 0) {
+      seq = g / p.blocks_per_seq;
+      blk = g % p.blocks_per_seq;
+    } else if (PREFIX && p.num_seqs > 1 && p.num_seqs <= 64 && gridDim.y % 8 == 0) {
+      // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD: the row blocks of the
+      // longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24 chunks of
+      // 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us; 19 prompts of 745 .. 1242 without
+      // context, whose blocks differ more than the prompts, 294 -> 302: they keep the order below).
+      int len = -1, nb = 0, before = 0;   // lane i: sequence i, its blocks, the blocks in front of them
+      bool over = false;
+      if (lane < p.num_seqs) {
+        const int ql = p.cu_seqlens_q[lane + 1] - p.cu_seqlens_q[lane];
+        len = p.seq_lens[lane];
+        nb = p.skip_decode && ql == 1 ? 0 : (ql + tpb - 1) / tpb;
+        over = len >= 3 * ql;
+      }
+      if (2 * __popcll(__ballot(nb > 0 && over)) >= __popcll(__ballot(nb > 0))) {
+        for (int j = 0; j < p.num_seqs; ++j) {
+          const int lj = __builtin_amdgcn_readlane(len, j), nj = __builtin_amdgcn_readlane(nb, j);
+          before += (lj > len || (lj == len && j < lane)) ? nj : 0;
+        }
+        const unsigned long long mine = __ballot(before <= gs && gs < before + nb);
+        if (mine == 0) return;            // the grid is an upper bound
+        seq = __builtin_amdgcn_readfirstlane(__ffsll((long long)mine) - 1);
+        blk = __builtin_amdgcn_readlane(nb, seq) - 1 - (gs - __builtin_amdgcn_readlane(before, seq));
+      }
+    }
+    if (blk < 0) {
+      seq = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] / tpb + i <= g; });
+      blk = g - (p.cu_seqlens_q[seq] / tpb + seq);
+      if (blk < 0) return;                // rows in front of the first sequence (cu_seqlens_q may start above 0)
+    }
   }
   const int tok0 = p.cu_seqlens_q[seq];
   const int qlen = p.cu_seqlens_q[seq + 1] - tok0;
@@ -232,6 +285,23 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // among the context keys (PREFIX)
   const int bound_new = rok ? (PREFIX ? rtok : ctx + rtok) : -1;
   const int bound_ctx = rok ? ctx - 1 : -1;
+
+  // tiles: ctx_tiles of the context (PREFIX), then the new domain's
+  const int ctx_tiles = PREFIX ? (ctx + BN - 1) / BN : 0;
+  const int new_tiles = ((PREFIX ? new_end : ctx + new_end) + BN - 1) / BN;
+  const int ntiles = ctx_tiles + new_tiles;
+  const int window = PREFIX ? 0 : p.window;          // keys (position - window, position] are visible; 0 = all
+  // (sliding window: the tiles left of the window of the workgroup's first row are not even staged)
+  const int t_start = window > 0 ? max(ctx + tok_base - window + 1, 0) / BN : 0;
+  // Split: this segment's share [t0, t1) of the block's tiles.  The host plans for the longest sequence it was told of -- of a
+  // decode beside the chunks, or for the width of the block table -- so a block of up to ONE_SEG tiles is one segment, which
+  // writes its output itself, segments without a tile leave here, and segment 0 tells the merge how many there are: -live in
+  // the last place of the sums, which is free unless all num_segments are live.
+  const int walk = ntiles - t_start;
+  const int per = !SPLIT || segs == 1 || walk <= ONE_SEG ? max(walk, 1) : (walk + segs - 1) / segs;
+  const int live = SPLIT ? max((walk + per - 1) / per, 1) : 1;
+  const int t0 = t_start + seg * per, t1 = min(t0 + per, ntiles);
+  if (seg >= live) return;
   // Q^T fragments (B operand of S^T): column m = this row, k = d = 16 ks + 8 hi + (0..7)
   u32x4 qf[KS];
   {
@@ -250,15 +320,10 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
 
   float kscale = 1.f, vscale = 1.f;
   if constexpr (FP8) { kscale = *p.k_scale; vscale = *p.v_scale; }
-  const int window = PREFIX ? 0 : p.window;          // keys (position - window, position] are visible; 0 = all
   const float sc2 = p.sm_scale * kLog2e;             // > 0 (host checks sm_scale)
   const float sc2k = sc2 * kscale;                   // fp8 keys: k_scale rides in the score scale
   const float vlog2 = FP8 ? log2f(vscale) : 0.f, vinv = FP8 ? 1.0f / vscale : 1.f;
 
-  // tiles: ctx_tiles of the context (PREFIX), then the new domain's
-  const int ctx_tiles = PREFIX ? (ctx + BN - 1) / BN : 0;
-  const int new_tiles = ((PREFIX ? new_end : ctx + new_end) + BN - 1) / BN;
-  const int ntiles = ctx_tiles + new_tiles;
   const int* bt = p.block_table + (int64_t)seq * p.bt_stride;
   const int last_page = PREFIX ? (ctx > 0 ? (ctx - 1) >> p.bs_shift : 0) : (seq_len - 1) >> p.bs_shift;
 
@@ -376,6 +441,24 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   uint8_t* v_wr = lds + V_OFF + skey * ROWB;
   const int kc0 = ((2 * spiece) ^ (skey & 15)) << 4, kc1 = ((2 * spiece + 1) ^ (skey & 15)) << 4;
   const int vc0 = ((2 * spiece) ^ ((skey & 3) << 2)) << 4, vc1 = ((2 * spiece + 1) ^ ((skey & 3) << 2)) << 4;
+  // PREFIX above head size 128: the offsets of a thread's first chunks (the second ones are at offset ^ 16), computed anew for
+  // every tile from a thread id that hipcc cannot trace back.  Kept over the loop they are spilled, and their reloads wait for
+  // the loads in flight (us, head 256: 32 x 128 tokens over 4096 16-bit 660 -> 538, fp8 440 -> 377; 2 x 2048 over 2048 fp8
+  // 299 -> 290).
+  constexpr bool WIDE = PREFIX && D > 128;
+  struct WideAt { int k, v; };
+  auto wide_at = [&](bool context) __attribute__((always_inline)) {
+    WideAt a = {0, 0};
+    if constexpr (WIDE) {
+      int t_ = tid;
+      asm volatile("" : "+v"(t_));
+      const int key = t_ / PPK, piece = t_ % PPK, kperm = (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1);   // (kperm: below)
+      const int kr = context ? kperm : key;
+      a.k = K_OFF + kr * ROWB + (((2 * piece) ^ (kr & 15)) << 4);
+      a.v = context ? V_OFF + t_ * 128 + (((t_ >> 1) & 7) << 4) : V_OFF + key * ROWB + (((2 * piece) ^ ((key & 3) << 2)) << 4);
+    }
+    return a;
+  };
   auto u4 = [](u32x4 v) __attribute__((always_inline)) { return make_uint4(v[0], v[1], v[2], v[3]); };
   // Slots past the sequence hold stale bytes (possibly NaN): K and V rows of such keys are zeroed (their scores are 0 + the
   // mask's -inf, their probabilities 0, and 0 * NaN = NaN), and so are the padding columns.  whole: every key of the tile
@@ -400,11 +483,17 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // rows of keys base + (0..63) of `keys` keys, K and V
   auto write_rows = [&](int t, int base, int keys, auto conv_c, auto whole) __attribute__((always_inline)) {
     const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
+    const WideAt at = wide_at(false);
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
       const bool live = base + skey + KSTEP * i < keys;
-      write_row(k_wr + kb_ + KSTEP * i * ROWB, kc0, kc1, kst[i], live, whole, conv_c);
-      write_row(v_wr + vb_ + KSTEP * i * ROWB, vc0, vc1, vst[i], live, whole, conv_c);
+      if constexpr (WIDE) {
+        write_row(lds + at.k + kb_ + KSTEP * i * ROWB, 0, (at.k ^ 16) - at.k, kst[i], live, whole, conv_c);
+        write_row(lds + at.v + vb_ + KSTEP * i * ROWB, 0, (at.v ^ 16) - at.v, vst[i], live, whole, conv_c);
+      } else {
+        write_row(k_wr + kb_ + KSTEP * i * ROWB, kc0, kc1, kst[i], live, whole, conv_c);
+        write_row(v_wr + vb_ + KSTEP * i * ROWB, vc0, vc1, vst[i], live, whole, conv_c);
+      }
     }
   };
   // Context tiles: LDS row i of K is key i with bits 2 and 3 swapped.  S^T row (r & 3) + 8 (r >> 2) + 4 hi, which lane half hi
@@ -415,9 +504,12 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   const int kc0_ctx = ((2 * spiece) ^ (kperm & 15)) << 4, kc1_ctx = ((2 * spiece + 1) ^ (kperm & 15)) << 4;
   auto write_ctx = [&](int t, auto whole) __attribute__((always_inline)) {
     const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
+    const WideAt at = wide_at(true);
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
-      write_row(k_wr_ctx + kb_ + KSTEP * i * ROWB, kc0_ctx, kc1_ctx, kst[i], t * BN + skey + KSTEP * i < ctx, whole, std::integral_constant<bool, FP8>{});
+      const bool live = t * BN + skey + KSTEP * i < ctx;
+      if constexpr (WIDE) write_row(lds + at.k + kb_ + KSTEP * i * ROWB, 0, (at.k ^ 16) - at.k, kst[i], live, whole, std::integral_constant<bool, FP8>{});
+      else write_row(k_wr_ctx + kb_ + KSTEP * i * ROWB, kc0_ctx, kc1_ctx, kst[i], live, whole, std::integral_constant<bool, FP8>{});
       // V^T: the item's 16 tokens of row vd = two 16-byte units
       const int vd = vd_of(i), vq = vq_of(i);
       const int valid = vd < dr ? ctx - (t * BN + 16 * vq) : 0;
@@ -434,10 +526,15 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
           hi4 = mask_halfs(hi4, valid - 8);
         }
       }
-      uint8_t* row = lds + V_OFF + vb_ + vd * 128;
-      const int f = (vd >> 1) & 7;
-      *reinterpret_cast<u32x4*>(row + (((2 * vq + 0) ^ f) << 4)) = (u32x4){lo.x, lo.y, lo.z, lo.w};
-      *reinterpret_cast<u32x4*>(row + (((2 * vq + 1) ^ f) << 4)) = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
+      if constexpr (WIDE) {      // (vd is the thread, vq is i)
+        *reinterpret_cast<u32x4*>(lds + (at.v ^ (32 * i)) + vb_) = (u32x4){lo.x, lo.y, lo.z, lo.w};
+        *reinterpret_cast<u32x4*>(lds + (at.v ^ (32 * i + 16)) + vb_) = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
+      } else {
+        uint8_t* row = lds + V_OFF + vb_ + vd * 128;
+        const int f = (vd >> 1) & 7;
+        *reinterpret_cast<u32x4*>(row + (((2 * vq + 0) ^ f) << 4)) = (u32x4){lo.x, lo.y, lo.z, lo.w};
+        *reinterpret_cast<u32x4*>(row + (((2 * vq + 1) ^ f) << 4)) = (u32x4){hi4.x, hi4.y, hi4.z, hi4.w};
+      }
     }
   };
   auto write_tile = [&](int t) __attribute__((always_inline)) {
@@ -619,11 +716,6 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // Registers hold tile t + 1 (loads in flight) while tile t is computed from LDS buffer t & 1; in interval t they
   // are written to buffer (t + 1) & 1 -- last read for tile t - 1, before the barrier that ended interval t - 1 --
   // and the loads of tile t + 2 are issued.  One barrier per tile.
-  // (sliding window: the tiles left of the window of the workgroup's first row are not even staged)
-  const int t_start = window > 0 ? max(ctx + tok_base - window + 1, 0) / BN : 0;
-  // (split: this segment's share [t0, t1) of the block's tiles, possibly none)
-  const int per = nseg > 1 ? (ntiles - t_start + nseg - 1) / nseg : ntiles - t_start;
-  const int t0 = t_start + seg * per, t1 = min(t0 + per, ntiles);
   if (t0 < t1) {
   Blk blk = load_blk(t0);
   issue_loads(t0, blk);
@@ -739,21 +831,21 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // ---- O^T / l -> out ------------------------------------------------------------------------------------------
   if (!rok) return;
   const float l = xsum(l_run);
-  if (nseg > 1) {   // this segment's partial: O unnormalised, running maximum (log2 domain; -inf: nothing visible), sum
+  if (SPLIT && seg == 0 && live < nseg && hi == 0)
+    p.segm_sum[((int64_t)(tok0 + rtok) * p.num_heads + rhead + 1) * nseg - 1] = -(float)live;
+  if (SPLIT && live > 1) {   // this segment's partial: O unnormalised, running maximum (log2 domain; -inf: nothing visible), sum
     const int64_t row = ((int64_t)(tok0 + rtok) * p.num_heads + rhead) * nseg + seg;
     if (hi == 0) {
       p.segm_max[row] = m_run;
       p.segm_sum[row] = l;
     }
-    if (t0 < t1) {
-      float* so = p.segm_out + row * dr + 4 * hi;
+    float* so = p.segm_out + row * dr + 4 * hi;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int rq = 0; rq < 4; ++rq)
-          if (32 * db + 8 * rq + 4 * hi < dr)
-            *reinterpret_cast<float4*>(so + 32 * db + 8 * rq) = make_float4(o[db][4 * rq], o[db][4 * rq + 1], o[db][4 * rq + 2], o[db][4 * rq + 3]);
-    }
+      for (int rq = 0; rq < 4; ++rq)
+        if (32 * db + 8 * rq + 4 * hi < dr)
+          *reinterpret_cast<float4*>(so + 32 * db + 8 * rq) = make_float4(o[db][4 * rq], o[db][4 * rq + 1], o[db][4 * rq + 2], o[db][4 * rq + 3]);
     return;
   }
   const float inv = l > 0.f ? 1.0f / l : 0.f;
@@ -784,8 +876,8 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
 }
 
 // Merge of a split launch: one wave per (token, q head).  Lane s holds segment s's maximum and sum; a half wave (D <= 128;
-// the whole wave above) reads one partial row per step, four rows in flight.  Segments that saw nothing were not written
-// and are not read.
+// the whole wave above) reads one partial row per step, four rows in flight.  Segments that saw nothing (maximum -inf) are
+// not read.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
   constexpr int LPR = D / 4, PAR = 64 / LPR;      // lanes per row, rows per step
@@ -799,22 +891,26 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
   }
   const int nseg = p.num_segments, dr = p.head_size;
   const int64_t row = ((int64_t)tok * p.num_heads + head) * nseg;
-  const float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
-  const float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
+  float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
+  float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
+  const float last = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ls), nseg - 1));
+  const int live = last < 0.f ? (int)-last : nseg;
+  if (live == 1) return;             // the only segment has written the output
+  if (lane >= live) { ms = -INFINITY; ls = 0.f; }
   const float mx = wave_max(ms);
   const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);
   const float l = wave_sum(ls * w);
   const int d = 4 * (lane % LPR), sub = lane / LPR;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   const float* base = p.segm_out + row * dr + (d < dr ? d : 0);
-  for (int s0 = 0; s0 < nseg; s0 += 4 * PAR) {
+  for (int s0 = 0; s0 < live; s0 += 4 * PAR) {
     float4 part[4];
     float ws[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int s = s0 + u * PAR + sub;
-      ws[u] = __shfl(w, s < nseg ? s : 0, 64);
-      if (s >= nseg) ws[u] = 0.f;
+      ws[u] = __shfl(w, s < live ? s : 0, 64);
+      if (s >= live) ws[u] = 0.f;
       part[u] = ws[u] > 0.f ? *reinterpret_cast<const float4*>(base + (int64_t)s * dr) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
@@ -851,9 +947,14 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st) {
   const bool wide = p.head_size > 128;                 // 128-row workgroups of four waves
   const int tpb = (wide ? 128 : 256) / p.pack;
   const unsigned gx = p.blocks_per_seq > 0 ? (unsigned)(p.blocks_per_seq * p.num_seqs) : (unsigned)(p.num_tokens / tpb + p.num_seqs);
-  const dim3 grid(gx * (unsigned)p.num_segments, (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads));
-#define FA_LAUNCH___(T_, F_, P_, D_, NW_, S_) \
-  hipLaunchKernelGGL((fa::fa_fwd_kernel<T_, F_, P_, D_, NW_, S_>), grid, dim3(64 * NW_), 0, st, p)
+  const unsigned gy = (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads);
+  const unsigned slots = p.num_segments > 1 ? (unsigned)p.seg_slots : 0u;
+  const dim3 grid(gx > slots ? gx : slots, gy);
+#define FA_LAUNCH___(T_, F_, P_, D_, NW_, S_)                                                                            \
+  do {                                                                                                                   \
+    if (p.num_segments > 1) hipLaunchKernelGGL((fa::fa_fwd_kernel<T_, F_, P_, D_, NW_, S_, true>), grid, dim3(64 * NW_), 0, st, p); \
+    else hipLaunchKernelGGL((fa::fa_fwd_kernel<T_, F_, P_, D_, NW_, S_, false>), grid, dim3(64 * NW_), 0, st, p);         \
+  } while (0)
 #define FA_LAUNCH__(T_, F_, P_, D_, NW_)                                                           \
   do {                                                                                             \
     if (!P_ && p.softcap > 0.f) FA_LAUNCH___(T_, F_, false, D_, NW_, true);                        \
