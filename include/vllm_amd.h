@@ -497,8 +497,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 workgroups of a CU paired long + short; same output bits)          */
 /*   "pf_segs":    key segments of the 256-row prefill kernel (0 = heuristic; at most the  */
 /*                 num_segments the caller brings scratch for)                            */
-/*   "mm_kernel":  scaled_mm kernel: 0 = heuristic,             1 = register-   */
-/*                 staged 128x128 tile, 2..10 = direct-to-LDS tile shapes       */
+/*   "mm_kernel":  scaled_mm kernel: 0 = heuristic, 1 = register-staged 128x128    */
+/*                 tile, 2..10 = direct-to-LDS tile shapes       */
 /*                 (256x256, 128x128, 128x64, 64x64, 64x32; even ids 4..10      */
 /*                 take 2 or 4 K blocks per barrier; scaled_mm_large.hip),      */
 /*                 11 = weight-streaming kernel (M <= 32 only),                 */
@@ -513,7 +513,9 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 26..28 = 64x64 / 128x64 tiles with deeper rings (no gain),       */
 /*                 29..36 = 18..25 with 256 x 192 tiles (the heuristic takes them  */
 /*                 where they save a round of workgroups: N 6144),                 */
-/*                 37 = scaled_mm_stream.hip (M <= 64, K a multiple of 128)         */
+/*                 37 = scaled_mm_stream.hip (M <= 64, K a multiple of 128),        */
+/*                 38 = scaled_mm_kgroup.hip (128x128 tiles, two K groups; 16-byte   */
+/*                 aligned output rows, K a multiple of 128)                         */
 /*   "mm_patch":   tile columns per super-column of the scaled_mm_pp tile order    */
 /*                 (default 8; <= 1 = column-major)                                  */
 /*   "mm_store":   scaled_mm_pp measurement: 3 = no output stores (garbage)         */
@@ -526,9 +528,12 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 that decode kernel (0 = heuristic, 1 = never, 2 / 4 = that    */
 /*                 many where the shape allows)                                  */
 /*   "pf_fa":      the 256-row kernel of unified_attention /                   */
-/*                 context_attention_fwd (prefill_fa.hip; head sizes 72 .. 256, */
-/*                 causal mask, unified: + sliding window, softcap): 0 = for launches whose longest query chunk fills */
-/*                 a row block (default), 1 = never, 2 = whenever it applies   */
+/*                 context_attention_fwd (prefill_fa.hip; causal mask, unified: + sliding  */
+/*                 window, softcap): 0 = where it pays (default): head sizes 72 .. 256     */
+/*                 with enough row blocks that the longest query chunk fills, head sizes   */
+/*                 8 .. 256 split over the keys where few row blocks have long key ranges; */
+/*                 1 = never, 2 = whenever it applies (head sizes 72 .. 256)               */
+/*   "pf_fa_abl":  accepted, without effect                                             */
 /*   "pf_fa_stagger": 0 = all eight waves of that kernel stage in step (1 =    */
 /*                 default: waves 4-7 at the top of the tile interval)         */
 /*   "cache_runs": 0 = reshape_and_cache always per token (no run detection)    */

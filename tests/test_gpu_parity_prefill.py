@@ -304,16 +304,16 @@ def test_prefill_long_chunk_repeats_bit_for_bit(dtype, kv, ctx):
 @pytest.mark.parametrize("block_size", [16, 32])
 @pytest.mark.parametrize("head_size", [128, 112, 256])
 def test_prefill_fa_kernel_whole_tiles(oracle, force_fa, head_size, block_size, kv):
-    """Runs of whole 64-key tiles are staged without checks while two more whole tiles of the same kind follow: contexts and
-    chunks of 0 .. 5 whole tiles, ending on a tile, one key before and one behind; a head size
-    with padding columns, which has no such run."""
-    qls = [320, 64, 129, 255, 192, 65, 257, 128]
-    ctxs = [0, 64, 128, 191, 192, 193, 256, 321]
-    c = make_prefill_case(qls, ctxs, 4, 2, head_size, block_size, torch.bfloat16, kv, seed=head_size + block_size, kv_scale=0.02)
-    out = run(c, kv)
-    assert not out.isnan().any()
-    torch.testing.assert_close(out.float(), run_oracle(oracle, c, kv).float(), atol=tol(torch.bfloat16), rtol=0)
-    torch.testing.assert_close(out.float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)
+    """Runs of at least four whole 64-key tiles with two more whole tiles of the same kind behind them are staged without checks:
+    contexts and chunks of 0 .. 5 whole tiles (no such run) and of 6 .. 9, ending on a tile, one key before and one behind; a
+    head size with padding columns, which has no such run."""
+    for qls, ctxs in (([320, 64, 129, 255, 192, 65, 257, 128], [0, 64, 128, 191, 192, 193, 256, 321]),
+                      ([449, 384, 33, 130, 64, 512, 383, 577], [0, 385, 383, 384, 447, 448, 449, 513])):
+        c = make_prefill_case(qls, ctxs, 4, 2, head_size, block_size, torch.bfloat16, kv, seed=head_size + block_size, kv_scale=0.02)
+        out = run(c, kv)
+        assert not out.isnan().any()
+        torch.testing.assert_close(out.float(), run_oracle(oracle, c, kv).float(), atol=tol(torch.bfloat16), rtol=0)
+        torch.testing.assert_close(out.float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)
 
 
 @pytest.fixture
@@ -443,3 +443,31 @@ def test_prefill_wide_block_table(tuning, kv, head_size, heads):
     assert lib.vllm_amd_context_attention_fwd_segments(4, *heads, head_size, 64, 65536, 146, 0, 0, 0) > 1
     c.update(b_loc=wide, max_seq_len=None)
     torch.testing.assert_close(run(c, kv).float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)
+
+
+@pytest.mark.parametrize("heads", [(16, 8), (16, 16)])
+@pytest.mark.parametrize("n", [2, 24, 63, 64, 65])
+@pytest.mark.parametrize("skip_decode", [False, True])
+@pytest.mark.parametrize("majority", [True, False])
+def test_prefill_longest_first_order(tuning, heads, n, skip_decode, majority):
+    """Unsplit launches over whole kv heads per XCD hand out the row blocks of the longest sequence first where most of the
+    chunks have contexts of at least twice their length (up to 64 sequences; just below that majority, and from 65 sequences
+    on, they keep the plain order): ties among the lengths, several blocks per sequence, no query, one token (skipped or not)."""
+    kv = "fp8" if n % 2 else "auto"
+    qls = [(150, 40, 300 if i < 8 else 20, 1, 0, 70)[i % 6] for i in range(n)]
+    ctxs = [2 * q + (0, 17)[i % 2] for i, q in enumerate(qls)]
+    if not majority:   # one chunk more without a context than with one
+        live = [i for i, q in enumerate(qls) if q > (1 if skip_decode else 0)]
+        for i in live[:len(live) // 2 + 1]:
+            ctxs[i] = 2 * qls[i] - 1
+    c = make_prefill_case(qls, ctxs, *heads, 128, 16, torch.bfloat16, kv, seed=n, kv_scale=0.02)
+    ref, at = prefill_reference(c), c["b_start_loc"].tolist()
+    if skip_decode:
+        for i, q in enumerate(qls):
+            if q == 1:
+                ref[at[i]] = 0.0
+    tuning("pf_fa", 2)
+    tuning("pf_segs", 1)
+    out = run(c, kv, skip_decode=skip_decode)
+    assert not out.isnan().any()
+    torch.testing.assert_close(out.float(), ref, atol=tol(torch.bfloat16), rtol=0)

@@ -506,12 +506,13 @@ def test_unified_fa_kernel_softcap(oracle, force_fa, soft_cap, D, fp8, window):
 @pytest.mark.parametrize("D", [128, 112, 256])
 @pytest.mark.parametrize("window", [None, 130])
 def test_unified_fa_kernel_whole_tiles(oracle, force_fa, window, D, fp8):
-    """Runs of whole 64-key tiles are staged without checks while two more follow: sequences of 1 .. 8 whole tiles, ending
-    on a tile, one key before and one behind, with and without keys before the chunk; a head size with padding columns,
-    which has no such run."""
-    lens = [(320, 320), (64, 128), (129, 257), (255, 446), (192, 384), (65, 258), (257, 513), (128, 449)]
-    c = make_unified_case(lens, 4, 2, D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
-    run(oracle, c, torch.bfloat16, fp8=fp8, window=window)
+    """Runs of at least four whole 64-key tiles are staged without checks while two more follow: sequences of 1 .. 12 whole
+    tiles, ending on a tile, one key before and one behind, with and without keys before the chunk; a head size with padding
+    columns, which has no such run."""
+    for lens in ([(320, 320), (64, 128), (129, 257), (255, 446), (192, 384), (65, 258), (257, 513), (128, 449)],
+                 [(449, 449), (384, 769), (33, 416), (130, 514), (512, 512), (64, 512), (383, 766), (577, 577)]):
+        c = make_unified_case(lens, 4, 2, D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
+        run(oracle, c, torch.bfloat16, fp8=fp8, window=window)
 
 
 @pytest.mark.parametrize("segs", [2, 5, 32])

@@ -38,7 +38,6 @@ extern int g_uni_decode;
 extern int g_pf_fa;
 extern int g_pf_segs;
 extern int g_pf_fa_stagger;
-extern int g_pf_fa_abl;
 
 template <typename cache_t> struct CacheTraits;
 template <> struct CacheTraits<float> { static constexpr int X = 4; };
@@ -588,7 +587,7 @@ extern "C" int vllm_amd_set_tuning(const char* key, int value) {
   if (strcmp(key, "uni_decode") == 0) { g_uni_decode = value; return VLLM_AMD_OK; }
   if (strcmp(key, "pf_fa") == 0) { g_pf_fa = value; return VLLM_AMD_OK; }
   if (strcmp(key, "pf_segs") == 0) { g_pf_segs = value; return VLLM_AMD_OK; }
-  if (strcmp(key, "pf_fa_abl") == 0) { g_pf_fa_abl = value; return VLLM_AMD_OK; }
+  if (strcmp(key, "pf_fa_abl") == 0) return VLLM_AMD_OK;   // (kept for old scripts: the ablations are compile-time)
   if (strcmp(key, "pf_fa_stagger") == 0) { g_pf_fa_stagger = value; return VLLM_AMD_OK; }
   VA_REQUIRE(false, VLLM_AMD_EINVAL, "set_tuning: unknown key %s", key);
 }

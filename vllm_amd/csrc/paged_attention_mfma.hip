@@ -888,7 +888,9 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       // a token (us, 1500 tokens: head 64 fp8 7.5, head 128 fp8 9.9, 16-bit 14.6), the chip 1 us per 6.2 MB; the batch is
       // taken to be 0.6 full.  Up to 10 us only: a long sequence among short ones has to be cut.  Measured, cut -> one piece:
       // 1 x 600 fp8 10.5 -> 8.7, 1 x 1000 11.6 -> 10.4, 32 x 1000 17.8 -> 13.8, 32 x 1500 23.1 -> 18.7, 16 x 600 16-bit
-      // 14.5 -> 11.1; kept cut: 1 x 1000 16-bit 12.0 (one piece 12.9), 1 x 1500 fp8 11.4 (13.2), head 256 1 x 1000 15.2 (15.8).
+      // 14.5 -> 11.1; kept cut: 1 x 1000 16-bit 12.0 (one piece 12.9), 1 x 1500 fp8 11.4 (13.2), head 256 1 x 1000 15.2 (15.8)
+      // (device time alone, batches of 1 .. 32: profiles/decode_one_piece.txt -- never above the cheaper form where it leaves
+      // the cut; up to 1.2 x are left where 16 sequences of 1000 .. 1500 tokens stay cut).
       if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
         const double tb = 2.0 * p.head_size * (p.kv_dtype == VLLM_AMD_KV_AUTO ? 2 : 1), t = 3.5e-3 + tb * 12.2e-6;
         const double alone = p.max_seq_len * t, stream = 0.6 * (double)base * p.max_seq_len * tb / 6.2e6;

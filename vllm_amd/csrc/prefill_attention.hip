@@ -29,7 +29,6 @@ constexpr int PF_BN = 64;
 int g_pf_rows = 0;   // tuning "pf_rows": query rows per workgroup (0 = default)
 int g_uni_decode = 1;   // tuning "uni_decode": 0 = decode-only launches take the packed tile kernel
 extern int g_pf_fa_stagger;   // prefill_fa.hip
-int g_pf_fa_abl = 0;    // tuning "pf_fa_abl": measurement only, see prefill_fa.cuh
 int g_pf_segs = 0;      // tuning "pf_segs": key segments of the 256-row kernel (0 = heuristic; needs the caller's scratch)
 int g_pf_fa = 0;        // tuning "pf_fa": 1 = unified_attention never takes the 256-row kernel (prefill_fa.hip), 2 = whenever it can
 
@@ -906,7 +905,6 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       f.prefix = 0; f.k_new = f.v_new = nullptr; f.k_stride_t = f.k_stride_h = f.v_stride_t = f.v_stride_h = 0;
       f.blocks_per_seq = 0;
       f.num_segments = plan.nseg; f.seg_slots = plan.seg_slots; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
-      f.abl = g_pf_fa_abl;
       f.stagger = g_pf_fa_stagger;
       return launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
     }
@@ -989,7 +987,7 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
       const int tpb = (head_size > 128 ? 128 : 256) / pack;
       f.blocks_per_seq = p.flat_batch > 0 ? 0 : (max_input_len + tpb - 1) / tpb;
       f.num_segments = plan.nseg; f.seg_slots = plan.seg_slots; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
-      f.abl = 0; f.stagger = g_pf_fa_stagger;
+      f.stagger = g_pf_fa_stagger;
       launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
       return;
     }

@@ -33,8 +33,6 @@ struct FaParams {
   // seg_slots: workgroups per grid.y to deal out to the row blocks, at least one each.
   int num_segments, seg_slots;
   float* segm_out; float* segm_max; float* segm_sum;
-  int abl;             // (unused; the kernel's ablations are compile-time: -DVA_FA_ABL=bits, garbage results: 1 no exp2,
-                       // 2 no staging after the first tiles, 4 no S^T MFMAs, 8 no PV MFMAs, 16 no barrier)
 };
 
 // dtype: VLLM_AMD_F16 / VLLM_AMD_BF16 (queries, output, and the cache unless fp8)

@@ -1,7 +1,8 @@
 // unified_attention (vllm/attention/ops/triton_unified_attention.py:52-272, 588-700) and context_attention_fwd
-// (vllm/attention/ops/prefix_prefill.py:36-288, 726-913; the PREFIX instantiation below) for LONG query chunks at head
-// sizes 72 .. 128 with the causal + padding mask (unified: + sliding window): the matrix-core-bound case of prefill_attention.hip,
-// re-built around what bounds that kernel (16 query rows per wave = one LDS fragment byte per
+// (vllm/attention/ops/prefix_prefill.py:36-288, 726-913; the PREFIX instantiation below) with the causal + padding mask
+// (unified: + sliding window, softcap): chunks that fill row blocks, at head sizes 72 .. 256, and -- split over the keys, head
+// sizes 8 .. 256 -- any chunk of more than one token where few row blocks have long key ranges (fa_plan in
+// prefill_attention.hip).  The matrix-core-bound case of prefill_attention.hip, re-built around what bounds that kernel (16 query rows per wave = one LDS fragment byte per
 // 32 flops and ~300 VALU per 32 MFMAs; a 64-row tile restages every K / V tile for 64 rows).
 //
 //   * a workgroup = 8 waves = 256 tile rows; a wave owns 32 rows and computes with v_mfma_f32_32x32x16:
@@ -138,7 +139,7 @@ __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];
 // [d][token] (16-byte units XOR-swizzled by d >> 1) and the PV MFMA's A operand is one plain 16-byte read; the new
 // tokens take the unified path's row-major image and transposing reads.  Dense k / v are never fp8.
 //
-// D_ = 128, NW_ = 8: head sizes 72 .. 128, eight waves = 256 rows, two waves per SIMD.
+// D_ = 128, NW_ = 8: head sizes 72 .. 128 (split over the keys: 8 .. 128), eight waves = 256 rows, two waves per SIMD.
 // D_ = 256, NW_ = 4: head sizes 136 .. 256: O^T alone is 128 registers for a wave's 32 rows and Q^T 64, so a wave takes a
 // whole SIMD's register file: four waves = 128 rows, one per SIMD, 32 KiB tiles (128 KiB of LDS), 32 + 32 MFMAs per tile.
 // SOFTCAP (unified_attention): scores softcap * tanh(score / softcap) (triton_unified_attention.py:219-221): a pass of
@@ -159,8 +160,8 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
-  // ablations are compile-time (-DVA_FA_ABL=n, tools/fa_stamps.sh; bits in prefill_fa.cuh): a run-time branch
-  // around every MFMA costs the schedule it is meant to measure
+  // ablations are compile-time (-DVA_FA_ABL=bits, tools/fa_stamps.sh; garbage results: 1 no exp2, 2 no staging after the first
+  // tiles, 4 no S^T MFMAs, 8 no PV MFMAs): a run-time branch around every MFMA costs the schedule it is meant to measure
 #ifndef VA_FA_ABL
 #define VA_FA_ABL 0
 #endif
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   if (p.skip_decode && qlen == 1) return;
   const int new_end = min(tok_base + tpb, qlen);
   const int kvh = pack > 1 ? y : y / (p.num_heads / p.num_kv_heads);
-  // head sizes 72 .. 128 (multiples of 8; 16 with an fp8 cache) run padded to 128: the columns d >= dr of Q, K and V are
+  // head sizes up to 128 (multiples of 8; 16 with an fp8 cache) run padded to 128, above to 256: the columns d >= dr of Q, K and V are
   // staged as zeros from clamped addresses, the output columns are not stored
   const int dr = p.head_size;
 
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     const T* qp = (const T*)p.q + (int64_t)(tok0 + (rok ? rtok : 0)) * p.q_stride_t + (int64_t)(rok ? rhead : 0) * p.q_stride_h;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const bool dok = 16 * ks + 8 * hi < dr;   // head sizes below 128: zero columns
+      const bool dok = 16 * ks + 8 * hi < dr;   // padded head sizes: zero columns
       const u32x4 v = *reinterpret_cast<const u32x4*>(qp + (dok ? 16 * ks + 8 * hi : 0));
       qf[ks] = (rok && dok) ? v : (u32x4){0, 0, 0, 0};
     }
@@ -777,7 +778,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
       // (behind the compute the fragment rings are dead: room for the conversion temporaries)
       if (!stage_first) stage(t, fast_c, vt_c);
       FA_T(0);
-      if (!(abl & 16)) __syncthreads();
+      __syncthreads();
       FA_T(5);
     }
   };

@@ -390,11 +390,11 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
           // profiles/r03_gemm_sweep_rotating.csv: the 64 x 64 tile with one K block per barrier wins at
           // every K: 4096 x 4096 at M 256 12.7 vs 15.2 us, 4096 x 6144 at M 128 13.4 vs 15.9 us)
           sel = (nt > 256 || K % (128 * t.kb) != 0 || i == 3) ? t.id : t.id_kb;
-          // Even the smallest tile leaves half the CUs idle and the K loop is long: two K
-          // slices (in-kernel fix-up, scaled_mm_large.hip).  The fix-up is a chain of three
-          // device-scope round trips (~2.5 us), so it pays only here: 14336x4096, M 16..64:
-          // 17.2 -> 15.2 us; everywhere else on the grid splitting loses
-          // (profiles/r01_gemm_sweep_splitk.csv; at K = 8192 it is 11.5 vs 11.1 us).
+          // Even the smallest tile leaves half the CUs idle and the K loop is long: two K slices (in-kernel fix-up,
+          // scaled_mm_large.hip).  The fix-up is a chain of three device-scope round trips (~2.5 us), so it pays only
+          // here.  (M <= 64 never comes this far, scaled_mm_stream_pays.)  M 65 .. 128, N 512 .. 2048, unsplit -> two
+          // slices: K 12288 15.1 .. 22.0 -> 12.6 .. 16.6 us, K 14336 16.8 .. 25.1 -> 13.6 .. 18.6, K 28672 33.4 .. 46.4 ->
+          // 22.0 .. 29.7 (profiles/gemm_two_slices.txt); at K 8192 it loses (profiles/r01_gemm_sweep_splitk.csv).
           if (i == 4 && nt <= 128 && K >= 12288 && want_splits == 0) splits = 2;
           break;
         }
