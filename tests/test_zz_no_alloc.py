@@ -41,9 +41,9 @@ def _call_static(a, w, sa, sb, splits):
 @pytest.mark.parametrize("splits", [0, 2, 4])
 def test_scaled_mm_static_matches_existing_entry(ops, splits):
     from vllm_amd import _lib
-    # the first two are the weight-streaming kernel's with splits = 0; the others the heuristic splits in two (M > 64, at
-    # most 128 tiles of 64 x 32, K >= 12288): the largest such grid, and ragged edges
-    for M, N, K in ((48, 2048, 14336), (17, 520, 12288), (100, 2048, 14336), (65, 520, 12288)):
+    # the second is the weight-streaming kernel's with splits = 0; the others the heuristic splits in two (at most 128 tiles
+    # of 64 x 32, K >= 12288, M K > 600000): the largest such grids, and ragged edges
+    for M, N, K in ((48, 2048, 14336), (17, 520, 12288), (100, 2048, 14336), (65, 520, 12288), (64, 4096, 12288), (42, 520, 14336)):
         a, w, sa, sb = _make(M, N, K, M + N)
         try:
             _lib.set_tuning("mm_splitk", 1)

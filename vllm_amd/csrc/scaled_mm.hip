@@ -272,6 +272,7 @@ int launch_scaled_mm_large(int shape, void* out, const void* a, const void* b,
                            int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
                            int out_dtype, bool vec, int splits, int ws_mode, hipStream_t st);
 bool scaled_mm_large_fits(int M, int N, int K, int64_t lda, int64_t ldb);
+bool scaled_mm_large_can_split(int M, int N, int bm, int bn, int splits, int ws_mode, hipStream_t st);
 // scaled_mm_stream.hip
 bool scaled_mm_stream_pays(int M, int N, int K);
 int launch_scaled_mm_stream(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
@@ -311,9 +312,15 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
              VLLM_AMD_EINVAL, "%s: scales must be per-tensor or per-row/per-column", op);
   const bool glds_ok = K % 128 == 0 && K >= 256 && scaled_mm_large_fits(M, N, K, lda, ldb);
   const int want_splits = req_splits > 0 ? req_splits : g_mm_splitk;   // 0 = heuristic
-  // M <= 64: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it)
+  const bool vec = (ldc % 4 == 0) && ((((uintptr_t)out) & 7) == 0);
+  // M <= 64: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it) -- but where the activations that
+  // every workgroup of it reads (M x K bytes) pass 600 KB and N is small, two K slices of the 64 x 32 tile (below) win if there
+  // is a workspace for them: N 4096, stream / slices in us, K 14336 at M 33 16.7 / 17.6, M 48 19.5 / 19.0, M 64 21.9 / 20.3;
+  // K 28672 at M 17 25.7 / 26.8, M 32 29.0 / 28.2, M 64 39.8 / 33.9 (profiles/gemm_stream.txt).
+  const bool slices = g_mm_kernel == 0 && want_splits == 0 && glds_ok && vec && K >= 12288 && ceil_div(N, 32) <= 128 &&
+                      M <= 64 && M * K > 600000 && scaled_mm_large_can_split(M, N, 64, 32, 2, ws_mode, st);
   if (glds_ok && M <= 64 &&
-      (g_mm_kernel == 37 || (g_mm_kernel == 0 && want_splits == 0 && scaled_mm_stream_pays(M, N, K)))) {
+      (g_mm_kernel == 37 || (g_mm_kernel == 0 && want_splits == 0 && !slices && scaled_mm_stream_pays(M, N, K)))) {
     launch_scaled_mm_stream(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel, out_dtype, st);
     VA_LAUNCH_CHECK(op);
     return VLLM_AMD_OK;
@@ -338,7 +345,6 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
     return VLLM_AMD_OK;
   }
   const int tiles = ceil_div(M, BM) * ceil_div(N, BN);
-  const bool vec = (ldc % 4 == 0) && ((((uintptr_t)out) & 7) == 0);
   if (glds_ok) {
     int sel = g_mm_kernel;
     int splits = want_splits > 0 ? want_splits : 1;
@@ -392,9 +398,9 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
           sel = (nt > 256 || K % (128 * t.kb) != 0 || i == 3) ? t.id : t.id_kb;
           // Even the smallest tile leaves half the CUs idle and the K loop is long: two K slices (in-kernel fix-up,
           // scaled_mm_large.hip).  The fix-up is a chain of three device-scope round trips (~2.5 us), so it pays only
-          // here.  (M <= 64 never comes this far, scaled_mm_stream_pays.)  M 65 .. 128, N 512 .. 2048, unsplit -> two
-          // slices: K 12288 15.1 .. 22.0 -> 12.6 .. 16.6 us, K 14336 16.8 .. 25.1 -> 13.6 .. 18.6, K 28672 33.4 .. 46.4 ->
-          // 22.0 .. 29.7 (profiles/gemm_two_slices.txt); at K 8192 it loses (profiles/r01_gemm_sweep_splitk.csv).
+          // here.  (M <= 64 comes this far for it only, see the stream kernel above.)  M 65 .. 128, N 512 .. 2048, unsplit -> two
+          // slices: K 12288 16.1 .. 22.7 -> 13.2 .. 17.1 us, K 14336 18.2 .. 25.4 -> 14.4 .. 18.8, K 28672 33.5 .. 48.1 ->
+          // 22.1 .. 30.5 (profiles/gemm_two_slices.txt); at K 8192 0.99 .. 1.19 x, not taken.
           if (i == 4 && nt <= 128 && K >= 12288 && want_splits == 0) splits = 2;
           break;
         }

@@ -239,9 +239,9 @@ __global__ __launch_bounds__(768) void scaled_mm_kgroup_kernel(const Params p) {
 
 // Single rounds of 128 x 128 tiles, 160 .. 256 of them.  Against the kernels of scaled_mm_large.hip that served these shapes
 // (the same tile with both waves of a SIMD in step, from 190 tiles on; 128 x 64 tiles below), weights from HBM, 145 shapes of
-// K 1024 .. 14336, N 1280 .. 28672, M 72 .. 3200 with that many tiles (profiles/gemm_kgroup.txt): 0.99 .. 1.09 x at K 1024,
-// 1.06 .. 1.21 at 2048 (but 2048 x 2048 at M 2000 0.94), 1.06 .. 1.31 at 4096, 1.06 .. 1.43 at 8192 and 14336.  Below 160 tiles the smaller tiles fill more CUs (144 tiles: 0.99 .. 1.25 x, 128: 0.73 .. 0.81), above 256
-// two workgroups of the smaller rings share a CU (320 and 448 tiles: 0.75 .. 1.03).
+// K 1024 .. 14336, N 1280 .. 28672, M 72 .. 3200 with that many tiles (profiles/gemm_kgroup.txt): 0.99 .. 1.10 x at K 1024,
+// 1.02 .. 1.24 at 2048, 1.02 .. 1.33 at 4096, 1.05 .. 1.37 at 8192, 1.05 .. 1.44 at 14336.  Below 160 tiles the smaller tiles fill more CUs (144 tiles: 0.96 .. 1.24 x, 128: 0.71 .. 0.77), above 256
+// two workgroups of the smaller rings share a CU (320 and 448 tiles: 0.81 .. 1.03).
 bool scaled_mm_kgroup_pays(int M, int N, int K) {
   const int64_t tiles = (int64_t)ceil_div(M, mmk::BM) * ceil_div(N, mmk::BN);
   return M > 64 && tiles >= 160 && tiles <= 256;

@@ -827,6 +827,15 @@ static int launch_glds_shape(int shape, const GldsArgs& g) {
   }
 }
 
+// Whether a launch of bm x bn tiles in `splits` K slices would get its scratch now (else launch_scaled_mm_large runs unsplit).
+bool scaled_mm_large_can_split(int M, int N, int bm, int bn, int splits, int ws_mode, hipStream_t st) {
+  if (ws_mode == 1) return true;   // (the static scratch holds every split of the heuristic, or the launch is an error)
+  const int tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  float* ws;
+  unsigned* ctr;
+  return split_workspace(st, (size_t)tiles * splits * bm * bn * sizeof(float), tiles, &ws, &ctr);
+}
+
 // The kernels address their operands with 32-bit byte offsets.
 bool scaled_mm_large_fits(int M, int N, int K, int64_t lda, int64_t ldb) {
   const int64_t lim = (int64_t)1 << 32;

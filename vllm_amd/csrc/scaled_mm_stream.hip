@@ -323,17 +323,22 @@ static void launch(const Params& p0, hipStream_t st) {
 
 }  // namespace mms
 
-// Whether launch_scaled_mm_stream is the better kernel (against the tile kernels, weights from HBM).  M <= 32: everywhere.
-// Above, a 32-column tile's stage is 3 .. 4 blocks of activations to 2 of weights, and the tile kernels, which share them
-// between more columns, win unless N is small (us, tiles -> stream: 14336 -> 4096 at M 64 27.5 -> 21.7, 8192 -> 7168 18.4 ->
-// 17.0), a workgroup can keep them (4096 -> 28672 30.1 -> 25.8) or M <= 48 leaves room (4096 -> 6144 9.8 -> 9.0); they keep
-// 4096 -> 6144 (10.7 : 10.3) and 3584 -> 8192 (10.2 : 10.3) at M 64, and 8192 -> 14336 from M 33 on (27.0 : 29.4).
+// Whether launch_scaled_mm_stream is the better kernel (against the tile kernels, weights from HBM; us, tiles -> stream; all
+// shapes: profiles/gemm_stream.txt).  M <= 32: up to 256 32-column tiles everywhere (0.98 .. 1.9 x).  With more, keeping the
+// activations costs a workgroup a start of 4 .. 5 us that K has to earn back: M 17, 1024 -> 14336 6.0 -> 9.1, 2048 -> 10240
+// 8.1 -> 9.3, 3072 -> 10240 10.7 -> 10.4, 4096 -> 28672 27.9 -> 21.0.
+// M > 32: a 32-column tile's stage is 3 .. 4 blocks of activations to 2 of weights, and the tile kernels, which share them
+// between more columns, win unless N is small (8192 -> 4096 at M 64 16.6 -> 13.5), a workgroup can keep them (4096 -> 28672
+// 29.7 -> 25.9; but 64 x 64 tiles that just make one round need K 4096: 3584 -> 14336 at M 49 13.0 -> 14.4, 4096 -> 14336
+// 15.5 -> 15.2) or M <= 48 leaves room (4096 -> 6144 8.7 -> 8.4, from K 3072 on: 2048 -> 8192 at M 48 6.3 -> 6.7); they keep
+// 4096 -> 6144 (10.4 : 10.3) and 3584 -> 8192 (9.8 : 10.1) at M 64, and more than 256 tiles over K above 4096 (8192 -> 14336 at
+// M 49, 64 27.9, 28.9 : 28.2, 30.9; not at M 33, 27.6 : 25.2).
 bool scaled_mm_stream_pays(int M, int N, int K) {
-  if (M <= 32) return true;
   if (M > 64) return false;
-  const int t32 = ceil_div(N, 32);
-  if (t32 < 160) return true;
-  return K <= 4096 ? M <= 48 || t32 > 256 : t32 <= 256;
+  const int t32 = ceil_div(N, 32), t64 = ceil_div(N, 64);
+  if (t32 > 256 && (K < 3072 || (M > 32 && K < 4096 && t64 >= 190 && t64 <= 256))) return false;
+  if (M <= 32 || t32 < 160) return true;
+  return K <= 4096 ? K >= 3072 && (M <= 48 || t32 > 256) : t32 <= 256;
 }
 
 // Caller guarantees 1 <= M <= 64, K % 128 == 0, 16-byte aligned operands and scaled_mm_large_fits() (32-bit offsets).

@@ -76,8 +76,8 @@ inline void* vptr(const OptTensor& t) { return t.has_value() ? t->data_ptr() : n
 // scaled_mm -- and before its first paged_attention_v1 only when the balanced form ("pa_balance" = 1,
 // off by default) is on: nothing else of that op uses it.  Without it the GEMM never splits over K.
 // One host synchronisation, in that first call.  Launches under stream capture never take a workspace
-// slot, so a captured GEMM runs unsplit: split-K (M above 64, few 64 x 32 tiles, K >= 12288: M 96, N 2048, K 14336
-// 20.4 -> 16.2 us) is an eager-launch optimisation; bench.py's graph-timed GEMM legs time the unsplit form.
+// slot, so a captured GEMM runs unsplit: split-K (M up to 128, few 64 x 32 tiles, K >= 12288: M 96, N 2048, K 14336
+// 20.5 -> 16.3 us) is an eager-launch optimisation; bench.py's graph-timed GEMM legs time the unsplit form.
 constexpr int64_t kWsBytes = (64ll << 20) + (512ll << 10);
 std::mutex g_ws_mu;
 Tensor g_ws[64];
