@@ -654,3 +654,14 @@ def test_unified_prefill_key_segments_among_decodes(oracle, n, fp8):
             run(oracle, c, torch.bfloat16, fp8=fp8)
         finally:
             _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,heads", [(80, (8, 2)), (128, (32, 8)), (256, (8, 4)), (64, (8, 2))])
+@pytest.mark.parametrize("window", [100, 600, 1500])
+@pytest.mark.parametrize("soft_cap", [None, 30.0])
+def test_unified_window_far_behind(oracle, fp8, D, heads, window, soft_cap):
+    """Windows that leave more than 16 key tiles of the longest sequence out: chunks of any length take the 256-row kernel, in
+    one piece (100), cut by the keys that a row block walks (600) or by all of them (1500); shorter sequences beside it."""
+    c = make_unified_case([(200, 2600), (3, 1500), (70, 70), (1, 700)], *heads, D, 16, torch.bfloat16, fp8=fp8, seed=D + window)
+    run(oracle, c, torch.bfloat16, window=window, softcap=soft_cap or 0.0, fp8=fp8)

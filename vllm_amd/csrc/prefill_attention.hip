@@ -770,11 +770,13 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 // kernel: 64 fresh tokens under a table for 8192 7.5 -> 13.3), ptok: query tokens of the chunks, nchunk: sequences among them
 // (a lower bound will do), cap: segments the caller has scratch for.
 //   * >= 128 row blocks, chunks of at least one: unsplit.  Without decodes beside the chunks from 64 on, over the flash-layout
-//     cache at head sizes up to 128 only in 16 bits and from 512 keys (min_blocks).  us, 64-row kernel -> this one: x-layout fp8
+//     cache at head sizes up to 128 only in 16 bits and from 512 keys (min_blocks; exactly 64, one round of the 64-row kernel,
+//     only with a context: 1 x 512 fresh 16-bit tokens 21.7 against 22.9, 560 24.7 -> 23.2).  us, 64-row kernel -> this one: x-layout fp8
 //     1000 tokens, 32 / 8 heads (120 blocks) 41.3 -> 33.1, 600 over 200 (72) 35.5 -> 31.5, head 256 900 tokens (112) 89.0 ->
 //     46.6; flash layout 16-bit 800 (96) 32.0 -> 28.5, head 256 600 over 200 (72) 58.9 -> 42.4; but fp8 1000 (120) 31.7 ->
 //     33.7, 2 x 500 24.4 -> 27.8, 16-bit 400 + 300 over 100 (80) 21.1 -> 22.8.  Windows narrower than half the keys count as
-//     16 bits: this kernel does not stage the tiles left of them (fp8, 900 tokens, window 128: 21.5 -> 15.6).
+//     16 bits: this kernel does not stage the tiles left of them (fp8, 900 tokens, window 128: 21.5 -> 15.6).  Windows that leave
+//     16 tiles out: any chunk (64 tokens over 8000 with a window of 128 105 -> 16, 16-bit 170 -> 16).
 //   * fewer: the 64-row kernel's four times as many workgroups finished sooner than that (chunk 256 over 4096 cached tokens
 //     among 255 decodes: 32 blocks, 82 against 150 us) and still left the chip idle behind one serial walk over the keys
 //     (2.1 us per 64-key tile).  Split, 256 workgroups are dealt out to the blocks there are; a segment is worth its start-up
@@ -782,19 +784,24 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 //     split: 35 tokens over 3723, 8 q / 1 kv head 123 -> 32; 512 over 8000, 32 / 8 208 -> 87; 1024 over 4000 139 -> 102; head
 //     64, 300 over 3000 87 -> 33; head 256, 2 x 300 over 3000 159 -> 60; x-layout prefix, 300 over 3000 106 -> 37.
 struct FaPlan { bool use; int nseg, seg_slots; };
-static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap,
-                      int64_t num_tokens, int num_seqs, int min_blocks = 128) {
+// flash: unified_attention's cache (at head sizes up to 64 its 64-row kernel is the faster one); window: 0 = none, as given
+static FaPlan fa_plan(bool flash, int head_size, int num_heads, int num_kv_heads, int max_q, int max_k, int64_t ptok, int nchunk, int cap,
+                      int64_t num_tokens, int num_seqs, int window = 0, int min_blocks = 128) {
   const int gqa = num_heads / num_kv_heads;
   const int pack = (gqa > 1 && gqa <= 16) ? gqa : 1;
   const int tpb = (head_size > 128 ? 128 : 256) / pack;
   const int y = pack > 1 ? num_kv_heads : num_heads;
   if (g_pf_fa == 1 || g_pf_rows != 0 || (max_q <= 1 && g_pf_fa != 2) || head_size > 256) return {false, 1, 0};
-  const bool whole = head_size > 64 && (g_pf_fa == 2 || (max_q >= tpb && ptok / tpb * y >= min_blocks));
+  const bool whole = head_size > 64 && (g_pf_fa == 2 || min_blocks == 0 || (max_q >= tpb && ptok * y >= (int64_t)min_blocks * tpb));
+  // Under a window this kernel walks the window and the block's own tokens, and is what a split competes with where it would
+  // run unsplit; the 64-row kernel stages every key.
+  const bool reach = whole && window > 0 && window < max_k - 255;
+  const int keys = reach ? window + 255 : max_k;
   int64_t blocks = (ptok + tpb - 1) / tpb;
   if (blocks < nchunk) blocks = nchunk;
   blocks *= y;
-  int nseg = blocks > 0 && blocks <= 128 && max_k >= 16 * PF_BN ? (int)(256 / blocks) : 1;
-  const int by_len = max_k / (3 * PF_BN);
+  int nseg = blocks > 0 && blocks <= 128 && keys >= (reach ? 8 : 16) * PF_BN ? (int)(256 / blocks) : 1;
+  const int by_len = keys / ((!reach ? 3 : blocks <= 16 ? 1 : 2) * PF_BN);
   if (nseg > by_len) nseg = by_len;
   if (nseg > cap) nseg = cap;
   if (nseg > FA_MAX_SEGMENTS) nseg = FA_MAX_SEGMENTS;
@@ -805,8 +812,21 @@ static FaPlan fa_plan(int head_size, int num_heads, int num_kv_heads, int max_q,
   // among 200 of 4096 400 / 319; and where max_k is a decode's, 100 fresh tokens among 60 of 3000 76 / 75, 500 over 100 among
   // 30 of 1500 48 / 45.
   const int64_t launched = (num_tokens / tpb + num_seqs) * y;
-  const double walk = (max_k - 0.5 * (max_q < max_k ? max_q : max_k)) / PF_BN;   // mean over the rows of the longest chunk
+  const double walk = (keys - 0.5 * (max_q < keys ? max_q : keys)) / PF_BN;   // mean over the rows of the longest chunk
   if (nseg > 1 && walk * 1.9 * (1.0 - 1.0 / nseg) < 2.0 * (4.0 + (double)(launched > 256 ? launched : 256) * 4.5e-3)) nseg = 1;
+  // ... and where the partials, written and read, do not cost more than it saves: many rows over few keys are faster in one
+  // piece.  Fitted to 680 launches in 2 .. 32 segments against the unsplit kernel (residual 2 us): what a tile less of the longest
+  // walk gives, what the split costs at all, per MB, and with q head groups above 4.  us, unsplit / split: 64 / 8 heads 512 over
+  // 512 37.5 / 47.3, over 1200 53.6 / 57.4; 32 / 8 1024 over 300 44.2 / 47.1, over 600 51.5 / 49.4, 2 x 512 over 600 39.7 / 44.1,
+  // 560 over 500 in three 36.7 / 35.3, 1024 over 6000 with a window of 128 19.0 / 34.5 (of 1024 40.5 / 46.4); head 64, 64-row
+  // kernel / split: 2 x 512 over 600 36.5 / 39.7.  Several chunks that the 64-row kernel would take are left to the rule above
+  // (8 x 100 over 1000 44.1 / 41.0), and so is the x layout at head sizes up to 64 (2 x 512 over 600 48.3 / 40.1).
+  if (nseg > 1 && (head_size > 64 ? whole || nchunk == 1 : flash)) {
+    const double mb = (double)ptok * num_heads * nseg * head_size * 8e-6, last = (double)keys / PF_BN * (1.0 - 1.0 / nseg);
+    const double gain = head_size > 128 ? 2.55 * last : 1.62 * last;
+    const double cost = (head_size > 128 ? 9.0 + 0.11 * mb : 5.0 + (head_size > 64 ? 0.22 : 0.36) * mb) + (gqa > 4 ? 3.0 : 0.0);
+    if (gain < cost * (nseg > 2 ? 0.95 : 1.0)) nseg = 1;
+  }
   int slots = 256 / y;
   if (g_pf_segs > 0) {   // every block that many, wherever there are tiles
     nseg = g_pf_segs < cap ? g_pf_segs : cap;
@@ -886,9 +906,13 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
                      p.kc_page_bytes < (1 << 27) && p.vc_page_bytes < (1 << 27);
     const int64_t ptok = mixed ? (int64_t)num_tokens - batch : (int64_t)num_tokens;   // ~ tokens of the chunks
     const bool narrow = p.sliding_window > 0 && 2 * (int64_t)p.sliding_window <= max_k;
-    const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
-                                num_tokens, batch,
-                                !mixed && (head_size > 128 || narrow || (!FP8 && max_k >= 512)) ? 64 : 128);
+    // (a window that leaves 16 tiles out: any chunk)
+    const int min_blocks = mixed ? 128
+                           : p.sliding_window > 0 && (int64_t)max_k - p.sliding_window >= 255 + 16 * PF_BN ? 0
+                           : head_size > 128 || narrow ? 64
+                           : !FP8 && max_k >= 512 ? (max_k < 600 ? 65 : 64) : 128;
+    const FaPlan plan = fa_plan(true, head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
+                                num_tokens, batch, p.sliding_window, min_blocks);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -965,8 +989,9 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
     const bool can = p.alibi_slopes == nullptr && p.sliding_window == 0 && p.sm_scale > 0.f &&
                      (block_size & (block_size - 1)) == 0 && p.k_stride_t < (1 << 27) && p.v_stride_t < (1 << 27);
     const int64_t ptok = p.flat_batch > 0 ? (int64_t)p.flat_tokens : (int64_t)max_input_len * batch;
-    const FaPlan plan = fa_plan(head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
-                                p.flat_batch > 0 ? p.num_segments : 1, ptok, batch, p.skip_decode ? 128 : 64);
+    const FaPlan plan = fa_plan(false, head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
+                                p.flat_batch > 0 ? p.num_segments : 1, ptok, batch, 0,
+                                p.skip_decode ? 128 : !FP8 && head_size <= 128 && max_k <= max_input_len ? 65 : 64);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -1292,7 +1317,7 @@ extern "C" int vllm_amd_context_attention_fwd_segments(int batch, int num_heads,
                                                        int max_seq_len, int num_tokens, int has_alibi, int sliding_window,
                                                        int skip_decode) {
   if (batch <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || num_tokens <= 0 || has_alibi || sliding_window > 0) return 1;
-  return fa_plan(head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch, FA_MAX_SEGMENTS,
+  return fa_plan(false, head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch, FA_MAX_SEGMENTS,
                  num_tokens, batch).nseg;
 }
 
@@ -1304,7 +1329,7 @@ extern "C" int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, 
   if (max_seqlen_q == 1) return num_seqs * num_kv_heads * ((num_heads / num_kv_heads + 15) / 16) < 1024 ? 16 : 1;
   if (has_alibi) return 1;
   const bool mixed = num_seqs >= 16 && (int64_t)num_tokens < (int64_t)num_seqs * max_seqlen_q;   // (launch_unified)
-  return fa_plan(head_size, num_heads, num_kv_heads, max_seqlen_q, max_seqlen_k, mixed ? num_tokens - num_seqs : num_tokens,
+  return fa_plan(true, head_size, num_heads, num_kv_heads, max_seqlen_q, max_seqlen_k, mixed ? num_tokens - num_seqs : num_tokens,
                  mixed ? 1 : num_seqs, FA_MAX_SEGMENTS, num_tokens, num_seqs).nseg;
 }
 
