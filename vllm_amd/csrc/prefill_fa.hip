@@ -187,19 +187,28 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   int seq = 0, blk = -1;   // sequence, row block in it
   int seg = 0, segs = 1;   // split launches: key segment, segments of this block
   int y, gs, g;
+  int tok0 = 0, qlen = 0, seq_len = 0;
   if constexpr (SPLIT) {
     // The row blocks there really are, and seg_slots workgroups dealt out to them: as num_segments workgroups for each
     // block there may be, a launch spent 2.2 ns on each one of a sequence that the decode kernel takes (100 fresh tokens among
     // 60 decodes of 3000 keys, 32 / 8 heads: 4032 workgroups, whole step 86.7 us, now 75.1; 200 over 3800 among 100 of 700: 91.7
     // -> 66.0).  The work goes evenly over the XCDs: a few blocks too many on one of them double up on its CUs (512 over 7488,
     // 8 q / 1 kv head: 60 against 40 us).
-    auto blocks_of = [&](int i) __attribute__((always_inline)) {
-      const int ql = i < p.num_seqs ? p.cu_seqlens_q[i + 1] - p.cu_seqlens_q[i] : 0;
-      return p.skip_decode && ql == 1 ? 0 : (ql + tpb - 1) / tpb;
+    struct Seq { int tok0, qlen, len, blocks; };
+    auto seq_at = [&](int i) __attribute__((always_inline)) {   // (lengths too: the found sequence's need no load of their own)
+      Seq q = {0, 0, 0, 0};
+      if (i < p.num_seqs) {
+        q.tok0 = p.cu_seqlens_q[i];
+        q.qlen = p.cu_seqlens_q[i + 1] - q.tok0;
+        q.len = p.seq_lens[i];
+        q.blocks = p.skip_decode && q.qlen == 1 ? 0 : (q.qlen + tpb - 1) / tpb;
+      }
+      return q;
     };
-    int n = blocks_of(lane), incl = wave_scan(n);             // the first 64 sequences stay in registers
+    Seq my = seq_at(lane);                                    // the first 64 sequences stay in registers
+    int incl = wave_scan(my.blocks);
     int here = __builtin_amdgcn_readlane(incl, 63), total = here;
-    for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(blocks_of(i + lane)), 63);
+    for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(seq_at(i + lane).blocks), 63);
     if (total == 0) return;
     const int work = max(total, min(p.seg_slots, total * nseg));   // per head
     const int w = xcd_order(work * (int)gridDim.y);
@@ -213,14 +222,17 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     b = total - 1 - b;                                        // later (longer) row blocks first
     for (int i = 0; i < p.num_seqs; i += 64) {
       if (i > 0) {
-        n = blocks_of(i + lane);
-        incl = wave_scan(n);
+        my = seq_at(i + lane);
+        incl = wave_scan(my.blocks);
         here = __builtin_amdgcn_readlane(incl, 63);
       }
       if (b < here) {
         const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(b < incl)) - 1);
         seq = i + l;
-        blk = b - __builtin_amdgcn_readlane(incl - n, l);
+        blk = b - __builtin_amdgcn_readlane(incl - my.blocks, l);
+        tok0 = __builtin_amdgcn_readlane(my.tok0, l);
+        qlen = __builtin_amdgcn_readlane(my.qlen, l);
+        seq_len = __builtin_amdgcn_readlane(my.len, l);
         break;
       }
       b -= here;
@@ -262,10 +274,10 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
       blk = g - (p.cu_seqlens_q[seq] / tpb + seq);
       if (blk < 0) return;                // rows in front of the first sequence (cu_seqlens_q may start above 0)
     }
+    tok0 = p.cu_seqlens_q[seq];
+    qlen = p.cu_seqlens_q[seq + 1] - tok0;
+    seq_len = p.seq_lens[seq];
   }
-  const int tok0 = p.cu_seqlens_q[seq];
-  const int qlen = p.cu_seqlens_q[seq + 1] - tok0;
-  const int seq_len = p.seq_lens[seq];
   const int ctx = seq_len - qlen;
   // first query token of this block
   const int tok_base = blk * tpb;
@@ -885,15 +897,17 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
   const int lane = threadIdx.x & 63;
   const int pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tok = pair / p.num_heads, head = pair % p.num_heads;
-  if (tok >= p.num_tokens || tok < p.cu_seqlens_q[0] || tok >= p.cu_seqlens_q[p.num_seqs]) return;
+  if (tok >= p.num_tokens) return;
+  const int nseg = p.num_segments, dr = p.head_size;
+  const int64_t row = ((int64_t)tok * p.num_heads + head) * nseg;
+  // (in front of the checks, not behind their loads; rows that nobody wrote are not used)
+  float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
+  float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
+  if (tok < p.cu_seqlens_q[0] || tok >= p.cu_seqlens_q[p.num_seqs]) return;
   if (p.skip_decode) {
     const int lo = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] <= tok; });
     if (p.cu_seqlens_q[lo + 1] - p.cu_seqlens_q[lo] == 1) return;   // the decode kernel's token
   }
-  const int nseg = p.num_segments, dr = p.head_size;
-  const int64_t row = ((int64_t)tok * p.num_heads + head) * nseg;
-  float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
-  float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
   const float last = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ls), nseg - 1));
   const int live = last < 0.f ? (int)-last : nseg;
   if (live == 1) return;             // the only segment has written the output
