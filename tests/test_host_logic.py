@@ -259,3 +259,18 @@ def test_fp8_linear_static_zero_dim_scale_is_not_sliced(monkeypatch):
     out = op.apply(torch.zeros((3, 32), dtype=torch.bfloat16), torch.zeros((32, 16), dtype=torch.float8_e4m3fn),
                    torch.ones(16, 1), input_scale=scale)
     assert out.shape == (3, 16) and seen["sa"] is scale
+
+
+def test_prefill_key_segments_plan():
+    """What the prefill launches answer about their split (host arithmetic): long contexts of few tokens are cut, many rows over
+    few keys, fresh prompts and decode-like calls are not, and the scratch of a mixed batch is bounded."""
+    from vllm_amd._lib import lib
+    uni, ctx = lib.vllm_amd_unified_attention_segments, lib.vllm_amd_context_attention_fwd_segments
+    assert uni(1, 32, 8, 128, 512, 8000, 512, 0) > 1 and ctx(1, 32, 8, 128, 512, 8000, 512, 0, 0, 0) > 1
+    assert uni(1, 64, 8, 128, 512, 1024, 512, 0) == 1 and ctx(1, 64, 8, 128, 512, 1024, 512, 0, 0, 0) == 1
+    assert uni(1, 32, 8, 128, 300, 300, 300, 0) == 1 and uni(1, 32, 8, 128, 512, 8000, 512, 1) == 1
+    assert ctx(1, 32, 8, 128, 512, 8000, 512, 0, 128, 0) == 1
+    for tokens, heads, d in ((2064, 32, 128), (4096, 64, 256), (600, 8, 64), (64, 32, 128)):
+        for n in (uni(tokens - 63, heads, 8, d, 64, 131072, tokens, 0), ctx(tokens - 63, heads, 8, d, 64, 131072, tokens, 0, 0, 1)):
+            assert 1 <= n <= 32 and (n == 1 or tokens * heads * n * (d + 2) * 4 <= 256 << 20)
+    assert uni(2001, 32, 8, 128, 64, 131072, 2064, 0) > 1

@@ -1312,25 +1312,33 @@ extern "C" int vllm_amd_context_attention_fwd_split(
   return context_attention(o, q, k, v, k_cache, v_cache, b_loc, b_start_loc, b_seq_len, k_scale, v_scale, alibi_slopes, fp8_out_scale, batch, num_heads, num_kv_heads, head_size, block_size, max_input_len, b_loc_stride, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h, kc_block_stride, kc_head_stride, vc_block_stride, vc_head_stride, sm_scale, sliding_window, skip_decode, num_tokens, dtype, kv_cache_dtype, stream, segm_output, segm_max, segm_expsum, num_segments, max_seq_len);
 }
 
+// Segments whose scratch stays within 256 MiB.  Chunks alone never need more than 34 MB, but it has a row for every token of
+// the batch: 64 tokens over a long context among 2000 decodes, 32 heads, would have asked for 1.1 GB.
+static int scratch_segments(int num_tokens, int num_heads, int head_size) {
+  const int64_t n = (256ll << 20) / ((int64_t)num_tokens * num_heads * (head_size + 2) * 4);
+  return n < FA_MAX_SEGMENTS ? (n > 1 ? (int)n : 1) : FA_MAX_SEGMENTS;
+}
+
 // Key segments that a launch of these sizes can use (1 = none; the caller then brings no scratch)
 extern "C" int vllm_amd_context_attention_fwd_segments(int batch, int num_heads, int num_kv_heads, int head_size, int max_input_len,
                                                        int max_seq_len, int num_tokens, int has_alibi, int sliding_window,
                                                        int skip_decode) {
-  if (batch <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || num_tokens <= 0 || has_alibi || sliding_window > 0) return 1;
-  return fa_plan(false, head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch, FA_MAX_SEGMENTS,
+  if (batch <= 0 || num_kv_heads <= 0 || num_heads <= 0 || head_size <= 0 || num_heads % num_kv_heads || num_tokens <= 0 || has_alibi || sliding_window > 0) return 1;
+  return fa_plan(false, head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch,
+                 scratch_segments(num_tokens, num_heads, head_size),
                  num_tokens, batch).nseg;
 }
 
 extern "C" int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, int num_kv_heads, int head_size, int max_seqlen_q,
                                                    int max_seqlen_k, int num_tokens, int has_alibi) {
-  if (num_seqs <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || num_tokens <= 0) return 1;
+  if (num_seqs <= 0 || num_kv_heads <= 0 || num_heads <= 0 || head_size <= 0 || num_heads % num_kv_heads || num_tokens <= 0) return 1;
   // decode batches of less than two rounds of workgroups: up to 16 segments (the reference's NUM_SEGMENTS,
   // triton_unified_attention.py:659-683)
   if (max_seqlen_q == 1) return num_seqs * num_kv_heads * ((num_heads / num_kv_heads + 15) / 16) < 1024 ? 16 : 1;
   if (has_alibi) return 1;
   const bool mixed = num_seqs >= 16 && (int64_t)num_tokens < (int64_t)num_seqs * max_seqlen_q;   // (launch_unified)
   return fa_plan(true, head_size, num_heads, num_kv_heads, max_seqlen_q, max_seqlen_k, mixed ? num_tokens - num_seqs : num_tokens,
-                 mixed ? 1 : num_seqs, FA_MAX_SEGMENTS, num_tokens, num_seqs).nseg;
+                 mixed ? 1 : num_seqs, scratch_segments(num_tokens, num_heads, head_size), num_tokens, num_seqs).nseg;
 }
 
 // unified_attention (vllm/attention/ops/triton_unified_attention.py:588-700): q over the new
