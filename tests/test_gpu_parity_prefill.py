@@ -471,3 +471,13 @@ def test_prefill_longest_first_order(tuning, heads, n, skip_decode, majority):
     out = run(c, kv, skip_decode=skip_decode)
     assert not out.isnan().any()
     torch.testing.assert_close(out.float(), ref, atol=tol(torch.bfloat16), rtol=0)
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("head_size,heads", [(256, (4, 2)), (160, (3, 3)), (192, (8, 1))])
+@pytest.mark.parametrize("qls,ctxs", [([5, 1, 33], [90, 300, 64]), ([100, 20], [0, 0]), ([17], [100]), ([1, 64, 0], [700, 0, 40]),
+                                      ([30, 31], [0, 0])])
+def test_prefill_wide_heads_short_chunks(kv, head_size, heads, qls, ctxs):
+    """Above head size 128 short chunks with a context, or of 100 tokens, take the 256-row kernel however few they are."""
+    c = make_prefill_case(qls, ctxs, *heads, head_size, 16, torch.bfloat16, kv, seed=head_size + len(qls), kv_scale=0.02)
+    torch.testing.assert_close(run(c, kv).float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)

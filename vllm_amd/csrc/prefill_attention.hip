@@ -777,6 +777,10 @@ static void launch_cfg(const PrefillParams& p, int block_size, int max_input_len
 //     33.7, 2 x 500 24.4 -> 27.8, 16-bit 400 + 300 over 100 (80) 21.1 -> 22.8.  Windows narrower than half the keys count as
 //     16 bits: this kernel does not stage the tiles left of them (fp8, 900 tokens, window 128: 21.5 -> 15.6).  Windows that leave
 //     16 tiles out: any chunk (64 tokens over 8000 with a window of 128 105 -> 16, 16-bit 170 -> 16).
+//     Short keys are the 64-row kernel's (64 blocks of 4 x 128 fresh tokens, x-layout fp8 12.8 against 14.7, flash fp8 head 256
+//     14.9 / 16.7, 4 x 200 over 100 24.2 / 25.7), but not above head size 128 in the x layout, where it has no registers to
+//     spare: any chunk with a context or of 100 tokens (head 256 16-bit 64 over 600 72.7 -> 47.4, 100 over 900 105 -> 61, 17 over
+//     100 23.9 -> 19.9; head 160 fp8 400 fresh 0.59 x; below that 64 fresh tokens 1.09 x).
 //   * fewer: the 64-row kernel's four times as many workgroups finished sooner than that (chunk 256 over 4096 cached tokens
 //     among 255 decodes: 32 blocks, 82 against 150 us) and still left the chip idle behind one serial walk over the keys
 //     (2.1 us per 64-key tile).  Split, 256 workgroups are dealt out to the blocks there are; a segment is worth its start-up
@@ -909,7 +913,8 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     // (a window that leaves 16 tiles out: any chunk)
     const int min_blocks = mixed ? 128
                            : p.sliding_window > 0 && (int64_t)max_k - p.sliding_window >= 255 + 16 * PF_BN ? 0
-                           : head_size > 128 || narrow ? 64
+                           : narrow ? 64
+                           : head_size > 128 ? (FP8 && max_k < 400 ? 128 : 64)
                            : !FP8 && max_k >= 512 ? (max_k < 600 ? 65 : 64) : 128;
     const FaPlan plan = fa_plan(true, head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
                                 num_tokens, batch, p.sliding_window, min_blocks);
@@ -989,9 +994,12 @@ static void launch_d(const PrefillParams& p, int head_size, int block_size, int 
     const bool can = p.alibi_slopes == nullptr && p.sliding_window == 0 && p.sm_scale > 0.f &&
                      (block_size & (block_size - 1)) == 0 && p.k_stride_t < (1 << 27) && p.v_stride_t < (1 << 27);
     const int64_t ptok = p.flat_batch > 0 ? (int64_t)p.flat_tokens : (int64_t)max_input_len * batch;
+    const int min_blocks = p.skip_decode ? 128
+                           : head_size > 128 ? (max_k >= max_input_len + 64 || max_input_len >= 100 ? 0 : 64)
+                           : max_k < 400 || (!FP8 && max_k <= max_input_len) ? 65 : 64;
     const FaPlan plan = fa_plan(false, head_size, p.num_heads, p.num_kv_heads, max_input_len, max_k, ptok, p.skip_decode ? 1 : batch,
                                 p.flat_batch > 0 ? p.num_segments : 1, ptok, batch, 0,
-                                p.skip_decode ? 128 : !FP8 && head_size <= 128 && max_k <= max_input_len ? 65 : 64);
+                                min_blocks);
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
