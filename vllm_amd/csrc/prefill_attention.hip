@@ -819,7 +819,7 @@ static FaPlan fa_plan(bool flash, int head_size, int num_heads, int num_kv_heads
   const double walk = (keys - 0.5 * (max_q < keys ? max_q : keys)) / PF_BN;   // mean over the rows of the longest chunk
   if (nseg > 1 && walk * 1.9 * (1.0 - 1.0 / nseg) < 2.0 * (4.0 + (double)(launched > 256 ? launched : 256) * 4.5e-3)) nseg = 1;
   // ... and where the partials, written and read, do not cost more than it saves: many rows over few keys are faster in one
-  // piece.  Fitted to 680 launches in 2 .. 32 segments against the unsplit kernel (residual 2 us): what a tile less of the longest
+  // piece.  Fitted to 340 launches at head size 128 (148 at 256) in 2 .. 32 segments against the unsplit kernel (residual 2 us; 4): what a tile less of the longest
   // walk gives, what the split costs at all, per MB, and with q head groups above 4.  us, unsplit / split: 64 / 8 heads 512 over
   // 512 37.5 / 47.3, over 1200 53.6 / 57.4; 32 / 8 1024 over 300 44.2 / 47.1, over 600 51.5 / 49.4, 2 x 512 over 600 39.7 / 44.1,
   // 560 over 500 in three 36.7 / 35.3, 1024 over 6000 with a window of 128 19.0 / 34.5 (of 1024 40.5 / 46.4); head 64, 64-row
@@ -1331,7 +1331,8 @@ static int scratch_segments(int num_tokens, int num_heads, int head_size) {
 extern "C" int vllm_amd_context_attention_fwd_segments(int batch, int num_heads, int num_kv_heads, int head_size, int max_input_len,
                                                        int max_seq_len, int num_tokens, int has_alibi, int sliding_window,
                                                        int skip_decode) {
-  if (batch <= 0 || num_kv_heads <= 0 || num_heads <= 0 || head_size <= 0 || num_heads % num_kv_heads || num_tokens <= 0 || has_alibi || sliding_window > 0) return 1;
+  if (batch <= 0 || num_kv_heads <= 0 || num_heads <= 0 || head_size <= 0 || num_heads % num_kv_heads || num_tokens <= 0) return 1;
+  if (has_alibi || sliding_window > 0) return 1;
   return fa_plan(false, head_size, num_heads, num_kv_heads, max_input_len, max_seq_len, num_tokens, skip_decode ? 1 : batch,
                  scratch_segments(num_tokens, num_heads, head_size),
                  num_tokens, batch).nseg;
