@@ -487,6 +487,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 registers in flight (not instantiated, measured slower)     */
 /*   "pa_sp":      reference partitions merged per workgroup in v2 / rocm      */
 /*                 launches (0 = heuristic, paged_attention_mfma.hip)          */
+/*   "pa_waves":   4 / 8 = waves per workgroup of the x-layout decode kernel at   */
+/*                 head sizes up to 128 (0 = heuristic)                        */
 /*   "pa_group":   XCD-grouped workgroup order of the decode kernel (0 = heuristic:   */
 /*                 >= 1024 workgroups and >= 2 kv heads, 1 = always, 2 = never)     */
 /*   "pa_balance": 1 = paged_attention_v1 cuts the concatenated sequences into equal    */

@@ -427,6 +427,23 @@ def test_v1_longest_first_order(ops, oracle, shape, kv):
         assert torch.equal(outs[0], outs[1]), name
 
 
+@pytest.mark.parametrize("version", ["v1", "v2", "rocm"])
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("head_size,block_size", [(64, 16), (128, 32), (80, 16)])
+def test_eight_waves(ops, oracle, version, kv, head_size, block_size):
+    """Eight waves per workgroup: sequences of fewer steps than waves (some waves have none), of exactly one step per wave, one
+    more and one less, and of a second round."""
+    from vllm_amd import _lib
+    lens = [1, 17, 31, 33, 63, 65, 255, 256, 257, 511, 512, 513, 1023, 1025]
+    c = make_attn_case(len(lens), 8, 2, head_size, block_size, torch.bfloat16, kv, lens, seed=head_size, kv_scale=1.0 if kv == "auto" else 0.5)
+    for waves in (8, 4):
+        _lib.set_tuning("pa_waves", waves)
+        try:
+            run_case(ops, oracle, c, version)
+        finally:
+            _lib.set_tuning("pa_waves", 0)
+
+
 @pytest.mark.parametrize("version", ["v2", "rocm"])
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 @pytest.mark.parametrize("head_size,max_len", [(64, 1290), (128, 600), (80, 513), (256, 520)])

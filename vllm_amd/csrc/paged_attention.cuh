@@ -42,6 +42,7 @@ int paged_attention_mfma(const PagedAttnParams& p);
 // tuning knob (A/B measurements): see vllm_amd_set_tuning
 void set_pa_variant(int v);
 void set_pa_sp(int v);
+void set_pa_waves(int v);
 void set_pa_group(int v);
 void set_pa_balance(int v);
 int get_pa_balance();

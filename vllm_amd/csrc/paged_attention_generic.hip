@@ -571,6 +571,7 @@ extern "C" int vllm_amd_set_tuning(const char* key, int value) {
   VA_REQUIRE(key != nullptr, VLLM_AMD_EINVAL, "set_tuning: null key");
   if (strcmp(key, "pa_variant") == 0) { set_pa_variant(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_sp") == 0) { set_pa_sp(value); return VLLM_AMD_OK; }
+  if (strcmp(key, "pa_waves") == 0) { set_pa_waves(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_group") == 0) { set_pa_group(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_balance") == 0) { set_pa_balance(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_order") == 0) { set_pa_order(value); return VLLM_AMD_OK; }

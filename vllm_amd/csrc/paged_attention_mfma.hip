@@ -728,6 +728,19 @@ static int g_pa_sp = 0;
 void set_pa_sp(int v) { g_pa_sp = v; }
 static int g_pa_group = 0;
 void set_pa_group(int v) { g_pa_group = v; }
+static int g_pa_waves = 0;   // tuning "pa_waves": 0 = pa_eight_waves, 4 / 8 = waves per workgroup
+void set_pa_waves(int v) { g_pa_waves = v; }
+
+// Eight waves per workgroup (head sizes up to 128) where the launch has no more workgroups than fit one to a CU: a sequence's
+// steps are then walked in half as many rounds, and the CU that would hold a second workgroup has none.  us, four -> eight
+// waves, one piece per sequence, fp8: 1 x 777 9.9 -> 8.9, 16 x 1500 14.5 -> 13.7, 32 x 1500 ragged 15.1 -> 14.4, head 64
+// 32 x 1500 12.4 -> 11.2; of 256 workgroups and more two of four waves share a CU and stream alike.  A 16-bit cache has twice the
+// bytes in flight per wave: 1 x 777 9.5 -> 8.6, level at 64 workgroups, 32 x 300 9.2 -> 9.7.  Pieces of 512 tokens and a merge
+// behind them gain up to 128 workgroups (1 x 3000 11.5 -> 11.2; 1 x 16000, 256 of them, 14.3 -> 14.7).
+static bool pa_eight_waves(int64_t workgroups, bool fp8, bool one_piece) {
+  if (g_pa_waves) return g_pa_waves == 8;
+  return workgroups <= (!fp8 ? 64 : one_piece ? 256 : 128);
+}
 
 #define PA_ARGS(A)                                                                                 \
   (A).out, (A).exp_sums, (A).max_logits, (A).q, (A).k_cache, (A).v_cache, (A).num_heads,           \
@@ -814,6 +827,15 @@ static int launch_mfma_v(const PagedAttnParams& p) {
       return VLLM_AMD_OK;
     }
   }
+  if constexpr (HS <= 128) {
+    if (pa_eight_waves((int64_t)grid.x * grid.y, FP8, grid.y == 1)) {
+      hipLaunchKernelGGL((pa_mfma_kernel<scalar_t, FP8, HS, BS, 8, VARIANT, PAD, false>), grid, dim3(8 * 64), 0,
+                         p.stream, PA_ARGS(A));
+      VA_LAUNCH_CHECK("paged_attention mfma launch");
+      if (part && !direct) return paged_attention_reduce(p);
+      return VLLM_AMD_OK;
+    }
+  }
   hipLaunchKernelGGL((pa_mfma_kernel<scalar_t, FP8, HS, BS, NW, VARIANT, PAD, false>), grid, dim3(NW * 64), 0,
                      p.stream, PA_ARGS(A));
   VA_LAUNCH_CHECK("paged_attention mfma launch");
@@ -891,11 +913,17 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       // 14.5 -> 11.1; kept cut: 1 x 1000 16-bit 12.0 (one piece 12.9), 1 x 1500 fp8 11.4 (13.2), head 256 1 x 1000 15.2 (15.8)
       // (device time alone, batches of 1 .. 32: profiles/decode_one_piece.txt -- never above the cheaper form where it leaves
       // the cut; up to 1.2 x are left where 16 sequences of 1000 .. 1500 tokens stay cut).
+      // With eight waves (pa_eight_waves) and an fp8 cache a token costs a workgroup 2.2 ns + 1 ns per 128 bytes and a launch
+      // 5.4 us around that, the merge 3.7 (1 x 777 / 1500 8.9 / 11.7 in one piece, 10.4 / 11.3 cut; head 64 1 x 1500 9.5, 10.1;
+      // 16 x 1500 13.7, 16.7).
       if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
-        const double tb = 2.0 * p.head_size * (p.kv_dtype == VLLM_AMD_KV_AUTO ? 2 : 1), t = 3.5e-3 + tb * 12.2e-6;
+        const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO;
+        const bool w8 = fp8 && p.head_size <= 128 && pa_eight_waves(base, true, true);
+        const double tb = 2.0 * p.head_size * (fp8 ? 1 : 2), t = w8 ? 2.2e-3 + tb * 7.8e-6 : 3.5e-3 + tb * 12.2e-6;
         const double alone = p.max_seq_len * t, stream = 0.6 * (double)base * p.max_seq_len * tb / 6.2e6;
         const double one = 1.05 * (alone > stream ? alone : stream), piece = (double)sp * p.partition_size * t;
-        if (alone <= 10.0 && (4.5 + one) * 1.03 < 4.5 + (piece > stream ? piece : stream) + 4.3) sp = P;
+        const double cut = piece > stream ? piece : stream;
+        if (alone <= 10.0 && (w8 ? 5.4 + one < 5.4 + cut + 3.7 : (4.5 + one) * 1.03 < 4.5 + cut + 4.3)) sp = P;
       }
     } else {
       // Enough pairs to fill the chip: few long pieces stream best (256 x 16k tokens: one piece per
