@@ -76,6 +76,11 @@ class PagedAttention:
         if use_v1 and max_num_partitions > 1:
             groups = num_kv_heads * ((num_heads // max(num_kv_heads, 1) + 15) // 16)
             use_v1 = num_seqs * groups >= 256
+        # ... and where the matrix-core kernel has two partitions it is faster in one piece (device, us, cut / whole: 1 x 777
+        # fp8 10.4 / 8.9, 16 x 777 16-bit 15.3 / 14.2, 8 x 777 13.1 / 11.6): v1, without the 5 us of host time for scratch
+        if (max_num_partitions == 2 and head_size <= 128 and head_size % 16 == 0 and block_size in (16, 32)
+                and query.dtype != torch.float32 and blocksparse_vert_stride <= 1):
+            use_v1 = True
         if use_v1:
             ops.paged_attention_v1(output, query, key_cache, value_cache, num_kv_heads, scale,
                                    block_tables, seq_lens, block_size, max_seq_len, alibi_slopes,
