@@ -497,6 +497,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*   "pa_order":   0 = unpartitioned decode launches keep the hardware's workgroup     */
 /*                 order (default 1: sequences handed out longest first, the two       */
 /*                 workgroups of a CU paired long + short; same output bits)          */
+/*   "pf_mixed":   0 = the decode tokens of a mixed unified_attention step have a         */
+/*                 launch of their own (default 1)                                      */
 /*   "pf_segs":    key segments of the 256-row prefill kernel (0 = heuristic; at most the  */
 /*                 num_segments the caller brings scratch for)                            */
 /*   "mm_kernel":  scaled_mm kernel: 0 = heuristic, 1 = register-staged 128x128    */

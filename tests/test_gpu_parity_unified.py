@@ -450,6 +450,26 @@ def test_unified_fa_kernel_features(oracle, force_fa, mode, fp8):
     run(oracle, c, torch.bfloat16, fp8=fp8, out_scale=torch.tensor([0.03]) if mode == "fp8_out" else None, view=view)
 
 
+@pytest.mark.parametrize("heads,D", [((8, 2), 128), ((32, 8), 80), ((24, 1), 128), ((4, 4), 128)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n,mode", [(16, "plain"), (19, "fp8_out"), (70, "plain")])
+def test_unified_mixed_one_launch(oracle, force_fa, heads, D, fp8, n, mode):
+    """Chunks and decode tokens in one launch (head-major cache memory): decodes of one key, of fewer steps than the eight waves,
+    of one step per wave and one key more, chunks in front of, among and behind them, groups of more than 16 q heads, row
+    blocks in a number that is no multiple of 8; with and without the longest-first order."""
+    from vllm_amd import _lib
+    seqs = [(1, (1, 16, 33, 255, 257, 512, 513, 900)[i % 8]) for i in range(n)]
+    seqs[0], seqs[n // 2], seqs[n - 1] = (70, 600), (65, 65), (130, 333)
+    c = make_unified_case(seqs, heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=n + D, kv_scale=0.5)
+    hnd = lambda t: t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+    for order in (1, 0) if n == 70 else (1,):
+        _lib.set_tuning("pa_order", order)
+        try:
+            run(oracle, c, torch.bfloat16, fp8=fp8, out_scale=torch.tensor([0.03]) if mode == "fp8_out" else None, view=hnd)
+        finally:
+            _lib.set_tuning("pa_order", 1)
+
+
 def test_unified_fa_kernel_sharp_rows(oracle, force_fa):
     """Rows whose maximum keeps growing along the keys (the lazy rescale must fire on some tiles and not on others):
     keys scaled up with their position."""

@@ -205,7 +205,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 // (position t of XCD x takes rank 8 t + x, or 8 t + 7 - x for odd t) so that every XCD gets the
 // same share of long sequences; the tail of the launch is then made of the shortest sequences.
 constexpr int kLptMaxSeqs = 1024;   // 16 registers of 64 lengths
-template <int NR = 4>   // NR registers of 64 lengths: S <= 64 NR
+// plain: a launch behind other workgroups, whose ids are handed out as CUs free up: longest first.
+template <int NR = 4, bool plain = false>   // NR registers of 64 lengths: S <= 64 NR
 __device__ __forceinline__ int pa_lpt_wg(const int* __restrict__ seq_lens, int S, int groups, int bits,
                                          int lane, int hw, int& seq_len_out, bool xcd_grouped = false) {
   int j, grp, srank;
@@ -219,7 +220,7 @@ __device__ __forceinline__ int pa_lpt_wg(const int* __restrict__ seq_lens, int S
     grp = hw - j * groups;
     int nf = (256 - grp + groups - 1) / groups;   // slots of this group with a hardware id below 256
     nf = nf < S ? nf : S;
-    srank = j < nf ? nf - 1 - j : j;
+    srank = j < nf && !plain ? nf - 1 - j : j;
   }
   const int kmax = (int)((1u << bits) - 1u);
   int len[NR], key[NR];

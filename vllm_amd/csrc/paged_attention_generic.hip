@@ -37,6 +37,7 @@ extern int g_pf_rows;   // prefill_attention.hip
 extern int g_uni_decode;
 extern int g_pf_fa;
 extern int g_pf_segs;
+extern int g_pf_mixed;
 extern int g_pf_fa_stagger;
 
 template <typename cache_t> struct CacheTraits;
@@ -587,6 +588,7 @@ extern "C" int vllm_amd_set_tuning(const char* key, int value) {
   if (strcmp(key, "pf_rows") == 0) { g_pf_rows = value; return VLLM_AMD_OK; }
   if (strcmp(key, "uni_decode") == 0) { g_uni_decode = value; return VLLM_AMD_OK; }
   if (strcmp(key, "pf_fa") == 0) { g_pf_fa = value; return VLLM_AMD_OK; }
+  if (strcmp(key, "pf_mixed") == 0) { g_pf_mixed = value; return VLLM_AMD_OK; }
   if (strcmp(key, "pf_segs") == 0) { g_pf_segs = value; return VLLM_AMD_OK; }
   if (strcmp(key, "pf_fa_abl") == 0) return VLLM_AMD_OK;   // (kept for old scripts: the ablations are compile-time)
   if (strcmp(key, "pf_fa_stagger") == 0) { g_pf_fa_stagger = value; return VLLM_AMD_OK; }

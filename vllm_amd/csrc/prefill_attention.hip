@@ -29,6 +29,7 @@ constexpr int PF_BN = 64;
 int g_pf_rows = 0;   // tuning "pf_rows": query rows per workgroup (0 = default)
 int g_uni_decode = 1;   // tuning "uni_decode": 0 = decode-only launches take the packed tile kernel
 extern int g_pf_fa_stagger;   // prefill_fa.hip
+int g_pf_mixed = 1;     // tuning "pf_mixed": 0 = the decode tokens of a mixed step have a launch of their own
 int g_pf_segs = 0;      // tuning "pf_segs": key segments of the 256-row kernel (0 = heuristic; needs the caller's scratch)
 int g_pf_fa = 0;        // tuning "pf_fa": 1 = unified_attention never takes the 256-row kernel (prefill_fa.hip), 2 = whenever it can
 
@@ -852,8 +853,9 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
   // whose query length is not 1, the tile kernel below then skips those whose length is.
   // num_tokens == batch * max_q means every query has max_q > 1 tokens: nothing to split off.
   const bool mixed = max_q > 1 && batch >= 16 && (int64_t)num_tokens < (int64_t)batch * max_q;
+  UniDecodeParams u;
+  bool beside = false;   // decode tokens that the tile kernel's launch may take along
   if ((max_q == 1 || mixed) && g_uni_decode && g_pf_rows != 1) {
-    UniDecodeParams u;
     u.out = p.o; u.q = p.q; u.k_cache = p.k_cache; u.v_cache = p.v_cache;
     u.cu_seqlens_q = p.b_start_loc; u.seq_lens = p.b_seq_len; u.block_table = p.b_loc;
     u.k_scale = p.k_scale; u.v_scale = p.v_scale; u.alibi_slopes = p.alibi_slopes;
@@ -896,8 +898,8 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     }
     u.num_segments = nseg;
     if (unified_decode_supported(u)) {
-      const int rc = unified_decode(u);
-      if (!mixed || rc != VLLM_AMD_OK) return rc;
+      if (!mixed) return unified_decode(u);
+      beside = true;
       p.skip_decode = 1;
     }
   }
@@ -918,6 +920,17 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
                            : !FP8 && max_k >= 512 ? (max_k < 600 ? 65 : 64) : 128;
     const FaPlan plan = fa_plan(true, head_size, p.num_heads, p.num_kv_heads, max_q, max_k, ptok, mixed ? 1 : batch, p.num_segments,
                                 num_tokens, batch, p.sliding_window, min_blocks);
+    // One launch for chunks and decodes (fa_mixed_kernel) where the row blocks fill the chip -- in few blocks cut into segments
+    // nothing hides the decodes (500 over 1500 among 63 of 4096 93 -> 100 us, 300 over 3000 among 200 of 500 74 -> 103) -- and up
+    // to 2.5 decode workgroups per CU: there they have a CU for themselves, and each one's start and merge (6 us) shows, where
+    // the decode kernel's own launch runs two or three side by side (2 x 1000 fresh among 127 of 250 58 -> 62 us, among 200 of
+    // 64 58 -> 76; 2000 over 1500 among 63 / 127 of 250 122 -> 113, 133 -> 125).
+    const bool one_launch = beside && can && plan.use && plan.nseg <= 1 && g_pf_mixed && head_size > 64 && head_size <= 128 &&
+                            u.hp == 1 && p.softcap == 0.f && p.sliding_window == 0 && unified_decode_pairs(u) <= 640;
+    if (beside && !one_launch) {
+      const int rc = unified_decode(u);
+      if (rc != VLLM_AMD_OK) return rc;
+    }
     if (can && plan.use) {
       FaParams f;
       f.o = p.o; f.q = p.q; f.k_cache = p.k_cache; f.v_cache = p.v_cache;
@@ -935,7 +948,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       f.blocks_per_seq = 0;
       f.num_segments = plan.nseg; f.seg_slots = plan.seg_slots; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
       f.stagger = g_pf_fa_stagger;
-      return launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st);
+      return launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st, one_launch ? &u : nullptr);
     }
   }
   // GQA: rows = (token, q head of the group) pairs, grid.y = kv heads ("pf_rows" = 1: off)

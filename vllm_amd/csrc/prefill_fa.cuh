@@ -35,8 +35,9 @@ struct FaParams {
   float* segm_out; float* segm_max; float* segm_sum;
 };
 
-// dtype: VLLM_AMD_F16 / VLLM_AMD_BF16 (queries, output, and the cache unless fp8)
-int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st);
+// dtype: VLLM_AMD_F16 / VLLM_AMD_BF16 (queries, output, and the cache unless fp8).  u: the decode tokens beside the chunks, taken
+// by the same launch (unified_attention without softcap, window or ALiBi, padded head size 128 for both, u->hp == 1).
+int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, const struct UniDecodeParams* u = nullptr);
 // largest num_segments
 constexpr int FA_MAX_SEGMENTS = 32;
 

@@ -28,6 +28,7 @@
 // v_scale in the softmax exponent (one rounding fewer than the reference's (fp8 * scale).to(dtype)).
 #include "mma.cuh"
 #include "prefill_fa.cuh"
+#include "unified_decode_kernel.cuh"
 
 #include <float.h>
 #include <type_traits>
@@ -145,8 +146,10 @@ __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];
 // SOFTCAP (unified_attention): scores softcap * tanh(score / softcap) (triton_unified_attention.py:219-221): a pass of
 // ~9 VALU per score between S^T and the softmax, in its own instantiation.
 // SPLIT: num_segments > 1, in its own instantiation (the 256-wide forms have no register to spare).
+// hw: the workgroup's hardware id in a grid of gx x gy (of the launch's first gx gy workgroups: ids go round-robin over the XCDs).
+template <int D_> constexpr int fa_lds() { return (KN + VN) * BN * 2 * D_; }   // 64 / 128 KiB
 template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP, bool SPLIT>
-__global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
+__device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw, int gx, int gy) {
   constexpr int NW = NW_, BM = 32 * NW, D = D_;
   constexpr int ROWB = 2 * D;       // bytes per LDS row (one key, D 16-bit values)
   constexpr int TILE = BN * ROWB;   // 16 / 32 KiB
@@ -156,7 +159,6 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   constexpr int PPK = D / 16;                     // 32-byte staging pieces per key
   constexpr int NTHR = 64 * NW, IPT = BN * PPK / NTHR, KSTEP = NTHR / PPK;   // staging items per thread, keys between them
   static_assert(IPT * NTHR == BN * PPK && (IPT == 1 || KSTEP % 16 == 0) && 4 * D == IPT * NTHR, "");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[(KN + VN) * TILE];   // 64 / 128 KiB
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
@@ -175,8 +177,8 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   // ---- workgroup -> (row block of some sequence, head).  Hardware ids go round-robin over the XCDs: the
   // bijective remap gives every XCD a contiguous range of logical ids (row blocks fastest, then heads), so the
   // row blocks and heads that read the same K / V share an L2; later (longer) row blocks first.
-  auto xcd_order = [](int nwg) __attribute__((always_inline)) {   // -1: more workgroups than work
-    const int hw = blockIdx.x + gridDim.x * blockIdx.y, q8 = nwg / 8, r8 = nwg % 8, xcd = hw % 8, idx = hw / 8;
+  auto xcd_order = [hw](int nwg) __attribute__((always_inline)) {   // -1: more workgroups than work
+    const int q8 = nwg / 8, r8 = nwg % 8, xcd = hw % 8, idx = hw / 8;
     return idx < q8 + (xcd < r8 ? 1 : 0) ? (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + idx : -1;
   };
   const int nseg = SPLIT ? p.num_segments : 1;
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
     for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(seq_at(i + lane).blocks), 63);
     if (total == 0) return;
     const int work = max(total, min(p.seg_slots, total * nseg));   // per head
-    const int w = xcd_order(work * (int)gridDim.y);
+    const int w = xcd_order(work * gy);
     if (w < 0) return;
     y = w / work;
     gs = w - y * work;
@@ -238,14 +240,14 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
       b -= here;
     }
   } else {
-    const int w = xcd_order(gridDim.x * gridDim.y);
-    y = w / gridDim.x;
-    gs = w % gridDim.x;
-    g = gridDim.x - 1 - gs;
+    const int w = xcd_order(gx * gy);
+    y = w / gx;
+    gs = w % gx;
+    g = gx - 1 - gs;
     if (p.blocks_per_seq > 0) {
       seq = g / p.blocks_per_seq;
       blk = g % p.blocks_per_seq;
-    } else if (PREFIX && p.num_seqs > 1 && p.num_seqs <= 64 && gridDim.y % 8 == 0) {
+    } else if (PREFIX && p.num_seqs > 1 && p.num_seqs <= 64 && gy % 8 == 0) {
       // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD: the row blocks of the
       // longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24 chunks of
       // 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us; 19 prompts of 745 .. 1242 without
@@ -888,6 +890,32 @@ __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   }
 }
 
+template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP, bool SPLIT>
+__global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[fa_lds<D_>()];
+  fa_body<T, FP8, PREFIX, D_, NW_, SOFTCAP, SPLIT>(p, lds, blockIdx.x + gridDim.x * blockIdx.y, gridDim.x, gridDim.y);
+}
+
+// A mixed step in one launch: the row blocks of the chunks first, behind them an eight-wave workgroup for every decode (sequence,
+// kv head) pair, longest first.  Row blocks of a chunk differ in length and so do the chunks: a launch of their own ended on a
+// few of them with most CUs idle (2000 tokens over 1500: 256 blocks of 24 .. 55 tiles), and the decode kernel, which waits for
+// bytes and not for the matrix cores, stood in front of it.  us, two launches -> one (32 / 8 heads, fp8, cache write included),
+// 2000 over 1500 among 63 decodes of up to 4096 keys 164 -> 148, of up to 1000 131 -> 114; 2 x 1000 fresh among 15 of 4000
+// 70.6 -> 43.7; 6000 fresh among 63 of 4000 371 -> 354.
+// (Tried: two groups of four waves per workgroup, 152 us in the first of these; several kv heads per workgroup one after the
+// other, 160.)
+template <typename T, bool FP8>
+__global__ __launch_bounds__(512) void fa_mixed_kernel(const FaParams p, const UniDecodeParams u, int gx, int gy, int nfa, int npairs, int sub_shift, int order) {
+  constexpr int DL = ua_decode_lds<FP8, 128, 8>(), LDS = DL > fa_lds<128>() ? DL : fa_lds<128>();
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS];
+  const int hw = blockIdx.x;
+  if (hw < nfa) {
+    if (hw < gx * gy) fa_body<T, FP8, false, 128, 8, false, false>(p, lds, hw, gx, gy);
+  } else {
+    ua_decode_body<T, FP8, 128, 8, false, true>(u, (char*)lds, sub_shift, 0, order, hw - nfa, npairs, 0);
+  }
+}
+
 // Merge of a split launch: one wave per (token, q head).  Lane s holds segment s's maximum and sum; a half wave (D <= 128;
 // the whole wave above) reads one partial row per step, four rows in flight.  Segments that saw nothing (maximum -inf) are
 // not read.
@@ -958,13 +986,24 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
 }  // namespace fa
 
 int g_pf_fa_stagger = 1;   // tuning "pf_fa_stagger": 0 = all eight waves stage at the bottom of the interval
-int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st) {
+int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, const UniDecodeParams* u) {
   const bool wide = p.head_size > 128;                 // 128-row workgroups of four waves
   const int tpb = (wide ? 128 : 256) / p.pack;
   const unsigned gx = p.blocks_per_seq > 0 ? (unsigned)(p.blocks_per_seq * p.num_seqs) : (unsigned)(p.num_tokens / tpb + p.num_seqs);
   const unsigned gy = (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads);
   const unsigned slots = p.num_segments > 1 ? (unsigned)p.seg_slots : 0u;
   const dim3 grid(gx > slots ? gx : slots, gy);
+  int npairs = 0, sub_shift = 0, order = 0;
+  if (u != nullptr) {
+    npairs = unified_decode_pairs(*u);
+    while ((16 << sub_shift) < u->block_size) ++sub_shift;
+    if (pa_order_enabled() && u->num_seqs <= kLptMaxSeqs)   // longest first (unified_decode)
+      for (order = 1; order < 30 && u->max_seq_len > 0 && (u->max_seq_len >> order) != 0;) ++order;
+  }
+  const unsigned nfa = (grid.x * grid.y + 7) / 8 * 8;   // (the ids behind them go round-robin over the XCDs too)
+#define FA_MIXED(T_, F_)                                                                                                  \
+  hipLaunchKernelGGL((fa::fa_mixed_kernel<T_, F_>), dim3(nfa + (unsigned)npairs), dim3(512), 0, st, p, *u, (int)grid.x, \
+                     (int)grid.y, (int)nfa, npairs, sub_shift, order)
 #define FA_LAUNCH___(T_, F_, P_, D_, NW_, S_)                                                                            \
   do {                                                                                                                   \
     if (p.num_segments > 1) hipLaunchKernelGGL((fa::fa_fwd_kernel<T_, F_, P_, D_, NW_, S_, true>), grid, dim3(64 * NW_), 0, st, p); \
@@ -983,7 +1022,11 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st) {
   do {                                                                      \
     if (p.prefix) FA_LAUNCH_(T_, F_, true); else FA_LAUNCH_(T_, F_, false); \
   } while (0)
-  if (dtype == VLLM_AMD_BF16) { if (fp8) FA_LAUNCH(bf16_t, true); else FA_LAUNCH(bf16_t, false); }
+  if (u != nullptr) {
+    if (dtype == VLLM_AMD_BF16) { if (fp8) FA_MIXED(bf16_t, true); else FA_MIXED(bf16_t, false); }
+    else { if (fp8) FA_MIXED(f16_t, true); else FA_MIXED(f16_t, false); }
+  }
+  else if (dtype == VLLM_AMD_BF16) { if (fp8) FA_LAUNCH(bf16_t, true); else FA_LAUNCH(bf16_t, false); }
   else { if (fp8) FA_LAUNCH(f16_t, true); else FA_LAUNCH(f16_t, false); }
   if (p.num_segments > 1) {
     const dim3 rgrid((unsigned)(((int64_t)p.num_tokens * p.num_heads + 3) / 4));
@@ -995,6 +1038,7 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st) {
     if (dtype == VLLM_AMD_BF16) FA_REDUCE(bf16_t); else FA_REDUCE(f16_t);
 #undef FA_REDUCE
   }
+#undef FA_MIXED
 #undef FA_LAUNCH
 #undef FA_LAUNCH_
 #undef FA_LAUNCH__

@@ -32,6 +32,10 @@ bool pa_order_enabled();   // tuning "pa_order" (paged_attention_mfma.hip)
 bool unified_decode_supported(const UniDecodeParams& p);
 // how many adjacent kv heads a workgroup row may take (1 = none): set UniDecodeParams::hp to it before unified_decode
 int unified_decode_heads_per_row(const UniDecodeParams& p);
+// (sequence, kv head, 16 q heads of its group) triples = workgroups of an unsplit launch
+inline int unified_decode_pairs(const UniDecodeParams& p) {
+  return p.num_seqs * (p.num_kv_heads / p.hp) * ((p.hp * (p.num_heads / p.num_kv_heads) + 15) / 16);
+}
 // main kernel and, with num_segments > 1 (at most 16), the merge of the segment partials
 int unified_decode(const UniDecodeParams& p);
 
