@@ -38,6 +38,8 @@ struct FaParams {
 // dtype: VLLM_AMD_F16 / VLLM_AMD_BF16 (queries, output, and the cache unless fp8).  u: the decode tokens beside the chunks, taken
 // by the same launch (unified_attention without softcap, window or ALiBi, padded head size 128 for both, u->hp == 1).
 int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, const struct UniDecodeParams* u = nullptr);
+// its part for head sizes above 128 (prefill_fa_wide.hip)
+void launch_fa_wide(const FaParams& p, int dtype, bool fp8, dim3 grid, hipStream_t st);
 // largest num_segments
 constexpr int FA_MAX_SEGMENTS = 32;
 
