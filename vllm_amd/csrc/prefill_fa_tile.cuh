@@ -359,11 +359,19 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   const int* bt = p.block_table + (int64_t)seq * p.bt_stride;
   const int last_page = PREFIX ? (ctx > 0 ? (ctx - 1) >> p.bs_shift : 0) : (seq_len - 1) >> p.bs_shift;
 
-  // ---- staging: item = tid + NTHR i -> (key = tid / PPK + KSTEP i, 32 bytes of 16-bit values = LDS chunks 2 piece,
-  // 2 piece + 1 with piece = tid % PPK) ----------------------------------------------------------------------------
-  const int skey = tid / PPK, spiece = tid % PPK;
-  const bool pv0 = 16 * spiece < dr, pv1 = 16 * spiece + 8 < dr;   // the thread's two 8-column chunks exist
-  const int spl = pv0 ? spiece : 0, o1 = pv1 ? 8 : 0;              // clamped piece / second chunk (16-bit elements)
+  // ---- staging: item = tid + NTHR i -> (key, two 8-column chunks ca and cb of its row), a wave's keys side by side ----------
+  // Eight lanes write 16 bytes each per LDS cycle, to banks 128 bytes apart at most: chunk numbers that differ modulo 8.  As 2 piece
+  // and 2 piece + 1 of one key every write took two cycles (SQ_LDS_BANK_CONFLICT: 256 cycles a tile).  PAIR (16 fp8 values of
+  // a load are two neighbouring chunks): four pieces each of two keys, whose swizzles differ in the lowest bit; else the eight
+  // lanes of a key write eight chunks in a row, and load 128 bytes in a row.
+  constexpr bool PAIR = FP8;
+  constexpr int WK = 64 / PPK;                                     // keys of a wave
+  const int lkey = PAIR ? ((lane >> 2) & 1) | ((lane / (2 * PPK)) << 1) : lane / PPK;
+  const int spiece = PAIR ? (lane & 3) | (((lane >> 3) & (PPK / 4 - 1)) << 2) : lane % PPK;
+  const int wkey = WK * wave, skey = wkey + lkey;
+  const int ca = PAIR ? 2 * spiece : spiece, cb = PAIR ? 2 * spiece + 1 : spiece + PPK;
+  const bool pv0 = 8 * ca < dr, pv1 = 8 * cb < dr;                 // the thread's two chunks exist
+  const int cal = pv0 ? ca : 0, cbl = pv1 ? cb : 0;                // clamped
   constexpr int NST = (FP8 && !PREFIX) ? 1 : 2;
   u32x4 kst[IPT][NST], vst[IPT][NST];
   // PREFIX, context V^T: item -> (d = item % D, tokens 16 vq .. of the tile with vq = item / D)
@@ -372,22 +380,20 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   // A wave's items are 64 / PPK = 8 (D = 256: 4) neighbouring keys and, for the context V^T, one group of 16 tokens: inside
   // one block of the cache (16 slots or more), so block ids and base addresses are wave-uniform -- scalar arithmetic -- and
   // a lane adds a 32-bit constant.  (Per-lane 64-bit products cost ~400 of the ~4100 cycles of a tile on every SIMD.)
-  constexpr int WK = 64 / PPK;
-  const int wkey = WK * wave, lkey = lane / PPK;                   // skey = wkey + lkey
   auto wvq_of = [&](int i) __attribute__((always_inline)) { return (64 * wave + NTHR * i) / D; };
   uint32_t koff, koff1 = 0, voff, voff1 = 0;                       // context / paged part: first and second 16 bytes
   uint32_t vtoff[IPT];
   if constexpr (PREFIX) {
-    koff = (uint32_t)((((FP8 ? spl : 2 * spl) << p.bs_shift) + lkey) << 4);
-    koff1 = FP8 ? 0 : (uint32_t)((((2 * spl + (pv1 ? 1 : 0)) << p.bs_shift) + lkey) << 4);
+    koff = (uint32_t)((((FP8 ? cal / 2 : cal) << p.bs_shift) + lkey) << 4);
+    koff1 = FP8 ? 0 : (uint32_t)(((cbl << p.bs_shift) + lkey) << 4);
 #pragma unroll
     for (int i = 0; i < IPT; ++i) vtoff[i] = (uint32_t)((min(vd_of(i), dr - 1) << p.bs_shift) * (FP8 ? 1 : 2));
     voff = 0;
   } else {
-    koff = (uint32_t)lkey * (uint32_t)p.kc_slot_bytes + 16 * NST * spl;
-    voff = (uint32_t)lkey * (uint32_t)p.vc_slot_bytes + 16 * NST * spl;
-    koff1 = koff + 2 * o1;
-    voff1 = voff + 2 * o1;
+    koff = (uint32_t)lkey * (uint32_t)p.kc_slot_bytes + (FP8 ? 8 : 16) * cal;
+    voff = (uint32_t)lkey * (uint32_t)p.vc_slot_bytes + (FP8 ? 8 : 16) * cal;
+    koff1 = (uint32_t)lkey * (uint32_t)p.kc_slot_bytes + 16 * cbl;
+    voff1 = (uint32_t)lkey * (uint32_t)p.vc_slot_bytes + 16 * cbl;
   }
   struct Blk { int k[IPT], v[IPT]; };
   auto load_blk = [&](int t) __attribute__((always_inline)) {
@@ -433,16 +439,16 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
         const int64_t row = tok0 + (t - ctx_tiles) * BN + wkey + KSTEP * i;
         const T* kb = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h;
         const T* vb = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h;
-        const uint32_t ko = (uint32_t)lkey * (uint32_t)p.k_stride_t + 16 * spl, vo = (uint32_t)lkey * (uint32_t)p.v_stride_t + 16 * spl;
-        kst[i][0] = ld16(kb + ko); kst[i][NST - 1] = ld16(kb + ko + 8);
-        vst[i][0] = ld16(vb + vo); vst[i][NST - 1] = ld16(vb + vo + 8);
+        const uint32_t ko = (uint32_t)lkey * (uint32_t)p.k_stride_t + 8 * ca, vo = (uint32_t)lkey * (uint32_t)p.v_stride_t + 8 * ca;
+        kst[i][0] = ld16(kb + ko); kst[i][NST - 1] = ld16(kb + ko + 8 * (cb - ca));
+        vst[i][0] = ld16(vb + vo); vst[i][NST - 1] = ld16(vb + vo + 8 * (cb - ca));
         continue;
       }
       const int64_t row = tok0 + min((t - ctx_tiles) * BN + skey + KSTEP * i, qlen - 1);
-      const T* kr = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h + 16 * spl;
-      const T* vr = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h + 16 * spl;
-      kst[i][0] = ld16(kr); kst[i][NST - 1] = ld16(kr + o1);
-      vst[i][0] = ld16(vr); vst[i][NST - 1] = ld16(vr + o1);
+      const T* kr = (const T*)p.k_new + row * p.k_stride_t + (int64_t)kvh * p.k_stride_h;
+      const T* vr = (const T*)p.v_new + row * p.v_stride_t + (int64_t)kvh * p.v_stride_h;
+      kst[i][0] = ld16(kr + 8 * cal); kst[i][NST - 1] = ld16(kr + 8 * cbl);
+      vst[i][0] = ld16(vr + 8 * cal); vst[i][NST - 1] = ld16(vr + 8 * cbl);
     }
   };
   auto issue_paged = [&](int t, const Blk& blk) __attribute__((always_inline)) {
@@ -465,29 +471,33 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     else if (t < ctx_tiles) issue_ctx(t, blk);
     else issue_new(t, std::false_type{});
   };
-  // K image: chunk ^= key & 15 (conflict-free ds_read_b128 of 32 keys x one chunk); V image: chunk ^= (key & 3) << 2
-  // (the four keys of a transposing read land in four different 64-byte bank ranges); context V^T image (PREFIX):
-  // rows of 128 bytes = 64 tokens of one d, 16-byte unit ^= (d >> 1) & 7 (16 rows x one unit: every bank once).
+  // K image: chunk ^= key & 15 (conflict-free ds_read_b128 of 32 keys x one chunk); V image: chunk ^= (key & 3) << 2 | (key & 1)
+  // (the four keys of a transposing read land in four different 64-byte bank ranges; the lowest bit is for the writes); context
+  // V^T image (PREFIX): rows of 128 bytes = 64 tokens of one d, 16-byte unit ^= (d >> 1) & 7 (16 rows x one unit: every bank once).
   // (the keys of a thread's items are KSTEP apart, a multiple of 16: one pair of swizzled chunk offsets for all)
   uint8_t* k_wr = lds + K_OFF + skey * ROWB;
   uint8_t* v_wr = lds + V_OFF + skey * ROWB;
-  const int kc0 = ((2 * spiece) ^ (skey & 15)) << 4, kc1 = ((2 * spiece + 1) ^ (skey & 15)) << 4;
-  const int vc0 = ((2 * spiece) ^ ((skey & 3) << 2)) << 4, vc1 = ((2 * spiece + 1) ^ ((skey & 3) << 2)) << 4;
-  // PREFIX above head size 128: the offsets of a thread's first chunks (the second ones are at offset ^ 16), computed anew for
+  auto vswz = [](int key) __attribute__((always_inline)) { return ((key & 3) << 2) | (key & 1); };
+  const int kc0 = (ca ^ (skey & 15)) << 4, kc1 = (cb ^ (skey & 15)) << 4;
+  const int vc0 = (ca ^ vswz(skey)) << 4, vc1 = (cb ^ vswz(skey)) << 4;
+  // PREFIX above head size 128: the offsets of a thread's first chunks (the second ones are at offset ^ CX), computed anew for
   // every tile from a thread id that hipcc cannot trace back.  Kept over the loop they are spilled, and their reloads wait for
   // the loads in flight (us, head 256: 32 x 128 tokens over 4096 16-bit 660 -> 538, fp8 440 -> 377; 2 x 2048 over 2048 fp8
   // 299 -> 290).
   constexpr bool WIDE = PREFIX && D > 128;
+  constexpr int CX = PAIR ? 16 : 16 * PPK;
   struct WideAt { int k, v; };
   auto wide_at = [&](bool context) __attribute__((always_inline)) {
     WideAt a = {0, 0};
     if constexpr (WIDE) {
       int t_ = tid;
       asm volatile("" : "+v"(t_));
-      const int key = t_ / PPK, piece = t_ % PPK, kperm = (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1);   // (kperm: below)
+      const int key = PAIR ? (t_ / 64) * WK + (((t_ >> 2) & 1) | (((t_ & 63) / (2 * PPK)) << 1)) : t_ / PPK;   // (as skey and ca)
+      const int chunk = PAIR ? 2 * ((t_ & 3) | (((t_ >> 3) & (PPK / 4 - 1)) << 2)) : t_ % PPK;
+      const int kperm = (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1);   // (below)
       const int kr = context ? kperm : key;
-      a.k = K_OFF + kr * ROWB + (((2 * piece) ^ (kr & 15)) << 4);
-      a.v = context ? V_OFF + t_ * 128 + (((t_ >> 1) & 7) << 4) : V_OFF + key * ROWB + (((2 * piece) ^ ((key & 3) << 2)) << 4);
+      a.k = K_OFF + kr * ROWB + ((chunk ^ (kr & 15)) << 4);
+      a.v = context ? V_OFF + t_ * 128 + (((t_ >> 1) & 7) << 4) : V_OFF + key * ROWB + ((chunk ^ vswz(key)) << 4);
     }
     return a;
   };
@@ -520,8 +530,8 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     for (int i = 0; i < IPT; ++i) {
       const bool live = base + skey + KSTEP * i < keys;
       if constexpr (WIDE) {
-        write_row(lds + at.k + kb_ + KSTEP * i * ROWB, 0, (at.k ^ 16) - at.k, kst[i], live, whole, conv_c);
-        write_row(lds + at.v + vb_ + KSTEP * i * ROWB, 0, (at.v ^ 16) - at.v, vst[i], live, whole, conv_c);
+        write_row(lds + at.k + kb_ + KSTEP * i * ROWB, 0, (at.k ^ CX) - at.k, kst[i], live, whole, conv_c);
+        write_row(lds + at.v + vb_ + KSTEP * i * ROWB, 0, (at.v ^ CX) - at.v, vst[i], live, whole, conv_c);
       } else {
         write_row(k_wr + kb_ + KSTEP * i * ROWB, kc0, kc1, kst[i], live, whole, conv_c);
         write_row(v_wr + vb_ + KSTEP * i * ROWB, vc0, vc1, vst[i], live, whole, conv_c);
@@ -533,14 +543,14 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   // of V^T is one 16-byte read (two 8-byte ones before: head 128 2 .. 5 %, head 256 5 .. 23 % slower).
   const int kperm = (skey & ~12) | ((skey & 4) << 1) | ((skey & 8) >> 1);
   uint8_t* k_wr_ctx = lds + K_OFF + kperm * ROWB;
-  const int kc0_ctx = ((2 * spiece) ^ (kperm & 15)) << 4, kc1_ctx = ((2 * spiece + 1) ^ (kperm & 15)) << 4;
+  const int kc0_ctx = (ca ^ (kperm & 15)) << 4, kc1_ctx = (cb ^ (kperm & 15)) << 4;
   auto write_ctx = [&](int t, auto whole) __attribute__((always_inline)) {
     const int kb_ = (t & (KN - 1)) * TILE, vb_ = (t & (VN - 1)) * TILE;
     const WideAt at = wide_at(true);
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
       const bool live = t * BN + skey + KSTEP * i < ctx;
-      if constexpr (WIDE) write_row(lds + at.k + kb_ + KSTEP * i * ROWB, 0, (at.k ^ 16) - at.k, kst[i], live, whole, std::integral_constant<bool, FP8>{});
+      if constexpr (WIDE) write_row(lds + at.k + kb_ + KSTEP * i * ROWB, 0, (at.k ^ CX) - at.k, kst[i], live, whole, std::integral_constant<bool, FP8>{});
       else write_row(k_wr_ctx + kb_ + KSTEP * i * ROWB, kc0_ctx, kc1_ctx, kst[i], live, whole, std::integral_constant<bool, FP8>{});
       // V^T: the item's 16 tokens of row vd = two 16-byte units
       const int vd = vd_of(i), vq = vq_of(i);
@@ -587,13 +597,13 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     const int q = (lane & 15) >> 2, pp = lane & 3, g1 = (lane >> 4) & 1;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
-      v_rd[db] = lds + V_OFF + (4 * hi + q) * ROWB + ((4 * (db ^ q) + 2 * g1 + (pp >> 1)) << 4) + 8 * (pp & 1);
+      v_rd[db] = lds + V_OFF + (4 * hi + q) * ROWB + ((4 * (db ^ q) + 2 * g1 + ((pp >> 1) ^ (q & 1))) << 4) + 8 * (pp & 1);
   }
 
   // (D = 256: the same addresses from one offset each, XORed with the k-step / d block / unit at the read)
   const int k_off0 = K_OFF + l32 * ROWB + ((hi ^ (l32 & 15)) << 4);
-  const int v_off0 = V_OFF + (4 * hi + ((lane & 15) >> 2)) * ROWB + ((4 * ((lane & 15) >> 2) + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) << 4) +
-                     8 * (lane & 1);
+  const int v_off0 = V_OFF + (4 * hi + ((lane & 15) >> 2)) * ROWB +
+                     ((4 * ((lane & 15) >> 2) + 2 * ((lane >> 4) & 1) + (((lane & 3) >> 1) ^ ((lane >> 2) & 1))) << 4) + 8 * (lane & 1);
   // context V^T (PREFIX): row d = 32 db + l32, unit 2 g16 + hi = tokens 16 g16 + 8 hi .. + 7
   int vt_o[4];
 #pragma unroll
