@@ -309,8 +309,7 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
         mx = fmaxf(mx, s[t][r]);
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor32(max_xor16(mx));
     const float m_new = fmaxf(m_run, mx);
     const float alpha = fast_exp2(m_run - m_new);   // first step: exp2(-huge) = 0
     m_run = m_new;
@@ -404,8 +403,7 @@ __device__ __forceinline__ void pa_piece(const PaK<scalar_t>& A, char* lds, cons
   }
 #endif
   // ---------------- merge the NW waves ------------------------------------------------
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = sum_xor32(sum_xor16(l_run));
   __syncthreads();   // P tiles are dead; LDS becomes the merge buffer
   // [NW][16 q heads][HEAD_SIZE + 4]: four consecutive d per 16-byte access, rows 16 bytes further along the banks than a
   // multiple of them.  (As [NW][HEAD_SIZE][16], 4 bytes at a time, the threads of a row read the same bank: 32-way conflicts

@@ -531,8 +531,7 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
             mx = fmaxf(mx, s[nt][mt][r]);
           }
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_xor32(max_xor16(mx));
       const float m_new = fmaxf(m_run[mt], mx);
       // a column with nothing visible yet keeps m = -inf; avoid (-inf) - (-inf)
       const float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -657,8 +656,7 @@ __global__ __launch_bounds__(64 * NW, (D > 128 ? 1 : 2)) void prefill_kernel(con
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     float l = l_run[mt];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = sum_xor32(sum_xor16(l));
     const int m = m_wave + 16 * mt + c16;
     if (!rok[mt]) continue;
     if (split) {

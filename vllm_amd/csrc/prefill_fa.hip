@@ -74,10 +74,10 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
     }
   }
   if constexpr (PAR == 2) {
-    acc.x += __shfl_xor(acc.x, 32, 64);
-    acc.y += __shfl_xor(acc.y, 32, 64);
-    acc.z += __shfl_xor(acc.z, 32, 64);
-    acc.w += __shfl_xor(acc.w, 32, 64);
+    acc.x = sum_xor32(acc.x);
+    acc.y = sum_xor32(acc.y);
+    acc.z = sum_xor32(acc.z);
+    acc.w = sum_xor32(acc.w);
   }
   if (sub != 0 || d >= dr) return;
   // (a row of NaN scores never raises its maximum from -inf: weight 0, but its sum is NaN, and so is the row, as unsplit)

@@ -71,22 +71,6 @@ constexpr int ONE_SEG = 3;        // a row block of up to this many tiles is not
 __device__ __forceinline__ float max3(float a, float b, float c) {
   return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
-// own value and the value of lane ^ 32, in some order.  v_permlane32_swap vdst, src exchanges lanes 32-63 of vdst
-// with lanes 0-31 of src; inline asm (with the two wait states a VALU write of an operand needs in front of it),
-// because hipcc folds the two results of __builtin_amdgcn_permlane32_swap into one when they are combined again.
-__device__ __forceinline__ void swap32(float& a, float& b) {
-  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-}
-__device__ __forceinline__ float xmax(float x) {
-  float a = x, b = x;
-  swap32(a, b);
-  return fmaxf(a, b);
-}
-__device__ __forceinline__ float xsum(float x) {
-  float a = x, b = x;
-  swap32(a, b);
-  return a + b;
-}
 __device__ __forceinline__ u32x2 lds_tr16(const uint8_t* p) {
   typedef __attribute__((ext_vector_type(4))) short s16x4;
   const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
@@ -717,7 +701,7 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     }
 #pragma unroll
     for (int r = 0; r < 16; r += 2) mx = max3(mx, s[1][r], s[1][r + 1]);
-    const float ms = xmax(mx) * sct;
+    const float ms = max_xor32(mx) * sct;
     if (__any(ms > m_run + THR)) {
       const float m_new = fmaxf(m_run, ms);
       const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
@@ -872,7 +856,7 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
 #endif
   // ---- O^T / l -> out ------------------------------------------------------------------------------------------
   if (!rok) return;
-  const float l = xsum(l_run);
+  const float l = sum_xor32(l_run);
   if (SPLIT && seg == 0 && live < nseg && hi == 0)
     p.segm_sum[((int64_t)(tok0 + rtok) * p.num_heads + rhead + 1) * nseg - 1] = -(float)live;
   if (SPLIT && live > 1) {   // this segment's partial: O unnormalised, running maximum (log2 domain; -inf: nothing visible), sum

@@ -46,12 +46,10 @@ __global__ __launch_bounds__(256) void ua_decode_reduce_kernel(const UniDecodePa
     for (int s2 = 0; s2 < 16; ++s2)
       part[s2] = dval ? *reinterpret_cast<const fv*>(p.segm_out + (row + min(s2, nseg - 1)) * dr + VPL * lane) : (fv)(0.f);
     float mx = ms;
-#pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    mx = row_max16(mx);
     const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);
     l = ls * w;
-#pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) l += __shfl_xor(l, m, 64);
+    l = row_sum16(l);
     l = __shfl(l, 0, 64);
 #pragma unroll
     for (int s2 = 0; s2 < 16; ++s2) {

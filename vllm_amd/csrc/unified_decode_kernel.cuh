@@ -303,8 +303,7 @@ __device__ __forceinline__ void ua_decode_body(const UniDecodeParams& p, char* l
         s[t][r] = x;
         mx = fmaxf(mx, x);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_xor32(max_xor16(mx));
     const float m_new = fmaxf(m_run, mx);
     const float alpha = fast_exp2(m_run - m_new);   // first step: exp2(-huge) = 0
     m_run = m_new;
@@ -383,8 +382,7 @@ __device__ __forceinline__ void ua_decode_body(const UniDecodeParams& p, char* l
   if (step < nsteps) do_step(step, std::false_type{});
 
   // ---------------- merge the NW waves ----------------------------------------------------
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = sum_xor32(sum_xor16(l_run));
   __syncthreads();   // the K images are dead; LDS becomes the merge buffer
   // [NW][16 q heads][D + 4], in 16-byte accesses, the rows 16 bytes further along the banks than a multiple of them (as
   // [NW][D][16] the threads of a row read the same bank).  Unscaled: the reader has every wave's maximum anyway.
