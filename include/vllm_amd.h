@@ -489,6 +489,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 launches (0 = heuristic, paged_attention_mfma.hip)          */
 /*   "pa_waves":   4 / 8 = waves per workgroup of the x-layout decode kernel at   */
 /*                 head sizes up to 128 (0 = heuristic)                        */
+/*   "pa_reduce":  1 = the merge of v2 / rocm partials always takes a workgroup per     */
+/*                 (sequence, q head) (default 0: a wave, up to 64 used slots)      */
 /*   "pa_group":   XCD-grouped workgroup order of the decode kernel (0 = heuristic:   */
 /*                 >= 1024 workgroups and >= 2 kv heads, 1 = always, 2 = never)     */
 /*   "pa_balance": 1 = paged_attention_v1 cuts the concatenated sequences into equal    */

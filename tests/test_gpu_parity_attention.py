@@ -427,6 +427,43 @@ def test_v1_longest_first_order(ops, oracle, shape, kv):
         assert torch.equal(outs[0], outs[1]), name
 
 
+@pytest.mark.parametrize("version", ["v2", "rocm"])
+@pytest.mark.parametrize("head_size,max_len", [(64, 4160), (128, 2049), (80, 1025), (256, 3000), (120, 700)])
+def test_merge_by_waves(ops, oracle, version, head_size, max_len):
+    """The merge with a wave per (sequence, q head): one slot, as many as a load has rows, one more, more than eight loads' worth,
+    none (a sequence of length 0), against the oracle and the merge with a workgroup each (fp32 sums in another order: the
+    results are those of one more rounding to 16 bits apart)."""
+    from vllm_amd import _lib
+    step = 512 if version == "v2" else 256
+    lens = [max_len, 1, step, step + 1, 2 * step, min(max_len, 4 * step), min(max_len, 4 * step + 1), min(max_len, 8 * step + 1)]
+    c = make_attn_case(len(lens), 8, 2, head_size, 16, torch.bfloat16, "auto", lens, seed=head_size)
+    q, kc, vc, bt = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt"))
+    sl = c["sl"].clone()
+    sl[1] = 0
+    P = -(-max_len // step)
+    one = torch.ones(1, device="cuda")
+    outs = []
+    _lib.set_tuning("pa_sp", 1)
+    try:
+        run_case(ops, oracle, c, version)
+        for mode in (0, 1):
+            _lib.set_tuning("pa_reduce", mode)
+            es = torch.full((len(lens), 8, P), float("nan"), device="cuda")
+            tmp = torch.full((len(lens), 8, P, head_size), float("nan"), dtype=torch.bfloat16, device="cuda")
+            out = torch.full_like(q, float("nan"))
+            if version == "v2":
+                ops.paged_attention_v2(out, es, es.clone(), tmp, q, kc, vc, 2, c["scale"], bt, sl.cuda(), 16, max_len, None, "auto", one, one)
+            else:
+                ops.paged_attention_rocm(out, es, es.clone(), tmp, q, kc, vc, 2, c["scale"], bt, sl.cuda(), None, 16, max_len, None,
+                                         "auto", one, one)
+            assert (out[1] == 0).all()
+            outs.append(out.float())
+    finally:
+        _lib.set_tuning("pa_sp", 0)
+        _lib.set_tuning("pa_reduce", 0)
+    assert ((outs[0] - outs[1]).abs() <= 2.0 ** -7 * outs[0].abs() + 1e-6).all()
+
+
 @pytest.mark.parametrize("version", ["v1", "v2", "rocm"])
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 @pytest.mark.parametrize("head_size,block_size", [(64, 16), (128, 32), (80, 16)])

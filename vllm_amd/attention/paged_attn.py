@@ -76,8 +76,9 @@ class PagedAttention:
         if use_v1 and max_num_partitions > 1:
             groups = num_kv_heads * ((num_heads // max(num_kv_heads, 1) + 15) // 16)
             use_v1 = num_seqs * groups >= 256
-        # ... and where the matrix-core kernel has two partitions it is faster in one piece (device, us, cut / whole: 1 x 777
-        # fp8 10.4 / 8.9, 16 x 777 16-bit 15.3 / 14.2, 8 x 777 13.1 / 11.6): v1, without the 5 us of host time for scratch
+        # ... and two partitions of the matrix-core kernel cost the device as much in one piece, or nearly (us, cut / whole:
+        # 1 x 777 fp8 9.1 / 8.7, 16 x 777 16-bit 13.6 / 12.9, 8 x 1000 16-bit 12.0 / 13.6): v1, without the 5 us of host time
+        # for scratch
         if (max_num_partitions == 2 and head_size <= 128 and head_size % 16 == 0 and block_size in (16, 32)
                 and query.dtype != torch.float32 and blocksparse_vert_stride <= 1):
             use_v1 = True

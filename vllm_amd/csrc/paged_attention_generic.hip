@@ -253,6 +253,8 @@ __global__ __launch_bounds__(kGenThreads) void pa_generic_kernel(
   }
 }
 
+static int g_pa_reduce = 0;   // tuning "pa_reduce": 1 = a workgroup per (sequence, q head) always
+
 // ---------------------------------------------------------------------------
 // Split-K reduce (v2: attention_kernels.cuh:562-664; rocm: rocm/attention.cu:1271-1475)
 // grid (num_heads, num_seqs), 128 threads.
@@ -333,8 +335,113 @@ __global__ __launch_bounds__(128) void pa_reduce_kernel(
   }
 }
 
+// The same merge with a wave per (sequence, q head), for up to 64 used slots of 16-bit partials: lane j holds slot j's maximum and
+// sum, LPR lanes read a row of the partials in 16-byte pieces, eight of them in flight.  Two memory round trips: lengths,
+// maxima and sums at once, then the rows.  (The kernel above chains four and reads its rows two bytes a thread; whole calls in us, that one -> this, fp8, 32 / 8
+// heads: 1 x 3000 11.2 -> 9.6, 20 x 1500 16.0 -> 13.9, 8 x 16000 ragged 37.3 -> 35.1; head 64 1 x 16000 12.8 -> 10.7.)
+template <typename scalar_t, bool ROCM, int LPR>
+__global__ __launch_bounds__(256) void pa_reduce_wave_kernel(
+    void* __restrict__ out_, const float* __restrict__ exp_sums, const float* __restrict__ max_logits,
+    const scalar_t* __restrict__ tmp_out, const int* __restrict__ seq_lens, const int* __restrict__ query_start_loc,
+    const float* __restrict__ fp8_out_scale, int num_seqs, int num_heads, int head_size, int partition_size,
+    int max_num_partitions, int slot_stride, int used, int window) {
+  constexpr int RPS = 64 / LPR, U = 8;                // rows per load, loads in flight
+  struct alignas(16) V8 { scalar_t e[8]; };
+  const int lane = threadIdx.x & 63;
+  const int pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (pair >= num_seqs * num_heads) return;
+  const int seq = pair / num_heads, head = pair - seq * num_heads;
+  const int64_t sidx = ((int64_t)seq * num_heads + head) * max_num_partitions;
+  // (in front of the checks; slots that nobody wrote are masked below)
+  float ml = -FLT_MAX, es = 0.f;
+  if (lane < used) {
+    ml = max_logits[sidx + (int64_t)lane * slot_stride];
+    es = exp_sums[sidx + (int64_t)lane * slot_stride];
+  }
+  const int seq_len = seq_lens[seq];
+  int64_t orow = seq;
+  if (query_start_loc) {
+    const int q0 = query_start_loc[seq];
+    if (query_start_loc[seq + 1] - q0 != 1) return;
+    orow = q0;
+  }
+  const int j0 = window > 0 ? max(0, seq_len - window) / partition_size : 0;
+  const int j1 = min((seq_len + partition_size - 1) / partition_size, used), np = j1 - j0;
+  const int sub = lane / LPR, d = 8 * (lane % LPR);
+  const bool mine = d < head_size;
+  const scalar_t* tp = tmp_out + sidx * head_size + (mine ? d : 0);
+  const int64_t row_elems = (int64_t)slot_stride * head_size;
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  float inv = 0.f;
+  bool copy = false;
+  if (np > 0) {
+    const bool live = lane >= j0 && lane < j1;
+    const float m = wave_max(live ? ml : -FLT_MAX);
+    const float w = live ? es * expf(ml - m) : 0.f;
+    inv = __fdividef(1.0f, wave_sum(w) + 1e-6f);
+    copy = !ROCM && np == 1;                          // :577-589
+    for (int b = j0; b < j1; b += RPS * U) {
+      V8 row[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = b + u * RPS + sub;
+        if (b + u * RPS < j1) row[u] = *reinterpret_cast<const V8*>(tp + (int64_t)(j < j1 ? j : j1 - 1) * row_elems);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = b + u * RPS + sub;
+        if (b + u * RPS >= j1) break;
+        float f = __shfl(w, j < 64 ? j : 63, 64);
+        if (!ROCM) f *= inv;
+        f = copy ? 1.f : f;
+        if (j < j1)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] = copy ? to_f32(row[u].e[e]) : acc[e] + to_f32(row[u].e[e]) * f;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (LPR <= 32) acc[e] = sum_xor32(acc[e]);
+      if constexpr (LPR <= 16) acc[e] = sum_xor16(acc[e]);
+      if constexpr (LPR <= 8) acc[e] += lane_dpp<0x128>(acc[e]);
+    }
+  }
+  if (sub != 0 || !mine) return;
+  const int64_t oi = (orow * num_heads + head) * head_size + d;
+  if (ROCM && fp8_out_scale) {
+    const float os = 1.0f / (*fp8_out_scale);
+    struct alignas(8) B8 { uint8_t e[8]; } o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o.e[e] = np > 0 ? f32_to_fp8(acc[e] * inv * os) : 0;
+    *reinterpret_cast<B8*>((uint8_t*)out_ + oi) = o;
+  } else {
+    V8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o.e[e] = from_f32<scalar_t>(ROCM ? acc[e] * inv : acc[e]);
+    *reinterpret_cast<V8*>((scalar_t*)out_ + oi) = o;
+  }
+}
+
 template <typename scalar_t>
 static int launch_reduce(const PagedAttnParams& p) {
+  const int used = ceil_div(p.max_num_partitions, p.sp_parts);
+  if constexpr (sizeof(scalar_t) == 2) {
+    if (used <= 64 && p.head_size % 8 == 0 && p.head_size <= 256 && (((uintptr_t)p.tmp_out | (uintptr_t)p.out) & 15) == 0 && g_pa_reduce != 1) {
+      const dim3 wgrid((unsigned)ceil_div((int64_t)p.num_seqs * p.num_heads, 4));
+#define RED(ROCM_, LPR_)                                                                                                    \
+  hipLaunchKernelGGL((pa_reduce_wave_kernel<scalar_t, ROCM_, LPR_>), wgrid, dim3(256), 0, p.stream, p.out, p.exp_sums,      \
+                     p.max_logits, (const scalar_t*)p.tmp_out, p.seq_lens, p.query_start_loc, p.fp8_out_scale, p.num_seqs,  \
+                     p.num_heads, p.head_size, p.partition_size * p.sp_parts, p.max_num_partitions, p.sp_parts, used, p.window)
+      const int lpr = p.head_size <= 64 ? 8 : p.head_size <= 128 ? 16 : 32;
+      if (p.rocm_semantics) { if (lpr == 8) RED(true, 8); else if (lpr == 16) RED(true, 16); else RED(true, 32); }
+      else { if (lpr == 8) RED(false, 8); else if (lpr == 16) RED(false, 16); else RED(false, 32); }
+#undef RED
+      VA_LAUNCH_CHECK("paged_attention reduce launch");
+      return VLLM_AMD_OK;
+    }
+  }
   dim3 grid(p.num_heads, p.num_seqs);
   size_t smem = sizeof(float) * (size_t)p.max_num_partitions;
   if (p.rocm_semantics)
@@ -572,6 +679,7 @@ extern "C" int vllm_amd_set_tuning(const char* key, int value) {
   VA_REQUIRE(key != nullptr, VLLM_AMD_EINVAL, "set_tuning: null key");
   if (strcmp(key, "pa_variant") == 0) { set_pa_variant(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_sp") == 0) { set_pa_sp(value); return VLLM_AMD_OK; }
+  if (strcmp(key, "pa_reduce") == 0) { g_pa_reduce = value; return VLLM_AMD_OK; }
   if (strcmp(key, "pa_waves") == 0) { set_pa_waves(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_group") == 0) { set_pa_group(value); return VLLM_AMD_OK; }
   if (strcmp(key, "pa_balance") == 0) { set_pa_balance(value); return VLLM_AMD_OK; }

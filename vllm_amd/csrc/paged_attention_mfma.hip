@@ -903,7 +903,7 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       const int64_t sp_min = p.partition_size >= 2048 ? 1 : 2048 / p.partition_size;
       sp = sp_fill < sp_min ? sp_fill : sp_min;
       if (sp < sp_bal) sp = sp_bal;
-      // Short sequences: one piece each, which writes the output itself -- no reduce kernel (~4.3 us with the gap in front
+      // Short sequences: one piece each, which writes the output itself -- no reduce kernel (~2.6 us with the gap in front
       // of it) -- where that costs less than the longest piece gains.  A workgroup alone takes 3.5 ns + 1 ns per 82 bytes for
       // a token (us, 1500 tokens: head 64 fp8 7.5, head 128 fp8 9.9, 16-bit 14.6), the chip 1 us per 6.2 MB; the batch is
       // taken to be 0.6 full.  Up to 10 us only: a long sequence among short ones has to be cut.  Measured, cut -> one piece:
@@ -911,17 +911,18 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       // 14.5 -> 11.1; kept cut: 1 x 1000 16-bit 12.0 (one piece 12.9), 1 x 1500 fp8 11.4 (13.2), head 256 1 x 1000 15.2 (15.8)
       // (device time alone, batches of 1 .. 32: profiles/decode_one_piece.txt -- never above the cheaper form where it leaves
       // the cut; up to 1.2 x are left where 16 sequences of 1000 .. 1500 tokens stay cut).
-      // With eight waves (pa_eight_waves) and an fp8 cache a token costs a workgroup 2.2 ns + 1 ns per 128 bytes and a launch
-      // 5.4 us around that, the merge 3.7 (1 x 777 / 1500 8.9 / 11.7 in one piece, 10.4 / 11.3 cut; head 64 1 x 1500 9.5, 10.1;
-      // 16 x 1500 13.7, 16.7).
+      // With eight waves (pa_eight_waves) a token costs a workgroup 2.2 ns + 1 ns per 128 bytes; the merge costs 2.1 us and 6 ns
+      // for each piece (us, one piece / cut, fp8: 1 x 1000 8.8 / 9.3, 1 x 1300 11.3 / 9.7, 8 x 1600 13.2 / 10.9, 16 x 1300
+      // ragged 12.3 / 12.8, 24 x 1600 15.8 / 20.4; head 64 1 x 1600 9.7 / 8.5, 16 x 1600 10.5 / 11.3; 16-bit 1 x 777 8.1 / 9.5, 8 x
+      // 1000 13.8 / 12.0).
       if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
         const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO;
-        const bool w8 = fp8 && p.head_size <= 128 && pa_eight_waves(base, true, true);
+        const bool w8 = p.head_size <= 128 && pa_eight_waves(base, fp8, true);
         const double tb = 2.0 * p.head_size * (fp8 ? 1 : 2), t = w8 ? 2.2e-3 + tb * 7.8e-6 : 3.5e-3 + tb * 12.2e-6;
         const double alone = p.max_seq_len * t, stream = 0.6 * (double)base * p.max_seq_len * tb / 6.2e6;
         const double one = 1.05 * (alone > stream ? alone : stream), piece = (double)sp * p.partition_size * t;
         const double cut = piece > stream ? piece : stream;
-        if (alone <= 10.0 && (w8 ? 5.4 + one < 5.4 + cut + 3.7 : (4.5 + one) * 1.03 < 4.5 + cut + 4.3)) sp = P;
+        if (alone <= 10.0 && (w8 ? one < cut + 2.1 + 0.006 * (double)(base * ((P + sp - 1) / sp)) : (4.5 + one) * 1.03 < 4.5 + cut + 2.6)) sp = P;
       }
     } else {
       // Enough pairs to fill the chip: few long pieces stream best (256 x 16k tokens: one piece per
