@@ -533,6 +533,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*   "uni_hp":     adjacent kv heads of a token-major cache taken as one row of  */
 /*                 that decode kernel (0 = heuristic, 1 = never, 2 / 4 = that    */
 /*                 many where the shape allows)                                  */
+/*   "uni_seg":    key segments of that decode kernel (0 = heuristic; at most the    */
+/*                 num_segments the caller brings scratch for)                   */
 /*   "pf_fa":      the 256-row kernel of unified_attention /                   */
 /*                 context_attention_fwd (prefill_fa.hip; causal mask, unified: + sliding  */
 /*                 window, softcap): 0 = where it pays (default): head sizes 72 .. 256     */

@@ -176,6 +176,22 @@ def test_unified_decode_kernel(oracle, dtype, block_size, fp8, nseq):
     run(oracle, c, dtype, fp8=fp8)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("D,nseq", [(64, 3), (128, 3), (128, 40), (256, 3), (256, 40)])
+@pytest.mark.parametrize("segs", [1, 2, 3, 16])
+def test_unified_decode_segments(oracle, fp8, D, nseq, segs):
+    """Every batch in one piece and cut, whichever of them the heuristic takes: more segments than a sequence has tiles, lengths
+    around the edges of a segment, one key."""
+    from vllm_amd import _lib
+    lens = [900, 1, 64, 65, 128, 129, 192, 383, 385, 577]
+    c = make_unified_case([(1, lens[i % len(lens)]) for i in range(nseq)], 8, 4, D, 16, torch.bfloat16, fp8=fp8, seed=nseq + segs, kv_scale=0.5)
+    _lib.set_tuning("uni_seg", segs)
+    try:
+        run(oracle, c, torch.bfloat16, fp8=fp8)
+    finally:
+        _lib.set_tuning("uni_seg", 0)
+
+
 @pytest.mark.parametrize("D", [32, 48, 80, 96, 112, 120, 136, 160, 192, 224, 256])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("nseq", [5, 260])

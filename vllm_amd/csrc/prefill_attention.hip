@@ -870,31 +870,8 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     u.segm_stride = p.segm_stride;
     u.dtype = std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16;
     u.fp8 = FP8; u.stream = st;
-    // Split over the keys (when the caller brought scratch).  The chip holds 512 workgroups at a
-    // time, so a launch of full-length workgroups takes ceil(wgs n / 512) / n rounds, and every
-    // workgroup pays ~4 us of prologue and merge next to ~25 ns per token of streaming: take the
-    // smallest segment count within 5 % of the best estimate (513..1023 workgroups: ~1.3
-    // rounds instead of 2); few sequences: as many segments of >= 256 tokens as allowed.
     u.hp = unified_decode_heads_per_row(u);
-    int nseg = 1;
-    if (p.num_segments > 1 && !mixed) {
-      const int wgs = batch * (p.num_kv_heads / u.hp) * ((gqa * u.hp + 15) / 16);
-      int cap = (max_k + 4 * PF_BN - 1) / (4 * PF_BN);
-      if (cap > p.num_segments) cap = p.num_segments;
-      if (cap > 16) cap = 16;
-      const float ovh = 160.f / (float)(max_k > 0 ? max_k : 1);
-      // rows above 128 elements: 256 workgroups carry the bytes in flight of 512 narrow ones (16-bit cache: one workgroup
-      // per CU; fp8: two of 32-token steps -- counting 512 slots there split 64 x 4096 in two: 93.8 against 89.9 us)
-      const int slots = head_size * u.hp > 128 ? 256 : 512;
-      auto cost = [&](int n) { return (float)((wgs * n + slots - 1) / slots) / n * (1.f + n * ovh); };
-      float best = 1e30f;
-      for (int n = 1; n <= cap; ++n) best = cost(n) < best ? cost(n) : best;
-      nseg = cap;
-      if (wgs * cap > slots)
-        for (int n = 1; n <= cap; ++n)
-          if (cost(n) <= best * 1.05f) { nseg = n; break; }
-    }
-    u.num_segments = nseg;
+    u.num_segments = unified_decode_segments(u, mixed ? 1 : p.num_segments);
     if (unified_decode_supported(u)) {
       if (!mixed) return unified_decode(u);
       beside = true;

@@ -36,6 +36,8 @@ int unified_decode_heads_per_row(const UniDecodeParams& p);
 inline int unified_decode_pairs(const UniDecodeParams& p) {
   return p.num_seqs * (p.num_kv_heads / p.hp) * ((p.hp * (p.num_heads / p.num_kv_heads) + 15) / 16);
 }
+// key segments of a launch (at most max_segments and 16); p.max_seq_len and p.hp are set
+int unified_decode_segments(const UniDecodeParams& p, int max_segments);
 // main kernel and, with num_segments > 1 (at most 16), the merge of the segment partials
 int unified_decode(const UniDecodeParams& p);
 

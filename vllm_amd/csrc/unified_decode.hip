@@ -2,6 +2,8 @@
 // unified_decode_kernel.cuh, and the merge of its key segments.
 #include "unified_decode_kernel.cuh"
 
+#include <algorithm>
+
 namespace va {
 
 extern int g_uni_decode;
@@ -151,6 +153,50 @@ int unified_decode_heads_per_row(const UniDecodeParams& p) {
     return hp;
   }
   return 1;
+}
+
+int g_uni_seg = 0;   // tuning "uni_seg": 0 = heuristic, n = that many key segments (at most those there is scratch for)
+
+int unified_decode_segments(const UniDecodeParams& p, int max_segments) {
+  // Split over the keys (when the caller brought scratch).  The chip holds 512 workgroups at a
+  // time, so a launch of full-length workgroups takes ceil(wgs n / 512) / n rounds, and every
+  // workgroup pays ~4 us of prologue and merge next to ~25 ns per token of streaming: take the
+  // smallest segment count within 5 % of the best estimate (513..1023 workgroups: ~1.3
+  // rounds instead of 2); few sequences: as many segments of >= 256 tokens as allowed.
+  const int max_k = p.max_seq_len, row = p.head_size * p.hp;
+  const int wgs = unified_decode_pairs(p);
+  if (max_segments <= 1 || max_k <= 0) return 1;
+  if (g_uni_seg > 0) return std::min(g_uni_seg, std::min(max_segments, 16));
+  int cap = (max_k + 255) / 256;
+  if (cap > max_segments) cap = max_segments;
+  if (cap > 16) cap = 16;
+  const float ovh = 160.f / (float)max_k;
+  // rows above 128 elements: 256 workgroups carry the bytes in flight of 512 narrow ones (16-bit cache: one workgroup
+  // per CU; fp8: two of 32-token steps -- counting 512 slots there split 64 x 4096 in two: 93.8 against 89.9 us)
+  const int slots = row > 128 ? 256 : 512;
+  auto cost = [&](int n) { return (float)((wgs * n + slots - 1) / slots) / n * (1.f + n * ovh); };
+  float best = 1e30f;
+  for (int n = 1; n <= cap; ++n) best = cost(n) < best ? cost(n) : best;
+  int nseg = cap;
+  if (wgs * cap > slots)
+    for (int n = 1; n <= cap; ++n)
+      if (cost(n) <= best * 1.05f) { nseg = n; break; }
+  // One piece all the same where what the cut gains does not pay for the merge behind it: 4.5 us and 4 ns for each workgroup.
+  // A workgroup alone takes 2.5 ns + 1 ns per 43 bytes for a token, the chip 1 us per 6.2 MB -- the batch taken to be 0.6 full --
+  // and both more where some of the 256 CUs have a workgroup more than others.  us, cut -> one piece (32 / 8 heads of 128, fp8):
+  // 1 x 500 11.9 -> 9.9, 16 x 777 14.7 -> 13.6, 24 x 500 14.9 -> 11.3, 32 x 1000 ragged 17.9 -> 14.4, 48 x 3000 ragged 40.2 -> 33.8,
+  // 96 x 1600 60.1 -> 53.6; 16-bit 32 x 500 19.0 -> 15.8.  Kept cut: 1 x 1600 11.8 (one piece 16.0), 8 x 3000 18.1 (24.2), 40 x 3000
+  // 46.7 (51.8), 40 x 3000 ragged 34.3 (30.8).  Over 1048 batches (1 .. 512 sequences of 300 .. 16000 tokens, head 64 / 128 / 256,
+  // both caches) 4.2 % on average, the worst 80 x 16000 of head 64 (212 -> 228; ragged 149 -> 128).
+  const double tb = 2.0 * row * (p.fp8 ? 1 : 2);
+  auto us = [&](int n) {
+    const int64_t tot = (int64_t)wgs * n;
+    const double alone = (double)(((max_k + 63) / 64 + n - 1) / n) * 64 * (2.5e-3 + tb * 2.3e-5);
+    const double stream = 0.6 * (double)wgs * max_k * tb / 6.2e6;
+    const double over = tot >= 256 ? (double)((tot + 255) / 256 * 256) / (double)tot - 1.0 : 0.0;
+    return (alone > stream ? alone : stream) * (1.0 + 1.6 * over * over) + (n > 1 ? 4.5 + 0.004 * (double)tot : 0.0);
+  };
+  return nseg > 1 && us(1) < 0.98 * us(nseg) ? 1 : nseg;
 }
 
 int unified_decode(const UniDecodeParams& p) {
