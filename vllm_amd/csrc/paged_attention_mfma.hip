@@ -941,6 +941,23 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
         if (cost < best * 0.97) { best = cost; sp = c; }
       }
     }
+    // One piece as well for batches that nearly fill the chip, where it beats the cut by the balance: extra workgroups and the merge of their pieces cost
+    // 4.7 us and 12 ns each; a workgroup takes 2 ns + 1 ns per 29 bytes for a token with the chip busy, the chip 1 us per 6.2 MB --
+    // the batch taken to be 0.84 full -- and both more where some of the 256 CUs have a workgroup more than others.  us, cut ->
+    // one piece (32 / 8 heads of 128): fp8 24 x 4096 39.3 -> 33.4, 48 x 2200 ragged 30.0 -> 23.7, 56 x 2200 48.7 -> 41.1 (ragged 36.0 ->
+    // 25.5), 96 x 4096 ragged 82.0 -> 73.8; 16-bit 24 x 2200 39.2 -> 34.6, 56 x 2200 93 -> 76; head 64 24 x 4096 23.5 -> 19.3.  Kept cut:
+    // 24 x 4096 ragged 29.0 (27.8), 40 x 4096 58.0 (63.5).  Not where the longest sequence may take a workgroup more than 24 us on
+    // an idle chip: among short ones it has to be cut; and fewer pairs are the rule above's (8 x 1600 of head 64 8.9, in one piece 9.7).
+    if (sp < P && base >= 160 && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
+      const double tb = 2.0 * p.head_size * (p.kv_dtype != VLLM_AMD_KV_AUTO ? 1 : 2);
+      auto us = [&](int64_t c) {
+        const int64_t tot = base * ((P + c - 1) / c), len = c < P ? c * p.partition_size : p.max_seq_len;
+        const double alone = (double)len * (2e-3 + tb * 3.5e-5), stream = 0.84 * (double)base * p.max_seq_len * tb / 6.2e6;
+        const double over = tot >= 256 ? (double)((tot + 255) / 256 * 256) / (double)tot - 1.0 : 0.0;
+        return (alone > stream ? alone : stream) * (1.0 + 1.05 * over * over) + (c < P ? 4.7 + 0.012 * (double)tot : 0.0);
+      };
+      if (p.max_seq_len * (2.5e-3 + tb * 1.2e-5) <= 24.0 && us(P) < 0.99 * us(sp)) sp = P;
+    }
     if (g_pa_sp > 0) sp = g_pa_sp;
     if (sp < 1) sp = 1;
     if (sp > p.max_num_partitions) sp = p.max_num_partitions;

@@ -187,7 +187,8 @@ int unified_decode_segments(const UniDecodeParams& p, int max_segments) {
   // 1 x 500 11.9 -> 9.9, 16 x 777 14.7 -> 13.6, 24 x 500 14.9 -> 11.3, 32 x 1000 ragged 17.9 -> 14.4, 48 x 3000 ragged 40.2 -> 33.8,
   // 96 x 1600 60.1 -> 53.6; 16-bit 32 x 500 19.0 -> 15.8.  Kept cut: 1 x 1600 11.8 (one piece 16.0), 8 x 3000 18.1 (24.2), 40 x 3000
   // 46.7 (51.8), 40 x 3000 ragged 34.3 (30.8).  Over 1048 batches (1 .. 512 sequences of 300 .. 16000 tokens, head 64 / 128 / 256,
-  // both caches) 4.2 % on average, the worst 80 x 16000 of head 64 (212 -> 228; ragged 149 -> 128).
+  // both caches) 4.0 % on average, none more than 2.5 % slower.  Not where the longest sequence may take a workgroup more than
+  // 24 us on an idle chip: among short ones it has to be cut.
   const double tb = 2.0 * row * (p.fp8 ? 1 : 2);
   auto us = [&](int n) {
     const int64_t tot = (int64_t)wgs * n;
@@ -196,7 +197,7 @@ int unified_decode_segments(const UniDecodeParams& p, int max_segments) {
     const double over = tot >= 256 ? (double)((tot + 255) / 256 * 256) / (double)tot - 1.0 : 0.0;
     return (alone > stream ? alone : stream) * (1.0 + 1.6 * over * over) + (n > 1 ? 4.5 + 0.004 * (double)tot : 0.0);
   };
-  return nseg > 1 && us(1) < 0.98 * us(nseg) ? 1 : nseg;
+  return nseg > 1 && max_k * (2.5e-3 + tb * 1.2e-5) <= 24.0 && us(1) < 0.98 * us(nseg) ? 1 : nseg;
 }
 
 int unified_decode(const UniDecodeParams& p) {
