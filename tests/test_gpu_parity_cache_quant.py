@@ -136,6 +136,53 @@ def test_reshape_and_cache_batched_prompts(ops, oracle, kv, lens, first):
     assert torch.equal(vc_d.cpu().view(torch.uint8), vc_o.view(torch.uint8))
 
 
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("BS", [16, 48])
+def test_reshape_and_cache_every_run(ops, oracle, kv, BS):
+    """Runs of 1 .. 33 slots from every offset of a 16-slot group, one behind the other: whole and partial tiles, one, two and more
+    segments among 16 tokens, a segment that ends behind them, slots that continue across a block by accident, padding."""
+    D, H, dtype = 64, 2, torch.float16
+    slots, blk = [], 1
+    for first in range(16):
+        for ln in (1, 2, 15, 16, 17, 18, 31, 33):
+            slots += [blk * BS + first + i for i in range(ln)]
+            blk += (first + ln + BS - 1) // BS + (first & 1)
+        slots += [-1] * (first % 3)
+    slots = torch.tensor(slots, dtype=torch.int64)
+    T, NB = len(slots), blk + 2
+    key, value = _kv_inputs(T, H, D, dtype, BS, strided=True)
+    x = x_of(dtype, kv)
+    cdt = dtype if kv == "auto" else torch.uint8
+    ks, vs = (0.05, 0.04) if kv != "auto" else (1.0, 1.0)
+    kc_o, vc_o = torch.zeros((NB, H, D // x, BS, x), dtype=cdt), torch.zeros((NB, H, D, BS), dtype=cdt)
+    kc_d, vc_d = kc_o.cuda(), vc_o.cuda()
+    oracle.reshape_and_cache(key, value, kc_o, vc_o, slots, kv, ks, vs)
+    ops.reshape_and_cache(key.cuda(), value.cuda(), kc_d, vc_d, slots.cuda(), kv,
+                          torch.tensor([ks], device="cuda"), torch.tensor([vs], device="cuda"))
+    assert torch.equal(kc_d.cpu().view(torch.uint8), kc_o.view(torch.uint8))
+    assert torch.equal(vc_d.cpu().view(torch.uint8), vc_o.view(torch.uint8))
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.37, -0.021, 3e-5, 300.0])
+def test_cache_write_every_half(ops, oracle, scale):
+    """The vectorised fp16 conversion over all finite halves: byte-exact, NaN codes of overflowing quotients up to their sign."""
+    h = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    h = torch.where(torch.isfinite(h), h, torch.zeros_like(h))
+    T, H, D, BS = 512, 1, 128, 16
+    key, value = h.view(T, H, D), h.flip(0).contiguous().view(T, H, D)
+    slots = torch.arange(T, dtype=torch.int64) + 5
+    kc_o = torch.zeros((T // BS + 2, H, D // 16, BS, 16), dtype=torch.uint8)
+    vc_o = torch.zeros((T // BS + 2, H, D, BS), dtype=torch.uint8)
+    kc_d, vc_d = kc_o.cuda(), vc_o.cuda()
+    oracle.reshape_and_cache(key, value, kc_o, vc_o, slots, "fp8", scale, scale)
+    sc = torch.tensor([scale], device="cuda")
+    ops.reshape_and_cache(key.cuda(), value.cuda(), kc_d, vc_d, slots.cuda(), "fp8", sc, sc)
+    for got, want in ((kc_d.cpu(), kc_o), (vc_d.cpu(), vc_o)):
+        nan = (want & 0x7f) == 0x7f
+        assert torch.equal(got[~nan], want[~nan])
+        assert ((got[nan] & 0x7f) == 0x7f).all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 @pytest.mark.parametrize("layout", ["NHD", "HND"])

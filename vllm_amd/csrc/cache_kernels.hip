@@ -63,14 +63,19 @@ __global__ void reshape_and_cache_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// reshape_and_cache for many tokens: one workgroup per (16 consecutive tokens, head).
-// Prefill and chunked prefill hand over runs of consecutive slots; for such a group the V
-// tile is transposed through LDS and every V row [d][16 tokens] leaves as ONE 16-byte
-// (fp8) store instead of 16 single-byte stores, and the K vectors of consecutive tokens
-// are contiguous 256-byte pieces.  A run may start anywhere in a block (chunk boundaries
-// do): the LDS columns keep the slots' alignment mod 16, partial 16-slot groups are
-// written as 4-byte units and single elements.  A group whose slots are not consecutive
-// (decode batches, padding slots < 0) takes the per-token scatter inside the same kernel.
+// reshape_and_cache for many tokens.  Prefill and chunked prefill hand over runs of consecutive
+// slots; the part of a run inside one 16-slot group of the cache ("segment") is one tile: its V
+// is transposed through LDS and every V row [d][16 slots] leaves as 16-byte stores instead of
+// single elements, and the K vectors of its tokens are contiguous 256-byte pieces.  A workgroup
+// (hpw heads) takes the segments that START among its 16 tokens -- so a run that begins anywhere
+// in a block (chunk boundaries do) is cut at the cache's groups and not at multiples of 16
+// tokens, and only its two ends are partial tiles, written as 4-byte units and single elements.
+// The first segment is blockIdx.z = 0's, a second one blockIdx.z = 1's (in one workgroup behind
+// each other 1.0 us more); more (decode batches) are scattered token by token.
+// Bound by latency: read and write phases of one round of workgroups (4 TB/s at 8192 aligned
+// tokens).  us, tiles at multiples of 16 tokens -> at the groups, 8 heads of 128: 8192 tokens from
+// slot 11 of a block fp8 20.4 -> 15.2, 16-bit 31.0 -> 16.9 (aligned 16.0 -> 14.2, 16.2 -> 16.6), 24 chunks
+// of up to 250 16.9 -> 13.9, 25.4 -> 14.9, 60 chunks of up to 33 9.0 -> 9.5, 9.9 -> 9.0.
 // Requires block_size % 16 == 0 and head_size <= 256.
 // ---------------------------------------------------------------------------
 template <typename scalar_t, typename cache_t, bool FP8>
@@ -82,13 +87,14 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
     const float* __restrict__ k_scale_p, const float* __restrict__ v_scale_p) {
   constexpr int CS = sizeof(cache_t);
   constexpr int X = 16 / CS;    // elements of one K cache vector
-  constexpr int G = 16;         // tokens per workgroup
+  constexpr int G = 16;         // tokens per workgroup, slots per tile
   constexpr int U = 4 / CS;     // elements of a 4-byte unit
   constexpr int W = 512;        // head elements (hpw * head_size <= W) per workgroup
-  constexpr int KI = W / X * G / 256, VI = W / 8 * G / 256, RI = W / 256;   // items per thread
-  __shared__ int64_t s_slot[G];
-  __shared__ __attribute__((aligned(16))) cache_t vt[G][W + X];   // [token][head, d], padded rows
-  const int tid = threadIdx.x;
+  constexpr int KI = W / X * G / 256, VI = W / 8 * G / 256;   // items per thread
+  __shared__ int64_t s_slot[2 * G];
+  __shared__ __attribute__((aligned(16))) cache_t vt[G][W + X];   // [slot of the group][head, d], padded rows
+  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+  const int tid = threadIdx.x, lane = tid & 63;
   // slot -> (block, offset): a shift for the usual power-of-two block sizes (a 64-bit
   // division per item otherwise)
   auto split = [&](int64_t slot, int64_t& blk, int64_t& off) {
@@ -96,187 +102,171 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
     else { blk = slot / block_size; off = slot % block_size; }
   };
   const int t0 = blockIdx.x * G, h0 = blockIdx.y * hpw;
-  const int n = num_tokens - t0 < G ? num_tokens - t0 : G;
   const int nh = num_heads - h0 < hpw ? num_heads - h0 : hpw;
   const int width = nh * head_size;   // contiguous source elements per token
-  if (tid < G) s_slot[tid] = tid < n ? slot_mapping[t0 + tid] : -1;
+  const scalar_t* const kbase = key + h0 * head_size;
+  const scalar_t* const vbase = value + h0 * head_size;
+  const int64_t blk_elems = (int64_t)num_heads * head_size * block_size;
+  const int64_t head_off = (int64_t)h0 * head_size * block_size;
 
-  // every load of the workgroup is issued before the first use (rows past n: token 0)
-  const scalar_t* kbase = key + (int64_t)t0 * key_stride + h0 * head_size;
-  const scalar_t* vbase = value + (int64_t)t0 * value_stride + h0 * head_size;
+  // every wave: slot of token t0 - 1 + lane (32 lanes); cont: it continues the token in front of it in the same group
+  const int tok = t0 - 1 + lane;
+  const int64_t sl = lane < 32 && tok >= 0 && tok < num_tokens ? slot_mapping[tok] : -1;
+  Divisor ks(1.f), vs(1.f);
+  if constexpr (FP8) { ks = Divisor(*k_scale_p); vs = Divisor(*v_scale_p); }
+  if (tid >= 1 && tid < 32) s_slot[tid - 1] = sl;
+  const int64_t before = __shfl_up((long long)sl, 1, 64);
+  const uint32_t cont = (uint32_t)__ballot(lane > 0 && sl >= 0 && before >= 0 && sl == before + 1 && (sl & 15) != 0) >> 1;
+  const uint32_t valid = (uint32_t)__ballot(sl >= 0) >> 1;   // bit i: token t0 + i
+  uint32_t starts = valid & ~cont & 0xffffu;
+  __syncthreads();
+
   const int cpt = width / X;          // K chunks per token
-  Vec<scalar_t, X> kreg[KI];
-#pragma unroll
-  for (int u = 0; u < KI; ++u) {      // item = (chunk, token), token fastest
-    const int it = tid + 256 * u;
-    const int i = it % G, c = it / G;
-    const bool ok = c < cpt && i < n;
-    kreg[u] = *reinterpret_cast<const Vec<scalar_t, X>*>(kbase + (ok ? (int64_t)i * key_stride + c * X : 0));
-  }
   const int cpv = width / 8;          // V chunks of 8 per token
   const int cpv_log2 = (cpv & (cpv - 1)) == 0 ? 31 - __clz(cpv) : -1;
   auto vitem = [&](int it, int& i, int& c) {   // item -> (token, chunk), chunk fastest
     if (cpv_log2 >= 0) { i = it >> cpv_log2; c = it & (cpv - 1); }
     else { i = it / cpv; c = it % cpv; }
   };
-  Vec<scalar_t, 8> vreg[VI];
+  // tokens t0 + i0 + [0, 16) of the bits in mask (one segment: its first n)
+  struct Rows { Vec<scalar_t, X> k[KI]; Vec<scalar_t, 8> v[VI]; };
+  auto load = [&](int i0, uint32_t mask, Rows& r) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < VI; ++u) {      // item = (token, chunk), chunk fastest
-    const int it = tid + 256 * u;
-    int i, c;
-    vitem(it, i, c);
-    const bool ok = i < n;
-    vreg[u] = *reinterpret_cast<const Vec<scalar_t, 8>*>(vbase + (ok ? (int64_t)i * value_stride + c * 8 : 0));
-  }
-  Divisor ks(1.f), vs(1.f);
-  if constexpr (FP8) { ks = Divisor(*k_scale_p); vs = Divisor(*v_scale_p); }
-  __syncthreads();
-
-  // a "run": consecutive slots up to the next multiple of 16 (segment A), then consecutive
-  // slots from a multiple of 16 (segment B: the sequence's next block, anywhere in the cache)
-  const int64_t slot0 = s_slot[0];
-  const int colbase = slot0 >= 0 ? (int)(slot0 % 16) : 0;
-  const int nA = n < 16 - colbase ? n : 16 - colbase;
-  const int64_t slotB = nA < n ? s_slot[nA] : 0;
-  bool run = slot0 >= 0 && slotB >= 0 && slotB % 16 == 0;
-  for (int i = 1; i < nA; ++i) run = run && s_slot[i] == slot0 + i;
-  for (int i = nA + 1; i < n; ++i) run = run && s_slot[i] == slotB + (i - nA);
-  auto conv = [](scalar_t v, Divisor sc) -> cache_t {
-    if constexpr (FP8) return f32_to_fp8(kv_quant_prep(v, sc));
-    else return v;
+    for (int u = 0; u < KI; ++u) {      // item = (chunk, token), token fastest
+      const int it = tid + 256 * u;
+      const int i = it % G, c = it / G;
+      const bool ok = c < cpt && ((mask >> i) & 1);
+      r.k[u] = *reinterpret_cast<const Vec<scalar_t, X>*>(kbase + (ok ? (int64_t)(t0 + i0 + i) * key_stride + c * X : 0));
+    }
+#pragma unroll
+    for (int u = 0; u < VI; ++u) {
+      int i, c;
+      vitem(tid + 256 * u, i, c);
+      const bool ok = i < G && ((mask >> i) & 1);
+      r.v[u] = *reinterpret_cast<const Vec<scalar_t, 8>*>(vbase + (ok ? (int64_t)(t0 + i0 + i) * value_stride + c * 8 : 0));
+    }
   };
-  const int64_t blk_elems = (int64_t)num_heads * head_size * block_size;
-  const int64_t head_off = (int64_t)h0 * head_size * block_size;
-
-  // K: a wave writes 256-byte pieces of a run (16 tokens x one 16-byte vector)
-  const int cph = head_size / X;
+  auto store = [&](int i0, uint32_t mask, bool run, const Rows& r) __attribute__((always_inline)) {
+    // K: a wave writes 256-byte pieces of a run (16 tokens x one 16-byte vector)
+    const int cph = head_size / X;
 #pragma unroll
-  for (int u = 0; u < KI; ++u) {
-    const int it = tid + 256 * u;
-    const int i = it % G, c = it / G;
-    const int64_t slot = s_slot[i];
-    if (c >= cpt || slot < 0) continue;   // slot < 0 also covers i >= n
+    for (int u = 0; u < KI; ++u) {
+      const int it = tid + 256 * u;
+      const int i = it % G, c = it / G;
+      if (c >= cpt || !((mask >> i) & 1)) continue;
+      int64_t blk, off;
+      split(s_slot[i0 + i], blk, off);
+      Vec<cache_t, X> kq;
+      if constexpr (FP8) {
+        kv_quant_vec(r.k[u], ks, kq);
+      } else {
+        kq = r.k[u];
+      }
+      const int hl = c / cph, xc = c % cph;
+      *reinterpret_cast<Vec<cache_t, X>*>(key_cache + blk * blk_elems + head_off +
+                                           ((int64_t)hl * head_size * block_size) +
+                                           ((int64_t)xc * block_size + off) * X) = kq;
+    }
+
+    // V: into the LDS tile (run) or scattered
+    const int col0 = run ? (int)(s_slot[i0] & 15) : 0;
+#pragma unroll
+    for (int u = 0; u < VI; ++u) {
+      int i, c;
+      vitem(tid + 256 * u, i, c);
+      if (i >= G || !((mask >> i) & 1)) continue;
+      Vec<cache_t, 8> vq;
+      if constexpr (FP8) {
+        kv_quant_vec(r.v[u], vs, vq);
+      } else {
+        vq = r.v[u];
+      }
+      if (run) {
+        *reinterpret_cast<Vec<cache_t, 8>*>(&vt[col0 + i][c * 8]) = vq;
+      } else {
+        int64_t blk, off;
+        split(s_slot[i0 + i], blk, off);
+        cache_t* dst = value_cache + blk * blk_elems + head_off + (int64_t)(c * 8) * block_size + off;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dst[(int64_t)j * block_size] = vq.v[j];
+      }
+    }
+    if (!run) return;
+    __syncthreads();
+
     int64_t blk, off;
-    split(slot, blk, off);
-    Vec<cache_t, X> kq;
-    if constexpr (FP8) {
-      kv_quant_vec(kreg[u], ks, kq);
-    } else {
+    split(s_slot[i0] - col0, blk, off);
+    cache_t* const vdst = value_cache + blk * blk_elems + head_off + off;
+    // a thread takes U consecutive d: one 4-byte LDS read per slot, a transpose in registers (v_perm_b32), rows of
+    // 16 / 32 bytes, or what there is of them (reads of single elements made this kernel bound by LDS issue)
+    const int lo = col0, hi = col0 + __popc(mask);
+    for (int w = tid; w < width / U; w += 256) {
+      uint32_t col[16];
 #pragma unroll
-      for (int j = 0; j < X; ++j) kq.v[j] = conv(kreg[u].v[j], ks);
-    }
-    const int hl = c / cph, xc = c % cph;
-    *reinterpret_cast<Vec<cache_t, X>*>(key_cache + blk * blk_elems + head_off +
-                                         ((int64_t)hl * head_size * block_size) +
-                                         ((int64_t)xc * block_size + off) * X) = kq;
-  }
-
-  // V: into the LDS tile (run) or scattered (anything else)
+      for (int p = 0; p < 16; ++p) col[p] = *reinterpret_cast<const uint32_t*>(&vt[p][w * U]);
 #pragma unroll
-  for (int u = 0; u < VI; ++u) {
-    const int it = tid + 256 * u;
-    int i, c;
-    vitem(it, i, c);
-    if (i >= G) continue;
-    const int64_t slot = s_slot[i];
-    if (slot < 0) continue;
-    Vec<cache_t, 8> vq;
-    if constexpr (FP8) {
-      kv_quant_vec(vreg[u], vs, vq);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) vq.v[j] = conv(vreg[u].v[j], vs);
-    }
-    if (run) {
-      *reinterpret_cast<Vec<cache_t, 8>*>(&vt[i][c * 8]) = vq;
-    } else {
-      int64_t blk, off;
-    split(slot, blk, off);
-      cache_t* dst = value_cache + blk * blk_elems + head_off + (int64_t)(c * 8) * block_size + off;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dst[(int64_t)j * block_size] = vq.v[j];
-    }
-  }
-  if (!run) return;
-  __syncthreads();
-
-  // rows of the transposed tile: column q = (slot0 % 16) + token keeps the slots' alignment,
-  // so columns [0,16) (segment A) and [16,32) (segment B) are 16-slot groups inside a block
-  if constexpr (CS == 1) {
-    // fp8, whole 16-slot groups (round 3): a thread takes FOUR consecutive d -- one 4-byte LDS read per token
-    // instead of four single-byte ones (the byte reads made this kernel LDS-issue bound: 16 ds_read_u8 per
-    // 16-byte row) -- transposes the 4 x 16 bytes in registers (v_perm_b32) and stores four 16-byte rows.
-    // Partial groups (the two ends of a run that starts mid-block) keep the per-row path below: the same
-    // scheme with 4-byte and single-byte stores measured slower there (32768 tokens 50.6 -> 79.5 us).
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int q0 = 16 * hh;
-      const int lo = colbase - q0 > 0 ? colbase - q0 : 0;
-      const int hi = colbase + n - q0 < 16 ? colbase + n - q0 : 16;
-      if (!(lo == 0 && hi == 16)) continue;   // uniform
-      const int64_t sbase = hh == 0 ? slot0 - colbase : slotB;
-      int64_t blk, off;
-      split(sbase, blk, off);
-      for (int dg = tid; dg < width / 4; dg += 256) {
-        uint32_t col[16];
-#pragma unroll
-        for (int p = 0; p < 16; ++p)
-          col[p] = *reinterpret_cast<const uint32_t*>(&vt[q0 + p - colbase][dg * 4]);
-        cache_t* dst = value_cache + blk * blk_elems + head_off + (int64_t)(dg * 4) * block_size + off;
-        typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
+      for (int e = 0; e < U; ++e) {
+        cache_t* dst = vdst + (int64_t)(w * U + e) * block_size;
+        uint32_t row[4 * CS];
+        if constexpr (CS == 1) {
           const uint32_t sel = 0x0c0c0000u | ((4u + e) << 8) | (uint32_t)e;   // byte e of (S1, S0)
-          u32x4 row;
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const uint32_t t0 = __builtin_amdgcn_perm(col[4 * k + 1], col[4 * k], sel);
-            const uint32_t t1 = __builtin_amdgcn_perm(col[4 * k + 3], col[4 * k + 2], sel);
-            row[k] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
+            const uint32_t a = __builtin_amdgcn_perm(col[4 * k + 1], col[4 * k], sel);
+            const uint32_t b = __builtin_amdgcn_perm(col[4 * k + 3], col[4 * k + 2], sel);
+            row[k] = __builtin_amdgcn_perm(b, a, 0x05040100u);
           }
-          *reinterpret_cast<u32x4*>(dst + (int64_t)e * block_size) = row;
+        } else {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) row[k] = __builtin_amdgcn_perm(col[(2 * k + 1) & 15], col[(2 * k) & 15], e ? 0x07060302u : 0x05040100u);
         }
-      }
-    }
-  }
+        if (mask == 0xffffu) {
 #pragma unroll
-  for (int u = 0; u < RI; ++u) {
-    const int d = tid + 256 * u;   // (head, d) row: rows of consecutive heads are contiguous
-    if (d >= width) continue;
+          for (int h = 0; h < CS; ++h)
+            *reinterpret_cast<u32x4*>(dst + 8 * h) = (u32x4){row[4 * h], row[4 * h + 1], row[4 * h + 2], row[4 * h + 3]};
+          continue;
+        }
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int q0 = 16 * hh;
-      const int lo = colbase - q0 > 0 ? colbase - q0 : 0;
-      const int hi = colbase + n - q0 < 16 ? colbase + n - q0 : 16;
-      if (hi <= lo) continue;   // uniform
-      if (CS == 1 && lo == 0 && hi == 16) continue;   // done above
-      const int64_t sbase = hh == 0 ? slot0 - colbase : slotB;   // first slot of the 16-slot group
-      int64_t blk, off;
-      split(sbase, blk, off);
-      cache_t* dst = value_cache + blk * blk_elems + head_off + (int64_t)d * block_size + off;
-      struct alignas(16) Row { cache_t e[16]; } row;
+        for (int h = 0; h < 2; ++h) {   // (uniform branches)
+          if (8 * h >= lo && 8 * h + 8 <= hi) {
+            if constexpr (CS == 1) *reinterpret_cast<uint2*>(dst + 8 * h) = make_uint2(row[2 * h], row[2 * h + 1]);
+            else *reinterpret_cast<u32x4*>(dst + 8 * h) = (u32x4){row[4 * h], row[4 * h + 1], row[4 * h + 2], row[4 * h + 3]};
+            continue;
+          }
 #pragma unroll
-      for (int p = 0; p < 16; ++p) {
-        const int i = q0 + p - colbase;
-        row.e[p] = (p >= lo && p < hi) ? vt[i][d] : cache_t{};
-      }
-      if (lo == 0 && hi == 16) {
-        *reinterpret_cast<Row*>(dst) = row;
-      } else {
+          for (int k = 0; k < 8 / U; ++k) {
+            const int q = 8 * h + U * k;
+            const uint32_t x = row[q / U];
+            if (q >= lo && q + U <= hi) {
+              *reinterpret_cast<uint32_t*>(dst + q) = x;
+            } else {
 #pragma unroll
-        for (int uu = 0; uu < 16 / U; ++uu) {
-          if (uu * U >= lo && uu * U + U <= hi) {
-            *reinterpret_cast<Vec<cache_t, U>*>(dst + uu * U) =
-                *reinterpret_cast<const Vec<cache_t, U>*>(&row.e[uu * U]);
-          } else {
-#pragma unroll
-            for (int j = 0; j < U; ++j)
-              if (uu * U + j >= lo && uu * U + j < hi) dst[uu * U + j] = row.e[uu * U + j];
+              for (int j = 0; j < U; ++j)
+                if (q + j >= lo && q + j < hi) __builtin_memcpy(dst + q + j, (const char*)&x + j * CS, CS);
+            }
           }
         }
       }
     }
+  };
+
+  Rows r;
+  if (__popc(starts) > 2) {
+    // token by token: z = 0 those of the first 16 that are not part of a segment that started in front, z = 1 the rest of the
+    // last segment behind them
+    const uint32_t tail = cont >> 16;   // bit 0: token t0 + 16 continues token t0 + 15
+    const uint32_t mask = blockIdx.z ? (1u << __builtin_ctz(~tail)) - 1u : valid & (0xffffu << __builtin_ctz(starts)) & 0xffffu;
+    if (mask == 0) return;
+    load(blockIdx.z ? G : 0, mask, r);
+    store(blockIdx.z ? G : 0, mask, false, r);
+    return;
   }
+  if (blockIdx.z) starts &= starts - 1;
+  if (starts == 0) return;
+  const int i0 = __builtin_ctz(starts);
+  const uint32_t mask = (2u << __builtin_ctz(~(cont >> (i0 + 1)))) - 1u;   // at most 16: a group's end is never continued
+  load(i0, mask, r);
+  store(i0, mask, true, r);
 }
 
 // Scalar fallback for layouts / alignments the vector kernel does not cover
@@ -425,12 +415,12 @@ static int launch_reshape_and_cache(const void* key, const void* value, void* kc
     int hpw = 512 / head_size;   // heads per workgroup: hpw * head_size <= 512 elements
     if (hpw > num_heads) hpw = num_heads;
     // fewer heads per workgroup while the launch would not fill the chip a few times over
-    // (round 3, with the 4-byte V path: 8192 tokens 19.8 us with 1 head per workgroup, 14.3 with 4; 2048 tokens 6.8 / 6.2
+    // (8192 tokens 19.8 us with 1 head per workgroup, 14.3 with 4; 2048 tokens 6.8 / 6.2
     // with 1 / 2: tools/bench_cache_hpw.py)
     while (hpw > 1 && (int64_t)((num_tokens + 15) / 16) * ((num_heads + hpw - 1) / hpw) < 512) hpw /= 2;
     if (g_cache_hpw > 0 && g_cache_hpw * head_size <= 512 && g_cache_hpw <= num_heads) hpw = g_cache_hpw;
     hipLaunchKernelGGL((reshape_and_cache_runs_kernel<scalar_t, cache_t, FP8>),
-                       dim3((num_tokens + 15) / 16, (num_heads + hpw - 1) / hpw), dim3(256), 0, st,
+                       dim3((num_tokens + 15) / 16, (num_heads + hpw - 1) / hpw, 2), dim3(256), 0, st,
                        (const scalar_t*)key, (const scalar_t*)value, (cache_t*)kc, (cache_t*)vc,
                        slot_mapping, key_stride, value_stride, num_tokens, num_heads, head_size,
                        block_size, bs_log2, hpw, ks, vs);

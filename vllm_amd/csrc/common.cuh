@@ -165,6 +165,39 @@ __device__ __forceinline__ void kv_quant_vec(const Vec<T, N>& in, Divisor d, Vec
       }
       o[i] = (uint32_t)word;
     }
+  } else if constexpr (__is_same(T, f16_t) && N % 4 == 0) {
+    // the same with the quotient's rounding to half in between (a quotient that overflows there: the scalar path)
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(&in);
+    const float as = fabsf(d.s), ay = fabsf(d.y);
+    const uint32_t sm = __float_as_uint(d.s) & 0x80000000u;
+    float q[N];
+    uint32_t mx = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float ax = fabsf((float)in.v[j]);
+      const float q0 = ax * ay;
+      float qf = fmaf(fmaf(-q0, as, ax), ay, q0);
+      asm("" : "+v"(qf));   // (v_fma_mixlo_f16, which hipcc makes of an fma rounded to half, rounds once instead of twice)
+      q[j] = (float)(f16_t)qf;
+      mx = mx > __float_as_uint(q[j]) ? mx : __float_as_uint(q[j]);
+    }
+    if (__builtin_expect(__any(mx >= 0x7f800000u), 0)) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) out.v[j] = f32_to_fp8(kv_quant_prep(in.v[j], d));
+      return;
+    }
+    uint32_t* o = reinterpret_cast<uint32_t*>(&out);
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t xw = w[2 * i + j / 2], sg = ((j & 1 ? xw : xw << 16) ^ sm) & 0x80000000u;
+        v[j] = __uint_as_float(__float_as_uint(fminf(q[4 * i + j], 448.0f)) | sg);
+      }
+      const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+      o[i] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo, true);
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < N; ++j) out.v[j] = f32_to_fp8(kv_quant_prep(in.v[j], d));
