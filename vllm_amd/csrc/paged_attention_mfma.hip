@@ -734,10 +734,13 @@ void set_pa_waves(int v) { g_pa_waves = v; }
 // waves, one piece per sequence, fp8: 1 x 777 9.9 -> 8.9, 16 x 1500 14.5 -> 13.7, 32 x 1500 ragged 15.1 -> 14.4, head 64
 // 32 x 1500 12.4 -> 11.2; of 256 workgroups and more two of four waves share a CU and stream alike.  A 16-bit cache has twice the
 // bytes in flight per wave: 1 x 777 9.5 -> 8.6, level at 64 workgroups, 32 x 300 9.2 -> 9.7.  Pieces of 512 tokens and a merge
-// behind them gain up to 128 workgroups (1 x 3000 11.5 -> 11.2; 1 x 16000, 256 of them, 14.3 -> 14.7).
-static bool pa_eight_waves(int64_t workgroups, bool fp8, bool one_piece) {
+// behind them gain up to 128 workgroups (1 x 3000 11.5 -> 11.2; 1 x 16000, 256 of them, 14.3 -> 14.7).  Up to 256 keys four
+// waves have one round or two and the other four only their part of the merge: 1 x 200 fp8 4.7 -> 5.1, 16-bit 5.2 -> 5.4, 1 x 300
+// 6.1 -> 5.9, 5.6 -> 5.5; up to 512 keys 256 workgroups are faster with four (32 x 500 7.9 -> 8.5).
+static bool pa_eight_waves(const PagedAttnParams& p, int64_t workgroups, bool fp8, bool one_piece) {
   if (g_pa_waves) return g_pa_waves == 8;
-  return workgroups <= (!fp8 ? 64 : one_piece ? 256 : 128);
+  if ((p.max_seq_len > 0 && p.max_seq_len <= 256) || (p.window > 0 && p.window <= 256)) return false;
+  return workgroups <= (!fp8 ? 64 : one_piece && !(p.max_seq_len > 0 && p.max_seq_len <= 512) ? 256 : 128);
 }
 
 #define PA_ARGS(A)                                                                                 \
@@ -826,7 +829,7 @@ static int launch_mfma_v(const PagedAttnParams& p) {
     }
   }
   if constexpr (HS <= 128) {
-    if (pa_eight_waves((int64_t)grid.x * grid.y, FP8, grid.y == 1)) {
+    if (pa_eight_waves(p, (int64_t)grid.x * grid.y, FP8, grid.y == 1)) {
       hipLaunchKernelGGL((pa_mfma_kernel<scalar_t, FP8, HS, BS, 8, VARIANT, PAD, false>), grid, dim3(8 * 64), 0,
                          p.stream, PA_ARGS(A));
       VA_LAUNCH_CHECK("paged_attention mfma launch");
@@ -917,7 +920,7 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       // 1000 13.8 / 12.0).
       if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
         const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO;
-        const bool w8 = p.head_size <= 128 && pa_eight_waves(base, fp8, true);
+        const bool w8 = p.head_size <= 128 && pa_eight_waves(p, base, fp8, true);
         const double tb = 2.0 * p.head_size * (fp8 ? 1 : 2), t = w8 ? 2.2e-3 + tb * 7.8e-6 : 3.5e-3 + tb * 12.2e-6;
         const double alone = p.max_seq_len * t, stream = 0.6 * (double)base * p.max_seq_len * tb / 6.2e6;
         const double one = 1.05 * (alone > stream ? alone : stream), piece = (double)sp * p.partition_size * t;
