@@ -912,8 +912,7 @@ int paged_attention_mfma(const PagedAttnParams& p0) {
       // taken to be 0.6 full.  Up to 10 us only: a long sequence among short ones has to be cut.  Measured, cut -> one piece:
       // 1 x 600 fp8 10.5 -> 8.7, 1 x 1000 11.6 -> 10.4, 32 x 1000 17.8 -> 13.8, 32 x 1500 23.1 -> 18.7, 16 x 600 16-bit
       // 14.5 -> 11.1; kept cut: 1 x 1000 16-bit 12.0 (one piece 12.9), 1 x 1500 fp8 11.4 (13.2), head 256 1 x 1000 15.2 (15.8)
-      // (device time alone, batches of 1 .. 32: profiles/decode_one_piece.txt -- never above the cheaper form where it leaves
-      // the cut; up to 1.2 x are left where 16 sequences of 1000 .. 1500 tokens stay cut).
+      // (Device time alone, both forms and this rule: profiles/decode_plans.txt.)
       // With eight waves (pa_eight_waves) a token costs a workgroup 2.2 ns + 1 ns per 128 bytes; the merge costs 2.1 us and 6 ns
       // for each piece (us, one piece / cut, fp8: 1 x 1000 8.8 / 9.3, 1 x 1300 11.3 / 9.7, 8 x 1600 13.2 / 10.9, 16 x 1300
       // ragged 12.3 / 12.8, 24 x 1600 15.8 / 20.4; head 64 1 x 1600 9.7 / 8.5, 16 x 1600 10.5 / 11.3; 16-bit 1 x 777 8.1 / 9.5, 8 x
