@@ -653,6 +653,28 @@ def test_unified_rows_in_front_of_the_first_sequence(oracle, kernel):
         _lib.set_tuning("pf_fa", 0)
 
 
+@pytest.mark.parametrize("segs", [1, 3, 6, 16])
+def test_unified_decode_rows_that_are_not_the_sequence_number(oracle, segs):
+    """Decode tokens behind rows of other sequences, and an empty sequence among them: the merge finds each one's own row."""
+    from vllm_amd import _lib
+    from vllm_amd.attention.ops import unified_attention
+    c = make_unified_case([(1, n) for n in (5, 300, 1100, 64, 900, 1025)], 8, 2, 128, 16, torch.bfloat16, seed=segs)
+    ref = torch.zeros_like(c["q"])
+    oracle.unified_attention(c["q"], c["k"], c["v"], ref, c["cu_seqlens_q"], 1, c["seqused_k"],
+                             c["max_seqlen_k"], 128 ** -0.5, True, (-1, -1), c["block_table"], 0.0, None, None, None, None, None)
+    d = {k: v.cuda() for k, v in c.items() if torch.is_tensor(v)}
+    cu, at = torch.tensor([2, 3, 3, 4, 5, 6], dtype=torch.int32, device="cuda"), torch.tensor([2, 0, 3, 4, 5], device="cuda")
+    out = torch.zeros_like(d["q"])
+    _lib.set_tuning("uni_seg", segs)
+    try:
+        unified_attention(d["q"], d["k"], d["v"], out, cu, 1, d["seqused_k"][at].contiguous(), c["max_seqlen_k"], 128 ** -0.5, True,
+                          (-1, -1), d["block_table"][at].contiguous(), 0.0, None, None, None)
+    finally:
+        _lib.set_tuning("uni_seg", 0)
+    ref[:2] = 0
+    torch.testing.assert_close(out.cpu().float(), ref.float(), atol=ATOL, rtol=RTOL)
+
+
 def test_unified_scales_of_an_unquantised_cache_are_not_read(oracle):
     """A cache in the query's type: k_descale / v_descale may be anywhere (a layer's scales on the host); with fp8 they may not."""
     from vllm_amd.attention.ops import unified_attention

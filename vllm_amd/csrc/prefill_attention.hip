@@ -868,6 +868,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     u.max_seq_len = max_k;
     u.segm_out = p.segm_out; u.segm_max = p.segm_max; u.segm_sum = p.segm_sum;
     u.segm_stride = p.segm_stride;
+    u.num_tokens = num_tokens;
     u.dtype = std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16;
     u.fp8 = FP8; u.stream = st;
     u.hp = unified_decode_heads_per_row(u);

@@ -20,35 +20,50 @@ __global__ __launch_bounds__(NW * 64, (D > 128 && !FP8 ? 1 : D == 128 && FP8 ? 3
 
 // Merge of the key segments of a split launch (reduce_segments,
 // triton_unified_attention.py:499-586): one wave per (sequence, q head).  Lane s holds the max /
-// sum of segment s (at most 16 segments), the weights come from two 16-lane butterflies, and
-// the 16 partial rows are loaded back to back (segments past the sequence's last one re-read
-// that last one with weight 0), so the kernel is two dependent memory round trips.
-template <typename T, int D>
+// sum of segment s (at most NS), the weights come from two 16-lane butterflies, and the NS partial
+// rows are loaded back to back.  Bound by its memory round trips: the rows of token `seq` are requested
+// together with the lengths that say which token and how many segments it is -- in a decode step of one
+// token per sequence that is the token; if not, they are loaded again -- and rows that no segment wrote
+// are left out afterwards.  us, two round trips -> one, with the main kernel and the cache write:
+// 1 x 1000 fp8 12.0 -> 11.1, 8 x 3000 ragged of head 64 14.4 -> 13.6, 16 x 6000 ragged 31.8 -> 30.9.
+template <typename T, int D, int NS>
 __global__ __launch_bounds__(256) void ua_decode_reduce_kernel(const UniDecodeParams p) {
   constexpr int VPL = D / 64;   // outputs per lane
   const int lane = threadIdx.x & 63;
-  const int pair = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (pair >= p.num_seqs * p.num_heads) return;
   const int seq = pair / p.num_heads, head = pair % p.num_heads;
+  const int dr = p.head_size;
+  const bool dval = VPL * lane < dr;
+  typedef __attribute__((ext_vector_type(VPL))) float fv;
+  fv part[NS];
+  float ms, ls;
+  auto load = [&](int tok) __attribute__((always_inline)) {
+    const int64_t row = ((int64_t)tok * p.num_heads + head) * p.segm_stride;
+    const int sl = lane < p.num_segments ? lane : 0;
+    ms = p.segm_max[row + sl];
+    ls = p.segm_sum[row + sl];
+#pragma unroll
+    for (int s2 = 0; s2 < NS; ++s2)
+      part[s2] = *reinterpret_cast<const fv*>(p.segm_out + (row + min(s2, p.num_segments - 1)) * dr + (dval ? VPL * lane : 0));
+  };
+  const int guess = min(seq, p.num_tokens - 1);
+  load(guess);
   const int qtok = p.cu_seqlens_q[seq];
   if (p.cu_seqlens_q[seq + 1] - qtok != 1) return;
   const int ntiles = (p.seq_lens[seq] + 63) >> 6;
+  if (qtok != guess) load(qtok);
   const int tps = (ntiles + p.num_segments - 1) / p.num_segments;
   const int nseg = tps > 0 ? (ntiles + tps - 1) / tps : 0;   // segments the main kernel wrote
-  const int64_t row = ((int64_t)qtok * p.num_heads + head) * p.segm_stride;
   float acc[VPL], l = 0.f;
 #pragma unroll
   for (int j = 0; j < VPL; ++j) acc[j] = 0.f;
-  const int dr = p.head_size;
-  const bool dval = VPL * lane < dr;
   if (nseg > 0) {
-    const float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
-    const float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
-    typedef __attribute__((ext_vector_type(VPL))) float fv;
-    fv part[16];
+    ms = lane < nseg ? ms : -INFINITY;
+    ls = lane < nseg ? ls : 0.f;
 #pragma unroll
-    for (int s2 = 0; s2 < 16; ++s2)
-      part[s2] = dval ? *reinterpret_cast<const fv*>(p.segm_out + (row + min(s2, nseg - 1)) * dr + VPL * lane) : (fv)(0.f);
+    for (int s2 = 0; s2 < NS; ++s2)
+      part[s2] = s2 < nseg ? part[s2] : (fv)(0.f);
     float mx = ms;
     mx = row_max16(mx);
     const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);
@@ -56,7 +71,7 @@ __global__ __launch_bounds__(256) void ua_decode_reduce_kernel(const UniDecodePa
     l = row_sum16(l);
     l = __shfl(l, 0, 64);
 #pragma unroll
-    for (int s2 = 0; s2 < 16; ++s2) {
+    for (int s2 = 0; s2 < NS; ++s2) {
       const float ws = __shfl(w, s2, 64);
 #pragma unroll
       for (int j = 0; j < VPL; ++j) acc[j] += part[s2][j] * ws;
@@ -97,8 +112,10 @@ int launch(const UniDecodeParams& p) {
     hipLaunchKernelGGL((ua_decode_kernel<T, FP8, D, NW, false>), grid, dim3(NW * 64), 0, p.stream, p, sub_shift, xcd_group, order);
   VA_LAUNCH_CHECK("unified_attention decode launch");
   if (p.num_segments > 1) {
-    hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D>), dim3((unsigned)((p.num_seqs * p.num_heads + 3) / 4)),
-                       dim3(256), 0, p.stream, p);
+    const dim3 rgrid((unsigned)((p.num_seqs * p.num_heads + 3) / 4));
+    if (p.num_segments <= 4) hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D, 4>), rgrid, dim3(256), 0, p.stream, p);
+    else if (p.num_segments <= 8) hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D, 8>), rgrid, dim3(256), 0, p.stream, p);
+    else hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D, 16>), rgrid, dim3(256), 0, p.stream, p);
     VA_LAUNCH_CHECK("unified_attention decode merge launch");
   }
   return VLLM_AMD_OK;
