@@ -86,6 +86,7 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
     int num_tokens, int num_heads, int head_size, int block_size, int bs_log2, int hpw,
     const float* __restrict__ k_scale_p, const float* __restrict__ v_scale_p) {
   constexpr int CS = sizeof(cache_t);
+  static_assert(sizeof(scalar_t) == 2 && (CS == 1 || CS == 2), "the transposes are of 1- and 2-byte elements");
   constexpr int X = 16 / CS;    // elements of one K cache vector
   constexpr int G = 16;         // tokens per workgroup, slots per tile
   constexpr int U = 4 / CS;     // elements of a 4-byte unit
@@ -406,25 +407,28 @@ static int launch_reshape_and_cache(const void* key, const void* value, void* kc
                       (key_stride % x == 0) && (value_stride % x == 0) &&
                       aligned(key, sizeof(scalar_t) * XN) && aligned(value, sizeof(scalar_t) * XN) &&
                       aligned(kc, 16);
-  // many tokens: the run-aware kernel (16 tokens x 1 head per workgroup)
-  const bool runs_ok = vec_ok && sizeof(scalar_t) == 2 && num_tokens >= 256 && block_size % 16 == 0 &&
-                       head_size % 8 == 0 && head_size <= 256 && aligned(vc, 16);
-  if (runs_ok && g_cache_runs) {
-    int bs_log2 = -1;
-    for (int i = 4; i < 16; ++i) if (block_size == (1 << i)) bs_log2 = i;
-    int hpw = 512 / head_size;   // heads per workgroup: hpw * head_size <= 512 elements
-    if (hpw > num_heads) hpw = num_heads;
-    // fewer heads per workgroup while the launch would not fill the chip a few times over
-    // (8192 tokens 19.8 us with 1 head per workgroup, 14.3 with 4; 2048 tokens 6.8 / 6.2
-    // with 1 / 2: tools/bench_cache_hpw.py)
-    while (hpw > 1 && (int64_t)((num_tokens + 15) / 16) * ((num_heads + hpw - 1) / hpw) < 512) hpw /= 2;
-    if (g_cache_hpw > 0 && g_cache_hpw * head_size <= 512 && g_cache_hpw <= num_heads) hpw = g_cache_hpw;
-    hipLaunchKernelGGL((reshape_and_cache_runs_kernel<scalar_t, cache_t, FP8>),
-                       dim3((num_tokens + 15) / 16, (num_heads + hpw - 1) / hpw, 2), dim3(256), 0, st,
-                       (const scalar_t*)key, (const scalar_t*)value, (cache_t*)kc, (cache_t*)vc,
-                       slot_mapping, key_stride, value_stride, num_tokens, num_heads, head_size,
-                       block_size, bs_log2, hpw, ks, vs);
-  } else if (vec_ok) {
+  // many tokens: the run-aware kernel
+  if constexpr (sizeof(scalar_t) == 2) {
+    if (vec_ok && num_tokens >= 256 && block_size % 16 == 0 && head_size % 8 == 0 && head_size <= 256 && aligned(vc, 16) && g_cache_runs) {
+      int bs_log2 = -1;
+      for (int i = 4; i < 16; ++i) if (block_size == (1 << i)) bs_log2 = i;
+      int hpw = 512 / head_size;   // heads per workgroup: hpw * head_size <= 512 elements
+      if (hpw > num_heads) hpw = num_heads;
+      // fewer heads per workgroup while the launch would not fill the chip a few times over
+      // (8192 tokens 19.8 us with 1 head per workgroup, 14.3 with 4; 2048 tokens 6.8 / 6.2
+      // with 1 / 2: tools/bench_cache_hpw.py)
+      while (hpw > 1 && (int64_t)((num_tokens + 15) / 16) * ((num_heads + hpw - 1) / hpw) < 512) hpw /= 2;
+      if (g_cache_hpw > 0 && g_cache_hpw * head_size <= 512 && g_cache_hpw <= num_heads) hpw = g_cache_hpw;
+      hipLaunchKernelGGL((reshape_and_cache_runs_kernel<scalar_t, cache_t, FP8>),
+                         dim3((num_tokens + 15) / 16, (num_heads + hpw - 1) / hpw, 2), dim3(256), 0, st,
+                         (const scalar_t*)key, (const scalar_t*)value, (cache_t*)kc, (cache_t*)vc,
+                         slot_mapping, key_stride, value_stride, num_tokens, num_heads, head_size,
+                         block_size, bs_log2, hpw, ks, vs);
+      VA_LAUNCH_CHECK("reshape_and_cache launch");
+      return VLLM_AMD_OK;
+    }
+  }
+  if (vec_ok) {
     const int nchunks = num_heads * head_size / x;
     int threads = nchunks < 256 ? ((nchunks + 63) / 64) * 64 : 256;
     hipLaunchKernelGGL((reshape_and_cache_kernel<scalar_t, cache_t, FP8, XN>), dim3(num_tokens),
