@@ -163,6 +163,37 @@ def test_reshape_and_cache_every_run(ops, oracle, kv, BS):
     assert torch.equal(vc_d.cpu().view(torch.uint8), vc_o.view(torch.uint8))
 
 
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("D,H,hpw", [(80, 5, 5), (80, 5, 2), (120, 4, 4), (256, 2, 2), (24, 3, 3), (16, 1, 1)])
+def test_reshape_and_cache_widths(ops, oracle, kv, D, H, hpw):
+    """Whole tiles and both halves of partial ones at rows of 16 .. 512 elements a workgroup: fewer rows than lanes, a number that is no
+    multiple of 64 or 256, a last workgroup of fewer heads."""
+    from vllm_amd import _lib
+    if kv != "auto" and D % 16:
+        pytest.skip("fp8 cache needs head_size % 16 == 0 (x = 16)")
+    dtype, BS = torch.bfloat16, 32
+    slots, blk = [], 1
+    for first, ln in ((0, 96), (5, 11), (5, 3), (8, 40), (16, 80), (31, 34), (3, 5), (0, 16)):
+        slots += [blk * BS + first + i for i in range(ln)]
+        blk += (first + ln + BS - 1) // BS
+    slots = torch.tensor(slots, dtype=torch.int64)
+    T, NB, x = len(slots), blk + 1, x_of(dtype, kv)
+    key, value = _kv_inputs(T, H, D, dtype, D, strided=False)
+    cdt = dtype if kv == "auto" else torch.uint8
+    s = 0.05 if kv != "auto" else 1.0
+    kc_o, vc_o = torch.zeros((NB, H, D // x, BS, x), dtype=cdt), torch.zeros((NB, H, D, BS), dtype=cdt)
+    kc_d, vc_d = kc_o.cuda(), vc_o.cuda()
+    oracle.reshape_and_cache(key, value, kc_o, vc_o, slots, kv, s, s)
+    _lib.set_tuning("cache_hpw", hpw)
+    try:
+        sc = torch.tensor([s], device="cuda")
+        ops.reshape_and_cache(key.cuda(), value.cuda(), kc_d, vc_d, slots.cuda(), kv, sc, sc)
+    finally:
+        _lib.set_tuning("cache_hpw", 0)
+    assert torch.equal(kc_d.cpu().view(torch.uint8), kc_o.view(torch.uint8))
+    assert torch.equal(vc_d.cpu().view(torch.uint8), vc_o.view(torch.uint8))
+
+
 @pytest.mark.parametrize("scale", [1.0, 0.37, -0.021, 3e-5, 300.0])
 def test_cache_write_every_half(ops, oracle, scale):
     """The vectorised fp16 conversion over all finite halves: byte-exact, NaN codes of overflowing quotients up to their sign."""

@@ -72,10 +72,10 @@ __global__ void reshape_and_cache_kernel(
 // tokens, and only its two ends are partial tiles, written as 4-byte units and single elements.
 // The first segment is blockIdx.z = 0's, a second one blockIdx.z = 1's (in one workgroup behind
 // each other 1.0 us more); more (decode batches) are scattered token by token.
-// Bound by latency: read and write phases of one round of workgroups (4 TB/s at 8192 aligned
+// Bound by latency: read and write phases of one round of workgroups (4.2 TB/s at 8192 aligned
 // tokens).  us, tiles at multiples of 16 tokens -> at the groups, 8 heads of 128: 8192 tokens from
-// slot 11 of a block fp8 20.4 -> 15.2, 16-bit 31.0 -> 16.9 (aligned 16.0 -> 14.2, 16.2 -> 16.6), 24 chunks
-// of up to 250 16.9 -> 13.9, 25.4 -> 14.9, 60 chunks of up to 33 9.0 -> 9.5, 9.9 -> 9.0.
+// slot 11 of a block fp8 20.1 -> 14.9, 16-bit 30.7 -> 14.7 (aligned 15.8 -> 13.8, 15.9 -> 14.9), 24 chunks
+// of up to 250 16.8 -> 13.4, 24.4 -> 13.1, 60 chunks of up to 33 9.0 -> 8.8, 9.8 -> 8.5.
 // Requires block_size % 16 == 0 and head_size <= 256.
 // ---------------------------------------------------------------------------
 template <typename scalar_t, typename cache_t, bool FP8>
@@ -198,53 +198,93 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
     int64_t blk, off;
     split(s_slot[i0] - col0, blk, off);
     cache_t* const vdst = value_cache + blk * blk_elems + head_off + off;
-    // a thread takes U consecutive d: one 4-byte LDS read per slot, a transpose in registers (v_perm_b32), rows of
-    // 16 / 32 bytes, or what there is of them (reads of single elements made this kernel bound by LDS issue)
-    const int lo = col0, hi = col0 + __popc(mask);
-    for (int w = tid; w < width / U; w += 256) {
-      uint32_t col[16];
+    // whole tiles, rows of 16 / 32 bytes
+    if (mask == 0xffffu) {
+      if constexpr (CS == 1) {
+        // a thread takes four consecutive d: one 4-byte LDS read per slot, a transpose in registers (reads of single elements made
+        // this kernel bound by LDS issue)
+        for (int w = tid; w < width / 4; w += 256) {
+          uint32_t col[16];
 #pragma unroll
-      for (int p = 0; p < 16; ++p) col[p] = *reinterpret_cast<const uint32_t*>(&vt[p][w * U]);
+          for (int p = 0; p < 16; ++p) col[p] = *reinterpret_cast<const uint32_t*>(&vt[p][w * 4]);
 #pragma unroll
-      for (int e = 0; e < U; ++e) {
-        cache_t* dst = vdst + (int64_t)(w * U + e) * block_size;
-        uint32_t row[4 * CS];
-        if constexpr (CS == 1) {
-          const uint32_t sel = 0x0c0c0000u | ((4u + e) << 8) | (uint32_t)e;   // byte e of (S1, S0)
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t sel = 0x0c0c0000u | ((4u + e) << 8) | (uint32_t)e;   // byte e of (S1, S0)
+            u32x4 row;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t x = __builtin_amdgcn_perm(col[4 * k + 1], col[4 * k], sel);
+              const uint32_t y = __builtin_amdgcn_perm(col[4 * k + 3], col[4 * k + 2], sel);
+              row[k] = __builtin_amdgcn_perm(y, x, 0x05040100u);
+            }
+            *reinterpret_cast<u32x4*>(vdst + (int64_t)(w * 4 + e) * block_size) = row;
+          }
+        }
+      } else {
+        // a lane takes two d and eight slots, and lanes 0, 1 of a quad trade their second row for the first one of lanes 2, 3, so that
+        // a store instruction covers 1 KiB in one piece (as 16 bytes a lane, 64 bytes apart, 8192 tokens took 16.6 us, now 14.9, 32768
+        // 56.9, now 52.6)
+        for (int it = tid; it < width; it += 256) {
+          const int w = it >> 1, h = it & 1;
+          const bool up = (it & 2) != 0;
+          uint32_t col[8];
+#pragma unroll
+          for (int p = 0; p < 8; ++p) col[p] = *reinterpret_cast<const uint32_t*>(&vt[8 * h + p][2 * w]);
+          u32x4 first, second;
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const uint32_t a = __builtin_amdgcn_perm(col[4 * k + 1], col[4 * k], sel);
-            const uint32_t b = __builtin_amdgcn_perm(col[4 * k + 3], col[4 * k + 2], sel);
-            row[k] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+            const uint32_t x = __builtin_amdgcn_perm(col[2 * k + 1], col[2 * k], 0x05040100u);   // rows 2 w, 2 w + 1
+            const uint32_t y = __builtin_amdgcn_perm(col[2 * k + 1], col[2 * k], 0x07060302u);
+            const uint32_t z = __builtin_amdgcn_update_dpp(0, up ? x : y, 0x4e, 0xf, 0xf, true);   // of lane ^ 2
+            first[k] = up ? z : x;
+            second[k] = up ? y : z;
           }
-        } else {
-#pragma unroll
-          for (int k = 0; k < 8; ++k) row[k] = __builtin_amdgcn_perm(col[(2 * k + 1) & 15], col[(2 * k) & 15], e ? 0x07060302u : 0x05040100u);
+          cache_t* dst = vdst + (int64_t)(2 * (w & ~1) + (up ? 1 : 0)) * block_size + 8 * h;
+          *reinterpret_cast<u32x4*>(dst) = first;
+          *reinterpret_cast<u32x4*>(dst + 2 * (int64_t)block_size) = second;
         }
-        if (mask == 0xffffu) {
+      }
+      return;
+    }
+    // what there is of a tile: a row per thread (four rows a thread left most of the workgroup idle behind a chain of small stores:
+    // 300 fp8 tokens from slot 11 6.0 us, now 5.2, 60 chunks of up to 33 9.4, now 8.8)
+    const int lo = col0, hi = col0 + __popc(mask);
+    for (int d = tid; d < width; d += 256) {
+      const int e = d % U;
+      cache_t* dst = vdst + (int64_t)d * block_size;
+      uint32_t col[16], row[4 * CS];
 #pragma unroll
-          for (int h = 0; h < CS; ++h)
-            *reinterpret_cast<u32x4*>(dst + 8 * h) = (u32x4){row[4 * h], row[4 * h + 1], row[4 * h + 2], row[4 * h + 3]};
+      for (int p = 0; p < 16; ++p) col[p] = *reinterpret_cast<const uint32_t*>(&vt[p][d - e]);
+      if constexpr (CS == 1) {
+        const uint32_t sel = 0x0c0c0000u | ((4u + e) << 8) | (uint32_t)e;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t x = __builtin_amdgcn_perm(col[4 * k + 1], col[4 * k], sel);
+          const uint32_t y = __builtin_amdgcn_perm(col[4 * k + 3], col[4 * k + 2], sel);
+          row[k] = __builtin_amdgcn_perm(y, x, 0x05040100u);
+        }
+      } else {
+        const uint32_t sel = e ? 0x07060302u : 0x05040100u;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) row[k] = __builtin_amdgcn_perm(col[2 * k + 1], col[2 * k], sel);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {   // (uniform branches)
+        if (8 * h >= lo && 8 * h + 8 <= hi) {
+          if constexpr (CS == 1) *reinterpret_cast<uint2*>(dst + 8 * h) = make_uint2(row[2 * h], row[2 * h + 1]);
+          else *reinterpret_cast<u32x4*>(dst + 8 * h) = (u32x4){row[4 * h], row[4 * h + 1], row[4 * h + 2], row[4 * h + 3]};
           continue;
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {   // (uniform branches)
-          if (8 * h >= lo && 8 * h + 8 <= hi) {
-            if constexpr (CS == 1) *reinterpret_cast<uint2*>(dst + 8 * h) = make_uint2(row[2 * h], row[2 * h + 1]);
-            else *reinterpret_cast<u32x4*>(dst + 8 * h) = (u32x4){row[4 * h], row[4 * h + 1], row[4 * h + 2], row[4 * h + 3]};
-            continue;
-          }
+        for (int k = 0; k < 8 / U; ++k) {
+          const int q = 8 * h + U * k;
+          const uint32_t x = row[q / U];
+          if (q >= lo && q + U <= hi) {
+            *reinterpret_cast<uint32_t*>(dst + q) = x;
+          } else {
 #pragma unroll
-          for (int k = 0; k < 8 / U; ++k) {
-            const int q = 8 * h + U * k;
-            const uint32_t x = row[q / U];
-            if (q >= lo && q + U <= hi) {
-              *reinterpret_cast<uint32_t*>(dst + q) = x;
-            } else {
-#pragma unroll
-              for (int j = 0; j < U; ++j)
-                if (q + j >= lo && q + j < hi) __builtin_memcpy(dst + q + j, (const char*)&x + j * CS, CS);
-            }
+            for (int j = 0; j < U; ++j)
+              if (q + j >= lo && q + j < hi) __builtin_memcpy(dst + q + j, (const char*)&x + j * CS, CS);
           }
         }
       }
