@@ -194,6 +194,36 @@ def test_reshape_and_cache_widths(ops, oracle, kv, D, H, hpw):
     assert torch.equal(vc_d.cpu().view(torch.uint8), vc_o.view(torch.uint8))
 
 
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,D,H,hpw,BS", [(512, 128, 8, 4, 16), (700, 80, 5, 5, 32), (513, 256, 3, 2, 48), (600, 16, 1, 1, 16), (511, 64, 2, 2, 16)])
+def test_reshape_and_cache_scattered(ops, oracle, kv, dtype, T, D, H, hpw, BS):
+    """Slots that do not follow each other, padding and a few short runs among them: a wave along d, from 512 tokens on."""
+    from vllm_amd import _lib
+    g = torch.Generator().manual_seed(T)
+    NB, x = 2 * T // BS + 2, x_of(dtype, kv)
+    slots = torch.randperm(NB * BS, generator=g)[:T]
+    slots[5::37] = -1
+    free = sorted(set(range(NB * BS)) - set(slots.tolist()))
+    runs = [a for a in free if a + 1 in free and a + 2 in free and a % 3 == 0][:8]
+    for n, a in enumerate(runs):   # (three slots in a row, all different)
+        slots[40 * n + 10:40 * n + 13] = torch.arange(a, a + 3)
+    key, value = _kv_inputs(T, H, D, dtype, D, strided=False)
+    cdt = dtype if kv == "auto" else torch.uint8
+    s = 0.05 if kv != "auto" else 1.0
+    kc_o, vc_o = torch.zeros((NB, H, D // x, BS, x), dtype=cdt), torch.zeros((NB, H, D, BS), dtype=cdt)
+    kc_d, vc_d = kc_o.cuda(), vc_o.cuda()
+    oracle.reshape_and_cache(key, value, kc_o, vc_o, slots, kv, s, s)
+    _lib.set_tuning("cache_hpw", hpw)
+    try:
+        sc = torch.tensor([s], device="cuda")
+        ops.reshape_and_cache(key.cuda(), value.cuda(), kc_d, vc_d, slots.cuda(), kv, sc, sc)
+    finally:
+        _lib.set_tuning("cache_hpw", 0)
+    assert torch.equal(kc_d.cpu().view(torch.uint8), kc_o.view(torch.uint8))
+    assert torch.equal(vc_d.cpu().view(torch.uint8), vc_o.view(torch.uint8))
+
+
 @pytest.mark.parametrize("scale", [1.0, 0.37, -0.021, 3e-5, 300.0])
 def test_cache_write_every_half(ops, oracle, scale):
     """The vectorised fp16 conversion over all finite halves: byte-exact, NaN codes of overflowing quotients up to their sign."""

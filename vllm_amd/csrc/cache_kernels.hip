@@ -78,8 +78,9 @@ __global__ void reshape_and_cache_kernel(
 // of up to 250 16.8 -> 13.4, 24.4 -> 13.1, 60 chunks of up to 33 9.0 -> 8.8, 9.8 -> 8.5.
 // Requires block_size % 16 == 0 and head_size <= 256.
 // ---------------------------------------------------------------------------
+// (five workgroups per CU: 96 registers, two less than hipcc takes for bf16 -> fp8 by itself)
 template <typename scalar_t, typename cache_t, bool FP8>
-__global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
+__global__ __launch_bounds__(256, 5) void reshape_and_cache_runs_kernel(
     const scalar_t* __restrict__ key, const scalar_t* __restrict__ value,
     cache_t* __restrict__ key_cache, cache_t* __restrict__ value_cache,
     const int64_t* __restrict__ slot_mapping, int64_t key_stride, int64_t value_stride,
@@ -147,7 +148,8 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
       r.v[u] = *reinterpret_cast<const Vec<scalar_t, 8>*>(vbase + (ok ? (int64_t)(t0 + i0 + i) * value_stride + c * 8 : 0));
     }
   };
-  auto store = [&](int i0, uint32_t mask, bool run, const Rows& r) __attribute__((always_inline)) {
+  // run: a segment; single (i0 = 0, no run): V through LDS, too
+  auto store = [&](int i0, uint32_t mask, bool run, bool single, const Rows& r) __attribute__((always_inline)) {
     // K: a wave writes 256-byte pieces of a run (16 tokens x one 16-byte vector)
     const int cph = head_size / X;
 #pragma unroll
@@ -169,7 +171,8 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
                                            ((int64_t)xc * block_size + off) * X) = kq;
     }
 
-    // V: into the LDS tile (run) or scattered
+    // V: into the LDS tile (run, single) or scattered
+    const bool tile = run || single;
     const int col0 = run ? (int)(s_slot[i0] & 15) : 0;
 #pragma unroll
     for (int u = 0; u < VI; ++u) {
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
       } else {
         vq = r.v[u];
       }
-      if (run) {
+      if (tile) {
         *reinterpret_cast<Vec<cache_t, 8>*>(&vt[col0 + i][c * 8]) = vq;
       } else {
         int64_t blk, off;
@@ -192,8 +195,31 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
         for (int j = 0; j < 8; ++j) dst[(int64_t)j * block_size] = vq.v[j];
       }
     }
-    if (!run) return;
+    if (!tile) return;
     __syncthreads();
+    if (!run) {
+      // element by element, a wave along d, four stores at a time
+      const int per = (width + 63) / 64, n = G * per;
+      for (int it = __builtin_amdgcn_readfirstlane(tid >> 6); it < n; it += 16) {
+        cache_t x[4];
+        cache_t* dst[4];
+        bool ok[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int i = (it + 4 * u) / per, d = 64 * (it + 4 * u - i * per) + lane;
+          ok[u] = it + 4 * u < n && ((mask >> i) & 1) && d < width;
+          const uint32_t slo = __builtin_amdgcn_readlane((int)sl, i + 1), shi = __builtin_amdgcn_readlane((int)(sl >> 32), i + 1);
+          int64_t blk, off;
+          split((int64_t)((uint64_t)shi << 32 | slo), blk, off);
+          dst[u] = value_cache + blk * blk_elems + head_off + (int64_t)d * block_size + off;
+          x[u] = vt[i & 15][d < width ? d : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (ok[u]) *dst[u] = x[u];
+      }
+      return;
+    }
 
     int64_t blk, off;
     split(s_slot[i0] - col0, blk, off);
@@ -299,7 +325,11 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
     const uint32_t mask = blockIdx.z ? (1u << __builtin_ctz(~tail)) - 1u : valid & (0xffffu << __builtin_ctz(starts)) & 0xffffu;
     if (mask == 0) return;
     load(blockIdx.z ? G : 0, mask, r);
-    store(blockIdx.z ? G : 0, mask, false, r);
+    // Slots that hardly ever follow each other (a decode batch) go through LDS: a thread that stores its own eight elements touches a
+    // line of the cache per lane and store, a wave along d eight (fp8) or sixteen.  us, by threads -> by waves: fp8 1024 tokens 11.4 ->
+    // 9.7, 2048 17.4 -> 13.2, 8192 65.3 -> 43.8, 16-bit 1024 12.5 -> 11.8, 8192 171.5 -> 165; below 512 tokens the longer way costs
+    // more (256: fp8 6.2 -> 6.5), and tokens in short runs share the lines that their thread touches.
+    store(blockIdx.z ? G : 0, mask, false, blockIdx.z == 0 && num_tokens >= 512 && __popc(starts) > 12, r);
     return;
   }
   if (blockIdx.z) starts &= starts - 1;
@@ -307,7 +337,7 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(
   const int i0 = __builtin_ctz(starts);
   const uint32_t mask = (2u << __builtin_ctz(~(cont >> (i0 + 1)))) - 1u;   // at most 16: a group's end is never continued
   load(i0, mask, r);
-  store(i0, mask, true, r);
+  store(i0, mask, true, false, r);
 }
 
 // Scalar fallback for layouts / alignments the vector kernel does not cover
