@@ -482,6 +482,21 @@ def test_eight_waves(ops, oracle, version, kv, head_size, block_size):
 
 
 @pytest.mark.parametrize("version", ["v2", "rocm"])
+@pytest.mark.parametrize("head_size,block_size", [(80, 16), (120, 32)])
+def test_padded_heads_in_many_pieces(ops, oracle, version, head_size, block_size):
+    """More than 512 pieces of padded rows over a 16-bit cache: two workgroups per CU, and some left to hand out."""
+    from vllm_amd import _lib
+    step = 512 if version == "v2" else 256
+    lens = [step * 3 - 7 * i if i % 3 else 1 + 40 * i for i in range(25)]
+    c = make_attn_case(len(lens), 16, 8, head_size, block_size, torch.bfloat16, "auto", lens, seed=head_size)
+    _lib.set_tuning("pa_sp", 1)
+    try:
+        run_case(ops, oracle, c, version)
+    finally:
+        _lib.set_tuning("pa_sp", 0)
+
+
+@pytest.mark.parametrize("version", ["v2", "rocm"])
 @pytest.mark.parametrize("kv", ["auto", "fp8"])
 @pytest.mark.parametrize("head_size,max_len", [(64, 1290), (128, 600), (80, 513), (256, 520)])
 def test_one_piece_per_sequence(ops, oracle, version, kv, head_size, max_len):

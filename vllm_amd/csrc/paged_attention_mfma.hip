@@ -837,7 +837,13 @@ static int launch_mfma_v(const PagedAttnParams& p) {
       return VLLM_AMD_OK;
     }
   }
-  hipLaunchKernelGGL((pa_mfma_kernel<scalar_t, FP8, HS, BS, NW, VARIANT, PAD, false>), grid, dim3(NW * 64), 0,
+  // Head sizes 72 .. 120 over a 16-bit cache have the registers of three workgroups per CU, and with 513 .. 768 pieces that is all of
+  // them at once: nothing is left to hand out as others finish, and a ragged batch ends on the CUs that drew three long ones.  20 KiB
+  // of LDS that nobody uses keep it at the two per CU that the pieces are cut for (us, three -> two per CU, ragged: 18 x 9102 of
+  // head 80 56.9 -> 45.2, 34 x 3194 of 112 57.4 -> 47.8, 36 x 2978 of 96 46.3 -> 41.7; all alike it is the other way round,
+  // 18 x 9102 74.0 -> 80.3, 39 x 2194 52.5 -> 54.8).
+  const bool two = PAD && HS == 128 && !FP8 && part && !direct && (int64_t)grid.x * grid.y > 512;
+  hipLaunchKernelGGL((pa_mfma_kernel<scalar_t, FP8, HS, BS, NW, VARIANT, PAD, false>), grid, dim3(NW * 64), two ? 20 * 1024 : 0,
                      p.stream, PA_ARGS(A));
   VA_LAUNCH_CHECK("paged_attention mfma launch");
   if (part && !direct) return paged_attention_reduce(p);
