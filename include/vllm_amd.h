@@ -87,6 +87,14 @@ int vllm_amd_paged_attention_v2(
     int blocksparse_vert_stride, int blocksparse_block_size,
     int blocksparse_head_sliding_step, void* stream);
 
+/* Pieces that vllm_amd_paged_attention_v2 would cut the sequences of such a call into (1: every sequence in one, and the
+ * scratch stays untouched -- the call may as well be vllm_amd_paged_attention_v1), max_num_partitions partitions each if the call is
+ * not the matrix-core kernel's.  Host arithmetic only. */
+int vllm_amd_paged_attention_v2_pieces(
+    const void* out, const void* query, int num_seqs, int num_heads, int head_size, int num_kv_heads, int block_size,
+    int max_seq_len, int max_num_partitions, int dtype, int kv_dtype, int64_t q_stride, int64_t kv_head_stride,
+    int blocksparse_vert_stride);
+
 /* Replaces torch.ops._rocm_C.paged_attention
  *   schema csrc/rocm/torch_bindings.cpp:42-56, entry csrc/rocm/attention.cu:3494-3539,
  *   launcher :3073-3228, python vllm/_custom_ops.py:100-126.

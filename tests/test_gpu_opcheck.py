@@ -181,6 +181,12 @@ def test_opcheck_call_operators():
     for per_token in (True, False):
         opcheck(torch.ops._vllm_amd_C.fp8_linear, (out, x, wq.t(), ws, None, r(64), per_token))
     i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    # one piece, and cut in two (scratch inside)
+    kx, vx, one = r(160, 2, 16, 16, 8), r(160, 2, 128, 16), torch.ones(1, device="cuda")
+    for n, lens in ((1, 600), (20, 1000)):
+        qd = r(n, 4, 128)
+        opcheck(torch.ops._vllm_amd_C.paged_attention_decode, (torch.empty_like(qd), qd, kx, vx, 2, 0.09, torch.randint(
+            160, (n, 64), dtype=torch.int32, device="cuda"), i32(*[lens] * n), 16, lens, None, "auto", one, one, 0, 0, 0, 64, 0))
     # 70 new tokens over 1100 (split over the keys: scratch inside) and a one-token sequence
     q, o = r(71, 4, 128), torch.empty((71, 4, 128), dtype=torch.bfloat16, device="cuda")
     table = torch.arange(160, dtype=torch.int32, device="cuda").view(2, 80)

@@ -481,6 +481,49 @@ def test_eight_waves(ops, oracle, version, kv, head_size, block_size):
             _lib.set_tuning("pa_waves", 0)
 
 
+@pytest.mark.parametrize("kv,S,head_size,block_size,dtype", [
+    ("fp8", 3, 128, 16, torch.bfloat16), ("auto", 3, 128, 32, torch.float16), ("auto", 9, 128, 16, torch.bfloat16), ("fp8", 20, 80, 16, torch.float16),
+    ("auto", 3, 256, 16, torch.bfloat16), ("auto", 3, 120, 8, torch.bfloat16), ("auto", 3, 64, 16, torch.float32)])
+def test_forward_decode_two_partitions(ops, oracle, kv, S, head_size, block_size, dtype):
+    """513 .. 1024 keys: in one piece and cut (9 sequences of a 16-bit cache), the generic kernel, eager and from a captured graph."""
+    from vllm_amd.attention import PagedAttention
+    lens = [(1000, 513, 1, 512, 700, 1024, 16, 900)[i % 8] for i in range(S)]
+    c = make_attn_case(S, 32, 8, head_size, block_size, dtype, kv, lens, seed=S, kv_scale=1.0 if kv == "auto" else 0.5)
+    ref = torch.zeros_like(c["q"])
+    oracle.paged_attention_v1(ref, c["q"], c["kc"], c["vc"], 8, c["scale"], c["bt"], c["sl"], block_size, c["max_len"], None, kv, c["kv_scale"],
+                              c["kv_scale"])
+    q, kc, vc, bt, sl = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt", "sl"))
+    sc = torch.tensor([c["kv_scale"]], device="cuda")
+    call = lambda: PagedAttention.forward_decode(q, kc, vc, bt, sl, c["max_len"], kv, 8, c["scale"], None, sc, sc)
+    out = call()
+    torch.testing.assert_close(out.cpu().float(), ref.float(), **TOL["auto" if kv == "auto" else "fp8"])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        captured = call()
+    for _ in range(3):
+        captured.zero_()
+        call()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, out)
+
+
+def test_forward_decode_unaligned_query_wide_table(ops, oracle):
+    """A query that is not 16-byte aligned is the generic kernel's, whose unpartitioned form has no room for the scores of a block table of
+    48000 tokens: two partitions of it have."""
+    from vllm_amd.attention import PagedAttention
+    c = make_attn_case(3, 8, 2, 128, 16, torch.bfloat16, "auto", [700, 513, 1], seed=4)
+    ref = torch.zeros_like(c["q"])
+    oracle.paged_attention_v1(ref, c["q"], c["kc"], c["vc"], 2, c["scale"], c["bt"], c["sl"], 16, c["max_len"], None, "auto", 1.0, 1.0)
+    q = torch.zeros(3 * 8 * 128 + 4, dtype=torch.bfloat16, device="cuda")[4:].view(3, 8, 128)
+    q.copy_(c["q"])
+    bt = torch.zeros((3, 3000), dtype=torch.int32)
+    bt[:, :c["bt"].shape[1]] = c["bt"]
+    one = torch.ones(1, device="cuda")
+    out = PagedAttention.forward_decode(q, c["kc"].cuda(), c["vc"].cuda(), bt.cuda(), c["sl"].cuda(), 700, "auto", 2, c["scale"], None, one, one)
+    torch.testing.assert_close(out.cpu().float(), ref.float(), **TOL["auto"])
+
+
 @pytest.mark.parametrize("version", ["v2", "rocm"])
 @pytest.mark.parametrize("head_size,block_size", [(80, 16), (120, 32)])
 def test_padded_heads_in_many_pieces(ops, oracle, version, head_size, block_size):

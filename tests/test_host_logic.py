@@ -58,6 +58,51 @@ def test_forward_decode_heuristic(monkeypatch, S, H, max_len, want, KVH):
         assert es.dtype == torch.float32 and tmp.dtype == q.dtype
 
 
+@pytest.mark.parametrize("S,H,KVH,D,BS,dtype,kv,want", [
+    (1, 32, 8, 128, 16, torch.bfloat16, "fp8", "decode"),
+    (8, 32, 8, 128, 16, torch.bfloat16, "auto", "decode"),
+    (8, 32, 8, 128, 8, torch.bfloat16, "auto", "decode"),
+    (4, 16, 8, 256, 32, torch.float16, "auto", "decode"),
+    (4, 16, 8, 64, 16, torch.float32, "auto", "decode"),
+    (40, 32, 8, 128, 16, torch.bfloat16, "auto", "v1"),       # 320 workgroups: one per CU and more
+    (200, 32, 1, 128, 16, torch.bfloat16, "fp8", "v1"),       # 32 q heads per kv head: two workgroups each
+])
+def test_forward_decode_two_partitions(monkeypatch, S, H, KVH, D, BS, dtype, kv, want):
+    """Between 513 and 1024 keys the operator that knows the plan decides, whatever the types and shapes; no scratch from here."""
+    from vllm_amd.attention import paged_attn
+    calls = {}
+    for mod, name, key in ((paged_attn.ops, "paged_attention_v1", "v1"), (paged_attn.ops, "paged_attention_v2", "v2"),
+                           (paged_attn._torch_ops, "paged_attention_decode", "decode")):
+        monkeypatch.setattr(mod, name, lambda *a, key=key, **k: calls.setdefault(key, a))
+    x = 16 // (torch.empty(0, dtype=dtype).element_size() if kv == "auto" else 1)
+    cdt = dtype if kv == "auto" else torch.uint8
+    q = torch.zeros((S, H, D), dtype=dtype)
+    kc, vc = torch.zeros((4, KVH, D // x, BS, x), dtype=cdt), torch.zeros((4, KVH, D, BS), dtype=cdt)
+    bt, sl, one = torch.zeros((S, 4096 // BS), dtype=torch.int32), torch.ones(S, dtype=torch.int32), torch.ones(1)
+    out = paged_attn.PagedAttention.forward_decode(q, kc, vc, bt, sl, 777, kv, KVH, 0.1, None, one, one, blocksparse_vert_stride=None)
+    assert out.shape == q.shape and list(calls) == [want]
+    if want == "decode":   # the arguments of v1
+        a = calls["decode"]
+        assert a[0] is out and a[1] is q and a[8:10] == (BS, 777) and a[11] == kv and len(a) == 19
+
+
+def test_paged_attention_v2_pieces():
+    """The plan without a device: one piece, two, and every call that is not the matrix-core kernel's."""
+    from vllm_amd._lib import BF16, F32, KV_AUTO, KV_FP8_E4M3, lib
+
+    def pieces(S=1, H=32, D=128, KVH=8, BS=16, L=777, P=2, dt=BF16, kv=KV_FP8_E4M3, out=1 << 20, q=1 << 21, q_stride=None, head_stride=None, vert=0):
+        return lib.vllm_amd_paged_attention_v2_pieces(out, q, S, H, D, KVH, BS, L, P, dt, kv, H * D if q_stride is None else q_stride,
+                                                      D * BS if head_stride is None else head_stride, vert)
+
+    assert pieces() == 1 and pieces(S=16, L=1000) == 1 and pieces(kv=KV_AUTO) == 1
+    assert pieces(S=8, L=1000, kv=KV_AUTO) == 2 and pieces(S=4, L=1024, kv=KV_AUTO) == 2
+    assert pieces(L=300, P=1) == 1 and pieces(S=0) == 1
+    for other in (dict(dt=F32, kv=KV_AUTO), dict(BS=8), dict(vert=2), dict(q=(1 << 21) + 8), dict(q_stride=32 * 128 + 4), dict(head_stride=128 * 16 + 16),
+                  dict(out=(1 << 20) + 8)):
+        assert pieces(**other) == 2, other
+    assert pieces(L=8000, P=16) > 1
+
+
 def test_shard_helpers():
     from vllm_amd.distributed import shard_kv_heads, shard_range
     assert shard_range(8192, 8, 3) == (3072, 4096)

@@ -26,6 +26,7 @@ SIGNATURES = {
     "vllm_amd_paged_attention_v2": [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp, _i, _i, _i, _i, _vp,
         _i, _i, _vp, _vp, _i64, _i64, _i64, _i, _i, _i, _i, _i, _vp],
+    "vllm_amd_paged_attention_v2_pieces": [_vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i64, _i],
     "vllm_amd_paged_attention_rocm": [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp, _vp, _i, _i, _i, _i,
         _vp, _i, _i, _vp, _vp, _vp, _i64, _i64, _i64, _vp],

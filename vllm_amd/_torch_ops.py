@@ -112,7 +112,9 @@ silu_and_mul_quant = torch.ops._C.silu_and_mul_quant
 #: device-side BlockTable.compute_slot_mapping (vllm/v1/worker/block_table.py:84-99); not a
 #: reference op -- the reference does this with numpy on the host
 compute_slot_mapping = torch.ops._vllm_amd_C.compute_slot_mapping
-#: dynamic activation quantisation + cutlass_scaled_mm; the attention calls behind attention/ops
+#: dynamic activation quantisation + cutlass_scaled_mm; decode in the form that paged_attention_v2's plan has; the attention calls
+#: behind attention/ops
 fp8_linear = torch.ops._vllm_amd_C.fp8_linear.default
+paged_attention_decode = torch.ops._vllm_amd_C.paged_attention_decode.default
 unified_attention = torch.ops._vllm_amd_C.unified_attention.default
 context_attention_fwd = torch.ops._vllm_amd_C.context_attention_fwd.default

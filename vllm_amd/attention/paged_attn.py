@@ -9,7 +9,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from .. import _custom_ops as ops
+from .. import _custom_ops as ops, _torch_ops
 
 # Same as PARTITION_SIZE of the v2 launcher (paged_attn.py:16)
 _PARTITION_SIZE = 512
@@ -76,18 +76,21 @@ class PagedAttention:
         if use_v1 and max_num_partitions > 1:
             groups = num_kv_heads * ((num_heads // max(num_kv_heads, 1) + 15) // 16)
             use_v1 = num_seqs * groups >= 256
-        # ... and two partitions of the matrix-core kernel cost the device as much in one piece, or nearly (us, cut / whole:
-        # 1 x 777 fp8 9.1 / 8.7, 16 x 777 16-bit 13.6 / 12.9, 8 x 1000 16-bit 12.0 / 13.6): v1, without the 5 us of host time
-        # for scratch
-        if (max_num_partitions == 2 and head_size <= 128 and head_size % 16 == 0 and block_size in (16, 32)
-                and query.dtype != torch.float32 and blocksparse_vert_stride <= 1):
-            use_v1 = True
         if use_v1:
             ops.paged_attention_v1(output, query, key_cache, value_cache, num_kv_heads, scale,
                                    block_tables, seq_lens, block_size, max_seq_len, alibi_slopes,
                                    kv_cache_dtype, k_scale, v_scale, tp_rank,
                                    blocksparse_local_blocks, blocksparse_vert_stride,
                                    blocksparse_block_size, blocksparse_head_sliding_step)
+        elif max_num_partitions == 2:
+            assert _PARTITION_SIZE % block_size == 0
+            # Two partitions are taken in one piece as often as not, which needs no scratch: one operator decides, and allocates
+            # only if they are cut (three allocations here cost 5 us of host time: 1 x 777 fp8 13.4 us a call, 8.4 so).
+            _torch_ops.paged_attention_decode(output, query, key_cache, value_cache, num_kv_heads, scale,
+                                              block_tables, seq_lens, block_size, max_seq_len,
+                                              alibi_slopes, kv_cache_dtype, k_scale, v_scale, tp_rank,
+                                              blocksparse_local_blocks, blocksparse_vert_stride,
+                                              blocksparse_block_size, blocksparse_head_sliding_step)
         else:
             assert _PARTITION_SIZE % block_size == 0
             tmp_output = torch.empty((num_seqs, num_heads, max_num_partitions, head_size),

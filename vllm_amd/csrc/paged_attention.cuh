@@ -39,6 +39,8 @@ int paged_attention_generic(const PagedAttnParams& p);
 // VLLM_AMD_EUNSUPPORTED *without touching memory* when the shape is not covered.
 bool paged_attention_mfma_supported(const PagedAttnParams& p);
 int paged_attention_mfma(const PagedAttnParams& p);
+// reference partitions that its v2 / rocm launch gives to one workgroup (max_num_partitions: one piece, which writes the output itself)
+int pa_partitions_per_piece(const PagedAttnParams& p);
 // tuning knob (A/B measurements): see vllm_amd_set_tuning
 void set_pa_variant(int v);
 void set_pa_sp(int v);

@@ -611,6 +611,19 @@ extern "C" int vllm_amd_paged_attention_v2(
   return run(p, "paged_attention_v2");
 }
 
+extern "C" int vllm_amd_paged_attention_v2_pieces(
+    const void* out, const void* query, int num_seqs, int num_heads, int head_size, int num_kv_heads, int block_size,
+    int max_seq_len, int max_num_partitions, int dtype, int kv_dtype, int64_t q_stride, int64_t kv_head_stride,
+    int blocksparse_vert_stride) {
+  if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || max_num_partitions <= 1) return 1;
+  PagedAttnParams p = {};
+  p.out = (void*)out; p.query = query; p.num_seqs = num_seqs; p.num_heads = num_heads; p.head_size = head_size;
+  p.num_kv_heads = num_kv_heads; p.block_size = block_size; p.max_seq_len = max_seq_len; p.partition_size = 512;
+  p.max_num_partitions = max_num_partitions; p.dtype = dtype; p.kv_dtype = kv_dtype; p.q_stride = q_stride;
+  p.kv_head_stride = kv_head_stride; p.bs_vert_stride = blocksparse_vert_stride;
+  return paged_attention_mfma_supported(p) ? ceil_div(max_num_partitions, pa_partitions_per_piece(p)) : max_num_partitions;
+}
+
 extern "C" int vllm_amd_paged_attention_rocm(
     void* out, float* exp_sums, float* max_logits, void* tmp_out, const void* query,
     const void* key_cache, const void* value_cache, int num_seqs, int num_heads, int head_size,

@@ -896,91 +896,92 @@ static int dispatch_mfma(const PagedAttnParams& p) {
 // partial into the first of its scratch slots, and the reduce kernel visits every sp-th
 // slot.  The scratch tensors are caller-allocated temporaries of the reference's shape;
 // only the slots we read are written.
+int pa_partitions_per_piece(const PagedAttnParams& p) {
+  const int chunks = ceil_div(p.num_heads / p.num_kv_heads, 16);
+  // The chip holds 512 of these workgroups (two per CU) and hands further ones out as others
+  // finish; the host does not know the batch's lengths (seq_lens live on the device).
+  const int64_t base = (int64_t)p.num_seqs * p.num_kv_heads * chunks;
+  const int64_t P = p.max_num_partitions;
+  const int64_t slots = p.head_size > 128 ? 256 : 512;   // head sizes above 128: one workgroup per CU
+  int64_t sp;
+  if (base < slots) {
+    // Fewer (sequence, head) pairs than workgroup slots: the sequences must be cut to fill the
+    // chip, and real batches are ragged, so aim at ~2048 workgroups of >= 2048 tokens -- the
+    // hardware hands them out as others finish (ragged 16 x U[8k, 64k] tokens: 215 us, against
+    // 239 us with the 512 longest pieces that a uniform batch would like best).
+    const int64_t total = base * P;
+    const int64_t sp_fill = (total + slots - 1) / slots, sp_bal = (total + 4 * slots - 1) / (4 * slots);
+    const int64_t sp_min = p.partition_size >= 2048 ? 1 : 2048 / p.partition_size;
+    sp = sp_fill < sp_min ? sp_fill : sp_min;
+    if (sp < sp_bal) sp = sp_bal;
+    // Short sequences: one piece each, which writes the output itself -- no reduce kernel (2 .. 2.4 us with the gap in front of it)
+    // -- where that costs less than the longest piece gains.  A workgroup alone takes 2 ns + 1 ns per 133 bytes for a token with
+    // eight waves, 2.2 ns + 1 ns per 78 bytes with four, 3.9 ns + 1 ns per 58 bytes above head size 128 (of rows padded to 64 / 128 / 192 /
+    // 256: the lanes of a padded row wait like the others), the chip 1 us per 6.2 MB; the batch is taken to be 0.56 / 0.66 / 0.91
+    // full, and a piece more costs the merge 0.5 .. 0.7 ns.  Up to 14 us only: a long sequence among short ones has to be cut.
+    // Over 6072 batches of up to 159 pairs (tools/sweep_decode_plans.py; profiles/decode_plans.txt has a few hundred) 0.2 % above the
+    // cheaper form on average, more than 3 % in one of 42.  us, one piece / cut, all sequences alike: fp8 1 x 777 8.7 / 9.1, 10 x 1551
+    // 13.2 / 11.4, 24 x 1000 11.3 / 14.4; 16-bit 1 x 600 7.3 / 9.6, 1 x 773 8.4 / 9.6, 6 x 704 10.5 / 9.2, 153 x 871 of one kv head 14.1 /
+    // 18.5; head 80 fp8 9 x 1478 13.2 / 10.4; head 64 1 x 1198 7.8 / 8.2; head 192 16-bit 2 x 423 8.5 / 9.0.
+    if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
+      const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO, wide = p.head_size > 128;
+      // (short whole rows over a 16-bit cache keep four waves, at no higher price than eight)
+      const bool w8 = !wide && (pa_eight_waves(p, base, fp8, true) || (!fp8 && base <= 64));
+      const int padded = p.head_size <= 64 ? 64 : !wide ? 128 : p.head_size == 192 ? 192 : 256;
+      const double es = fp8 ? 1.0 : 2.0, tb = 2.0 * p.head_size * es, row = 2.0 * padded * es;
+      const double t = w8 ? 2e-3 + row * 7.5e-6 : wide ? 3.9e-3 + row * 17.3e-6 : 2.2e-3 + row * 12.9e-6;
+      const double alone = p.max_seq_len * t, piece = (double)sp * p.partition_size * t;
+      const double stream = (w8 ? 0.56 : wide ? 0.91 : 0.66) * (double)base * p.max_seq_len * tb / 6.2e6;
+      const double merge = (w8 ? 2.4 : 2.0) + (w8 ? 0.5e-3 : 0.7e-3) * (double)(base * ((P + sp - 1) / sp));
+      const double one = (w8 ? 1.04 : wide ? 0.89 : 1.02) * (alone > stream ? alone : stream);
+      if (alone <= 14.0 && one < (piece > stream ? piece : stream) + merge) sp = P;
+    }
+  } else {
+    // Enough pairs to fill the chip: few long pieces stream best (256 x 16k tokens: one piece per
+    // sequence 81.3 % of peak, sp 16 80.3 %, sp 8 78.5 %, sp 4 76.0 %) and a ragged batch is
+    // balanced by the longest-first order of one-piece launches (pa_lpt_wg; 64 x U[2k, 16k]:
+    // 2048-token pieces 218 us, one piece 209 us; 64 x U[8k, 64k]: 755 -> 725 us).  What is left is
+    // the quantisation into rounds of 512 workgroups: with all lengths at max_seq_len a launch of
+    // `pieces` per pair costs ceil(base pieces / 512) rounds of (sp partition_size + ~256 tokens
+    // of prologue and merge); take the cheapest, the longest pieces within 3 %, none below 2048
+    // tokens.  profiles/r02_decode_order.txt §7.
+    sp = P;
+    double best = 1e300;
+    for (int64_t c = P; c >= 1 && c * p.partition_size >= 2048; --c) {
+      const int64_t pieces = (P + c - 1) / c, rounds = (base * pieces + slots - 1) / slots;
+      const double cost = (double)rounds * (double)(c * p.partition_size + 256);
+      if (cost < best * 0.97) { best = cost; sp = c; }
+    }
+  }
+  // One piece as well for batches that nearly fill the chip, where it beats the cut by the balance: extra workgroups and the merge
+  // of their pieces cost 4.7 us and 12 ns each; a workgroup takes 2 ns + 1 ns per 29 bytes for a token with the chip busy, the chip
+  // 1 us per 6.2 MB -- the batch taken to be 0.84 full -- and both more where some of the 256 CUs have a workgroup more than
+  // others.  (Below 256 pairs a padded row of a 16-bit cache counts whole: 20 x 1923 of head 80 25.9 us cut, 30.4 in one piece.)  us,
+  // cut -> one piece (32 / 8 heads of 128): fp8 48 x 2200 ragged 29.6 -> 24.3, 56 x 2200 48.7 -> 42.9 (ragged 35.7 -> 26.6), 96 x 4096 ragged
+  // 81.6 -> 74.4; 16-bit 24 x 2200 39.2 -> 34.6, 56 x 2200 93.3 -> 75.9; head 64 24 x 4096 23.5 -> 19.5.  Kept cut: 40 x 4096 58.0 (63.9), and
+  // with it, for its price of a busy chip, what one workgroup per CU streams faster: 24 x 4096 39.3 (33.2; ragged 28.9, 29.2).  Not where
+  // the longest sequence may take a workgroup more than 24 us on an idle chip: among short ones it has to be cut; and fewer
+  // pairs are the rule above's (8 x 1600 of head 64 8.9, in one piece 9.7).
+  if (sp < P && base >= 160 && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
+    const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO;
+    const double tb = 2.0 * (!fp8 && base < 256 && p.head_size > 64 && p.head_size < 128 ? 128 : p.head_size) * (fp8 ? 1 : 2);
+    auto us = [&](int64_t c) {
+      const int64_t tot = base * ((P + c - 1) / c), len = c < P ? c * p.partition_size : p.max_seq_len;
+      const double alone = (double)len * (2e-3 + tb * 3.5e-5), stream = 0.84 * (double)base * p.max_seq_len * tb / 6.2e6;
+      const double over = tot >= 256 ? (double)((tot + 255) / 256 * 256) / (double)tot - 1.0 : 0.0;
+      return (alone > stream ? alone : stream) * (1.0 + 1.05 * over * over) + (c < P ? 4.7 + 0.012 * (double)tot : 0.0);
+    };
+    if (p.max_seq_len * (2.5e-3 + tb * 1.2e-5) <= 24.0 && us(P) < 0.99 * us(sp)) sp = P;
+  }
+  if (g_pa_sp > 0) sp = g_pa_sp;
+  if (sp < 1) sp = 1;
+  if (sp > p.max_num_partitions) sp = p.max_num_partitions;
+  return (int)sp;
+}
+
 int paged_attention_mfma(const PagedAttnParams& p0) {
   PagedAttnParams p = p0;
-  p.sp_parts = 1;
-  if (p.partition_size > 0) {
-    const int chunks = ceil_div(p.num_heads / p.num_kv_heads, 16);
-    // The chip holds 512 of these workgroups (two per CU) and hands further ones out as others
-    // finish; the host does not know the batch's lengths (seq_lens live on the device).
-    const int64_t base = (int64_t)p.num_seqs * p.num_kv_heads * chunks;
-    const int64_t P = p.max_num_partitions;
-    const int64_t slots = p.head_size > 128 ? 256 : 512;   // head sizes above 128: one workgroup per CU
-    int64_t sp;
-    if (base < slots) {
-      // Fewer (sequence, head) pairs than workgroup slots: the sequences must be cut to fill the
-      // chip, and real batches are ragged, so aim at ~2048 workgroups of >= 2048 tokens -- the
-      // hardware hands them out as others finish (ragged 16 x U[8k, 64k] tokens: 215 us, against
-      // 239 us with the 512 longest pieces that a uniform batch would like best).
-      const int64_t total = base * P;
-      const int64_t sp_fill = (total + slots - 1) / slots, sp_bal = (total + 4 * slots - 1) / (4 * slots);
-      const int64_t sp_min = p.partition_size >= 2048 ? 1 : 2048 / p.partition_size;
-      sp = sp_fill < sp_min ? sp_fill : sp_min;
-      if (sp < sp_bal) sp = sp_bal;
-      // Short sequences: one piece each, which writes the output itself -- no reduce kernel (2 .. 2.4 us with the gap in front of it)
-      // -- where that costs less than the longest piece gains.  A workgroup alone takes 2 ns + 1 ns per 133 bytes for a token with
-      // eight waves, 2.2 ns + 1 ns per 78 bytes with four, 3.9 ns + 1 ns per 58 bytes above head size 128 (of rows padded to 64 / 128 / 192 /
-      // 256: the lanes of a padded row wait like the others), the chip 1 us per 6.2 MB; the batch is taken to be 0.56 / 0.66 / 0.91
-      // full, and a piece more costs the merge 0.5 .. 0.7 ns.  Up to 14 us only: a long sequence among short ones has to be cut.
-      // Over 6072 batches of up to 159 pairs (tools/sweep_decode_plans.py; profiles/decode_plans.txt has a few hundred) 0.2 % above the
-      // cheaper form on average, more than 3 % in one of 42.  us, one piece / cut, all sequences alike: fp8 1 x 777 8.7 / 9.1, 10 x 1551
-      // 13.2 / 11.4, 24 x 1000 11.3 / 14.4; 16-bit 1 x 600 7.3 / 9.6, 1 x 773 8.4 / 9.6, 6 x 704 10.5 / 9.2, 153 x 871 of one kv head 14.1 /
-      // 18.5; head 80 fp8 9 x 1478 13.2 / 10.4; head 64 1 x 1198 7.8 / 8.2; head 192 16-bit 2 x 423 8.5 / 9.0.
-      if (sp < P && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
-        const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO, wide = p.head_size > 128;
-        // (short whole rows over a 16-bit cache keep four waves, at no higher price than eight)
-        const bool w8 = !wide && (pa_eight_waves(p, base, fp8, true) || (!fp8 && base <= 64));
-        const int padded = p.head_size <= 64 ? 64 : !wide ? 128 : p.head_size == 192 ? 192 : 256;
-        const double es = fp8 ? 1.0 : 2.0, tb = 2.0 * p.head_size * es, row = 2.0 * padded * es;
-        const double t = w8 ? 2e-3 + row * 7.5e-6 : wide ? 3.9e-3 + row * 17.3e-6 : 2.2e-3 + row * 12.9e-6;
-        const double alone = p.max_seq_len * t, piece = (double)sp * p.partition_size * t;
-        const double stream = (w8 ? 0.56 : wide ? 0.91 : 0.66) * (double)base * p.max_seq_len * tb / 6.2e6;
-        const double merge = (w8 ? 2.4 : 2.0) + (w8 ? 0.5e-3 : 0.7e-3) * (double)(base * ((P + sp - 1) / sp));
-        const double one = (w8 ? 1.04 : wide ? 0.89 : 1.02) * (alone > stream ? alone : stream);
-        if (alone <= 14.0 && one < (piece > stream ? piece : stream) + merge) sp = P;
-      }
-    } else {
-      // Enough pairs to fill the chip: few long pieces stream best (256 x 16k tokens: one piece per
-      // sequence 81.3 % of peak, sp 16 80.3 %, sp 8 78.5 %, sp 4 76.0 %) and a ragged batch is
-      // balanced by the longest-first order of one-piece launches (pa_lpt_wg; 64 x U[2k, 16k]:
-      // 2048-token pieces 218 us, one piece 209 us; 64 x U[8k, 64k]: 755 -> 725 us).  What is left is
-      // the quantisation into rounds of 512 workgroups: with all lengths at max_seq_len a launch of
-      // `pieces` per pair costs ceil(base pieces / 512) rounds of (sp partition_size + ~256 tokens
-      // of prologue and merge); take the cheapest, the longest pieces within 3 %, none below 2048
-      // tokens.  profiles/r02_decode_order.txt §7.
-      sp = P;
-      double best = 1e300;
-      for (int64_t c = P; c >= 1 && c * p.partition_size >= 2048; --c) {
-        const int64_t pieces = (P + c - 1) / c, rounds = (base * pieces + slots - 1) / slots;
-        const double cost = (double)rounds * (double)(c * p.partition_size + 256);
-        if (cost < best * 0.97) { best = cost; sp = c; }
-      }
-    }
-    // One piece as well for batches that nearly fill the chip, where it beats the cut by the balance: extra workgroups and the merge
-    // of their pieces cost 4.7 us and 12 ns each; a workgroup takes 2 ns + 1 ns per 29 bytes for a token with the chip busy, the chip
-    // 1 us per 6.2 MB -- the batch taken to be 0.84 full -- and both more where some of the 256 CUs have a workgroup more than
-    // others.  (Below 256 pairs a padded row of a 16-bit cache counts whole: 20 x 1923 of head 80 25.9 us cut, 30.4 in one piece.)  us,
-    // cut -> one piece (32 / 8 heads of 128): fp8 48 x 2200 ragged 29.6 -> 24.3, 56 x 2200 48.7 -> 42.9 (ragged 35.7 -> 26.6), 96 x 4096 ragged
-    // 81.6 -> 74.4; 16-bit 24 x 2200 39.2 -> 34.6, 56 x 2200 93.3 -> 75.9; head 64 24 x 4096 23.5 -> 19.5.  Kept cut: 40 x 4096 58.0 (63.9), and
-    // with it, for its price of a busy chip, what one workgroup per CU streams faster: 24 x 4096 39.3 (33.2; ragged 28.9, 29.2).  Not where
-    // the longest sequence may take a workgroup more than 24 us on an idle chip: among short ones it has to be cut; and fewer
-    // pairs are the rule above's (8 x 1600 of head 64 8.9, in one piece 9.7).
-    if (sp < P && base >= 160 && p.max_seq_len > 0 && p.fp8_out_scale == nullptr) {
-      const bool fp8 = p.kv_dtype != VLLM_AMD_KV_AUTO;
-      const double tb = 2.0 * (!fp8 && base < 256 && p.head_size > 64 && p.head_size < 128 ? 128 : p.head_size) * (fp8 ? 1 : 2);
-      auto us = [&](int64_t c) {
-        const int64_t tot = base * ((P + c - 1) / c), len = c < P ? c * p.partition_size : p.max_seq_len;
-        const double alone = (double)len * (2e-3 + tb * 3.5e-5), stream = 0.84 * (double)base * p.max_seq_len * tb / 6.2e6;
-        const double over = tot >= 256 ? (double)((tot + 255) / 256 * 256) / (double)tot - 1.0 : 0.0;
-        return (alone > stream ? alone : stream) * (1.0 + 1.05 * over * over) + (c < P ? 4.7 + 0.012 * (double)tot : 0.0);
-      };
-      if (p.max_seq_len * (2.5e-3 + tb * 1.2e-5) <= 24.0 && us(P) < 0.99 * us(sp)) sp = P;
-    }
-    if (g_pa_sp > 0) sp = g_pa_sp;
-    if (sp < 1) sp = 1;
-    if (sp > p.max_num_partitions) sp = p.max_num_partitions;
-    p.sp_parts = (int)sp;
-  }
+  p.sp_parts = p.partition_size > 0 ? pa_partitions_per_piece(p) : 1;
   if (p.dtype == VLLM_AMD_F16) return dispatch_mfma<f16_t>(p);
   return dispatch_mfma<bf16_t>(p);
 }

@@ -14,6 +14,7 @@
 #include <torch/library.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
@@ -467,6 +468,31 @@ struct Segments {
   }
 };
 
+// paged_attention_v1 where v2 would take every sequence in one piece, else v2 with scratch of its own (vllm/attention/ops/
+// paged_attn.py:131-193)
+void paged_attention_decode(Tensor& out, const Tensor& query, const Tensor& key_cache, const Tensor& value_cache,
+                            int64_t num_kv_heads, double scale, const Tensor& block_tables, const Tensor& seq_lens,
+                            int64_t block_size, int64_t max_seq_len, const OptTensor& alibi_slopes,
+                            const std::string& kv_cache_dtype, const Tensor& k_scale, const Tensor& v_scale,
+                            int64_t tp_rank, int64_t bs_local_blocks, int64_t bs_vert_stride, int64_t bs_block_size,
+                            int64_t bs_head_sliding_step) {
+  TORCH_CHECK(query.dim() == 3, "query.dim() == 3");
+  const int64_t s = query.size(0), h = query.size(1), d = query.size(2), parts = (max_seq_len + 511) / 512;
+  if (vllm_amd_paged_attention_v2_pieces(out.data_ptr(), query.data_ptr(), (int)s, (int)h, (int)d, (int)num_kv_heads, (int)block_size,
+                                         (int)max_seq_len, (int)parts, dt(query), kv(kv_cache_dtype), query.stride(0),
+                                         key_cache.stride(1), (int)bs_vert_stride) == 1) {
+    paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size, max_seq_len,
+                       alibi_slopes, kv_cache_dtype, k_scale, v_scale, tp_rank, bs_local_blocks, bs_vert_stride, bs_block_size,
+                       bs_head_sliding_step);
+    return;
+  }
+  Tensor sums = at::empty({s, h, parts}, query.options().dtype(at::kFloat)), max = at::empty_like(sums);
+  Tensor tmp = at::empty({s, h, parts, d}, out.options());
+  paged_attention_v2(out, sums, max, tmp, query, key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size,
+                     max_seq_len, alibi_slopes, kv_cache_dtype, k_scale, v_scale, tp_rank, bs_local_blocks, bs_vert_stride,
+                     bs_block_size, bs_head_sliding_step);
+}
+
 inline int kv_of_cache(const Tensor& k) { return is_fp8(k) ? VLLM_AMD_KV_FP8_E4M3 : VLLM_AMD_KV_AUTO; }
 
 // vllm/attention/ops/triton_unified_attention.py:588-700 (the arguments are checked in the Python mirror)
@@ -630,6 +656,9 @@ void register_all() {
        "compute_slot_mapping(Tensor! slot_mapping, Tensor block_table, Tensor req_indices,"
        " Tensor positions, int block_size) -> ()",
        &compute_slot_mapping);
+  x.op("paged_attention_decode",
+       "paged_attention_decode(Tensor! out, Tensor query, Tensor key_cache, Tensor value_cache," PA_TAIL,
+       &paged_attention_decode);
   x.op("fp8_linear",
        "fp8_linear(Tensor! out, Tensor input, Tensor weight, Tensor weight_scale, Tensor? scale_ub, Tensor? bias,"
        " bool per_token) -> ()",
