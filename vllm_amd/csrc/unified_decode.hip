@@ -10,10 +10,10 @@ extern int g_uni_decode;
 
 namespace {
 
-// (head 128 with an fp8 cache sits at the 168 registers of three workgroups per CU: 172 sequences x 80 keys, 1376 workgroups,
-// 16.4 us against 19.6 at two)
+// (head 128 sits at the 168 registers of three workgroups per CU: 172 sequences x 80 fp8 keys, 1376 workgroups, 16.4 us against
+// 19.6 at two)
 template <typename T, bool FP8, int D, int NW, bool GEN>
-__global__ __launch_bounds__(NW * 64, (D > 128 && !FP8 ? 1 : D == 128 && FP8 ? 3 : 2)) void ua_decode_kernel(const UniDecodeParams p, int sub_shift, int xcd_group, int order) {
+__global__ __launch_bounds__(NW * 64, (D > 128 && !FP8 ? 1 : D == 128 ? 3 : 2)) void ua_decode_kernel(const UniDecodeParams p, int sub_shift, int xcd_group, int order) {
   __shared__ __attribute__((aligned(16))) char lds[ua_decode_lds<FP8, D, NW>()];
   ua_decode_body<T, FP8, D, NW, GEN, false>(p, lds, sub_shift, xcd_group, order, blockIdx.x, gridDim.x, blockIdx.y);
 }
