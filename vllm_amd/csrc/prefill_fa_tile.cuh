@@ -107,7 +107,7 @@ __device__ __forceinline__ int wave_last(int n, int lane, F&& le) {
 // the wave's tiles: 0 K ring fill + staging (LDS writes of tile t + 1, loads of t + 2), 2 S^T, 4 softmax + PV,
 // 5 barrier, 6 tiles computed, 7 whole kernel
 #ifdef VA_PROBES
-static __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];
+static __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];   // (one for each file that launches the kernel, with its reader)
 #define FA_T(i)                                                   \
   do {                                                            \
     const unsigned long long now__ = __builtin_readcyclecounter(); \
@@ -849,9 +849,9 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   }   // t0 < t1
 
 #ifdef VA_PROBES
-  if (lane == 0 && blockIdx.y == 0 && blockIdx.x < 2048) {
+  if (lane == 0 && hw < 2048) {
     acc__[7] = __builtin_readcyclecounter() - t_entry__;
-    for (int i = 0; i < 8; ++i) g_fa_stamps[((size_t)blockIdx.x * 8 + wave) * 8 + i] = acc__[i];
+    for (int i = 0; i < 8; ++i) g_fa_stamps[((size_t)hw * 8 + wave) * 8 + i] = acc__[i];
   }
 #endif
   // ---- O^T / l -> out ------------------------------------------------------------------------------------------

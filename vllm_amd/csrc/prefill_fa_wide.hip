@@ -31,3 +31,9 @@ void launch_fa_wide(const FaParams& p, int dtype, bool fp8, dim3 grid, hipStream
 }
 
 }  // namespace va
+
+#ifdef VA_PROBES
+extern "C" int vllm_amd_probe_fa_wide_stamps(unsigned long long* dst, int nwg) {
+  return hipMemcpyFromSymbol(dst, HIP_SYMBOL(va::fa::g_fa_stamps), (size_t)nwg * 8 * 8 * 8) == hipSuccess ? 0 : -3;
+}
+#endif
