@@ -559,7 +559,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /*                 vllm_amd_set_workspace; unsplit without one)                 */
 /* ------------------------------------------------------------------------- */
 int vllm_amd_set_tuning(const char* key, int value);
-/* current value of "pa_balance" / "mm_kernel" / "mm_splitk" (the torch layer asks before it allocates) */
+/* current value of "pa_balance" / "mm_kernel" / "mm_splitk" (the torch layer asks before it allocates); "pf_mixed_launches": how many
+ * mixed unified_attention steps went out as one launch so far, in this process */
 int vllm_amd_get_tuning(const char* key, int* value);
 
 #ifdef __cplusplus

@@ -486,6 +486,45 @@ def test_unified_mixed_one_launch(oracle, force_fa, heads, D, fp8, n, mode):
             _lib.set_tuning("pa_order", 1)
 
 
+def _mixed_launches():
+    import ctypes
+    from vllm_amd import _lib
+    n = ctypes.c_int()
+    _lib.check(_lib.lib.vllm_amd_get_tuning(b"pf_mixed_launches", ctypes.byref(n)))
+    return n.value
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,D,BS", [((8, 2), 128, 32), ((32, 8), 80, 64), ((24, 1), 96, 16), ((4, 4), 128, 128)])
+def test_unified_mixed_forms(oracle, force_fa, heads, D, BS, dtype, fp8):
+    """The same mixed step in one launch and in two, which each is looked up: both 16-bit types, pages of more than one 16-slot tile."""
+    from vllm_amd import _lib
+    seqs = [(1, (1, 16, 31, 33, 64, 129, 257, 512, 700)[i % 9]) for i in range(19)]
+    seqs[0], seqs[9], seqs[18] = (70, 300), (65, 65), (130, 190)
+    c = make_unified_case(seqs, heads[0], heads[1], D, BS, dtype, fp8=fp8, seed=BS + D, kv_scale=0.5)
+    hnd = lambda t: t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+    for mixed in (1, 0):
+        _lib.set_tuning("pf_mixed", mixed)
+        try:
+            before = _mixed_launches()
+            run(oracle, c, dtype, fp8=fp8, view=hnd)
+            assert _mixed_launches() - before == mixed
+        finally:
+            _lib.set_tuning("pf_mixed", 1)
+
+
+@pytest.mark.parametrize("n,one", [(80, 1), (81, 0)])
+def test_unified_mixed_launch_limit(oracle, force_fa, n, one):
+    """640 (sequence, kv head) pairs go along with the chunks, 648 have a launch of their own."""
+    seqs = [(1, 1 + 3 * i % 70) for i in range(n)]
+    seqs[5], seqs[n - 1] = (66, 80), (35, 35)
+    c = make_unified_case(seqs, 8, 8, 128, 16, torch.bfloat16, seed=n)
+    before = _mixed_launches()
+    run(oracle, c, torch.bfloat16, view=lambda t: t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3))
+    assert _mixed_launches() - before == one
+
+
 def test_unified_fa_kernel_sharp_rows(oracle, force_fa):
     """Rows whose maximum keeps growing along the keys (the lazy rescale must fire on some tiles and not on others):
     keys scaled up with their position."""

@@ -20,6 +20,7 @@
 #include "paged_attention.cuh"
 
 #include <float.h>
+#include <atomic>
 #include <string.h>
 
 namespace va {
@@ -39,6 +40,7 @@ extern int g_uni_decode;
 extern int g_pf_fa;
 extern int g_pf_segs;
 extern int g_pf_mixed;
+extern std::atomic<int> g_pf_mixed_launches;   // prefill_fa.hip
 extern int g_pf_fa_stagger;
 
 template <typename cache_t> struct CacheTraits;
@@ -725,5 +727,6 @@ extern "C" int vllm_amd_get_tuning(const char* key, int* value) {
   if (strcmp(key, "pa_balance") == 0) { *value = get_pa_balance(); return VLLM_AMD_OK; }
   if (strcmp(key, "mm_kernel") == 0) { *value = g_mm_kernel; return VLLM_AMD_OK; }
   if (strcmp(key, "mm_splitk") == 0) { *value = g_mm_splitk; return VLLM_AMD_OK; }
+  if (strcmp(key, "pf_mixed_launches") == 0) { *value = g_pf_mixed_launches.load(std::memory_order_relaxed); return VLLM_AMD_OK; }
   VA_REQUIRE(false, VLLM_AMD_EINVAL, "get_tuning: unknown key %s", key);
 }

@@ -2,6 +2,8 @@
 #include "prefill_fa_tile.cuh"
 #include "unified_decode_kernel.cuh"
 
+#include <atomic>
+
 namespace va {
 namespace fa {
 
@@ -95,6 +97,7 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
 }  // namespace fa
 
 int g_pf_fa_stagger = 1;   // tuning "pf_fa_stagger": 0 = all eight waves stage at the bottom of the interval
+std::atomic<int> g_pf_mixed_launches{0};   // get_tuning "pf_mixed_launches"
 int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, const UniDecodeParams* u) {
   const bool wide = p.head_size > 128;                 // 128-row workgroups of four waves
   const int tpb = (wide ? 128 : 256) / p.pack;
@@ -129,6 +132,7 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, co
     if (p.prefix) FA_LAUNCH_(T_, F_, true); else FA_LAUNCH_(T_, F_, false); \
   } while (0)
   if (u != nullptr) {
+    g_pf_mixed_launches.fetch_add(1, std::memory_order_relaxed);
     if (dtype == VLLM_AMD_BF16) { if (fp8) FA_MIXED(bf16_t, true); else FA_MIXED(bf16_t, false); }
     else { if (fp8) FA_MIXED(f16_t, true); else FA_MIXED(f16_t, false); }
   }
