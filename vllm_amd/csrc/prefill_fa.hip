@@ -11,9 +11,9 @@ namespace fa {
 // kv head) pair, longest first.  Row blocks of a chunk differ in length and so do the chunks: a launch of their own ended on a
 // few of them with most CUs idle (2000 tokens over 1500: 256 blocks of 24 .. 55 tiles), and the decode kernel, which waits for
 // bytes and not for the matrix cores, stood in front of it.  us, two launches -> one (32 / 8 heads, fp8, cache write included),
-// 2000 over 1500 among 63 decodes of up to 4096 keys 164 -> 148, of up to 1000 131 -> 114; 2 x 1000 fresh among 15 of 4000
+// 2000 over 1500 among 63 decodes of up to 4096 keys 158 -> 144, of up to 1000 131 -> 114; 2 x 1000 fresh among 15 of 4000
 // 70.6 -> 43.7; 6000 fresh among 63 of 4000 371 -> 354.
-// (Tried: two groups of four waves per workgroup, 152 us in the first of these; several kv heads per workgroup one after the
+// (Tried, where the first of these took 148: two groups of four waves per workgroup 152; several kv heads per workgroup one after the
 // other, 160.)
 template <typename T, bool FP8>
 __global__ __launch_bounds__(512) void fa_mixed_kernel(const FaParams p, const UniDecodeParams u, int gx, int gy, int nfa, int npairs, int sub_shift, int order) {

@@ -175,8 +175,8 @@ int unified_decode_heads_per_row(const UniDecodeParams& p) {
 int g_uni_seg = 0;   // tuning "uni_seg": 0 = heuristic, n = that many key segments (at most those there is scratch for)
 
 int unified_decode_segments(const UniDecodeParams& p, int max_segments) {
-  // Split over the keys (when the caller brought scratch).  The chip holds 512 workgroups at a
-  // time, so a launch of full-length workgroups takes ceil(wgs n / 512) / n rounds, and every
+  // Split over the keys (when the caller brought scratch).  With the chip counted as 512 slots (two workgroups per CU, as it was
+  // fitted; rows of 128 fit three by now, of 64 four) a launch of full-length ones takes ceil(wgs n / 512) / n rounds, and every
   // workgroup pays ~4 us of prologue and merge next to ~25 ns per token of streaming: take the
   // smallest segment count within 5 % of the best estimate (513..1023 workgroups: ~1.3
   // rounds instead of 2); few sequences: as many segments of >= 256 tokens as allowed.
@@ -203,8 +203,10 @@ int unified_decode_segments(const UniDecodeParams& p, int max_segments) {
   // and both more where some of the 256 CUs have a workgroup more than others.  us, cut -> one piece (32 / 8 heads of 128, fp8):
   // 1 x 500 11.9 -> 9.9, 16 x 777 14.7 -> 13.6, 24 x 500 14.9 -> 11.3, 32 x 1000 ragged 17.9 -> 14.4, 48 x 3000 ragged 40.2 -> 33.8,
   // 96 x 1600 60.1 -> 53.6; 16-bit 32 x 500 19.0 -> 15.8.  Kept cut: 1 x 1600 11.8 (one piece 16.0), 8 x 3000 18.1 (24.2), 40 x 3000
-  // 46.7 (51.8), 40 x 3000 ragged 34.3 (30.8).  Over 1048 batches (1 .. 512 sequences of 300 .. 16000 tokens, head 64 / 128 / 256,
-  // both caches) 4.0 % on average, none more than 2.5 % slower.  Not where the longest sequence may take a workgroup more than
+  // 46.7 (51.8), 40 x 3000 ragged 34.3 (30.8).  Over 4625 batches (1 .. 1023 pairs, 257 .. 9000 tokens, head 64 .. 256, both caches;
+  // tools/sweep_decode_plans.py, 237 of them in profiles/decode_plans.txt) 3.7 % below always cutting and 0.5 % above the cheaper
+  // form on average; more than 2.5 % slower than the cut in 2.4 % of them, since the merge now costs 0.3 .. 1.1 us less than when the
+  // price was fitted (4 x 1281 fp8 of 12 heads of 64 11.6 cut, 13.1 so).  Not where the longest sequence may take a workgroup more than
   // 24 us on an idle chip: among short ones it has to be cut.
   const double tb = 2.0 * row * (p.fp8 ? 1 : 2);
   auto us = [&](int n) {

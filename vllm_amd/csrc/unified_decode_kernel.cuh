@@ -1,9 +1,9 @@
 // The decode kernel of unified_attention as a device function: its own launch is in unified_decode.hip, the one it shares with
-// the tile kernel in prefill_fa.hip.  The bandwidth kernel of paged_attention_mfma.hip re-laid for the FLASH cache layout [block][slot][kv head][d] of the
-// V1 engine (vllm/attention/ops/triton_unified_attention.py:52-272 for the maths; caller
+// the tile kernel in prefill_fa.hip.  The bandwidth kernel of paged_attention_mfma.hip re-laid for the FLASH cache layout
+// [block][slot][kv head][d] of the V1 engine (vllm/attention/ops/triton_unified_attention.py:52-272 for the maths; caller
 // vllm/v1/attention/backends/triton_attn.py:297-317).
 //
-// One workgroup (4 waves) per (sequence, kv head[, key segment]) serves the whole GQA group (16 q
+// One workgroup (four waves, eight in a mixed step's launch) per (sequence, kv head[, key segment]) serves the whole GQA group (16 q
 // heads of it at a time), so every K / V byte is read once.  Waves stride over steps of 16 KiB of KV (fp8: 64 tokens,
 // 16-bit: 32), each with a private online softmax; one merge through LDS at the end.
 //
