@@ -1,5 +1,5 @@
 #!/bin/bash
-# Probe builds of the 256-row prefill kernel with compile-time ablations (run HERE, before gpurun):
+# Probe builds of the 256-row prefill kernel with compile-time ablations (no GPU needed):
 #   tools/fa_stamps.sh 0 12 2 31   ->  vllm_amd/csrc/libvllm_amd_probe_abl<N>.so
 # then on the GPU: VLLM_AMD_LIB=vllm_amd/csrc/libvllm_amd_probe_abl12.so python tools/fa_stamps.py
 set -e

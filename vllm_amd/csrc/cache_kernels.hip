@@ -71,7 +71,7 @@ __global__ void reshape_and_cache_kernel(
 // in a block (chunk boundaries do) is cut at the cache's groups and not at multiples of 16
 // tokens, and only its two ends are partial tiles, written as 4-byte units and single elements.
 // The first segment is blockIdx.z = 0's, a second one blockIdx.z = 1's (in one workgroup behind
-// each other 1.0 us more); more (decode batches) are scattered token by token.
+// each other 1 .. 3 us more); more (decode batches) are scattered token by token.
 // Bound by latency: read and write phases of one round of workgroups (4.2 TB/s at 8192 aligned
 // tokens).  us, tiles at multiples of 16 tokens -> at the groups, 8 heads of 128: 8192 tokens from
 // slot 11 of a block fp8 20.1 -> 14.9, 16-bit 30.7 -> 14.7 (aligned 15.8 -> 13.8, 15.9 -> 14.9), 24 chunks

@@ -898,11 +898,12 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
                                 num_tokens, batch, p.sliding_window, min_blocks);
     // One launch for chunks and decodes (fa_mixed_kernel) where the row blocks fill the chip -- in few blocks cut into segments
     // nothing hides the decodes (500 over 1500 among 63 of 4096 93 -> 100 us, 300 over 3000 among 200 of 500 74 -> 103) -- and up
-    // to 2.5 decode workgroups per CU: there they have a CU for themselves, and each one's start and merge (6 us) shows, where
-    // the decode kernel's own launch runs two or three side by side (2 x 1000 fresh among 127 of 250 58 -> 62 us, among 200 of
-    // 64 58 -> 76; 2000 over 1500 among 63 / 127 of 250 122 -> 113, 133 -> 125).
+    // to two decode workgroups per CU: here they have a CU for themselves, and each one's start and merge (6 us) shows, where
+    // the decode kernel's own launch runs two or three side by side.  Of 1143 random steps up to 640 pairs, one launch / two: below 384
+    // pairs 0.91 (six of 807 more than 2 % slower), 384 .. 512 0.95 (19 of 201), 513 .. 640 0.98 (44 of 135, 16 of them by 7 .. 26 %: 6 x
+    // 205 fresh among 71 of 191 30.8 -> 38.7 us; 2 x 1000 fresh among 200 of 64 58 -> 76).
     const bool one_launch = beside && can && plan.use && plan.nseg <= 1 && g_pf_mixed && head_size > 64 && head_size <= 128 &&
-                            u.hp == 1 && p.softcap == 0.f && p.sliding_window == 0 && unified_decode_pairs(u) <= 640;
+                            u.hp == 1 && p.softcap == 0.f && p.sliding_window == 0 && unified_decode_pairs(u) <= 512;
     if (beside && !one_launch) {
       const int rc = unified_decode(u);
       if (rc != VLLM_AMD_OK) return rc;
