@@ -734,17 +734,20 @@ void set_pa_waves(int v) { g_pa_waves = v; }
 // waves, one piece per sequence, fp8: 1 x 777 9.9 -> 8.9, 16 x 1500 14.5 -> 13.7, 32 x 1500 ragged 15.1 -> 14.4, head 64
 // 32 x 1500 12.4 -> 11.2; of 256 workgroups and more two of four waves share a CU and stream alike.  A 16-bit cache has twice the
 // bytes in flight per wave: 1 x 777 9.5 -> 8.6, level at 64 workgroups, 32 x 300 9.2 -> 9.7.  Pieces of 512 tokens and a merge
-// behind them gain up to 128 workgroups (1 x 3000 11.5 -> 11.2; 1 x 16000, 256 of them, 14.3 -> 14.7).  Up to 256 keys a workgroup
+// behind them gain up to 128 workgroups (fp8 rows of 64 2.5 .. 4 %, of 96 8 %; 256 workgroups lose 2 %).  Up to 256 keys a workgroup
 // -- short sequences, a window, the rocm op's pieces -- four waves have one round or two and the other four only their part of the
 // merge: 1 x 200 fp8 4.7 -> 5.1, 16-bit 5.2 -> 5.4, pieces of 256 fp8 and 16-bit 4 .. 9 % slower with eight (but rows padded to 128 over a
 // 16-bit cache 5 % faster), 1 x 300 6.1 -> 5.9; up to 512 keys 256 workgroups are faster with four (32 x 500 7.9 -> 8.5), and so are
-// whole rows of 128 over a 16-bit cache (8 .. 64 workgroups, 260 .. 512 keys 0 .. 6 %, pieces of 512 2 .. 3 %).
+// whole rows of 128 over a 16-bit cache (8 .. 64 workgroups, 260 .. 512 keys 0 .. 6 %, pieces of 512 2 .. 3 %).  Pieces of 512 of
+// whole fp8 rows of 128 gain 0 .. 2.6 % where they are full and lose as much as the merge gained where the lengths are short, as in a
+// graph captured at a long maximum (1 x 68 keys, planned for 8192, 6.9 -> 7.3): four too.
 static bool pa_eight_waves(const PagedAttnParams& p, int64_t workgroups, bool fp8, bool one_piece) {
   if (g_pa_waves) return g_pa_waves == 8;
   int64_t keys = p.max_seq_len > 0 ? p.max_seq_len : 1 << 30;   // a workgroup's, at most
   if (p.window > 0 && p.window < keys) keys = p.window;
   if (!one_piece && (int64_t)p.sp_parts * p.partition_size < keys) keys = (int64_t)p.sp_parts * p.partition_size;
-  if (keys <= (fp8 || p.head_size <= 64 ? 256 : p.head_size < 128 ? 255 : 512)) return false;
+  const bool whole = p.head_size == 128;
+  if (keys <= (whole && !(fp8 && one_piece) ? 512 : p.head_size > 64 && !whole && !fp8 ? 255 : 256)) return false;
   return workgroups <= (!fp8 ? 64 : one_piece && keys > 512 ? 256 : 128);
 }
 
