@@ -481,3 +481,22 @@ def test_prefill_wide_heads_short_chunks(kv, head_size, heads, qls, ctxs):
     """Above head size 128 short chunks with a context, or of 100 tokens, take the 256-row kernel however few they are."""
     c = make_prefill_case(qls, ctxs, *heads, head_size, 16, torch.bfloat16, kv, seed=head_size + len(qls), kv_scale=0.02)
     torch.testing.assert_close(run(c, kv).float(), prefill_reference(c), atol=tol(torch.bfloat16), rtol=0)
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("lens,ctx,heads", [
+    ([33, 32, 96, 129, 200, 1, 64], [0, 0, 70, 0, 300, 40, 130], (8, 2)),            # 2, 1, 3, 5, 7, 1, 2 halves of 32 tokens
+    ([129, 257, 300], [0, 140, 64], (4, 4)),                                          # halves of 128 tokens
+    ([43, 86, 171], [0, 200, 0], (6, 2)),                                             # a group that does not divide 128 rows
+    ([2 + i for i in range(32)], [7 * i for i in range(32)], (8, 8)),                 # one round of row blocks: pairs
+    ([2 + i for i in range(33)], [300 + 7 * i for i in range(33)], (8, 8)),           # more: the longest sequences first
+    ([2 + i % 30 for i in range(70)], [3 * i for i in range(70)], (4, 2)),            # more sequences than lanes
+])
+def test_prefill_row_blocks(oracle, tuning, kv, lens, ctx, heads):
+    """The unsplit 256-row kernel where its row blocks are dealt out, in the order of each rule."""
+    tuning("pf_fa", 2)
+    tuning("pf_segs", 1)
+    c = make_prefill_case(lens, ctx, heads[0], heads[1], 128, 16, torch.float16, kv, seed=len(lens), kv_scale=0.02)
+    out = run(c, kv)
+    assert not out.isnan().any()
+    torch.testing.assert_close(out.float(), run_oracle(oracle, c, kv).float(), atol=tol(torch.float16), rtol=0)

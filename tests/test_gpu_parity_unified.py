@@ -762,3 +762,30 @@ def test_unified_window_far_behind(oracle, fp8, D, heads, window, soft_cap):
     one piece (100), cut by the keys that a row block walks (600) or by all of them (1500); shorter sequences beside it."""
     c = make_unified_case([(200, 2600), (3, 1500), (70, 70), (1, 700)], *heads, D, 16, torch.bfloat16, fp8=fp8, seed=D + window)
     run(oracle, c, torch.bfloat16, window=window, softcap=soft_cap or 0.0, fp8=fp8)
+
+
+# (query, key) lengths -> row blocks of 256 / group tokens and their halves
+ROW_BLOCKS = {
+    "halves": ([(33, 33), (32, 32), (96, 96), (129, 129), (200, 500), (1, 70), (64, 65), (2, 300)], (8, 2)),     # 1, 2, 3, 5, 7 halves of 32 tokens
+    "one head": ([(129, 129), (257, 400), (128, 300), (300, 300)], (4, 4)),                                       # halves of 128 tokens
+    "group of 16": ([(9, 9), (8, 80), (17, 17), (40, 200)], (16, 1)),
+    "group of 3": ([(43, 43), (85, 85), (86, 300), (171, 171)], (6, 2)),                                          # does not divide 128: no pairs
+    "one round": ([(2 + i, 10 + 3 * i) for i in range(32)], (8, 8)),                                              # 256 row blocks
+    "past one round": ([(2 + i, 10 + 3 * i) for i in range(33)], (8, 8)),                                         # 264
+    "past 64 sequences": ([(2 + i % 40, 3 + 2 * i) if i % 7 else (1, 50) for i in range(80)], (4, 2)),
+}
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("blocks", ROW_BLOCKS)
+def test_unified_row_blocks(oracle, force_fa, fp8, blocks):
+    """The unsplit 256-row kernel where its row blocks are dealt out: half blocks paired from the front and the back of a chunk up to
+    one round of workgroups, whole ones above, more sequences than lanes."""
+    from vllm_amd import _lib
+    seqs, heads = ROW_BLOCKS[blocks]
+    c = make_unified_case(seqs, heads[0], heads[1], 128, 16, torch.bfloat16, fp8=fp8, seed=len(seqs), kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        run(oracle, c, torch.bfloat16, fp8=fp8)
+    finally:
+        _lib.set_tuning("pf_segs", 0)

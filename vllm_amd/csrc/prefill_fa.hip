@@ -21,10 +21,25 @@ __global__ __launch_bounds__(512) void fa_mixed_kernel(const FaParams p, const U
   __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS];
   const int hw = blockIdx.x;
   if (hw < nfa) {
-    if (hw < gx * gy) fa_body<T, FP8, false, 128, 8, false, false>(p, lds, hw, gx, gy);
+    if (hw < gx * gy) fa_body<T, FP8, false, 128, 8, false, false, true>(p, lds, hw, gy);
   } else {
     ua_decode_body<T, FP8, 128, 8, false, true>(u, (char*)lds, sub_shift, 0, order, hw - nfa, npairs, 0);
   }
+}
+
+// The last i of [0, n) for which le(i) holds (it holds for all i up to that one; 0 if it holds for none): 64 candidates per
+// step, so that 64 sequences take one load and 4096 two, where a binary search chains 6 and 12.
+template <typename F>
+__device__ __forceinline__ int wave_last(int n, int lane, F&& le) {
+  int lo = 0;
+  while (n > 1) {
+    const int step = (n + 63) >> 6, i = lane * step;
+    const int m = (int)__popcll(__ballot(i < n && le(lo + (i < n ? i : 0))));   // (popcll is unsigned)
+    const int c = m > 0 ? m - 1 : 0;
+    lo += c * step;
+    n = min(step, n - c * step);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
 }
 
 // Merge of a split launch: one wave per (token, q head).  Lane s holds segment s's maximum and sum; a half wave (D <= 128;

@@ -88,21 +88,6 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
-// The last i of [0, n) for which le(i) holds (it holds for all i up to that one; 0 if it holds for none): 64 candidates per
-// step, so that 64 sequences take one load and 4096 two, where a binary search chains 6 and 12.
-template <typename F>
-__device__ __forceinline__ int wave_last(int n, int lane, F&& le) {
-  int lo = 0;
-  while (n > 1) {
-    const int step = (n + 63) >> 6, i = lane * step;
-    const int m = (int)__popcll(__ballot(i < n && le(lo + (i < n ? i : 0))));   // (popcll is unsigned)
-    const int c = m > 0 ? m - 1 : 0;
-    lo += c * step;
-    n = min(step, n - c * step);
-  }
-  return __builtin_amdgcn_readfirstlane(lo);
-}
-
 // -DVA_PROBES (tools/fa_stamps.py): shader-clock time per wave spent in each part of the tile loop, summed over
 // the wave's tiles: 0 K ring fill + staging (LDS writes of tile t + 1, loads of t + 2), 2 S^T, 4 softmax + PV,
 // 5 barrier, 6 tiles computed, 7 whole kernel
@@ -119,12 +104,16 @@ static __device__ unsigned long long g_fa_stamps[2048 * 8 * 8];   // (one for ea
 #endif
 
 // Where a workgroup works: row block `blk` of sequence `seq` (its first query token tok0, its lengths), grid row y, and in split
-// launches the key segment `seg` of `segs`.
-struct FaAt { bool some = false; int seq, blk, y, seg, segs, tok0, qlen, seq_len; };
+// launches the key segment `seg` of `segs`.  pair: not rows of one row block, but of the blk-th half block from the front and the
+// blk-th from the back.
+struct FaAt { bool some = false, pair = false; int seq, blk, y, seg, segs, tok0, qlen, seq_len; };
 
-// hw: the workgroup's hardware id in a grid of gx x gy (of the launch's first gx gy workgroups: ids go round-robin over the XCDs).
-template <bool PREFIX, bool SPLIT, int BM>
-__device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int gx, int gy) {
+// hw: the workgroup's hardware id in a grid of gx x gy (of the launch's first gx gy workgroups: ids go round-robin over the XCDs),
+// an upper bound of the row blocks there are (gx = num_tokens / tpb + num_seqs, or blocks_per_seq * num_seqs where the caller did
+// not say how many query tokens there are).
+// MIXED: behind the row blocks the launch has a workgroup for every (decode, kv head).
+template <bool PREFIX, bool SPLIT, bool MIXED, int BM>
+__device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int gy) {
   // ---- workgroup -> (row block of some sequence, head).  Hardware ids go round-robin over the XCDs: the
   // bijective remap gives every XCD a contiguous range of logical ids (row blocks fastest, then heads), so the
   // row blocks and heads that read the same K / V share an L2; later (longer) row blocks first.
@@ -134,106 +123,92 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
   };
   const int nseg = SPLIT ? p.num_segments : 1;
   const int tpb = BM / p.pack;                // tokens per workgroup
-  // grid.x enumerates the row blocks of ALL sequences (num_tokens / tpb + num_seqs is an upper bound); the
-  // sequence is the last one whose first block cu[i] / tpb + i is <= g (find_seq_idx, :33-48)
-  // (blocks_per_seq > 0: the caller did not say how many query tokens there are; every sequence gets that many blocks)
   FaAt at;
-  int seq = 0, blk = -1;
-  int seg = 0, segs = 1;
-  int y, gs, g;
-  int tok0 = 0, qlen = 0, seq_len = 0;
-  if constexpr (SPLIT) {
-    // The row blocks there really are, and seg_slots workgroups dealt out to them: as num_segments workgroups for each
-    // block there may be, a launch spent 2.2 ns on each one of a sequence that the decode kernel takes (100 fresh tokens among
-    // 60 decodes of 3000 keys, 32 / 8 heads: 4032 workgroups, whole step 86.7 us, now 75.1; 200 over 3800 among 100 of 700: 91.7
-    // -> 66.0).  The work goes evenly over the XCDs: a few blocks too many on one of them double up on its CUs (512 over 7488,
-    // 8 q / 1 kv head: 60 against 40 us).
-    struct Seq { int tok0, qlen, len, blocks; };
-    auto seq_at = [&](int i) __attribute__((always_inline)) {   // (lengths too: the found sequence's need no load of their own)
-      Seq q = {0, 0, 0, 0};
-      if (i < p.num_seqs) {
-        q.tok0 = p.cu_seqlens_q[i];
-        q.qlen = p.cu_seqlens_q[i + 1] - q.tok0;
-        q.len = p.seq_lens[i];
-        q.blocks = p.skip_decode && q.qlen == 1 ? 0 : (q.qlen + tpb - 1) / tpb;
-      }
-      return q;
-    };
-    Seq my = seq_at(lane);                                    // the first 64 sequences stay in registers
-    int incl = wave_scan(my.blocks);
-    int here = __builtin_amdgcn_readlane(incl, 63), total = here;
-    for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(seq_at(i + lane).blocks), 63);
-    if (total == 0) return at;
-    const int work = max(total, min(p.seg_slots, total * nseg));   // per head
-    const int w = xcd_order(work * gy);
-    if (w < 0) return at;
-    y = w / work;
-    gs = w - y * work;
-    seg = gs / total;
-    int b = gs - seg * total;                                 // (a segment's row blocks are adjacent, they read the same K / V)
-    segs = work / total;
-    segs += b < work - segs * total ? 1 : 0;
-    b = total - 1 - b;                                        // later (longer) row blocks first
-    for (int i = 0; i < p.num_seqs; i += 64) {
-      if (i > 0) {
-        my = seq_at(i + lane);
-        incl = wave_scan(my.blocks);
-        here = __builtin_amdgcn_readlane(incl, 63);
-      }
-      if (b < here) {
-        const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(b < incl)) - 1);
-        seq = i + l;
-        blk = b - __builtin_amdgcn_readlane(incl - my.blocks, l);
-        tok0 = __builtin_amdgcn_readlane(my.tok0, l);
-        qlen = __builtin_amdgcn_readlane(my.qlen, l);
-        seq_len = __builtin_amdgcn_readlane(my.len, l);
-        break;
-      }
-      b -= here;
+  at.seg = 0;
+  at.segs = 1;
+  // The row blocks there really are, and in split launches seg_slots workgroups dealt out to them: as num_segments workgroups for
+  // each block there may be, a launch spent 2.2 ns on each one of a sequence that the decode kernel takes (100 fresh tokens among
+  // 60 decodes of 3000 keys, 32 / 8 heads: 4032 workgroups, whole step 86.7 us, now 75.1; 200 over 3800 among 100 of 700: 91.7
+  // -> 66.0).  The work goes evenly over the XCDs: a few blocks too many on one of them double up on its CUs (512 over 7488,
+  // 8 q / 1 kv head: 60 against 40 us), and so do those of a launch in whose grid every other workgroup is empty (32 chunks of 64
+  // tokens over 6000 keys, one row block each, in a grid of 64 a head: 232 -> 180; 16 of 60 .. 100 over 1500 .. 3000 among 40 decodes
+  // 119 -> 101).
+  struct Seq { int tok0, qlen, len, blocks; };
+  auto seq_at = [&](int i) __attribute__((always_inline)) {   // (lengths too: the found sequence's need no load of their own)
+    Seq q = {0, 0, 0, 0};
+    if (i < p.num_seqs) {
+      q.tok0 = p.cu_seqlens_q[i];
+      q.qlen = p.cu_seqlens_q[i + 1] - q.tok0;
+      q.len = p.seq_lens[i];
+      q.blocks = p.skip_decode && q.qlen == 1 ? 0 : (q.qlen + tpb - 1) / tpb;
     }
-  } else {
-    const int w = xcd_order(gx * gy);
-    y = w / gx;
-    gs = w % gx;
-    g = gx - 1 - gs;
-    if (p.blocks_per_seq > 0) {
-      seq = g / p.blocks_per_seq;
-      blk = g % p.blocks_per_seq;
-    } else if (PREFIX && p.num_seqs > 1 && p.num_seqs <= 64 && gy % 8 == 0) {
-      // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD: the row blocks of the
-      // longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24 chunks of
-      // 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us; 19 prompts of 745 .. 1242 without
-      // context, whose blocks differ more than the prompts, 294 -> 302: they keep the order below).
-      int len = -1, nb = 0, before = 0;   // lane i: sequence i, its blocks, the blocks in front of them
-      bool over = false;
-      if (lane < p.num_seqs) {
-        const int ql = p.cu_seqlens_q[lane + 1] - p.cu_seqlens_q[lane];
-        len = p.seq_lens[lane];
-        nb = p.skip_decode && ql == 1 ? 0 : (ql + tpb - 1) / tpb;
-        over = len >= 3 * ql;
-      }
-      if (2 * __popcll(__ballot(nb > 0 && over)) >= __popcll(__ballot(nb > 0))) {
-        for (int j = 0; j < p.num_seqs; ++j) {
-          const int lj = __builtin_amdgcn_readlane(len, j), nj = __builtin_amdgcn_readlane(nb, j);
-          before += (lj > len || (lj == len && j < lane)) ? nj : 0;
-        }
-        const unsigned long long mine = __ballot(before <= gs && gs < before + nb);
-        if (mine == 0) return at;            // the grid is an upper bound
-        seq = __builtin_amdgcn_readfirstlane(__ffsll((long long)mine) - 1);
-        blk = __builtin_amdgcn_readlane(nb, seq) - 1 - (gs - __builtin_amdgcn_readlane(before, seq));
+    return q;
+  };
+  Seq my = seq_at(lane);                                    // the first 64 sequences stay in registers
+  int incl = wave_scan(my.blocks);
+  int here = __builtin_amdgcn_readlane(incl, 63), total = here;
+  for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(seq_at(i + lane).blocks), 63);
+  if (total == 0) return at;
+  const int work = SPLIT ? max(total, min(p.seg_slots, total * nseg)) : total;   // per head
+  const int w = xcd_order(work * gy);
+  if (w < 0) return at;
+  at.y = w / work;
+  const int gs = w - at.y * work;
+  auto take = [&](int l) __attribute__((always_inline)) {
+    at.some = true;
+    at.tok0 = __builtin_amdgcn_readlane(my.tok0, l);
+    at.qlen = __builtin_amdgcn_readlane(my.qlen, l);
+    at.seq_len = __builtin_amdgcn_readlane(my.len, l);
+  };
+  if constexpr (!SPLIT) {
+    // One round of workgroups ends with its longest one, and under the causal mask the rows of a block differ in length by up to the
+    // chunk: each takes four waves' rows from the front of the chunk and four from its back, which all add up to the same.
+    // (A SIMD's second wave is done early; the first one then walks on alone at 1.2 us a tile, two take 1.9.)
+    // us, 32 / 8 heads, with the cache write: 2000 fresh tokens 69.5 -> 61.5, 1700 over 300 68 -> 60, 2000 over 1500 116 -> 107; 8 / 1
+    // heads 6000 fresh 198 -> 172.  Beside decodes the CUs
+    // of short row blocks do not idle, and row blocks of one length leave the decodes to the end (2000 over 1500 among 63 of up to
+    // 4096 keys 143 -> 152 us, 2048 fresh among 48 of 2000 69 -> 81; with few of them 1300 fresh among 16 of 1000 47 -> 41).
+    at.pair = !MIXED && BM == 256 && p.window == 0 && 128 % p.pack == 0 && total * gy <= 256;
+    // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD, more than one round: the row
+    // blocks of the longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24
+    // chunks of 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us, the flash layout 260 -> 250; 19 prompts of 745 .. 1242 without
+    // context, whose blocks differ more than the prompts, 294 -> 302: they keep the order below).
+    if (!MIXED && !at.pair && p.num_seqs > 1 && p.num_seqs <= 64 && gy % 8 == 0) {
+      const bool over = my.len >= 3 * my.qlen;
+      if (2 * __popcll(__ballot(my.blocks > 0 && over)) >= __popcll(__ballot(my.blocks > 0))) {
+        int before = 0;                        // blocks of longer sequences
+        const uint32_t key = (uint32_t)my.len << 6 | (uint32_t)(63 - lane);   // (no two alike)
+#pragma unroll 4
+        for (int j = 0; j < p.num_seqs; ++j)
+          before += (uint32_t)__builtin_amdgcn_readlane((int)key, j) > key ? __builtin_amdgcn_readlane(my.blocks, j) : 0;
+        const unsigned long long mine = __ballot(before <= gs && gs < before + my.blocks);
+        at.seq = __builtin_amdgcn_readfirstlane(__ffsll((long long)mine) - 1);
+        at.blk = __builtin_amdgcn_readlane(my.blocks, at.seq) - 1 - (gs - __builtin_amdgcn_readlane(before, at.seq));
+        take(at.seq);
+        return at;
       }
     }
-    if (blk < 0) {
-      seq = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] / tpb + i <= g; });
-      blk = g - (p.cu_seqlens_q[seq] / tpb + seq);
-      if (blk < 0) return at;                // rows in front of the first sequence (cu_seqlens_q may start above 0)
-    }
-    tok0 = p.cu_seqlens_q[seq];
-    qlen = p.cu_seqlens_q[seq + 1] - tok0;
-    seq_len = p.seq_lens[seq];
   }
-  at.some = true;
-  at.seq = seq; at.blk = blk; at.y = y; at.seg = seg; at.segs = segs; at.tok0 = tok0; at.qlen = qlen; at.seq_len = seq_len;
+  at.seg = gs / total;
+  int b = gs - at.seg * total;                              // (a segment's row blocks are adjacent, they read the same K / V)
+  at.segs = work / total;
+  at.segs += b < work - at.segs * total ? 1 : 0;
+  b = total - 1 - b;                                        // later (longer) row blocks first
+  for (int i = 0; i < p.num_seqs; i += 64) {
+    if (i > 0) {
+      my = seq_at(i + lane);
+      incl = wave_scan(my.blocks);
+      here = __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (b < here) {
+      const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(b < incl)) - 1);
+      at.seq = i + l;
+      at.blk = b - __builtin_amdgcn_readlane(incl - my.blocks, l);
+      take(l);
+      break;
+    }
+    b -= here;
+  }
   return at;
 }
 
@@ -250,8 +225,8 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
 // ~9 VALU per score between S^T and the softmax, in its own instantiation.
 // SPLIT: num_segments > 1, in its own instantiation (the 256-wide forms have no register to spare).
 template <int D_> constexpr int fa_lds() { return (KN + VN) * BN * 2 * D_; }   // 64 / 128 KiB
-template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP, bool SPLIT>
-__device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw, int gx, int gy) {
+template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP, bool SPLIT, bool MIXED = false>
+__device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw, int gy) {
   constexpr int NW = NW_, BM = 32 * NW, D = D_;
   constexpr int ROWB = 2 * D;       // bytes per LDS row (one key, D 16-bit values)
   constexpr int TILE = BN * ROWB;   // 16 / 32 KiB
@@ -276,7 +251,7 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   unsigned long long last__ = t_entry__;
 #endif
 
-  const FaAt at = fa_find<PREFIX, SPLIT, BM>(p, lane, hw, gx, gy);
+  const FaAt at = fa_find<PREFIX, SPLIT, MIXED, BM>(p, lane, hw, gy);
   if (!at.some) return;
   const int nseg = SPLIT ? p.num_segments : 1;
   const int pack = p.pack, tpb = BM / pack;   // tokens per workgroup
@@ -284,19 +259,26 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   const int ctx = seq_len - qlen;
   // first query token of this block
   const int tok_base = blk * tpb;
-  if (tok_base >= qlen) return;
-  if (p.skip_decode && qlen == 1) return;
-  const int new_end = min(tok_base + tpb, qlen);
+  // The rows of this wave: those of its half of the workgroup (waves 0-3 and 4-7, where the group divides into 128 rows) from row
+  // hrow0 and token htok on
+  const bool halves = NW == 8 && 128 % pack == 0;
+  const int htpb = halves ? tpb / 2 : tpb, hrow0 = halves && wave >= 4 ? 128 : 0;
+  int htok = tok_base + hrow0 / pack, new_end = min(tok_base + tpb, qlen);
+  if (at.pair) {
+    const int front = blk * htpb, back = ((qlen + htpb - 1) / htpb - 1 - blk) * htpb;
+    htok = wave < 4 ? back : (front < back ? front : qlen);   // (the middle half of an odd number: nothing for waves 4-7)
+    new_end = min(back + htpb, qlen);
+  }
   const int kvh = pack > 1 ? y : y / (p.num_heads / p.num_kv_heads);
   // head sizes up to 128 (multiples of 8; 16 with an fp8 cache) run padded to 128, above to 256: the columns d >= dr of Q, K and V are
   // staged as zeros from clamped addresses, the output columns are not stored
   const int dr = p.head_size;
 
   // ---- this lane's query row: tile row 32 wave + l32 -> (token, head) ----------------------------------------
-  const int mloc = 32 * wave + l32;
-  const int rtok = tok_base + mloc / pack;
-  const int rhead = pack > 1 ? kvh * pack + mloc % pack : y;
-  const bool rok = mloc < tpb * pack && rtok < qlen;
+  const int wrow = 32 * wave - hrow0, hrow = wrow + l32;
+  const int rtok = htok + hrow / pack;
+  const int rhead = pack > 1 ? kvh * pack + hrow % pack : y;
+  const bool rok = hrow < htpb * pack && rtok < qlen;
   // last visible key: among the new-domain keys (UNI: every key, by position; PREFIX: the new tokens, by index) and
   // among the context keys (PREFIX)
   const int bound_new = rok ? (PREFIX ? rtok : ctx + rtok) : -1;
@@ -330,9 +312,9 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     }
   }
   // wave-uniform: the tokens of the wave's rows
-  const bool w_rows = 32 * wave < tpb * pack && tok_base + (32 * wave) / pack < qlen;
-  const int w_lo = (PREFIX ? 0 : ctx) + tok_base + (32 * wave) / pack;
-  const int w_hi = (PREFIX ? 0 : ctx) + min(tok_base + (32 * wave + 31) / pack, new_end - 1);
+  const bool w_rows = wrow < htpb * pack && htok + wrow / pack < qlen;
+  const int w_lo = (PREFIX ? 0 : ctx) + htok + wrow / pack;
+  const int w_hi = (PREFIX ? 0 : ctx) + min(htok + (wrow + 31) / pack, min(htok + htpb, qlen) - 1);
 
   float kscale = 1.f, vscale = 1.f;
   if constexpr (FP8) { kscale = *p.k_scale; vscale = *p.v_scale; }
@@ -844,7 +826,9 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     tile_loop(b1, bf, INTERIOR, std::false_type{}, std::true_type{});
     tile_loop(bf, b2, INTERIOR, std::false_type{}, std::false_type{});
     tile_loop(b2, e2, MASKED_, std::false_type{}, std::false_type{});
-    tile_loop(e2, ntiles, SKIP, std::false_type{}, std::false_type{});
+    const int sf = fast_end(e2, ntiles, seq_len / BN);
+    tile_loop(e2, sf, SKIP, std::false_type{}, std::true_type{});
+    tile_loop(sf, ntiles, SKIP, std::false_type{}, std::false_type{});
   }
   }   // t0 < t1
 
@@ -904,7 +888,7 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
 template <typename T, bool FP8, bool PREFIX, int D_, int NW_, bool SOFTCAP, bool SPLIT>
 __global__ __launch_bounds__(64 * NW_) void fa_fwd_kernel(const FaParams p) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[fa_lds<D_>()];
-  fa_body<T, FP8, PREFIX, D_, NW_, SOFTCAP, SPLIT>(p, lds, blockIdx.x + gridDim.x * blockIdx.y, gridDim.x, gridDim.y);
+  fa_body<T, FP8, PREFIX, D_, NW_, SOFTCAP, SPLIT>(p, lds, blockIdx.x + gridDim.x * blockIdx.y, gridDim.y);
 }
 
 }  // namespace fa
