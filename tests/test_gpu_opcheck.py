@@ -197,3 +197,35 @@ def test_opcheck_call_operators():
     one = torch.ones(1, device="cuda")
     opcheck(torch.ops._vllm_amd_C.context_attention_fwd, (q, k, k, o, kx, vx, table, i32(0, 70, 71), i32(1170, 40), 1280, 70,
                                                           one, one, None, 0, 0.09, False, None))
+
+
+@pytest.mark.parametrize("m", [1, 17])
+def test_fp8_linear_new_equals_the_steps(ops, m):
+    """The linear operator that allocates its output: opcheck, and the bytes of quantisation and GEMM called one by one, from 2-D
+    and 3-D inputs."""
+    from vllm_amd.quantization import PTPCFp8LinearMethod
+    g = torch.Generator().manual_seed(m)
+    r = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).cuda()
+    x, b, ub = r(m, 256), r(64), torch.tensor([1.5], device="cuda")
+    w, ws = PTPCFp8LinearMethod.process_weights_after_loading(r(64, 256))
+    opcheck(torch.ops._vllm_amd_C.fp8_linear_new, (x, w, ws, torch.bfloat16, ub, b, True))
+    for per_token in (True, False):
+        q, s = ops.scaled_fp8_quant(x, scale_ub=ub if per_token else None, use_per_token_if_dynamic=per_token)
+        ref = ops.cutlass_scaled_mm(q, w, s, ws, torch.bfloat16, b)
+        assert torch.equal(ops.fp8_linear(x, w, ws, torch.bfloat16, ub if per_token else None, b, per_token), ref)
+    out = PTPCFp8LinearMethod().apply(w, ws, x.view(1, m, 256), b)
+    assert out.shape == (1, m, 64) and torch.equal(out[0], PTPCFp8LinearMethod().apply(w, ws, x, b))
+    assert PTPCFp8LinearMethod().apply(w, ws, x[:0].view(1, 0, 256)).shape == (1, 0, 64)
+
+
+@pytest.mark.parametrize("max_len", [1025, 3000])
+def test_forward_decode_scratch_equals_v2(ops, max_len):
+    """forward_decode, whose scratch is one buffer inside the operator, against paged_attention_v2 with the caller's tensors."""
+    from vllm_amd.attention import PagedAttention
+    c = make_attn_case(3, 8, 2, 128, 16, torch.bfloat16, "fp8", [1, 700, max_len], seed=max_len, kv_scale=0.5)
+    q, kc, vc, bt, sl = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt", "sl"))
+    sc, parts = torch.tensor([0.5], device="cuda"), (max_len + 511) // 512
+    out, es = torch.empty_like(q), torch.empty((3, 8, parts), device="cuda")
+    ops.paged_attention_v2(out, es, torch.empty_like(es), torch.empty((3, 8, parts, 128), dtype=q.dtype, device="cuda"), q, kc, vc,
+                           2, c["scale"], bt, sl, 16, max_len, None, "fp8", sc, sc)
+    assert torch.equal(PagedAttention.forward_decode(q, kc, vc, bt, sl, max_len, "fp8", 2, c["scale"], None, sc, sc), out)

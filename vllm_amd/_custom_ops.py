@@ -206,11 +206,8 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor
     """``cutlass_scaled_mm(*scaled_fp8_quant(x), ...)`` as one operator: x [M, K] quantised dynamically per token (or
     per tensor), weight fp8 [K, N] column-major.  (The reference does this in Fp8LinearOp.apply, w8a8_utils.py:297-377.)"""
     assert out_dtype is torch.bfloat16 or out_dtype is torch.float16
-    n = weight.shape[1]
-    assert bias is None or (bias.shape[0] == n and bias.dtype == out_dtype)
-    out = torch.empty((x.shape[0], n), dtype=out_dtype, device=x.device)
-    _torch_ops.fp8_linear(out, x, weight, weight_scale, scale_ub, bias, per_token)
-    return out
+    assert bias is None or (bias.shape[0] == weight.shape[1] and bias.dtype == out_dtype)
+    return _torch_ops.fp8_linear_new(x, weight, weight_scale, out_dtype, scale_ub, bias, per_token)
 
 
 # vllm/_custom_ops.py:1501-1508

@@ -128,6 +128,26 @@ void paged_attention_v1(Tensor& out, const Tensor& query, const Tensor& key_cach
       (int)bs_block_size, (int)bs_head_sliding_step, stream_of(query)));
 }
 
+// (scratch as pointers: the operator's tensors, or one buffer of paged_attention_decode)
+void paged_attention_v2_at(Tensor& out, float* exp_sums, float* max_logits, void* tmp_out, int64_t parts, const Tensor& query,
+                           const Tensor& key_cache, const Tensor& value_cache, int64_t num_kv_heads, double scale,
+                           const Tensor& block_tables, const Tensor& seq_lens, int64_t block_size, int64_t max_seq_len,
+                           const OptTensor& alibi_slopes, const std::string& kv_cache_dtype, const Tensor& k_scale,
+                           const Tensor& v_scale, int64_t tp_rank, int64_t bs_local_blocks, int64_t bs_vert_stride,
+                           int64_t bs_block_size, int64_t bs_head_sliding_step) {
+  TORCH_CHECK(block_tables.scalar_type() == at::kInt && seq_lens.scalar_type() == at::kInt,
+              "block_tables / seq_lens must be int32");
+  DevGuard g(query.device());
+  check(vllm_amd_paged_attention_v2(
+      out.data_ptr(), exp_sums, max_logits, tmp_out,
+      query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), (int)query.size(0), (int)query.size(1),
+      (int)query.size(2), (int)num_kv_heads, (float)scale, (const int*)block_tables.data_ptr(),
+      (const int*)seq_lens.data_ptr(), (int)block_tables.size(1), (int)block_size, (int)max_seq_len,
+      (int)parts, fptr(alibi_slopes), dt(query), kv(kv_cache_dtype), fptr(k_scale), fptr(v_scale),
+      query.stride(0), key_cache.stride(0), key_cache.stride(1), (int)tp_rank, (int)bs_local_blocks,
+      (int)bs_vert_stride, (int)bs_block_size, (int)bs_head_sliding_step, stream_of(query)));
+}
+
 void paged_attention_v2(Tensor& out, Tensor& exp_sums, Tensor& max_logits, Tensor& tmp_out, const Tensor& query,
                         const Tensor& key_cache, const Tensor& value_cache, int64_t num_kv_heads, double scale,
                         const Tensor& block_tables, const Tensor& seq_lens, int64_t block_size, int64_t max_seq_len,
@@ -140,17 +160,10 @@ void paged_attention_v2(Tensor& out, Tensor& exp_sums, Tensor& max_logits, Tenso
                   max_logits.is_contiguous(), "out / tmp_out / exp_sums / max_logits must be contiguous");
   TORCH_CHECK(exp_sums.scalar_type() == at::kFloat && max_logits.scalar_type() == at::kFloat,
               "exp_sums / max_logits must be float32");
-  TORCH_CHECK(block_tables.scalar_type() == at::kInt && seq_lens.scalar_type() == at::kInt,
-              "block_tables / seq_lens must be int32");
-  DevGuard g(query.device());
-  check(vllm_amd_paged_attention_v2(
-      out.data_ptr(), (float*)exp_sums.data_ptr(), (float*)max_logits.data_ptr(), tmp_out.data_ptr(),
-      query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), (int)query.size(0), (int)query.size(1),
-      (int)query.size(2), (int)num_kv_heads, (float)scale, (const int*)block_tables.data_ptr(),
-      (const int*)seq_lens.data_ptr(), (int)block_tables.size(1), (int)block_size, (int)max_seq_len,
-      (int)exp_sums.size(-1), fptr(alibi_slopes), dt(query), kv(kv_cache_dtype), fptr(k_scale), fptr(v_scale),
-      query.stride(0), key_cache.stride(0), key_cache.stride(1), (int)tp_rank, (int)bs_local_blocks,
-      (int)bs_vert_stride, (int)bs_block_size, (int)bs_head_sliding_step, stream_of(query)));
+  paged_attention_v2_at(out, (float*)exp_sums.data_ptr(), (float*)max_logits.data_ptr(), tmp_out.data_ptr(), exp_sums.size(-1), query,
+                        key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size, max_seq_len, alibi_slopes,
+                        kv_cache_dtype, k_scale, v_scale, tp_rank, bs_local_blocks, bs_vert_stride, bs_block_size,
+                        bs_head_sliding_step);
 }
 
 void paged_attention_rocm(Tensor& out, const Tensor& exp_sums, const Tensor& max_logits, const Tensor& tmp_out,
@@ -296,28 +309,37 @@ void dynamic_per_token_scaled_fp8_quant(Tensor& result, const Tensor& input, Ten
 
 // ---- GEMM --------------------------------------------------------------------------------
 // csrc/quantization/cutlass_w8a8/scaled_mm_entry.cu checks, restated
+// Checks of everything but the activations, which come as the fp8 values and scales [M, K] of `a`, one row after the other with
+// `lda` between them.
+void scaled_mm_at(Tensor& out, const void* a, int64_t M, int64_t K, int64_t lda, const Tensor& b, const float* a_scales,
+                  int64_t a_scale_numel, const Tensor& b_scales, const OptTensor& bias) {
+  TORCH_CHECK(b.dim() == 2 && out.dim() == 2, "a.dim() == 2 && b.dim() == 2 && c.dim() == 2");
+  const int64_t N = b.size(1);
+  TORCH_CHECK(out.size(0) == M && b.size(0) == K && out.size(1) == N,
+              "c.size(0) == a.size(0) && a.size(1) == b.size(0) && b.size(1) == c.size(1)");
+  TORCH_CHECK(out.stride(1) == 1, "a.stride(1) == 1 && c.stride(1) == 1");  // row major
+  TORCH_CHECK(b.stride(0) == 1, "b.stride(0) == 1");                        // column major
+  TORCH_CHECK(is_fp8(b), "scaled_mm: only fp8 e4m3 x fp8 e4m3 is implemented on gfx950");
+  TORCH_CHECK(b_scales.scalar_type() == at::kFloat, "scales must be float32");
+  TORCH_CHECK(b_scales.is_contiguous(), "a_scales.is_contiguous() && b_scales.is_contiguous()");
+  TORCH_CHECK(!bias.has_value() || (bias->numel() == N && bias->is_contiguous() && bias->dim() == 1 &&
+                                    bias->scalar_type() == out.scalar_type()),
+              "bias.numel() == b.size(1) && bias.is_contiguous() && bias.dim() == 1");
+  DevGuard g(out.device());
+  check(vllm_amd_scaled_mm(out.data_ptr(), a, b.data_ptr(), a_scales, fptr(b_scales), vptr(bias), (int)M, (int)N, (int)K, lda,
+                           b.stride(1), out.stride(0), (int)a_scale_numel, (int)b_scales.numel(), dt(out), stream_of(out)));
+}
+
 void cutlass_scaled_mm(Tensor& out, const Tensor& a, const Tensor& b, const Tensor& a_scales,
                        const Tensor& b_scales, const OptTensor& bias) {
   need_devs(out, a, b, a_scales, b_scales, bias);
   ensure_workspace(a);
-  TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2, "a.dim() == 2 && b.dim() == 2 && c.dim() == 2");
-  const int64_t M = a.size(0), K = a.size(1), N = b.size(1);
-  TORCH_CHECK(out.size(0) == M && b.size(0) == K && out.size(1) == N,
-              "c.size(0) == a.size(0) && a.size(1) == b.size(0) && b.size(1) == c.size(1)");
-  TORCH_CHECK(a.stride(1) == 1 && out.stride(1) == 1, "a.stride(1) == 1 && c.stride(1) == 1");  // row major
-  TORCH_CHECK(b.stride(0) == 1, "b.stride(0) == 1");                                             // column major
-  TORCH_CHECK(is_fp8(a) && is_fp8(b), "scaled_mm: only fp8 e4m3 x fp8 e4m3 is implemented on gfx950");
-  TORCH_CHECK(a_scales.scalar_type() == at::kFloat && b_scales.scalar_type() == at::kFloat,
-              "scales must be float32");
-  TORCH_CHECK(a_scales.is_contiguous() && b_scales.is_contiguous(),
-              "a_scales.is_contiguous() && b_scales.is_contiguous()");
-  TORCH_CHECK(!bias.has_value() || (bias->numel() == N && bias->is_contiguous() && bias->dim() == 1 &&
-                                    bias->scalar_type() == out.scalar_type()),
-              "bias.numel() == b.size(1) && bias.is_contiguous() && bias.dim() == 1");
-  DevGuard g(a.device());
-  check(vllm_amd_scaled_mm(out.data_ptr(), a.data_ptr(), b.data_ptr(), fptr(a_scales), fptr(b_scales), vptr(bias),
-                           (int)M, (int)N, (int)K, a.stride(0), b.stride(1), out.stride(0), (int)a_scales.numel(),
-                           (int)b_scales.numel(), dt(out), stream_of(a)));
+  TORCH_CHECK(a.dim() == 2, "a.dim() == 2 && b.dim() == 2 && c.dim() == 2");
+  TORCH_CHECK(a.stride(1) == 1, "a.stride(1) == 1 && c.stride(1) == 1");
+  TORCH_CHECK(is_fp8(a), "scaled_mm: only fp8 e4m3 x fp8 e4m3 is implemented on gfx950");
+  TORCH_CHECK(a_scales.scalar_type() == at::kFloat, "scales must be float32");
+  TORCH_CHECK(a_scales.is_contiguous(), "a_scales.is_contiguous() && b_scales.is_contiguous()");
+  scaled_mm_at(out, a.data_ptr(), a.size(0), a.size(1), a.stride(0), b, fptr(a_scales), a_scales.numel(), b_scales, bias);
 }
 
 void wvSplitKQ(const Tensor& in_a, const Tensor& in_b, Tensor& out_c, const Tensor& scale_a, const Tensor& scale_b,
@@ -429,27 +451,47 @@ void compute_slot_mapping(Tensor& slot_mapping, const Tensor& block_table, const
 
 // Dynamic activation quantisation (per token, or per tensor) + scaled_mm: vllm/model_executor/layers/quantization/utils/
 // w8a8_utils.py:297-377.  As two operators with three allocations from Python a call cost 18 us of host time, whatever
-// the GEMM took (17 tokens, 4096 -> 6144: 10 us on the GPU).
+// the GEMM took (17 tokens, 4096 -> 6144: 9 us on the GPU); with one allocation here and the output's below 10.4.
 void fp8_linear(Tensor& out, const Tensor& input, const Tensor& weight, const Tensor& weight_scale, const OptTensor& scale_ub,
                 const OptTensor& bias, bool per_token) {
   need_devs(out, input, weight, weight_scale, scale_ub, bias);
   TORCH_CHECK(input.dim() == 2, "input.ndim == 2");
   const Tensor x = input.contiguous();
   const int64_t m = x.size(0), k = x.size(1);
+  if (per_token) {
+    ensure_workspace(x);
+    // scales and quantised rows in one buffer (a tensor of each cost 0.7 us more)
+    const int64_t scales = (m * (int64_t)sizeof(float) + 255) / 256 * 256;
+    const Tensor buf = at::empty({scales + m * k}, x.options().dtype(at::kByte));
+    float* const scale = (float*)buf.data_ptr();
+    void* const q = (char*)buf.data_ptr() + scales;
+    DevGuard g(x.device());
+    check(vllm_amd_dynamic_per_token_scaled_fp8_quant(q, x.data_ptr(), scale, fptr(scale_ub), m, (int)k, dt(x), stream_of(x)));
+    scaled_mm_at(out, q, m, k, k, weight, scale, m, weight_scale, bias);
+    return;
+  }
   const Tensor q = at::empty({m, k}, x.options().dtype(at::kFloat8_e4m3fn));
-  Tensor scale = at::empty({per_token ? m : 1}, x.options().dtype(at::kFloat));
+  Tensor scale = at::empty({1}, x.options().dtype(at::kFloat));
   {
     DevGuard g(x.device());
-    if (per_token) {
-      check(vllm_amd_dynamic_per_token_scaled_fp8_quant(q.data_ptr(), x.data_ptr(), (float*)scale.data_ptr(), fptr(scale_ub),
-                                                        m, (int)k, dt(x), stream_of(x)));
-    } else {
-      scale.zero_();   // the kernel's atomic maximum starts there
-      check(vllm_amd_dynamic_scaled_fp8_quant(q.data_ptr(), x.data_ptr(), (float*)scale.data_ptr(), m, (int)k, dt(x),
-                                              stream_of(x)));
-    }
+    scale.zero_();   // the kernel's atomic maximum starts there
+    check(vllm_amd_dynamic_scaled_fp8_quant(q.data_ptr(), x.data_ptr(), (float*)scale.data_ptr(), m, (int)k, dt(x), stream_of(x)));
   }
   cutlass_scaled_mm(out, q, weight, scale, weight_scale, bias);
+}
+
+// ... with an output of its own (1 us less of host time than one from Python)
+Tensor fp8_linear_new(const Tensor& input, const Tensor& weight, const Tensor& weight_scale, at::ScalarType out_dtype,
+                      const OptTensor& scale_ub, const OptTensor& bias, bool per_token) {
+  TORCH_CHECK(input.dim() == 2, "input.ndim == 2");
+  TORCH_CHECK(weight.dim() == 2, "a.dim() == 2 && b.dim() == 2 && c.dim() == 2");
+  Tensor out = at::empty({input.size(0), weight.size(1)}, input.options().dtype(out_dtype));
+  fp8_linear(out, input, weight, weight_scale, scale_ub, bias, per_token);
+  return out;
+}
+Tensor fp8_linear_new_meta(const Tensor& input, const Tensor& weight, const Tensor& weight_scale, at::ScalarType out_dtype,
+                           const OptTensor& scale_ub, const OptTensor& bias, bool per_token) {
+  return at::empty_symint({input.sym_size(0), weight.sym_size(1)}, input.options().dtype(out_dtype));
 }
 
 // One buffer for the partial outputs, maxima and sums of `nseg` key segments.
@@ -468,8 +510,9 @@ struct Segments {
   }
 };
 
-// paged_attention_v1 where v2 would take every sequence in one piece, else v2 with scratch of its own (vllm/attention/ops/
-// paged_attn.py:131-193)
+// vllm/attention/ops/paged_attn.py:131-193.  Two partitions: paged_attention_v1 where v2 would take every sequence in one piece,
+// which needs no scratch.  Else v2 with scratch of its own, maxima, sums and partial outputs in one buffer (three tensors from
+// Python cost 3.5 us of host time: 1 x 3000 fp8 tokens 15.3 -> 11.8 us a call).
 void paged_attention_decode(Tensor& out, const Tensor& query, const Tensor& key_cache, const Tensor& value_cache,
                             int64_t num_kv_heads, double scale, const Tensor& block_tables, const Tensor& seq_lens,
                             int64_t block_size, int64_t max_seq_len, const OptTensor& alibi_slopes,
@@ -478,7 +521,8 @@ void paged_attention_decode(Tensor& out, const Tensor& query, const Tensor& key_
                             int64_t bs_head_sliding_step) {
   TORCH_CHECK(query.dim() == 3, "query.dim() == 3");
   const int64_t s = query.size(0), h = query.size(1), d = query.size(2), parts = (max_seq_len + 511) / 512;
-  if (vllm_amd_paged_attention_v2_pieces(out.data_ptr(), query.data_ptr(), (int)s, (int)h, (int)d, (int)num_kv_heads, (int)block_size,
+  if (parts >= 1 && parts <= 2 &&
+      vllm_amd_paged_attention_v2_pieces(out.data_ptr(), query.data_ptr(), (int)s, (int)h, (int)d, (int)num_kv_heads, (int)block_size,
                                          (int)max_seq_len, (int)parts, dt(query), kv(kv_cache_dtype), query.stride(0),
                                          key_cache.stride(1), (int)bs_vert_stride) == 1) {
     paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size, max_seq_len,
@@ -486,11 +530,14 @@ void paged_attention_decode(Tensor& out, const Tensor& query, const Tensor& key_
                        bs_head_sliding_step);
     return;
   }
-  Tensor sums = at::empty({s, h, parts}, query.options().dtype(at::kFloat)), max = at::empty_like(sums);
-  Tensor tmp = at::empty({s, h, parts, d}, out.options());
-  paged_attention_v2(out, sums, max, tmp, query, key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size,
-                     max_seq_len, alibi_slopes, kv_cache_dtype, k_scale, v_scale, tp_rank, bs_local_blocks, bs_vert_stride,
-                     bs_block_size, bs_head_sliding_step);
+  need_devs(out, query, key_cache, value_cache, block_tables, seq_lens, alibi_slopes, k_scale, v_scale);
+  TORCH_CHECK(out.is_contiguous(), "out must be contiguous");
+  const int64_t rows = s * h * parts, stats = (2 * rows * (int64_t)sizeof(float) + 255) / 256 * 256;
+  const Tensor buf = at::empty({stats + rows * d * (int64_t)out.element_size()}, query.options().dtype(at::kByte));
+  float* const sums = (float*)buf.data_ptr();
+  paged_attention_v2_at(out, sums, sums + rows, (char*)buf.data_ptr() + stats, parts, query, key_cache, value_cache, num_kv_heads,
+                        scale, block_tables, seq_lens, block_size, max_seq_len, alibi_slopes, kv_cache_dtype, k_scale, v_scale,
+                        tp_rank, bs_local_blocks, bs_vert_stride, bs_block_size, bs_head_sliding_step);
 }
 
 inline int kv_of_cache(const Tensor& k) { return is_fp8(k) ? VLLM_AMD_KV_FP8_E4M3 : VLLM_AMD_KV_AUTO; }
@@ -556,6 +603,7 @@ struct Registrar {
   torch::Library* impl;
   torch::Library* impl_any;
   torch::Library* impl_grad;
+  torch::Library* impl_meta;
   template <class F>
   void op(const char* name, const char* schema, F* fn, bool any_device = false) {
     try {
@@ -580,7 +628,8 @@ Registrar open_ns(const char* ns) {
   return Registrar{ns, mk(torch::Library::FRAGMENT, std::nullopt),
                    mk(torch::Library::IMPL, c10::DispatchKey::CUDA),
                    mk(torch::Library::IMPL, c10::DispatchKey::CompositeExplicitAutograd),
-                   mk(torch::Library::IMPL, c10::DispatchKey::AutogradCUDA)};
+                   mk(torch::Library::IMPL, c10::DispatchKey::AutogradCUDA),
+                   mk(torch::Library::IMPL, c10::DispatchKey::Meta)};
 }
 
 void register_all() {
@@ -663,6 +712,11 @@ void register_all() {
        "fp8_linear(Tensor! out, Tensor input, Tensor weight, Tensor weight_scale, Tensor? scale_ub, Tensor? bias,"
        " bool per_token) -> ()",
        &fp8_linear);
+  x.op_no_grad("fp8_linear_new",
+               "fp8_linear_new(Tensor input, Tensor weight, Tensor weight_scale, ScalarType out_dtype, Tensor? scale_ub, Tensor? bias,"
+               " bool per_token) -> Tensor",
+               &fp8_linear_new);
+  x.impl_meta->impl("fp8_linear_new", &fp8_linear_new_meta);
   // (no gradient passes through these two, as under the inference mode the reference runs them in)
   x.op_no_grad("unified_attention",
        "unified_attention(Tensor q, Tensor k, Tensor v, Tensor! out, Tensor cu_seqlens_q, int max_seqlen_q,"
