@@ -789,3 +789,22 @@ def test_unified_row_blocks(oracle, force_fa, fp8, blocks):
         run(oracle, c, torch.bfloat16, fp8=fp8)
     finally:
         _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,D,seqs", [
+    ((8, 2), 128, [(40 + 31 * (i % 5), 40 + 31 * (i % 5) + 7 * (i % 3)) for i in range(60)]),           # 2 heads: 4 XCDs each, 300 blocks
+    ((16, 1), 128, [(100 + 53 * (i % 4), 150 + 61 * (i % 4)) for i in range(25)]),                      # 1 head, halves of 8 tokens, 300 blocks
+    ((16, 4), 128, [(300 + i, 300 + i) for i in range(15)] + [(1, 9)]),                                 # 4 heads, 304 blocks, the last of one token
+    ((8, 8), 128, [(1 + 17 * i % 290, 20 + 29 * i) for i in range(36)]),                                # whole heads per XCD, short and long contexts
+    ((16, 8), 256, [(3 + 40 * (i % 6), 3 + 40 * (i % 6)) for i in range(14)]),                          # 128-row blocks
+])
+def test_unified_row_block_order(oracle, force_fa, fp8, heads, D, seqs):
+    """More than one round of row blocks: in the order of their last keys, in shares per XCD for few heads; every block once."""
+    from vllm_amd import _lib
+    c = make_unified_case(seqs, heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=len(seqs), kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        run(oracle, c, torch.bfloat16, fp8=fp8)
+    finally:
+        _lib.set_tuning("pf_segs", 0)

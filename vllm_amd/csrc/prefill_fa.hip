@@ -119,7 +119,8 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, co
   const unsigned gx = p.blocks_per_seq > 0 ? (unsigned)(p.blocks_per_seq * p.num_seqs) : (unsigned)(p.num_tokens / tpb + p.num_seqs);
   const unsigned gy = (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads);
   const unsigned slots = p.num_segments > 1 ? (unsigned)p.seg_slots : 0u;
-  const dim3 grid(gx > slots ? gx : slots, gy);
+  const unsigned per = gy == 1 || gy == 2 || gy == 4 ? 8 / gy : 1;   // (fa_find)
+  const dim3 grid(((gx > slots ? gx : slots) + per - 1) / per * per, gy);
   int npairs = 0, sub_shift = 0, order = 0;
   if (u != nullptr) {
     npairs = unified_decode_pairs(*u);

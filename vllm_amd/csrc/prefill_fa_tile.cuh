@@ -88,6 +88,16 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
+__device__ __forceinline__ int wave_max_i(int v) {   // (lanes without a source keep their own value)
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // -DVA_PROBES (tools/fa_stamps.py): shader-clock time per wave spent in each part of the tile loop, summed over
 // the wave's tiles: 0 K ring fill + staging (LDS writes of tile t + 1, loads of t + 2), 2 S^T, 4 softmax + PV,
 // 5 barrier, 6 tiles computed, 7 whole kernel
@@ -110,7 +120,7 @@ struct FaAt { bool some = false, pair = false; int seq, blk, y, seg, segs, tok0,
 
 // hw: the workgroup's hardware id in a grid of gx x gy (of the launch's first gx gy workgroups: ids go round-robin over the XCDs),
 // an upper bound of the row blocks there are (gx = num_tokens / tpb + num_seqs, or blocks_per_seq * num_seqs where the caller did
-// not say how many query tokens there are).
+// not say how many query tokens there are; 1, 2 or 4 heads: gx gy a multiple of 8).
 // MIXED: behind the row blocks the launch has a workgroup for every (decode, kv head).
 template <bool PREFIX, bool SPLIT, bool MIXED, int BM>
 __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int gy) {
@@ -150,10 +160,32 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
   for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(seq_at(i + lane).blocks), 63);
   if (total == 0) return at;
   const int work = SPLIT ? max(total, min(p.seg_slots, total * nseg)) : total;   // per head
-  const int w = xcd_order(work * gy);
-  if (w < 0) return at;
-  at.y = w / work;
-  const int gs = w - at.y * work;
+  // Most chunks are short ones over contexts at least twice as long: a sequence's blocks read the same keys, and belong together.
+  const unsigned long long chunks = __ballot(my.blocks > 0);
+  const bool over = !SPLIT && 2 * __popcll(__ballot(my.blocks > 0 && my.len >= 3 * my.qlen)) >= __popcll(chunks);
+  // One round of workgroups ends with its longest one, and under the causal mask the rows of a block differ in length by up to the
+  // chunk: each takes four waves' rows from the front of the chunk and four from its back, which all add up to the same.
+  // (A SIMD's second wave is done early; the first one then walks on alone at 1.2 us a tile, two take 1.9.)
+  // us, 32 / 8 heads, with the cache write: 2000 fresh tokens 69.5 -> 61.5, 1700 over 300 68 -> 60, 2000 over 1500 116 -> 107; 8 / 1
+  // heads 6000 fresh 198 -> 172.  Beside decodes the CUs of short row blocks do not idle, and row blocks of one length leave the
+  // decodes to the end (2000 over 1500 among 63 of up to 4096 keys 143 -> 152 us, 2048 fresh among 48 of 2000 69 -> 81; with few of
+  // them 1300 fresh among 16 of 1000 47 -> 41).
+  at.pair = !SPLIT && !MIXED && BM == 256 && p.window == 0 && 128 % p.pack == 0 && total * gy <= 256;
+  // 1, 2 or 4 heads, several rounds: every XCD takes its share of a head's blocks one by one.  In runs the long ones meet on the
+  // first XCDs (8 / 1 heads, 10000 fresh tokens 483 -> 277 us, 3 x 5000 231 -> 155; 16 / 4, 6000 229 -> 184).
+  const bool few = !SPLIT && !at.pair && !over && (gy == 1 || gy == 2 || gy == 4);
+  int gs;
+  if (few) {
+    const int per = 8 / gy, xcd = hw % 8;
+    at.y = xcd / per;
+    gs = hw / 8 * per + xcd % per;
+    if (gs >= work) return at;
+  } else {
+    const int w = xcd_order(work * gy);
+    if (w < 0) return at;
+    at.y = w / work;
+    gs = w - at.y * work;
+  }
   auto take = [&](int l) __attribute__((always_inline)) {
     at.some = true;
     at.tok0 = __builtin_amdgcn_readlane(my.tok0, l);
@@ -161,21 +193,38 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
     at.seq_len = __builtin_amdgcn_readlane(my.len, l);
   };
   if constexpr (!SPLIT) {
-    // One round of workgroups ends with its longest one, and under the causal mask the rows of a block differ in length by up to the
-    // chunk: each takes four waves' rows from the front of the chunk and four from its back, which all add up to the same.
-    // (A SIMD's second wave is done early; the first one then walks on alone at 1.2 us a tile, two take 1.9.)
-    // us, 32 / 8 heads, with the cache write: 2000 fresh tokens 69.5 -> 61.5, 1700 over 300 68 -> 60, 2000 over 1500 116 -> 107; 8 / 1
-    // heads 6000 fresh 198 -> 172.  Beside decodes the CUs
-    // of short row blocks do not idle, and row blocks of one length leave the decodes to the end (2000 over 1500 among 63 of up to
-    // 4096 keys 143 -> 152 us, 2048 fresh among 48 of 2000 69 -> 81; with few of them 1300 fresh among 16 of 1000 47 -> 41).
-    at.pair = !MIXED && BM == 256 && p.window == 0 && 128 % p.pack == 0 && total * gy <= 256;
-    // Short chunks over long contexts (most of them at least twice as long), whole kv heads per XCD, more than one round: the row
-    // blocks of the longest sequence first -- an XCD's workgroups start in this order, and a ragged batch ends on short ones (24
-    // chunks of 150 .. 250 over 1500 .. 3000 tokens, three rounds of workgroups: 266 -> 257 us, the flash layout 260 -> 250; 19 prompts of 745 .. 1242 without
-    // context, whose blocks differ more than the prompts, 294 -> 302: they keep the order below).
-    if (!MIXED && !at.pair && p.num_seqs > 1 && p.num_seqs <= 64 && gy % 8 == 0) {
-      const bool over = my.len >= 3 * my.qlen;
-      if (2 * __popcll(__ballot(my.blocks > 0 && over)) >= __popcll(__ballot(my.blocks > 0))) {
+    if (!at.pair && p.num_seqs <= 64 && (few || gy % 8 == 0) && __popcll(chunks) > 1) {
+      // Several chunks: an XCD's workgroups start in this order, and what it ends on should be short.  The row blocks in the order of
+      // their last keys, those with most of them first, in 64 steps of the range: lane l counts the blocks of its step and the ones
+      // before it.  Up to two rounds and a bit; above that, and over long contexts, the blocks of a sequence stay together at head size
+      // 128, whose tiles take too little time for keys from farther than the L2 (us: 8 x 300 .. 500 over 250 .. 500 70 -> 66, 5 x 540 ..
+      // 900 fresh 61 -> 57, head 256 5 x 550 .. 917 fresh 76 -> 68, 3 x 1200 .. 2000 143 -> 132; but 19 x 745 .. 1242 fresh 284 -> 292, 6 x
+      // 600 .. 1000 over 500 .. 1000 141 -> 143, 16 x 180 .. 300 over 750 .. 1500 134 -> 143).
+      if (128 % p.pack == 0 && (few || (!over && (BM == 128 || total * gy <= 576)))) {
+        const int sh = __builtin_ctz(tpb), ctx = my.len - my.qlen;
+        const int top = wave_max_i(my.blocks > 0 ? ctx + (my.blocks << sh) : 0), low = -wave_max_i(my.blocks > 0 ? -ctx : -top);
+        const int step = ((top - low) >> 6) + 1;
+        // blocks of a sequence whose last key is beyond `end`
+        auto beyond = [&](int end, int ctx_, int n) __attribute__((always_inline)) { return n - min(max((end - ctx_) >> sh, 0), n); };
+        int upto = 0;
+        const int end = top - (lane + 1) * step;
+        for (unsigned long long m = chunks; m != 0; m &= m - 1) {
+          const int j = __ffsll((long long)m) - 1;
+          upto += beyond(end, __builtin_amdgcn_readlane(ctx, j), __builtin_amdgcn_readlane(my.blocks, j));
+        }
+        const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(upto > gs)) - 1);
+        const int r = gs - (l > 0 ? __builtin_amdgcn_readlane(upto, l - 1) : 0);
+        const int before = beyond(top - l * step, ctx, my.blocks), n = beyond(top - (l + 1) * step, ctx, my.blocks) - before;
+        const int sum = wave_scan(n);
+        at.seq = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(r < sum)) - 1);
+        at.blk = __builtin_amdgcn_readlane(my.blocks - 1 - before + (sum - n), at.seq) - r;
+        take(at.seq);
+        return at;
+      }
+      // Short chunks over long contexts: the row blocks of the longest sequence first (24 chunks of 150 .. 250 over 1500 .. 3000 tokens,
+      // three rounds of workgroups: 266 -> 257 us, the flash layout 260 -> 250; 19 prompts of 745 .. 1242 without context, whose
+      // blocks differ more than the prompts, 294 -> 302: they keep the order below).
+      if (over && !MIXED) {
         int before = 0;                        // blocks of longer sequences
         const uint32_t key = (uint32_t)my.len << 6 | (uint32_t)(63 - lane);   // (no two alike)
 #pragma unroll 4
@@ -189,10 +238,13 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
       }
     }
   }
-  at.seg = gs / total;
-  int b = gs - at.seg * total;                              // (a segment's row blocks are adjacent, they read the same K / V)
-  at.segs = work / total;
-  at.segs += b < work - at.segs * total ? 1 : 0;
+  int b = gs;
+  if constexpr (SPLIT) {
+    at.seg = gs / total;
+    b = gs - at.seg * total;                                // (a segment's row blocks are adjacent, they read the same K / V)
+    at.segs = work / total;
+    at.segs += b < work - at.segs * total ? 1 : 0;
+  }
   b = total - 1 - b;                                        // later (longer) row blocks first
   for (int i = 0; i < p.num_seqs; i += 64) {
     if (i > 0) {
