@@ -407,3 +407,25 @@ def test_scaled_mm_kgroup_edges(ops, force_kernel, M, N, K):
         torch.ops._C.cutlass_scaled_mm(buf[:, pad:pad + N], a8, w8.t(), one, one, None)
         assert torch.equal(buf[:, pad:pad + N], prod.to(torch.bfloat16))
         assert (buf[:, :pad] == 7).all() and (buf[:, pad + N:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K,forced", [
+    (1101, 8184, 1024, 32),   # 256 x 192 tiles in one round, not 128 x 128 in three; ragged rows and columns
+    (700, 14336, 512, 32),
+    (289, 6136, 4096, 7),     # 64 x 64, not 128 x 64
+    (384, 6144, 2048, 38),    # 128 x 128 in one round, not 128 x 64
+    (1101, 8180, 1024, 3),    # rows that are no multiple of 16 bytes: the table's tile
+])
+def test_scaled_mm_by_rounds(ops, force_kernel, M, N, K, forced):
+    """Tiles chosen by the cost of whole rounds: small integers, so that sums are exact in any order, against the forced kernel and
+    a float32 product."""
+    g = torch.Generator().manual_seed(M)
+    a = torch.randint(-2, 3, (M, K), generator=g).float().cuda()
+    w = torch.randint(-2, 3, (N, K), generator=g).float().cuda()
+    a[:, 0], w[:, 1] = torch.arange(M, device="cuda") % 7, torch.arange(N, device="cuda") % 5
+    one = torch.ones((1, 1), device="cuda")
+    a8, w8 = a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn)
+    out = ops.cutlass_scaled_mm(a8, w8.t(), one, one, torch.bfloat16)
+    assert torch.equal(out, (a @ w.t()).to(torch.bfloat16))
+    force_kernel(forced)
+    assert torch.equal(out, ops.cutlass_scaled_mm(a8, w8.t(), one, one, torch.bfloat16))

@@ -294,6 +294,47 @@ int g_mm_tail = 0;     // tuning key kept for old scripts; the tail split went a
 
 using namespace va;
 
+// Above M 64 a launch takes whole rounds of tiles on 256 CUs, and which tile wastes the least of its last one is seldom the largest
+// that fills the chip (1024 x 8192 -> 10240: 320 tiles of 128 x 128 in two rounds 127.6 us, 216 of 256 x 192 in one 74.0).  us of a launch:
+// c + rounds (a + b nb), nb = K / 128; the kernels whose workgroups share a CU in pairs: pairs of rounds, and a last odd one.  Fitted to 810
+// launches (18 weight shapes of K 1024 .. 16384, N 1280 .. 28672, M 65 .. 4096, weights from HBM, each kernel forced; 9 .. 13 % rms).
+// Taken where it is 5 % below the tile that the table below would take.  715 other launches: 93 of them change, to 0.62 .. 1.00 of
+// the time (128 x 128 -> 256 x 192 0.76 on average, 128 x 64 -> 128 x 128 in one round 0.80, -> 64 x 64 0.83); profiles/gemm_rounds.txt.
+constexpr int kWide192 = 39;   // scaled_mm_pp.hip's 256 x 192 tiles
+struct TileCost { int sel, bm, bn; double c, a, b, a_odd, b_odd; };   // a_odd < 0: one workgroup per CU
+constexpr TileCost kTileCost[] = {
+    {38, 128, 128, 0.14, 4.57, 0.463, -1, 0},      // scaled_mm_kgroup.hip
+    {2, 256, 256, 1.85, 4.53, 1.307, -1, 0},       // scaled_mm_pp.hip
+    {kWide192, 256, 192, 1.17, 4.97, 1.096, -1, 0},
+    {3, 128, 128, 0.33, 4.90, 0.931, 3.13, 0.764},   // scaled_mm_large.hip
+    {7, 64, 64, 2.62, 1.00, 0.397, 0.97, 0.238},
+    // (those that only the table takes)
+    {4, 128, 128, 0.14, 4.57, 0.463, -1, 0},
+    {5, 128, 64, 1.44, 1.90, 0.660, 2.17, 0.367},
+    {6, 128, 64, 1.24, 2.29, 0.341, -1, 0},
+    {9, 64, 32, 3.45, 0.17, 0.272, -0.13, 0.178},
+    {10, 64, 32, 2.35, 1.05, 0.153, -1, 0},
+};
+static double tile_cost(const TileCost& t, int M, int N, int K) {
+  const int64_t rounds = ((int64_t)ceil_div(M, t.bm) * ceil_div(N, t.bn) + 255) / 256;
+  const double nb = K / 128;
+  if (t.a_odd == -1) return t.c + (double)rounds * (t.a + t.b * nb);
+  return t.c + (double)(rounds / 2) * (t.a + t.b * nb) + (double)(rounds % 2) * (t.a_odd + t.b_odd * nb);
+}
+// sel: what the table takes
+static int scaled_mm_by_rounds(int sel, int M, int N, int K) {
+  double own = 0.0, best = 1e30;
+  int pick = sel;
+  for (int i = 0; i < (int)(sizeof(kTileCost) / sizeof(kTileCost[0])); ++i) {
+    const double us = tile_cost(kTileCost[i], M, N, K);
+    if (kTileCost[i].sel == sel) own = us;
+    // (64 x 64 instead of 128 x 128 tiles: 0.996 of the time on average, up to 1.10)
+    const bool may = i < 4 || (i == 4 && (sel == 5 || sel == 6 || sel == 9 || sel == 10));
+    if (may && us < best) { best = us; pick = kTileCost[i].sel; }
+  }
+  return best < 0.95 * own ? pick : sel;
+}
+
 static int launch_scaled_mm(void* out, const void* a, const void* b, const float* a_scales,
                             const float* b_scales, const void* bias, int M, int N, int K,
                             int64_t lda, int64_t ldb, int64_t ldc, int a_scale_numel,
@@ -361,15 +402,13 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
       }
       sel = 2;
     }
+    // 16-byte row-contiguous stores
+    const bool vec16 = ldc % 8 == 0 && N % 8 == 0 && (((uintptr_t)out) & 15) == 0;
+    const bool chosen = sel != 0;
     // a single round of 128 x 128 tiles: scaled_mm_kgroup.hip ("mm_kernel" 38 forces it)
-    if ((sel == 38 || (sel == 0 && want_splits == 0 && scaled_mm_kgroup_pays(M, N, K))) && ldc % 8 == 0 && N % 8 == 0 &&
-        (((uintptr_t)out) & 15) == 0) {
-      launch_scaled_mm_kgroup(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel,
-                              out_dtype, st);
-      VA_LAUNCH_CHECK(op);
-      return VLLM_AMD_OK;
-    }
-    if (sel == 0 || sel == 11 || sel > 36) {
+    if (sel == 0 && want_splits == 0 && vec16 && scaled_mm_kgroup_pays(M, N, K)) sel = 38;
+    if (sel == 38 && !vec16) sel = 0;
+    if (sel == 0 || sel == 11 || (sel > 36 && sel != 38)) {
       // Largest tile that still yields ~3/4 of a full wave of workgroups (256 CUs); rows of
       // a tile beyond M are wasted MFMA work, so BM <= 2 M.  With more than one wave of tiles the
       // variant that fits several workgroups per CU wins, below that the variant that takes
@@ -406,23 +445,21 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
         }
       }
     }
+    if (!chosen && want_splits == 0 && splits == 1 && vec16 && M > 64) sel = scaled_mm_by_rounds(sel, M, N, K);
+    if (sel == 38) {
+      launch_scaled_mm_kgroup(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel,
+                              out_dtype, st);
+      VA_LAUNCH_CHECK(op);
+      return VLLM_AMD_OK;
+    }
     if (sel >= 2) {
-      // 16-byte row-contiguous stores through LDS
-      const bool vec16 = ldc % 8 == 0 && N % 8 == 0 && ((((uintptr_t)out) & 15) == 0);
-      // MFMA-bound problems (the heuristic's 256 x 256 choice): the staggered, persistent kernel of
+      // MFMA-bound problems (256 x 256 or 256 x 192 tiles): the staggered, persistent kernel of
       // scaled_mm_pp.hip -- waves 4-7 half a K block behind waves 0-3, one workgroup per CU walking its
       // XCD's share of the tiles (4096^3 55.9 -> 49.3 us, K 14336 170.7 -> 154.0, N 28672 405 -> 334,
-      // N 6144 100 (92.7 with the tail split below) -> 85.1: profiles/r03_gemm_pp.txt).  It writes 16-byte
+      // N 6144 100 -> 85.1: profiles/r03_gemm_pp.txt).  It writes 16-byte
       // pieces of rows, so outputs that do not allow them keep the kernel of scaled_mm_large.hip.
-      if (sel == 2 && g_mm_kernel == 0 && splits == 1 && vec16) {
-        // 256 x 192 tiles where they save a round of workgroups: a 192-wide tile costs ~7/8 of a 256-wide one (it
-        // stages 56 instead of 64 KiB per K block), so N 6144 (the fused qkv projection) at M 3072 -- 288 tiles = 2
-        // rounds against 384 narrow ones = 2 x 7/8 -- goes 90.2 -> 78.9 us, at M 4096 / 2048 91.5 / 52.3 -> 89.2 /
-        // 50.7 us; everywhere else on the benchmark grid the wide tile has fewer or equal rounds (profiles/r03_gemm_pp.txt 13)
-        const int tm = ceil_div(M, 256);
-        const int r256 = ceil_div(tm * ceil_div(N, 256), 256), r192 = ceil_div(tm * ceil_div(N, 192), 256);
-        const int variant = (8 * r256 > 7 * r192) ? (3 | 8) : 3;
-        launch_scaled_mm_pp(variant, out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc,
+      if ((sel == 2 || sel == kWide192) && g_mm_kernel == 0 && splits == 1 && vec16) {
+        launch_scaled_mm_pp(sel == kWide192 ? (3 | 8) : 3, out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc,
                             a_scale_numel, b_scale_numel, out_dtype, st);
         VA_LAUNCH_CHECK(op);
         return VLLM_AMD_OK;
