@@ -429,3 +429,25 @@ def test_scaled_mm_by_rounds(ops, force_kernel, M, N, K, forced):
     assert torch.equal(out, (a @ w.t()).to(torch.bfloat16))
     force_kernel(forced)
     assert torch.equal(out, ops.cutlass_scaled_mm(a8, w8.t(), one, one, torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (17, 1280, 1024), (48, 1267, 384),      # groups of 16 rows, 16 columns
+    (49, 1280, 1024), (255, 509, 1024),     # 32 rows
+    (33, 2560, 512), (40, 2556, 256),       # 16 rows, 32 columns
+    (100, 1278, 1024), (145, 1024, 1152),   # 48 rows
+    (112, 2048, 1024), (52, 4096, 256), (256, 1016, 1024),   # 32 rows, 32 columns
+])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
+def test_scaled_mm_row_groups(ops, M, N, K, out_dtype):
+    """Few columns: the weight-stream kernel with the rows in groups, on the shapes of each group size with ragged last groups; small
+    integers, so that sums are exact in any order."""
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randint(-2, 3, (M, K), generator=g).float().cuda()
+    w = torch.randint(-2, 3, (N, K), generator=g).float().cuda()
+    a[:, 0], w[:, 1] = torch.arange(M, device="cuda") % 7, torch.arange(N, device="cuda") % 5
+    sa = 2.0 ** (torch.arange(M, device="cuda") % 4).float().view(-1, 1)
+    sb, bias = 2.0 ** -(torch.arange(N, device="cuda") % 3).float().view(-1, 1), (torch.arange(N, device="cuda") % 9).to(out_dtype)
+    out = ops.cutlass_scaled_mm(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn).t(), sa, sb, out_dtype, bias)
+    ref = ((a @ w.t()) * sa * sb.view(1, -1)).to(out_dtype) + bias
+    assert torch.equal(out, ref)

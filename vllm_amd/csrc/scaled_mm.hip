@@ -275,6 +275,7 @@ bool scaled_mm_large_fits(int M, int N, int K, int64_t lda, int64_t ldb);
 bool scaled_mm_large_can_split(int M, int N, int bm, int bn, int splits, int ws_mode, hipStream_t st);
 // scaled_mm_stream.hip
 bool scaled_mm_stream_pays(int M, int N, int K);
+bool scaled_mm_stream_small(int M, int N);
 int launch_scaled_mm_stream(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
                             const void* bias, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
                             int out_dtype, hipStream_t st);
@@ -354,14 +355,14 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
   const bool glds_ok = K % 128 == 0 && K >= 256 && scaled_mm_large_fits(M, N, K, lda, ldb);
   const int want_splits = req_splits > 0 ? req_splits : g_mm_splitk;   // 0 = heuristic
   const bool vec = (ldc % 4 == 0) && ((((uintptr_t)out) & 7) == 0);
-  // M <= 64: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it) -- but where the activations that
-  // every workgroup of it reads (M x K bytes) pass 600 KB and N is small, two K slices of the 64 x 32 tile (below) win if there
+  // Few rows: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it up to M 64) -- but where the activations that
+  // every workgroup of it reads (M x K bytes) pass 600 KB and N is small, not so that groups of rows help, two K slices of the 64 x 32 tile (below) win if there
   // is a workspace for them: N 4096, stream / slices in us, K 14336 at M 33 16.7 / 17.6, M 48 19.5 / 19.0, M 64 21.9 / 20.3;
   // K 28672 at M 17 25.7 / 26.8, M 32 29.0 / 28.2, M 64 39.8 / 33.9 (profiles/gemm_stream.txt).
   const bool slices = g_mm_kernel == 0 && want_splits == 0 && glds_ok && vec && K >= 12288 && ceil_div(N, 32) <= 128 &&
-                      M <= 64 && M * K > 600000 && scaled_mm_large_can_split(M, N, 64, 32, 2, ws_mode, st);
-  if (glds_ok && M <= 64 &&
-      (g_mm_kernel == 37 || (g_mm_kernel == 0 && want_splits == 0 && !slices && scaled_mm_stream_pays(M, N, K)))) {
+                      M <= 64 && M * K > 600000 && !scaled_mm_stream_small(M, N) && scaled_mm_large_can_split(M, N, 64, 32, 2, ws_mode, st);
+  if (glds_ok &&
+      ((g_mm_kernel == 37 && M <= 64) || (g_mm_kernel == 0 && want_splits == 0 && !slices && scaled_mm_stream_pays(M, N, K)))) {
     launch_scaled_mm_stream(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel, out_dtype, st);
     VA_LAUNCH_CHECK(op);
     return VLLM_AMD_OK;

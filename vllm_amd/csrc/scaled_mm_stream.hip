@@ -1,8 +1,9 @@
-// fp8 scaled GEMM for gfx950, M <= 64: the decode step's projections, bound by the weight stream (N x K bytes of HBM).
+// fp8 scaled GEMM for gfx950, few rows: the decode step's projections, bound by the weight stream (N x K bytes of HBM).
 //
 //   out[M,N] = ((sa (.) A[M,K]) . (sb (.) W[N,K]^T)).to(out_t) (+ bias)      K % 128 == 0
 //
-// A workgroup owns 16 NT output columns and ALL rows (MT blocks of 16); its waves split K (wave w takes the 128-byte
+// A workgroup owns 16 NT output columns and MT blocks of 16 rows -- all of them, or one of several groups of rows where the column
+// tiles alone leave CUs idle (stream_rows) --; its waves split K (wave w takes the 128-byte
 // K blocks w, w + NW, ...) and every wave runs a pipeline of its own: a wave-private ring in LDS, filled with
 // global_load_lds 16 bytes per lane, no barrier until the partial sums are combined at the end of a tile.  What bounded
 // the forms before it (us at M 16: 14336 -> 4096 19.1, here 12.7; 4096 -> 28672 28.3, here 21.6; M 1: 15.8 / 28.8, here 11.0 / 20.8 =
@@ -44,6 +45,7 @@ struct Params {
   int M, N, K;
   int64_t lda, ldb, ldc;
   int asn, bsn, ntiles;
+  int groups;   // of 16 MT rows
   int vec;   // 8-byte aligned output rows, N % 4 == 0
 };
 
@@ -92,8 +94,23 @@ constexpr int MAXT = 16;   // tiles per workgroup (their column scales sit in LD
 
 // KBW = 0: weights and activations both travel through the ring (D stages of NT + MT blocks per wave).  KBW > 0
 // (RESIDENT): a wave has at most KBW K blocks and keeps their activations in registers; ring stages of NT blocks.
-template <typename out_t, int MT, int NT, int NW, int D, int KBW>
-__global__ __launch_bounds__(64 * NW) void scaled_mm_stream_kernel(const Params p) {
+// GROUPS: p.groups of 16 MT rows, one column tile per workgroup; else M <= 16 MT.
+template <typename out_t, int MT, int NT, int NW, int D, int KBW, bool GROUPS>
+__global__ __launch_bounds__(64 * NW) void scaled_mm_stream_kernel(const Params p_) {
+  Params p = p_;
+  int wg = blockIdx.x;
+  if constexpr (GROUPS) {
+    // Hardware workgroup i runs on XCD i % 8: all groups of a column tile on one XCD, one after the other, so that its weights leave
+    // HBM once (with the groups as grid.y, 33 .. 48 rows of N 2192 took as long as two passes over the weights).
+    const int idx = wg >> 3, grp = idx % p.groups;
+    wg = (wg & 7) + 8 * (idx / p.groups);
+    if (wg >= p.ntiles) return;
+    const int m0 = grp * 16 * MT;
+    p.a += (int64_t)m0 * p.lda;
+    p.out = (out_t*)p.out + (int64_t)m0 * p.ldc;
+    if (p.asn != 1) p.sa += m0;
+    p.M = min(p.M - m0, 16 * MT);
+  }
   constexpr bool RES = KBW > 0;
   constexpr int F = RES ? NT : NT + MT;            // blocks per ring stage
   constexpr int STAGE = F * 2048, L = 2 * F;       // bytes, load instructions per stage
@@ -111,7 +128,7 @@ __global__ __launch_bounds__(64 * NW) void scaled_mm_stream_kernel(const Params 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g4 = lane >> 4, r8 = lane >> 3;
-  const int M = p.M, N = p.N, G = gridDim.x, wg = blockIdx.x;
+  const int M = p.M, N = p.N, G = GROUPS ? p.ntiles : (int)gridDim.x;
   const int nkb = p.K / 128;
   const int spt = (nkb - wave + NW - 1) / NW;            // K blocks of this wave (0: it only takes part in the sums)
   const int mytiles = (p.ntiles - wg + G - 1) / G;
@@ -289,6 +306,30 @@ __global__ __launch_bounds__(64 * NW) void scaled_mm_stream_kernel(const Params 
   if constexpr (RES) wait_vm<0>();   // T < D: loads that no step waited for have landed before the LDS is given back
 }
 
+// Row groups: N up to 4096 has at most 256 column tiles of 16, and a workgroup pulls 128 (16 MT + 16 NT) bytes per K block at the same
+// ~90 GB/s whatever its neighbours do.  So the smallest MT + NT with which all rows still make one round of workgroups: the weights go
+// to several of them, through L2, and the activations to none twice.  us, all rows in one workgroup (M > 64: the tile kernels) ->
+// groups: 8192 -> 1280 at M 32 9.3 -> 7.2, M 63 12.3 -> 9.1, M 94 12.0 -> 9.3; 15360 -> 1248 at M 40 18.4 -> 11.0, M 81 20.4 -> 14.7;
+// 4096 -> 1024 at M 64 7.7 -> 5.1; 8192 -> 2048 at M 64 12.6 -> 9.5; 4096 -> 4096 at M 63 8.2 -> 8.1; of 849 launches with N up to 4096
+// and M 9 .. 330 the 340 that it takes 0.78 (profiles/gemm_row_groups.txt).  A second round costs more than it spreads: 8192 -> 1280 at
+// M 49 as 320 workgroups of 16 rows 10.4, as 160 of 32 8.7; and a round is 32 workgroups on each XCD, in whole column tiles: 12672 ->
+// 2624 at M 44 as 82 x 3, 33 on two of them, 17.0 -> 24.7.  32 rows x 32 columns only above M 48 (48 rows x 16 in one group there: 0.94 of it).
+// mt = 0: all rows in one workgroup.
+struct Rows { int mt, nt; };
+static Rows stream_rows(int M, int N) {
+  if (M <= 16 || N > 4096) return {0, 0};
+  auto wgs = [&](int mt, int nt) { return (int64_t)ceil_div(ceil_div(N, 16 * nt), 8) * 8 * ceil_div(M, 16 * mt); };
+  if (wgs(1, 1) <= 256) return {1, 1};
+  if (M <= 32) return {0, 0};
+  if (wgs(2, 1) <= 256) return {2, 1};
+  if (wgs(1, 2) <= 256) return {1, 2};
+  if (M <= 48) return {0, 0};
+  if (wgs(2, 2) <= 256 && wgs(2, 2) >= wgs(3, 1)) return {2, 2};
+  if (wgs(3, 1) <= 256) return {3, 1};
+  if (wgs(2, 2) <= 256) return {2, 2};
+  return {0, 0};
+}
+
 template <typename out_t>
 static void launch(const Params& p0, hipStream_t st) {
   Params p = p0;
@@ -298,8 +339,24 @@ static void launch(const Params& p0, hipStream_t st) {
     p.ntiles = ceil_div(p.N, 16 * NT);                                                                        \
     int grid = p.ntiles < (GRID) ? p.ntiles : (GRID);                                                         \
     if (grid * MAXT < p.ntiles) grid = ceil_div(p.ntiles, MAXT);                                              \
-    hipLaunchKernelGGL((scaled_mm_stream_kernel<out_t, MT, NT, NW, D, KBW>), dim3(grid), dim3(64 * NW), 0, st, p); \
+    hipLaunchKernelGGL((scaled_mm_stream_kernel<out_t, MT, NT, NW, D, KBW, false>), dim3(grid), dim3(64 * NW), 0, st, p); \
   } while (0)
+#define VA_STREAM_ROWS(MT, NT, NW, D)                                                                         \
+  do {                                                                                                        \
+    p.ntiles = ceil_div(p.N, 16 * NT);                                                                        \
+    p.groups = ceil_div(p.M, 16 * MT);                                                                        \
+    hipLaunchKernelGGL((scaled_mm_stream_kernel<out_t, MT, NT, NW, D, 0, true>), dim3(ceil_div(p.ntiles, 8) * 8 * p.groups), \
+                       dim3(64 * NW), 0, st, p);                                                              \
+  } while (0)
+  const Rows rows = stream_rows(p.M, p.N);
+  if (rows.mt > 0) {
+    if (rows.mt == 1 && rows.nt == 1) VA_STREAM_ROWS(1, 1, 4, 3);
+    else if (rows.mt == 2 && rows.nt == 1) VA_STREAM_ROWS(2, 1, 4, 2);
+    else if (rows.mt == 1) VA_STREAM_ROWS(1, 2, 8, 2);
+    else if (rows.mt == 2) VA_STREAM_ROWS(2, 2, 4, 2);
+    else VA_STREAM_ROWS(3, 1, 4, 2);
+    return;
+  }
   // 32-column tiles from 160 of them on (N 5120): fewer, the 16-column ones fill the CUs better (N 4096 at M 16: 5.5 us
   // against 6.6; N 6144: 7.7 against 6.8).
   const bool wide = t32 >= 160, k4 = p.K <= 4 * 8 * 128, k8 = p.K <= 8 * 8 * 128;
@@ -318,6 +375,7 @@ static void launch(const Params& p0, hipStream_t st) {
   else if (mt == 2) VA_STREAM(2, 1, 4, 2, 0, 1024);
   else if (mt == 3) VA_STREAM(3, 1, 4, 2, 0, 512);
   else VA_STREAM(4, 1, 4, 2, 0, 512);
+#undef VA_STREAM_ROWS
 #undef VA_STREAM
 }
 
@@ -334,19 +392,25 @@ static void launch(const Params& p0, hipStream_t st) {
 // 4096 -> 6144 (10.4 : 10.3) and 3584 -> 8192 (9.8 : 10.1) at M 64, and more than 256 tiles over K above 4096 (8192 -> 14336 at
 // M 49, 64 27.9, 28.9 : 28.2, 30.9; not at M 33, 27.6 : 25.2).
 bool scaled_mm_stream_pays(int M, int N, int K) {
-  if (M > 64) return false;
+  if (M > 64) return K >= 1024 && mms::stream_rows(M, N).mt > 0;
   const int t32 = ceil_div(N, 32), t64 = ceil_div(N, 64);
   if (t32 > 256 && (K < 3072 || (M > 32 && K < 4096 && t64 >= 190 && t64 <= 256))) return false;
   if (M <= 32 || t32 < 160) return true;
   return K <= 4096 ? K >= 3072 && (M <= 48 || t32 > 256) : t32 <= 256;
 }
 
-// Caller guarantees 1 <= M <= 64, K % 128 == 0, 16-byte aligned operands and scaled_mm_large_fits() (32-bit offsets).
+// The groups of rows are so small that nothing the tile kernels have for these shapes comes near, K slices included.
+bool scaled_mm_stream_small(int M, int N) {
+  const mms::Rows r = mms::stream_rows(M, N);
+  return r.mt > 0 && r.mt + r.nt <= 3;
+}
+
+// Caller guarantees M >= 1, above 64 scaled_mm_stream_pays(), K % 128 == 0, 16-byte aligned operands and scaled_mm_large_fits() (32-bit offsets).
 int launch_scaled_mm_stream(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
                             const void* bias, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
                             int out_dtype, hipStream_t st) {
   const int vec = ldc % 4 == 0 && N % 4 == 0 && (((uintptr_t)out) & 7) == 0;
-  const mms::Params p{(const uint8_t*)a, (const uint8_t*)b, a_scales, b_scales, bias, out, M, N, K, lda, ldb, ldc, asn, bsn, 0, vec};
+  const mms::Params p{(const uint8_t*)a, (const uint8_t*)b, a_scales, b_scales, bias, out, M, N, K, lda, ldb, ldc, asn, bsn, 0, 1, vec};
   if (out_dtype == VLLM_AMD_BF16) mms::launch<bf16_t>(p, st);
   else mms::launch<f16_t>(p, st);
   return VLLM_AMD_OK;
