@@ -196,11 +196,12 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
     if (!at.pair && p.num_seqs <= 64 && (few || gy % 8 == 0) && __popcll(chunks) > 1) {
       // Several chunks: an XCD's workgroups start in this order, and what it ends on should be short.  The row blocks in the order of
       // their last keys, those with most of them first, in 64 steps of the range: lane l counts the blocks of its step and the ones
-      // before it.  Up to two rounds and a bit; above that, and over long contexts, the blocks of a sequence stay together at head size
+      // before it.  Up to two rounds and 16 chunks; above that, and over long contexts, the blocks of a sequence stay together at head size
       // 128, whose tiles take too little time for keys from farther than the L2 (us: 8 x 300 .. 500 over 250 .. 500 70 -> 66, 5 x 540 ..
       // 900 fresh 61 -> 57, head 256 5 x 550 .. 917 fresh 76 -> 68, 3 x 1200 .. 2000 143 -> 132; but 19 x 745 .. 1242 fresh 284 -> 292, 6 x
-      // 600 .. 1000 over 500 .. 1000 141 -> 143, 16 x 180 .. 300 over 750 .. 1500 134 -> 143).
-      if (128 % p.pack == 0 && (few || (!over && (BM == 128 || total * gy <= 576)))) {
+      // 600 .. 1000 over 500 .. 1000 141 -> 143, 16 x 180 .. 300 over 750 .. 1500 134 -> 143, 19 x 138 .. 230 fresh, 520 blocks, 43 -> 46,
+      // 8 x 403 .. 671 over 198 .. 395, 568 blocks, 86 -> 91, 20 x 56 .. 93 fresh, 280 blocks, 26.4 -> 28.5).
+      if (128 % p.pack == 0 && (few || (!over && (BM == 128 || (total * gy <= 512 && (int)__popcll(chunks) <= 16))))) {
         const int sh = __builtin_ctz(tpb), ctx = my.len - my.qlen;
         const int top = wave_max_i(my.blocks > 0 ? ctx + (my.blocks << sh) : 0), low = -wave_max_i(my.blocks > 0 ? -ctx : -top);
         const int step = ((top - low) >> 6) + 1;
@@ -878,9 +879,9 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
     tile_loop(b1, bf, INTERIOR, std::false_type{}, std::true_type{});
     tile_loop(bf, b2, INTERIOR, std::false_type{}, std::false_type{});
     tile_loop(b2, e2, MASKED_, std::false_type{}, std::false_type{});
-    const int sf = fast_end(e2, ntiles, seq_len / BN);
-    tile_loop(e2, sf, SKIP, std::false_type{}, std::true_type{});
-    tile_loop(sf, ntiles, SKIP, std::false_type{}, std::false_type{});
+    // (waves without rows, too, with the checks: without them they get in the way of a single wave that has some, 160 tiles of one
+    // query token 172 -> 184 us, and pairs gain nothing)
+    tile_loop(e2, ntiles, SKIP, std::false_type{}, std::false_type{});
   }
   }   // t0 < t1
 
