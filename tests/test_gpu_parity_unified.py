@@ -525,6 +525,40 @@ def test_unified_mixed_launch_limit(oracle, force_fa, n, one):
     assert _mixed_launches() - before == one
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,D", [((8, 2), 128), ((32, 8), 80), ((24, 1), 96)])
+@pytest.mark.parametrize("seqs,one", [
+    ([(1, 700), (130, 190)], 1), ([(70, 300), (1, 1), (65, 65), (1, 513)], 1), ([(1, 900), (1, 5), (1, 257), (450, 450)], 1),
+    ([(40, 500), (90, 90), (3, 7)], 1),           # no decode, and nothing that tells
+    ([(90, 500), (91, 91)], 0), ([(1, 99)] + [(50, 50)] * 5, 0),   # none, and too many tokens for one; one that does not matter
+])
+def test_unified_few_sequences_one_launch(oracle, force_fa, heads, D, fp8, seqs, one):
+    """Fewer than 16 sequences: decodes that may be among the chunks go along as workgroups of the decode kernel."""
+    from vllm_amd import _lib
+    c = make_unified_case(seqs, heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=len(seqs) + D, kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        before = _mixed_launches()
+        run(oracle, c, torch.bfloat16, fp8=fp8, view=lambda t: t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3))
+        assert _mixed_launches() - before == one
+    finally:
+        _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,D", [((8, 2), 64), ((16, 8), 256), ((4, 4), 128)])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_unified_few_sequences_decodes_apart(oracle, heads, D, fp8, softcap):
+    """The same, where the chunks' kernel takes no decodes along: the decode kernel in front of it, and every token written once."""
+    from vllm_amd import _lib
+    c = make_unified_case([(1, 2100), (300, 310), (1, 1), (2, 900)], heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        run(oracle, c, torch.bfloat16, fp8=fp8, softcap=softcap)
+    finally:
+        _lib.set_tuning("pf_segs", 0)
+
+
 def test_unified_fa_kernel_sharp_rows(oracle, force_fa):
     """Rows whose maximum keeps growing along the keys (the lazy rescale must fire on some tiles and not on others):
     keys scaled up with their position."""

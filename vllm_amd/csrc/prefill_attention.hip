@@ -851,9 +851,16 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
   // whose query length is not 1, the tile kernel below then skips those whose length is.
   // num_tokens == batch * max_q means every query has max_q > 1 tokens: nothing to split off.
   const bool mixed = max_q > 1 && batch >= 16 && (int64_t)num_tokens < (int64_t)batch * max_q;
+  // Fewer sequences, of which one or more may be decodes: as rows of a row block of its own such a token walks its keys at 1.1 us
+  // per 64 (2 in the 64-row kernel), and a step ends when the longest is done; a workgroup of the decode kernel takes 0.2 .. 0.3.
+  // us, 8 / 1 heads, 7 x 654 fresh among 4 of 10303 172 -> 62; 32 / 8, 2000 among 3 of 4000 97 -> 71, 3 x 1200 among one of 16000
+  // 288 -> 128.  Where no walk is longer than the chunks' own (two waves a SIMD, 1.9 us a tile) there is nothing to win, and the
+  // workgroups that find no decode cost 1 .. 2 us (6 x 673 .. 1122 fresh among 5 of up to 474 84 -> 87).
+  const bool maybe = !mixed && max_q > 1 && (int64_t)num_tokens <= (int64_t)(batch - 1) * max_q + 1 &&
+                     max_k >= 2 * (int64_t)max_q;
   UniDecodeParams u;
   bool beside = false;   // decode tokens that the tile kernel's launch may take along
-  if ((max_q == 1 || mixed) && g_uni_decode && g_pf_rows != 1) {
+  if ((max_q == 1 || mixed || maybe) && g_uni_decode && g_pf_rows != 1) {
     u.out = p.o; u.q = p.q; u.k_cache = p.k_cache; u.v_cache = p.v_cache;
     u.cu_seqlens_q = p.b_start_loc; u.seq_lens = p.b_seq_len; u.block_table = p.b_loc;
     u.k_scale = p.k_scale; u.v_scale = p.v_scale; u.alibi_slopes = p.alibi_slopes;
@@ -872,11 +879,10 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     u.dtype = std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16;
     u.fp8 = FP8; u.stream = st;
     u.hp = unified_decode_heads_per_row(u);
-    u.num_segments = unified_decode_segments(u, mixed ? 1 : p.num_segments);
+    u.num_segments = unified_decode_segments(u, max_q > 1 ? 1 : p.num_segments);
     if (unified_decode_supported(u)) {
-      if (!mixed) return unified_decode(u);
+      if (max_q == 1) return unified_decode(u);
       beside = true;
-      p.skip_decode = 1;
     }
   }
   // Query chunks with only the causal mask (+ window, softcap): the 256-row kernel (prefill_fa.hip; rows = (token, q head of
@@ -904,7 +910,12 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     // 205 fresh among 71 of 191 30.8 -> 38.7 us; 2 x 1000 fresh among 200 of 64 58 -> 76).
     const bool one_launch = beside && can && plan.use && plan.nseg <= 1 && g_pf_mixed && head_size > 64 && head_size <= 128 &&
                             u.hp == 1 && p.softcap == 0.f && p.sliding_window == 0 && unified_decode_pairs(u) <= 512;
-    if (beside && !one_launch) {
+    // In a launch of their own: always with 16 sequences and more; below that where the tile kernel would walk many more keys for one of
+    // them than for a chunk (us, head 64, 32 / 8, 2 x 1500 over 500 among 5 of 8000 213 -> 95, 2000 among 3 of 4000 105 -> 76; head 256,
+    // 16 / 8, 312 -> 168, 164 -> 132), and not split (the segments spread the walk).
+    const bool apart = beside && !one_launch && (mixed || (plan.nseg <= 1 && max_q >= 256 && max_k >= 2048));
+    p.skip_decode = one_launch || apart;
+    if (apart) {
       const int rc = unified_decode(u);
       if (rc != VLLM_AMD_OK) return rc;
     }

@@ -167,10 +167,11 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
   // chunk: each takes four waves' rows from the front of the chunk and four from its back, which all add up to the same.
   // (A SIMD's second wave is done early; the first one then walks on alone at 1.2 us a tile, two take 1.9.)
   // us, 32 / 8 heads, with the cache write: 2000 fresh tokens 69.5 -> 61.5, 1700 over 300 68 -> 60, 2000 over 1500 116 -> 107; 8 / 1
-  // heads 6000 fresh 198 -> 172.  Beside decodes the CUs of short row blocks do not idle, and row blocks of one length leave the
-  // decodes to the end (2000 over 1500 among 63 of up to 4096 keys 143 -> 152 us, 2048 fresh among 48 of 2000 69 -> 81; with few of
-  // them 1300 fresh among 16 of 1000 47 -> 41).
-  at.pair = !SPLIT && !MIXED && BM == 256 && p.window == 0 && 128 % p.pack == 0 && total * gy <= 256;
+  // heads 6000 fresh 198 -> 172.  Beside more decodes than the same round has CUs for, those of short row blocks do not idle, and row blocks
+  // of one length leave the decodes to the end (2000 over 1500 among 63 of up to 4096 keys 143 -> 152 us, 2048 fresh among 48 of 2000
+  // 69 -> 81); up to that, 8 / 1 heads, 5000 fresh among 40 of 1000 138 -> 109, 2 x 3000 among 20 of 3000 87 -> 71.
+  const int decodes = !MIXED ? 0 : p.num_seqs > 64 ? p.num_seqs : (int)__popcll(__ballot(my.qlen == 1));
+  at.pair = !SPLIT && BM == 256 && p.window == 0 && 128 % p.pack == 0 && (total + decodes) * gy <= 256;
   // 1, 2 or 4 heads, several rounds: every XCD takes its share of a head's blocks one by one.  In runs the long ones meet on the
   // first XCDs (8 / 1 heads, 10000 fresh tokens 483 -> 277 us, 3 x 5000 231 -> 155; 16 / 4, 6000 229 -> 184).
   const bool few = !SPLIT && !at.pair && !over && (gy == 1 || gy == 2 || gy == 4);
@@ -225,7 +226,7 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
       // Short chunks over long contexts: the row blocks of the longest sequence first (24 chunks of 150 .. 250 over 1500 .. 3000 tokens,
       // three rounds of workgroups: 266 -> 257 us, the flash layout 260 -> 250; 19 prompts of 745 .. 1242 without context, whose
       // blocks differ more than the prompts, 294 -> 302: they keep the order below).
-      if (over && !MIXED) {
+      if (over && decodes == 0) {
         int before = 0;                        // blocks of longer sequences
         const uint32_t key = (uint32_t)my.len << 6 | (uint32_t)(63 - lane);   // (no two alike)
 #pragma unroll 4
