@@ -16,14 +16,20 @@ namespace fa {
 // (Tried, where the first of these took 148: two groups of four waves per workgroup 152; several kv heads per workgroup one after the
 // other, 160.)
 template <typename T, bool FP8>
-__global__ __launch_bounds__(512) void fa_mixed_kernel(const FaParams p, const UniDecodeParams u, int gx, int gy, int nfa, int npairs, int sub_shift, int order) {
+__global__ __launch_bounds__(512) void fa_mixed_kernel(const FaParams p, const UniDecodeParams u, int gx, int gy, int nfa, int npairs, int first, int early, int sub_shift, int order) {
   constexpr int DL = ua_decode_lds<FP8, 128, 8>(), LDS = DL > fa_lds<128>() ? DL : fa_lds<128>();
   __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS];
-  const int hw = blockIdx.x;
-  if (hw < nfa) {
-    if (hw < gx * gy) fa_body<T, FP8, false, 128, 8, false, false, true>(p, lds, hw, gy);
+  // the decodes `pair` < early come behind the first `first` row blocks, the others behind all of them
+  int id = blockIdx.x, pair = -1;
+  if (id >= first) {
+    if (id < first + early) pair = id - first;
+    else id -= early;
+  }
+  if (pair < 0 && id >= nfa) pair = id - nfa + early;
+  if (pair < 0) {
+    if (id < gx * gy) fa_body<T, FP8, false, 128, 8, false, false, true>(p, lds, id, gy);
   } else {
-    ua_decode_body<T, FP8, 128, 8, false, true>(u, (char*)lds, sub_shift, 0, order, hw - nfa, npairs, 0);
+    ua_decode_body<T, FP8, 128, 8, false, true>(u, (char*)lds, sub_shift, 0, order, pair, npairs, 0);
   }
 }
 
@@ -129,9 +135,14 @@ int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, co
       for (order = 1; order < 30 && u->max_seq_len > 0 && (u->max_seq_len >> order) != 0;) ++order;
   }
   const unsigned nfa = (grid.x * grid.y + 7) / 8 * 8;   // (the ids behind them go round-robin over the XCDs too)
+  // Fewer than 16 sequences have a decode with at least twice the longest chunk's keys here, if any: not behind all row blocks but
+  // behind the 24 of every XCD that start first (us, 32 / 8 heads, 2 x 1500 over 500 among 5 of 8000 99 -> 78, 3 x 1200 among one of
+  // 16000 127 -> 98, 2 x 4000 among 10 of 10000 252 -> 233; 16-bit 126 -> 88, 181 -> 155, 291 -> 238).  With more sequences the longest
+  // may be a chunk's context, and what starts late a row block: 64 / 8, 3 x 540 over 4000 among 40 of 2566 183 -> 200.
+  const int first = nfa < 8 * 24 ? (int)nfa : 8 * 24, early = p.num_seqs < 16 ? npairs / 8 * 8 : 0;
 #define FA_MIXED(T_, F_)                                                                                                  \
   hipLaunchKernelGGL((fa::fa_mixed_kernel<T_, F_>), dim3(nfa + (unsigned)npairs), dim3(512), 0, st, p, *u, (int)grid.x, \
-                     (int)grid.y, (int)nfa, npairs, sub_shift, order)
+                     (int)grid.y, (int)nfa, npairs, first, early, sub_shift, order)
 #define FA_LAUNCH___(T_, F_, P_, D_, NW_, S_)                                                                            \
   do {                                                                                                                   \
     if (p.num_segments > 1) hipLaunchKernelGGL((fa::fa_fwd_kernel<T_, F_, P_, D_, NW_, S_, true>), grid, dim3(64 * NW_), 0, st, p); \
