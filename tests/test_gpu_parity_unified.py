@@ -559,6 +559,17 @@ def test_unified_few_sequences_decodes_apart(oracle, heads, D, fp8, softcap):
         _lib.set_tuning("pf_segs", 0)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,D", [((8, 1), 128), ((16, 2), 64), ((8, 2), 256), ((24, 1), 80)])
+@pytest.mark.parametrize("window,out8", [(None, False), (700, False), (None, True)])
+def test_unified_decodes_cut_beside_segments(oracle, heads, D, fp8, window, out8):
+    """Few decodes beside a chunk whose keys are cut into segments: cut too, and merged by the chunk's merge; pieces without a key, of
+    one tile and one key more, chunks in front of and behind the decodes."""
+    seqs = [(40, 2300)] + [(1, (1, 63, 64, 65, 128, 129, 900, 2200, 1025)[i % 9]) for i in range(15)] + [(9, 30)]
+    c = make_unified_case(seqs, heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
+    run(oracle, c, torch.bfloat16, fp8=fp8, window=window, out_scale=torch.tensor([0.03]) if out8 else None)
+
+
 def test_unified_fa_kernel_sharp_rows(oracle, force_fa):
     """Rows whose maximum keeps growing along the keys (the lazy rescale must fire on some tiles and not on others):
     keys scaled up with their position."""

@@ -914,6 +914,15 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
     // them than for a chunk (us, head 64, 32 / 8, 2 x 1500 over 500 among 5 of 8000 213 -> 95, 2000 among 3 of 4000 105 -> 76; head 256,
     // 16 / 8, 312 -> 168, 164 -> 132), and not split (the segments spread the walk).
     const bool apart = beside && !one_launch && (mixed || (plan.nseg <= 1 && max_q >= 256 && max_k >= 2048));
+    // Beside chunks in segments, few decodes are cut like a batch of their own, and the chunks' merge takes theirs along (a merge of
+    // their own is 2 us where they turn out short).  us, 8 / 1 heads, 500 among 20 of 8000 69 -> 35, 3 x 1000 among 30 of 10605 127 -> 72,
+    // 16-bit 1000 over 2000 among 40 of 4000 76 -> 53, 600 over 1000 among 16 of 5105 76 -> 39; 500 over 8000 among 30 of 200, short
+    // decodes, 51.4 -> 51.1.  Not more of them, which fill the chip, nor fewer keys.
+    if (apart && can && plan.use && plan.nseg > 1 && max_k >= 2048 && unified_decode_pairs(u) <= 64) {
+      u.num_segments = unified_decode_segments(u, plan.nseg);
+      u.segm_stride = plan.nseg;
+      u.merge = false;
+    }
     p.skip_decode = one_launch || apart;
     if (apart) {
       const int rc = unified_decode(u);
@@ -934,6 +943,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       f.window = p.sliding_window; f.softcap = p.softcap;
       f.prefix = 0; f.k_new = f.v_new = nullptr; f.k_stride_t = f.k_stride_h = f.v_stride_t = f.v_stride_h = 0;
       f.blocks_per_seq = 0;
+      f.decode_segments = apart ? u.num_segments : 1;
       f.num_segments = plan.nseg; f.seg_slots = plan.seg_slots; f.segm_out = p.segm_out; f.segm_max = p.segm_max; f.segm_sum = p.segm_sum;
       f.stagger = g_pf_fa_stagger;
       return launch_unified_fa(f, std::is_same<T, f16_t>::value ? VLLM_AMD_F16 : VLLM_AMD_BF16, FP8, st, one_launch ? &u : nullptr);

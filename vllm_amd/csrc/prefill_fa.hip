@@ -64,13 +64,20 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
   float ms = lane < nseg ? p.segm_max[row + lane] : -INFINITY;
   float ls = lane < nseg ? p.segm_sum[row + lane] : 0.f;
   if (tok < p.cu_seqlens_q[0] || tok >= p.cu_seqlens_q[p.num_seqs]) return;
+  int live = -1;
   if (p.skip_decode) {
     const int lo = wave_last(p.num_seqs, lane, [&](int i) { return p.cu_seqlens_q[i] <= tok; });
-    if (p.cu_seqlens_q[lo + 1] - p.cu_seqlens_q[lo] == 1) return;   // the decode kernel's token
+    if (p.cu_seqlens_q[lo + 1] - p.cu_seqlens_q[lo] == 1) {           // the decode kernel's token
+      if (p.decode_segments <= 1) return;
+      const int tiles = (p.seq_lens[lo] + 63) >> 6, per = (tiles + p.decode_segments - 1) / p.decode_segments;
+      live = per > 0 ? (tiles + per - 1) / per : 0;
+    }
   }
-  const float last = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ls), nseg - 1));
-  const int live = last < 0.f ? (int)-last : nseg;
-  if (live == 1) return;             // the only segment has written the output
+  if (live < 0) {
+    const float last = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ls), nseg - 1));
+    live = last < 0.f ? (int)-last : nseg;
+    if (live == 1) return;             // the only segment has written the output
+  }
   if (lane >= live) { ms = -INFINITY; ls = 0.f; }
   const float mx = wave_max(ms);
   const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);

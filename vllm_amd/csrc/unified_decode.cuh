@@ -19,6 +19,7 @@ struct UniDecodeParams {
   // cdiv(cdiv(seq_len, 64), num_segments) -- the partition unified_reduce_kernel assumes
   float* segm_out; float* segm_max; float* segm_sum;
   int num_segments, segm_stride;
+  bool merge = true;     // false: the partials are left to fa_reduce_kernel (prefill_fa.hip)
   int num_tokens;        // rows of q, out and (times num_heads) of the segm_* buffers
   int dtype;             // VLLM_AMD_F16 / VLLM_AMD_BF16
   bool fp8;              // e4m3 cache

@@ -111,7 +111,7 @@ int launch(const UniDecodeParams& p) {
   else
     hipLaunchKernelGGL((ua_decode_kernel<T, FP8, D, NW, false>), grid, dim3(NW * 64), 0, p.stream, p, sub_shift, xcd_group, order);
   VA_LAUNCH_CHECK("unified_attention decode launch");
-  if (p.num_segments > 1) {
+  if (p.num_segments > 1 && p.merge) {
     const dim3 rgrid((unsigned)((p.num_seqs * p.num_heads + 3) / 4));
     if (p.num_segments <= 4) hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D, 4>), rgrid, dim3(256), 0, p.stream, p);
     else if (p.num_segments <= 8) hipLaunchKernelGGL((ua_decode_reduce_kernel<T, D, 8>), rgrid, dim3(256), 0, p.stream, p);
