@@ -299,7 +299,7 @@ using namespace va;
 // that fills the chip (1024 x 8192 -> 10240: 320 tiles of 128 x 128 in two rounds 127.6 us, 216 of 256 x 192 in one 74.0).  us of a launch:
 // c + rounds (a + b nb), nb = K / 128; the kernels whose workgroups share a CU in pairs: pairs of rounds, and a last odd one.  Fitted to 810
 // launches (18 weight shapes of K 1024 .. 16384, N 1280 .. 28672, M 65 .. 4096, weights from HBM, each kernel forced; 9 .. 13 % rms).
-// Taken where it is 5 % below the tile that the table below would take.  715 other launches: 93 of them change, to 0.62 .. 1.00 of
+// Taken where it is 5 % below the tile that the table below would take.  715 other launches: some 90 of them change, to 0.62 .. 1.00 of
 // the time (128 x 128 -> 256 x 192 0.76 on average, 128 x 64 -> 128 x 128 in one round 0.80, -> 64 x 64 0.83); profiles/gemm_rounds.txt.
 constexpr int kWide192 = 39;   // scaled_mm_pp.hip's 256 x 192 tiles
 struct TileCost { int sel, bm, bn; double c, a, b, a_odd, b_odd; };   // a_odd < 0: one workgroup per CU
@@ -329,8 +329,9 @@ static int scaled_mm_by_rounds(int sel, int M, int N, int K) {
   for (int i = 0; i < (int)(sizeof(kTileCost) / sizeof(kTileCost[0])); ++i) {
     const double us = tile_cost(kTileCost[i], M, N, K);
     if (kTileCost[i].sel == sel) own = us;
-    // (64 x 64 instead of 128 x 128 tiles: 0.996 of the time on average, up to 1.10)
-    const bool may = i < 4 || (i == 4 && (sel == 5 || sel == 6 || sel == 9 || sel == 10));
+    // (64 x 64 instead of 128 x 128 tiles: 0.996 of the time on average, up to 1.10; instead of 64 x 32 ones, of which up to 288 share
+    // their CUs: 6400 -> 1696 at M 303, 265 tiles, 14.7 -> 16.7 us, 7936 -> 2176 at M 220, 272 tiles, 18.7 -> 19.6; from 300 on 0.80 .. 0.96)
+    const bool may = i < 4 || (i == 4 && (sel == 5 || sel == 6 || sel == 10 || (sel == 9 && ceil_div(M, 64) * ceil_div(N, 32) > 288)));
     if (may && us < best) { best = us; pick = kTileCost[i].sel; }
   }
   return best < 0.95 * own ? pick : sel;
