@@ -219,13 +219,15 @@ def test_fp8_linear_new_equals_the_steps(ops, m):
 
 
 @pytest.mark.parametrize("max_len", [1025, 3000])
-def test_forward_decode_scratch_equals_v2(ops, max_len):
-    """forward_decode, whose scratch is one buffer inside the operator, against paged_attention_v2 with the caller's tensors."""
-    from vllm_amd.attention import PagedAttention
+def test_decode_scratch_equals_v2(ops, max_len):
+    """paged_attention_decode, whose scratch is one buffer inside the operator, against paged_attention_v2 with the caller's tensors."""
+    from vllm_amd import _torch_ops
     c = make_attn_case(3, 8, 2, 128, 16, torch.bfloat16, "fp8", [1, 700, max_len], seed=max_len, kv_scale=0.5)
     q, kc, vc, bt, sl = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt", "sl"))
     sc, parts = torch.tensor([0.5], device="cuda"), (max_len + 511) // 512
     out, es = torch.empty_like(q), torch.empty((3, 8, parts), device="cuda")
     ops.paged_attention_v2(out, es, torch.empty_like(es), torch.empty((3, 8, parts, 128), dtype=q.dtype, device="cuda"), q, kc, vc,
                            2, c["scale"], bt, sl, 16, max_len, None, "fp8", sc, sc)
-    assert torch.equal(PagedAttention.forward_decode(q, kc, vc, bt, sl, max_len, "fp8", 2, c["scale"], None, sc, sc), out)
+    got = torch.empty_like(q)
+    _torch_ops.paged_attention_decode(got, q, kc, vc, 2, c["scale"], bt, sl, 16, max_len, None, "fp8", sc, sc, 0, 0, 0, 64, 0)
+    assert torch.equal(got, out)
