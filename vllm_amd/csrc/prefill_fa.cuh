@@ -16,6 +16,7 @@ struct FaParams {
   int bs_shift;        // log2(block size)
   int skip_decode;     // sequences of query length 1 were taken by the decode kernel
   int decode_segments = 1;   // > 1: in that many pieces of whole 64-key tiles, which this launch's merge takes along (same stride)
+  int tpb = 0;         // tokens per row block (set by launch_unified_fa)
   int pack;            // q heads per tile-row group: the GQA group (rows = (token, head) pairs) or 1
   int64_t bt_stride, q_stride_t, q_stride_h, o_stride_t, o_stride_h;
   int64_t kc_block_bytes, kc_slot_bytes, kc_head_bytes, vc_block_bytes, vc_slot_bytes, vc_head_bytes;

@@ -126,9 +126,10 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
 
 int g_pf_fa_stagger = 1;   // tuning "pf_fa_stagger": 0 = all eight waves stage at the bottom of the interval
 std::atomic<int> g_pf_mixed_launches{0};   // get_tuning "pf_mixed_launches"
-int launch_unified_fa(const FaParams& p, int dtype, bool fp8, hipStream_t st, const UniDecodeParams* u) {
+int launch_unified_fa(const FaParams& given, int dtype, bool fp8, hipStream_t st, const UniDecodeParams* u) {
+  FaParams p = given;
   const bool wide = p.head_size > 128;                 // 128-row workgroups of four waves
-  const int tpb = (wide ? 128 : 256) / p.pack;
+  const int tpb = p.tpb = (wide ? 128 : 256) / p.pack;
   const unsigned gx = p.blocks_per_seq > 0 ? (unsigned)(p.blocks_per_seq * p.num_seqs) : (unsigned)(p.num_tokens / tpb + p.num_seqs);
   const unsigned gy = (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads);
   const unsigned slots = p.num_segments > 1 ? (unsigned)p.seg_slots : 0u;

@@ -132,7 +132,8 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
     return idx < q8 + (xcd < r8 ? 1 : 0) ? (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + idx : -1;
   };
   const int nseg = SPLIT ? p.num_segments : 1;
-  const int tpb = BM / p.pack;                // tokens per workgroup
+  const int tpb = p.tpb;                      // tokens per workgroup
+  const int tsh = (tpb & (tpb - 1)) == 0 ? __builtin_ctz(tpb) : -1;   // (a division here is 1 % of a short row block)
   FaAt at;
   at.seg = 0;
   at.segs = 1;
@@ -150,7 +151,7 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
       q.tok0 = p.cu_seqlens_q[i];
       q.qlen = p.cu_seqlens_q[i + 1] - q.tok0;
       q.len = p.seq_lens[i];
-      q.blocks = p.skip_decode && q.qlen == 1 ? 0 : (q.qlen + tpb - 1) / tpb;
+      q.blocks = p.skip_decode && q.qlen == 1 ? 0 : tsh >= 0 ? (q.qlen + tpb - 1) >> tsh : (q.qlen + tpb - 1) / tpb;
     }
     return q;
   };
@@ -308,7 +309,7 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   const FaAt at = fa_find<PREFIX, SPLIT, MIXED, BM>(p, lane, hw, gy);
   if (!at.some) return;
   const int nseg = SPLIT ? p.num_segments : 1;
-  const int pack = p.pack, tpb = BM / pack;   // tokens per workgroup
+  const int pack = p.pack, tpb = p.tpb;       // tokens per workgroup
   const int seq = at.seq, blk = at.blk, y = at.y, seg = at.seg, segs = at.segs, tok0 = at.tok0, qlen = at.qlen, seq_len = at.seq_len;
   const int ctx = seq_len - qlen;
   // first query token of this block
