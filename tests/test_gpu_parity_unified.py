@@ -843,6 +843,7 @@ def test_unified_row_blocks(oracle, force_fa, fp8, blocks):
     ((16, 4), 128, [(300 + i, 300 + i) for i in range(15)] + [(1, 9)]),                                 # 4 heads, 304 blocks, the last of one token
     ((8, 8), 128, [(1 + 17 * i % 290, 20 + 29 * i) for i in range(36)]),                                # whole heads per XCD, short and long contexts
     ((16, 8), 256, [(3 + 40 * (i % 6), 3 + 40 * (i % 6)) for i in range(14)]),                          # 128-row blocks
+    ((128, 8), 128, [(530, 530), (512, 512)]),                                                          # two prompts, 528 blocks
 ])
 def test_unified_row_block_order(oracle, force_fa, fp8, heads, D, seqs):
     """More than one round of row blocks: in the order of their last keys, in shares per XCD for few heads; every block once."""

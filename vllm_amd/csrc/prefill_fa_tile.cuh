@@ -202,8 +202,11 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
       // 128, whose tiles take too little time for keys from farther than the L2 (us: 8 x 300 .. 500 over 250 .. 500 70 -> 66, 5 x 540 ..
       // 900 fresh 61 -> 57, head 256 5 x 550 .. 917 fresh 76 -> 68, 3 x 1200 .. 2000 143 -> 132; but 19 x 745 .. 1242 fresh 284 -> 292, 6 x
       // 600 .. 1000 over 500 .. 1000 141 -> 143, 16 x 180 .. 300 over 750 .. 1500 134 -> 143, 19 x 138 .. 230 fresh, 520 blocks, 43 -> 46,
-      // 8 x 403 .. 671 over 198 .. 395, 568 blocks, 86 -> 91, 20 x 56 .. 93 fresh, 280 blocks, 26.4 -> 28.5).
-      if (128 % p.pack == 0 && (few || (!over && (BM == 128 || (total * gy <= 512 && (int)__popcll(chunks) <= 16))))) {
+      // 8 x 403 .. 671 over 198 .. 395, 568 blocks, 86 -> 91, 20 x 56 .. 93 fresh, 280 blocks, 26.4 -> 28.5).  And two prompts without a
+      // context at any length (3600 + 6000 429 -> 420, 3001 + 5003 317 -> 312; three of 3000 194 : 195, two of 4000 over 1500 331 -> 340).
+      const int n = (int)__popcll(chunks);
+      const bool in_order = BM == 128 || (total * gy <= 512 ? n <= 16 : n == 2 && __ballot(my.blocks > 0 && my.len > my.qlen) == 0);
+      if (128 % p.pack == 0 && (few || (!over && in_order))) {
         const int sh = __builtin_ctz(tpb), ctx = my.len - my.qlen;
         const int top = wave_max_i(my.blocks > 0 ? ctx + (my.blocks << sh) : 0), low = -wave_max_i(my.blocks > 0 ? -ctx : -top);
         const int step = ((top - low) >> 6) + 1;
