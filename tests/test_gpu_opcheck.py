@@ -231,3 +231,39 @@ def test_decode_scratch_equals_v2(ops, max_len):
     got = torch.empty_like(q)
     _torch_ops.paged_attention_decode(got, q, kc, vc, 2, c["scale"], bt, sl, 16, max_len, None, "fp8", sc, sc, 0, 0, 0, 64, 0)
     assert torch.equal(got, out)
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+def test_decode_two_partitions_equals_v2(ops, kv):
+    """Two partitions, as forward_decode sends them: cut in two pieces over a 16-bit cache (scratch inside), one piece over an fp8 one."""
+    from vllm_amd import _lib
+    from vllm_amd.attention import PagedAttention
+    lens = [1000, 513, 1, 700, 512, 1024, 64, 900]
+    c = make_attn_case(8, 32, 8, 128, 16, torch.bfloat16, kv, lens, seed=8, kv_scale=0.5 if kv == "fp8" else 1.0)
+    q, kc, vc, bt, sl = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt", "sl"))
+    sc = torch.tensor([0.5 if kv == "fp8" else 1.0], device="cuda")
+    code = _lib.KV_FP8_E4M3 if kv == "fp8" else _lib.KV_AUTO
+    pieces = _lib.lib.vllm_amd_paged_attention_v2_pieces(q.data_ptr(), q.data_ptr(), 8, 32, 128, 8, 16, 1024, 2, _lib.BF16, code,
+                                                         q.stride(0), kc.stride(1), 0)
+    assert pieces == (1 if kv == "fp8" else 2)
+    out, es = torch.empty_like(q), torch.empty((8, 32, 2), device="cuda")
+    ops.paged_attention_v2(out, es, torch.empty_like(es), torch.empty((8, 32, 2, 128), dtype=q.dtype, device="cuda"), q, kc, vc,
+                           8, c["scale"], bt, sl, 16, 1024, None, kv, sc, sc)
+    assert torch.equal(PagedAttention.forward_decode(q, kc, vc, bt, sl, 1024, kv, 8, c["scale"], None, sc, sc), out)
+
+
+@pytest.mark.parametrize("n,max_len,takes", [(20, 1100, 0), (8, 1600, 1)])
+def test_decode_one_piece_takes_no_scratch(ops, n, max_len, takes):
+    """The operator itself over three and more partitions: in one piece without an allocation, cut with one."""
+    from vllm_amd import _torch_ops
+    c = make_attn_case(n, 32, 8, 128, 16, torch.bfloat16, "fp8", [max_len - 40 * i for i in range(n)], seed=n, kv_scale=0.5)
+    q, kc, vc, bt, sl = (to_dev(c[k]) for k in ("q", "kc", "vc", "bt", "sl"))
+    sc, parts, got = torch.tensor([0.5], device="cuda"), (max_len + 511) // 512, torch.empty_like(q)
+    out, es = torch.empty_like(q), torch.empty((n, 32, parts), device="cuda")
+    ops.paged_attention_v2(out, es, torch.empty_like(es), torch.empty((n, 32, parts, 128), dtype=q.dtype, device="cuda"), q, kc, vc,
+                           8, c["scale"], bt, sl, 16, max_len, None, "fp8", sc, sc)
+    made = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = made()
+    _torch_ops.paged_attention_decode(got, q, kc, vc, 8, c["scale"], bt, sl, 16, max_len, None, "fp8", sc, sc, 0, 0, 0, 64, 0)
+    assert made() - before == takes
+    assert torch.equal(got, out)

@@ -510,8 +510,8 @@ struct Segments {
   }
 };
 
-// vllm/attention/ops/paged_attn.py:131-193, two partitions: paged_attention_v1 where v2 would take every sequence in one piece,
-// which needs no scratch.  Else v2 with scratch of its own, maxima, sums and partial outputs in one buffer.
+// vllm/attention/ops/paged_attn.py:131-193: paged_attention_v1 where v2 would take every sequence in one piece, which needs no scratch,
+// else v2 with scratch of its own, maxima, sums and partial outputs in one buffer.  (forward_decode comes here with two partitions.)
 void paged_attention_decode(Tensor& out, const Tensor& query, const Tensor& key_cache, const Tensor& value_cache,
                             int64_t num_kv_heads, double scale, const Tensor& block_tables, const Tensor& seq_lens,
                             int64_t block_size, int64_t max_seq_len, const OptTensor& alibi_slopes,
@@ -520,8 +520,7 @@ void paged_attention_decode(Tensor& out, const Tensor& query, const Tensor& key_
                             int64_t bs_head_sliding_step) {
   TORCH_CHECK(query.dim() == 3, "query.dim() == 3");
   const int64_t s = query.size(0), h = query.size(1), d = query.size(2), parts = (max_seq_len + 511) / 512;
-  if (parts >= 1 && parts <= 2 &&
-      vllm_amd_paged_attention_v2_pieces(out.data_ptr(), query.data_ptr(), (int)s, (int)h, (int)d, (int)num_kv_heads, (int)block_size,
+  if (vllm_amd_paged_attention_v2_pieces(out.data_ptr(), query.data_ptr(), (int)s, (int)h, (int)d, (int)num_kv_heads, (int)block_size,
                                          (int)max_seq_len, (int)parts, dt(query), kv(kv_cache_dtype), query.stride(0),
                                          key_cache.stride(1), (int)bs_vert_stride) == 1) {
     paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size, max_seq_len,
