@@ -216,6 +216,12 @@ int vllm_amd_scaled_mm(void* out, const void* a, const void* b,
                        int64_t ldb, int64_t ldc, int a_scale_numel,
                        int b_scale_numel, int out_dtype, void* stream);
 
+/* The kernel that vllm_amd_scaled_mm takes for such sizes where no tuning key forces one and the output rows are 16-byte aligned (N
+ * and ldc multiples of 8): its "mm_kernel" number, 39 = 256 x 192 tiles of scaled_mm_pp.hip, 3700 + 10 r + c = the weight stream with the rows
+ * in groups, 16 r rows x 16 c columns a workgroup, 1000 more = in two K slices (workspace: whether there is one for them); 0 = one of
+ * the others.  Host arithmetic only. */
+int vllm_amd_scaled_mm_kernel(int M, int N, int K, int workspace);
+
 /* No counterpart in the reference (its libraries own their workspaces): registers (ws != NULL)
  * or removes (ws == NULL) the CURRENT device's workspace -- `bytes` of caller-owned device
  * memory, 256-byte aligned, valid until replaced or removed; at least 513 KiB, sized for full use

@@ -451,3 +451,17 @@ def test_scaled_mm_row_groups(ops, M, N, K, out_dtype):
     out = ops.cutlass_scaled_mm(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn).t(), sa, sb, out_dtype, bias)
     ref = ((a @ w.t()) * sa * sb.view(1, -1)).to(out_dtype) + bias
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("M,N,K,rows,cols", [
+    (17, 1280, 256, 16, 16), (48, 1272, 384, 16, 16), (64, 1024, 4096, 16, 16),
+    (33, 2560, 1408, 16, 32), (40, 2552, 1280, 16, 32), (47, 2560, 15360, 16, 32), (65, 1360, 1024, 16, 32),
+    (49, 1280, 256, 32, 16), (255, 512, 1024, 32, 16),
+    (145, 1024, 1152, 48, 16), (100, 1280, 1024, 48, 16),
+    (52, 4096, 2048, 32, 32), (112, 2048, 1024, 32, 32), (56, 4088, 14336, 32, 32), (256, 1016, 1024, 32, 32),
+])
+def test_scaled_mm_row_groups_taken(ops, M, N, K, rows, cols):
+    """The same, sizes of which the rule says that they take each form, up to a last group of one row."""
+    from vllm_amd._lib import lib
+    assert lib.vllm_amd_scaled_mm_kernel(M, N, K, 0) == 3700 + 10 * (rows // 16) + cols // 16
+    test_scaled_mm_row_groups(ops, M, N, K, torch.bfloat16)

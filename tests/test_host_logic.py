@@ -103,6 +103,35 @@ def test_paged_attention_v2_pieces():
     assert pieces(L=8000, P=16) > 1
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (32, 1280, 8192, 3711), (64, 1024, 4096, 3711), (40, 1248, 15360, 3711), (64, 2048, 8192, 3721), (40, 2480, 1536, 3712),
+    (94, 1280, 8192, 3721), (84, 2048, 16384, 3731), (63, 4096, 4096, 3722), (150, 1280, 1152, 3722), (138, 1296, 1024, 3722),
+    # 32 columns over a short K: all rows in one workgroup
+    (39, 2560, 1024, 37), (48, 2144, 1152, 37), (48, 2144, 1280, 3712), (50, 3504, 512, 37), (56, 3280, 1920, 37), (56, 3280, 2048, 3722),
+    # a nearly empty last group over a long one
+    (33, 2192, 14336, 37), (35, 2192, 14336, 37), (36, 2192, 14336, 3712), (36, 2560, 20480, 37), (37, 2560, 20480, 3712),
+    (33, 2240, 8192, 3712), (33, 2192, 13312, 3712), (53, 4096, 15360, 37), (55, 3584, 20480, 37), (56, 3584, 20480, 3722), (54, 3888, 14336, 3722),
+    (53, 4096, 10240, 3722), (49, 2560, 15360, 3722), (66, 2560, 16384, 3722), (66, 2192, 20480, 10), (83, 2192, 20480, 10), (84, 2192, 20480, 3722),
+    # ... and beside tile kernels with four K blocks per barrier
+    (91, 2560, 3584, 10), (91, 2560, 3456, 3722), (91, 2560, 4096, 3722), (100, 2048, 1024, 3722), (91, 2048, 1536, 3731),
+    # one group, more rounds than one, too many columns
+    (16, 1280, 8192, 37), (32, 4096, 4096, 37), (48, 4096, 4096, 37), (48, 6144, 4096, 37), (60, 4160, 4096, 37),
+])
+def test_scaled_mm_row_groups_rule(M, N, K, kernel):
+    """The rows of the weight stream in groups: 3700 + 10 (rows / 16) + columns / 16 of a workgroup, 37 in one."""
+    from vllm_amd._lib import lib
+    assert lib.vllm_amd_scaled_mm_kernel(M, N, K, 0) == kernel
+
+
+def test_scaled_mm_two_slices_rule():
+    """Two K slices (1000 + tile) instead of the weight stream where there is a workspace, not instead of small groups of rows."""
+    from vllm_amd._lib import lib
+    k = lib.vllm_amd_scaled_mm_kernel
+    assert k(48, 4096, 14336, 1) == 1010 and k(48, 4096, 14336, 0) == 37 and k(32, 4096, 14336, 1) == 37
+    assert k(40, 1248, 15360, 1) == 3711 and k(44, 2192, 14336, 1) == 3712 and k(60, 2560, 14336, 1) == 1010 and k(60, 2560, 14336, 0) == 3722
+    assert k(100, 512, 12288, 1) == 3711 and k(0, 512, 1024, 1) == k(8, 512, 128, 1) == k(8, 516, 1024, 1) == 0
+
+
 def test_shard_helpers():
     from vllm_amd.distributed import shard_kv_heads, shard_range
     assert shard_range(8192, 8, 3) == (3072, 4096)

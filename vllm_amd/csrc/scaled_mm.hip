@@ -275,7 +275,8 @@ bool scaled_mm_large_fits(int M, int N, int K, int64_t lda, int64_t ldb);
 bool scaled_mm_large_can_split(int M, int N, int bm, int bn, int splits, int ws_mode, hipStream_t st);
 // scaled_mm_stream.hip
 bool scaled_mm_stream_pays(int M, int N, int K);
-bool scaled_mm_stream_small(int M, int N);
+int scaled_mm_stream_groups(int M, int N, int K);
+bool scaled_mm_stream_small(int M, int N, int K);
 int launch_scaled_mm_stream(void* out, const void* a, const void* b, const float* a_scales, const float* b_scales,
                             const void* bias, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int asn, int bsn,
                             int out_dtype, hipStream_t st);
@@ -337,6 +338,59 @@ static int scaled_mm_by_rounds(int sel, int M, int N, int K) {
   return best < 0.95 * own ? pick : sel;
 }
 
+// Two K slices of the 64 x 32 tile instead of the weight stream: where the activations that every workgroup of that reads (M x K bytes)
+// pass 600 KB and N is small, not so that groups of rows help.  N 4096, stream / slices in us, K 14336 at M 33 16.7 / 17.6, M 48 19.5 /
+// 19.0, M 64 21.9 / 20.3; K 28672 at M 17 25.7 / 26.8, M 32 29.0 / 28.2, M 64 39.8 / 33.9 (profiles/gemm_stream.txt).
+static bool scaled_mm_slices_pay(int M, int N, int K) {
+  return K >= 12288 && ceil_div(N, 32) <= 128 && M <= 64 && M * K > 600000 && !scaled_mm_stream_small(M, N, K);
+}
+
+// The tile kernel of a launch that takes one ("mm_kernel" numbers; kWide192).  forced: "mm_kernel" asks for none of the others;
+// may_split: the number of K slices (`splits`, set to 2 where they pay) is open.
+static int scaled_mm_tile(int M, int N, int K, bool vec16, bool forced, bool may_split, int& splits) {
+  // a single round of 128 x 128 tiles: scaled_mm_kgroup.hip ("mm_kernel" 38 forces it)
+  int sel = !forced && may_split && vec16 && scaled_mm_kgroup_pays(M, N, K) ? 38 : 0;
+  if (sel == 0) {
+    // Largest tile that still yields ~3/4 of a full wave of workgroups (256 CUs); rows of
+    // a tile beyond M are wasted MFMA work, so BM <= 2 M.  With more than one wave of tiles the
+    // variant that fits several workgroups per CU wins, below that the variant that takes
+    // KB K-blocks per barrier (measured: tools/sweep_gemm.py, profiles/r01_gemm_sweep.csv).
+    struct GldsTile { int id, id_kb, bm, bn, kb; };
+    static const GldsTile tiles_tab[5] = {{2, 2, 256, 256, 1}, {3, 4, 128, 128, 2},
+                                          {5, 6, 128, 64, 2},  {7, 8, 64, 64, 4},
+                                          {9, 10, 64, 32, 4}};
+    for (int i = 0; i < 5; ++i) {
+      const GldsTile& t = tiles_tab[i];
+      if (i < 4 && t.bm > 64 && M <= t.bm / 2) continue;
+      const int nt = ceil_div(M, t.bm) * ceil_div(N, t.bn);
+      // (128 x 64 tiles of few rows already from 160 on: 4096 x 10240 at M 96 19.8 -> 17.7 us, 8192 x 5120 at M 256 36.0 ->
+      // 29.5; not where a quarter of the rows is padding, M 160 12.3 -> 13.7, nor above, 8192 x 2048 at M 640 25.2 -> 26.1)
+      const int enough = i == 2 && M <= 256 && (M <= 128 || M > 192) ? 160 : 190;
+      if (nt >= enough || i == 4) {
+        // (the 64 x 64 tile with 4 K blocks per barrier loses on long K loops: 14336 x 4096 at
+        // M 192 / 256 31.1 vs 25.3 / 27.5 us, 8192 x 4096 18.2 / 19.0 vs 16.0 / 16.6 us; at K 4096
+        // it wins, 8.5 vs 9.1 us -- profiles/r02_gemm_sweep_mid.csv)
+        // (more than one round of tiles: the variant that fits two workgroups per CU -- 4096 x 6144
+        // at M 768 = 288 tiles of 128 x 128: 38.6 -> 30.2 us, at M 384 = 288 tiles of 128 x 64: 24.4 ->
+        // 20.6 us)
+        // (weights streamed from HBM as in a model -- bench.py rotates them now,
+        // profiles/r03_gemm_sweep_rotating.csv: the 64 x 64 tile with one K block per barrier wins at
+        // every K: 4096 x 4096 at M 256 12.7 vs 15.2 us, 4096 x 6144 at M 128 13.4 vs 15.9 us)
+        sel = (nt > 256 || K % (128 * t.kb) != 0 || i == 3) ? t.id : t.id_kb;
+        // Even the smallest tile leaves half the CUs idle and the K loop is long: two K slices (in-kernel fix-up,
+        // scaled_mm_large.hip).  The fix-up is a chain of three device-scope round trips (~2.5 us), so it pays only
+        // here.  (M <= 64 comes this far for it only, see the stream kernel above.)  M 65 .. 128, N 512 .. 2048, unsplit -> two
+        // slices: K 12288 16.1 .. 22.7 -> 13.2 .. 17.1 us, K 14336 18.2 .. 25.4 -> 14.4 .. 18.8, K 28672 33.5 .. 48.1 ->
+        // 22.1 .. 30.5 (profiles/gemm_two_slices.txt); at K 8192 0.99 .. 1.19 x, not taken.
+        if (i == 4 && nt <= 128 && K >= 12288 && may_split) splits = 2;
+        break;
+      }
+    }
+  }
+  if (!forced && may_split && splits == 1 && vec16 && M > 64) sel = scaled_mm_by_rounds(sel, M, N, K);
+  return sel;
+}
+
 static int launch_scaled_mm(void* out, const void* a, const void* b, const float* a_scales,
                             const float* b_scales, const void* bias, int M, int N, int K,
                             int64_t lda, int64_t ldb, int64_t ldc, int a_scale_numel,
@@ -356,12 +410,9 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
   const bool glds_ok = K % 128 == 0 && K >= 256 && scaled_mm_large_fits(M, N, K, lda, ldb);
   const int want_splits = req_splits > 0 ? req_splits : g_mm_splitk;   // 0 = heuristic
   const bool vec = (ldc % 4 == 0) && ((((uintptr_t)out) & 7) == 0);
-  // Few rows: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it up to M 64) -- but where the activations that
-  // every workgroup of it reads (M x K bytes) pass 600 KB and N is small, not so that groups of rows help, two K slices of the 64 x 32 tile (below) win if there
-  // is a workspace for them: N 4096, stream / slices in us, K 14336 at M 33 16.7 / 17.6, M 48 19.5 / 19.0, M 64 21.9 / 20.3;
-  // K 28672 at M 17 25.7 / 26.8, M 32 29.0 / 28.2, M 64 39.8 / 33.9 (profiles/gemm_stream.txt).
-  const bool slices = g_mm_kernel == 0 && want_splits == 0 && glds_ok && vec && K >= 12288 && ceil_div(N, 32) <= 128 &&
-                      M <= 64 && M * K > 600000 && !scaled_mm_stream_small(M, N) && scaled_mm_large_can_split(M, N, 64, 32, 2, ws_mode, st);
+  // Few rows: bound by the weight stream, scaled_mm_stream.hip ("mm_kernel" 37 forces it up to M 64)
+  const bool slices = g_mm_kernel == 0 && want_splits == 0 && glds_ok && vec && scaled_mm_slices_pay(M, N, K) &&
+                      scaled_mm_large_can_split(M, N, 64, 32, 2, ws_mode, st);
   if (glds_ok &&
       ((g_mm_kernel == 37 && M <= 64) || (g_mm_kernel == 0 && want_splits == 0 && !slices && scaled_mm_stream_pays(M, N, K)))) {
     launch_scaled_mm_stream(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel, out_dtype, st);
@@ -407,47 +458,8 @@ static int launch_scaled_mm(void* out, const void* a, const void* b, const float
     // 16-byte row-contiguous stores
     const bool vec16 = ldc % 8 == 0 && N % 8 == 0 && (((uintptr_t)out) & 15) == 0;
     const bool chosen = sel != 0;
-    // a single round of 128 x 128 tiles: scaled_mm_kgroup.hip ("mm_kernel" 38 forces it)
-    if (sel == 0 && want_splits == 0 && vec16 && scaled_mm_kgroup_pays(M, N, K)) sel = 38;
     if (sel == 38 && !vec16) sel = 0;
-    if (sel == 0 || sel == 11 || (sel > 36 && sel != 38)) {
-      // Largest tile that still yields ~3/4 of a full wave of workgroups (256 CUs); rows of
-      // a tile beyond M are wasted MFMA work, so BM <= 2 M.  With more than one wave of tiles the
-      // variant that fits several workgroups per CU wins, below that the variant that takes
-      // KB K-blocks per barrier (measured: tools/sweep_gemm.py, profiles/r01_gemm_sweep.csv).
-      struct GldsTile { int id, id_kb, bm, bn, kb; };
-      static const GldsTile tiles_tab[5] = {{2, 2, 256, 256, 1}, {3, 4, 128, 128, 2},
-                                            {5, 6, 128, 64, 2},  {7, 8, 64, 64, 4},
-                                            {9, 10, 64, 32, 4}};
-      for (int i = 0; i < 5; ++i) {
-        const GldsTile& t = tiles_tab[i];
-        if (i < 4 && t.bm > 64 && M <= t.bm / 2) continue;
-        const int nt = ceil_div(M, t.bm) * ceil_div(N, t.bn);
-        // (128 x 64 tiles of few rows already from 160 on: 4096 x 10240 at M 96 19.8 -> 17.7 us, 8192 x 5120 at M 256 36.0 ->
-        // 29.5; not where a quarter of the rows is padding, M 160 12.3 -> 13.7, nor above, 8192 x 2048 at M 640 25.2 -> 26.1)
-        const int enough = i == 2 && M <= 256 && (M <= 128 || M > 192) ? 160 : 190;
-        if (nt >= enough || i == 4) {
-          // (the 64 x 64 tile with 4 K blocks per barrier loses on long K loops: 14336 x 4096 at
-          // M 192 / 256 31.1 vs 25.3 / 27.5 us, 8192 x 4096 18.2 / 19.0 vs 16.0 / 16.6 us; at K 4096
-          // it wins, 8.5 vs 9.1 us -- profiles/r02_gemm_sweep_mid.csv)
-          // (more than one round of tiles: the variant that fits two workgroups per CU -- 4096 x 6144
-          // at M 768 = 288 tiles of 128 x 128: 38.6 -> 30.2 us, at M 384 = 288 tiles of 128 x 64: 24.4 ->
-          // 20.6 us)
-          // (weights streamed from HBM as in a model -- bench.py rotates them now,
-          // profiles/r03_gemm_sweep_rotating.csv: the 64 x 64 tile with one K block per barrier wins at
-          // every K: 4096 x 4096 at M 256 12.7 vs 15.2 us, 4096 x 6144 at M 128 13.4 vs 15.9 us)
-          sel = (nt > 256 || K % (128 * t.kb) != 0 || i == 3) ? t.id : t.id_kb;
-          // Even the smallest tile leaves half the CUs idle and the K loop is long: two K slices (in-kernel fix-up,
-          // scaled_mm_large.hip).  The fix-up is a chain of three device-scope round trips (~2.5 us), so it pays only
-          // here.  (M <= 64 comes this far for it only, see the stream kernel above.)  M 65 .. 128, N 512 .. 2048, unsplit -> two
-          // slices: K 12288 16.1 .. 22.7 -> 13.2 .. 17.1 us, K 14336 18.2 .. 25.4 -> 14.4 .. 18.8, K 28672 33.5 .. 48.1 ->
-          // 22.1 .. 30.5 (profiles/gemm_two_slices.txt); at K 8192 0.99 .. 1.19 x, not taken.
-          if (i == 4 && nt <= 128 && K >= 12288 && want_splits == 0) splits = 2;
-          break;
-        }
-      }
-    }
-    if (!chosen && want_splits == 0 && splits == 1 && vec16 && M > 64) sel = scaled_mm_by_rounds(sel, M, N, K);
+    if (sel == 0 || sel == 11 || (sel > 36 && sel != 38)) sel = scaled_mm_tile(M, N, K, vec16, chosen, want_splits == 0, splits);
     if (sel == 38) {
       launch_scaled_mm_kgroup(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc, a_scale_numel, b_scale_numel,
                               out_dtype, st);
@@ -492,6 +504,19 @@ extern "C" int vllm_amd_scaled_mm(void* out, const void* a, const void* b, const
   return launch_scaled_mm(out, a, b, a_scales, b_scales, bias, M, N, K, lda, ldb, ldc,
                           a_scale_numel, b_scale_numel, out_dtype, (hipStream_t)stream,
                           "scaled_mm");
+}
+
+// The kernel that such a call takes where nothing is forced and the output rows are 16-byte aligned: no device, no launch.
+extern "C" int vllm_amd_scaled_mm_kernel(int M, int N, int K, int workspace) {
+  if (M <= 0 || N <= 0 || K < 256 || K % 128 != 0 || N % 8 != 0) return 0;
+  const bool slices = workspace && scaled_mm_slices_pay(M, N, K);
+  if (!slices && scaled_mm_stream_pays(M, N, K)) {
+    const int groups = scaled_mm_stream_groups(M, N, K);
+    return groups > 0 ? 3700 + groups : 37;
+  }
+  int splits = 1;
+  const int sel = scaled_mm_tile(M, N, K, true, false, true, splits);
+  return workspace && splits == 2 ? 1000 + sel : sel;
 }
 
 // The variant of vllm_amd_scaled_mm for callers that cannot allocate or register memory: split-K

@@ -306,27 +306,42 @@ __global__ __launch_bounds__(64 * NW) void scaled_mm_stream_kernel(const Params 
   if constexpr (RES) wait_vm<0>();   // T < D: loads that no step waited for have landed before the LDS is given back
 }
 
-// Row groups: N up to 4096 has at most 256 column tiles of 16, and a workgroup pulls 128 (16 MT + 16 NT) bytes per K block at the same
-// ~90 GB/s whatever its neighbours do.  So the smallest MT + NT with which all rows still make one round of workgroups: the weights go
-// to several of them, through L2, and the activations to none twice.  us, all rows in one workgroup (M > 64: the tile kernels) ->
-// groups: 8192 -> 1280 at M 32 9.3 -> 7.2, M 63 12.3 -> 9.1, M 94 12.0 -> 9.3; 15360 -> 1248 at M 40 18.4 -> 11.0, M 81 20.4 -> 14.7;
-// 4096 -> 1024 at M 64 7.7 -> 5.1; 8192 -> 2048 at M 64 12.6 -> 9.5; 4096 -> 4096 at M 63 8.2 -> 8.1; of 849 launches with N up to 4096
-// and M 9 .. 330 the 340 that it takes 0.78 (profiles/gemm_row_groups.txt).  A second round costs more than it spreads: 8192 -> 1280 at
-// M 49 as 320 workgroups of 16 rows 10.4, as 160 of 32 8.7; and a round is 32 workgroups on each XCD, in whole column tiles: 12672 ->
-// 2624 at M 44 as 82 x 3, 33 on two of them, 17.0 -> 24.7.  32 rows x 32 columns only above M 48 (48 rows x 16 in one group there: 0.94 of it).
+// Row groups: N up to 4096 has at most 256 column tiles of 16, and a workgroup that pulls 128 (16 MT + 16 NT) bytes per K block gets
+// 70 GB/s of them while half the CUs are idle, 55 (16 x 16) .. 49 (32 x 32) in a full round.  So the smallest MT + NT with which all rows
+// still make one round of workgroups: the weights go to several of them, through L2, and the activations to none twice.  us, all rows in
+// one workgroup (M > 64: the tile kernels) -> groups: 8192 -> 1280 at M 32 9.3 -> 7.2, M 63 12.3 -> 9.1, M 94 12.0 -> 9.3; 15360 -> 1248
+// at M 40 18.4 -> 11.0, M 81 20.4 -> 14.7; 4096 -> 1024 at M 64 7.7 -> 5.1; 8192 -> 2048 at M 64 12.6 -> 9.5; 4096 -> 4096 at M 63 8.2 ->
+// 8.1; of 849 launches with N up to 4096 and M 9 .. 330 the 340 that it takes 0.78 (profiles/gemm_row_groups.txt).  A second round costs
+// more than it spreads: 8192 -> 1280 at M 49 as 320 workgroups of 16 rows 10.4, as 160 of 32 8.7; and a round is 32 workgroups on each XCD,
+// in whole column tiles: 12672 -> 2624 at M 44 as 82 x 3, 33 on two of them, 17.0 -> 24.7.  32 rows x 32 columns only above M 48 (48 rows x
+// 16 in one group there: 0.94 of it).
+// 32 columns pull no less than all rows in one workgroup do, only with more of them: up to M 64 that takes K 1280 (16 rows; 1024 -> 2560 at
+// M 40 4.2 -> 4.4, 1536 -> 2192 at M 44 4.8 -> 4.6) or 2048 (32 rows; 512 -> 3504 at M 50 3.9 -> 4.2, 1280 -> 3280 at M 56 5.0 -> 5.2,
+// 2048 -> 4096 at M 64 6.3 -> 5.7).  The tile kernels above it, which three groups of 32 rows stand against, take four K blocks per barrier
+// where K is a multiple of 512, and are ahead up to K 4096 (1536 -> 2560 at M 88 4.8 -> 5.2, 3584 -> 2560 at M 91 7.0 -> 7.6; 1280 -> 2560 at
+// M 78 5.0 -> 4.8, 8192 -> 2560 at M 83 12.7 -> 11.4).  Over a long K the activations of a nearly empty last group cost more than it takes
+// off the others: 16 rows from K 14336 on want K / 4096 in it (14336 -> 2192 at M 33 16.4 -> 17.6, 15616 -> 2192 at M 34 18.3 -> 18.9, M 36
+// 18.1 -> 16.8), two groups of 32 rows 24 where a full round reads most (15360 -> 4096 at M 53 25.2 -> 26.4, M 62 24.8 -> 23.2; 20480 -> 3584 at
+// M 49 30.7 -> 33.4; 14336 -> 3888 at M 54 22.7 -> 21.1) and three of them from K 20480 on 20 (20480 -> 2560 at M 75 27.9 -> 30.9, M 80 28.6 ->
+// 29.8, M 91 29.9 -> 28.0; 16384 -> 2192 at M 65 22.0 -> 20.6).
 // mt = 0: all rows in one workgroup.
 struct Rows { int mt, nt; };
-static Rows stream_rows(int M, int N) {
+static Rows stream_rows(int M, int N, int K) {
   if (M <= 16 || N > 4096) return {0, 0};
   auto wgs = [&](int mt, int nt) { return (int64_t)ceil_div(ceil_div(N, 16 * nt), 8) * 8 * ceil_div(M, 16 * mt); };
+  auto last = [&](int mt) { return (M - 1) % (16 * mt) + 1; };   // rows of the last group
+  // (32 columns do not pay)
+  const bool no12 = (M <= 64 && K < 1280) || (M <= 48 && K >= 14336 && last(1) * 4096 < K);
+  const bool no22 = M <= 64 ? K < 2048 || ((int64_t)ceil_div(N, 32) * 2 * K > 3600000 && last(2) < 24)
+                           : M <= 96 && wgs(2, 2) > 200 && ((K < 4096 && K % 512 == 0) || (K >= 20480 && last(2) < 20));
   if (wgs(1, 1) <= 256) return {1, 1};
   if (M <= 32) return {0, 0};
   if (wgs(2, 1) <= 256) return {2, 1};
-  if (wgs(1, 2) <= 256) return {1, 2};
+  if (wgs(1, 2) <= 256) return no12 ? Rows{0, 0} : Rows{1, 2};
   if (M <= 48) return {0, 0};
-  if (wgs(2, 2) <= 256 && wgs(2, 2) >= wgs(3, 1)) return {2, 2};
+  if (wgs(2, 2) <= 256 && wgs(2, 2) >= wgs(3, 1)) return no22 ? Rows{0, 0} : Rows{2, 2};
   if (wgs(3, 1) <= 256) return {3, 1};
-  if (wgs(2, 2) <= 256) return {2, 2};
+  if (wgs(2, 2) <= 256) return no22 ? Rows{0, 0} : Rows{2, 2};
   return {0, 0};
 }
 
@@ -348,7 +363,7 @@ static void launch(const Params& p0, hipStream_t st) {
     hipLaunchKernelGGL((scaled_mm_stream_kernel<out_t, MT, NT, NW, D, 0, true>), dim3(ceil_div(p.ntiles, 8) * 8 * p.groups), \
                        dim3(64 * NW), 0, st, p);                                                              \
   } while (0)
-  const Rows rows = stream_rows(p.M, p.N);
+  const Rows rows = stream_rows(p.M, p.N, p.K);
   if (rows.mt > 0) {
     if (rows.mt == 1 && rows.nt == 1) VA_STREAM_ROWS(1, 1, 4, 3);
     else if (rows.mt == 2 && rows.nt == 1) VA_STREAM_ROWS(2, 1, 4, 2);
@@ -392,16 +407,22 @@ static void launch(const Params& p0, hipStream_t st) {
 // 4096 -> 6144 (10.4 : 10.3) and 3584 -> 8192 (9.8 : 10.1) at M 64, and more than 256 tiles over K above 4096 (8192 -> 14336 at
 // M 49, 64 27.9, 28.9 : 28.2, 30.9; not at M 33, 27.6 : 25.2).
 bool scaled_mm_stream_pays(int M, int N, int K) {
-  if (M > 64) return K >= 1024 && mms::stream_rows(M, N).mt > 0;
+  if (M > 64) return K >= 1024 && mms::stream_rows(M, N, K).mt > 0;
   const int t32 = ceil_div(N, 32), t64 = ceil_div(N, 64);
   if (t32 > 256 && (K < 3072 || (M > 32 && K < 4096 && t64 >= 190 && t64 <= 256))) return false;
   if (M <= 32 || t32 < 160) return true;
   return K <= 4096 ? K >= 3072 && (M <= 48 || t32 > 256) : t32 <= 256;
 }
 
+// 16 x rows and columns of a workgroup where the rows go in groups, 10 mt + nt; 0 where a workgroup takes all of them.
+int scaled_mm_stream_groups(int M, int N, int K) {
+  const mms::Rows r = mms::stream_rows(M, N, K);
+  return 10 * r.mt + r.nt;
+}
+
 // The groups of rows are so small that nothing the tile kernels have for these shapes comes near, K slices included.
-bool scaled_mm_stream_small(int M, int N) {
-  const mms::Rows r = mms::stream_rows(M, N);
+bool scaled_mm_stream_small(int M, int N, int K) {
+  const mms::Rows r = mms::stream_rows(M, N, K);
   return r.mt > 0 && r.mt + r.nt <= 3;
 }
 
