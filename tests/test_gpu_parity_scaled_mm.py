@@ -465,3 +465,20 @@ def test_scaled_mm_row_groups_taken(ops, M, N, K, rows, cols):
     from vllm_amd._lib import lib
     assert lib.vllm_amd_scaled_mm_kernel(M, N, K, 0) == 3700 + 10 * (rows // 16) + cols // 16
     test_scaled_mm_row_groups(ops, M, N, K, torch.bfloat16)
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (1101, 8184, 1024, 39), (700, 14336, 512, 39), (289, 6136, 4096, 7), (384, 6144, 2048, 38),
+    (2852, 2000, 256, 3), (1100, 11960, 256, 2), (1600, 11960, 256, 39), (467, 11720, 384, 3), (8474, 1896, 1024, 39), (66, 27848, 384, 38), (66, 28240, 256, 3),
+])
+def test_scaled_mm_tile_taken(ops, M, N, K, kernel):
+    """The tile that the rule says, at the edges of where it was fitted: every output once, exact sums."""
+    from vllm_amd._lib import lib
+    assert lib.vllm_amd_scaled_mm_kernel(M, N, K, 0) == kernel
+    g = torch.Generator().manual_seed(M)
+    a = torch.randint(-2, 3, (M, K), generator=g).float().cuda()
+    w = torch.randint(-2, 3, (N, K), generator=g).float().cuda()
+    a[:, 0], w[:, 1] = torch.arange(M, device="cuda") % 7, torch.arange(N, device="cuda") % 5
+    one = torch.ones((1, 1), device="cuda")
+    out = ops.cutlass_scaled_mm(a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn).t(), one, one, torch.bfloat16)
+    assert torch.equal(out, (a @ w.t()).to(torch.bfloat16))

@@ -123,6 +123,21 @@ def test_scaled_mm_row_groups_rule(M, N, K, kernel):
     assert lib.vllm_amd_scaled_mm_kernel(M, N, K, 0) == kernel
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (4096, 4096, 4096, 2), (3072, 6144, 4096, 39), (2048, 6144, 4096, 39), (512, 7168, 8192, 38), (128, 6144, 4096, 7),
+    (1024, 10240, 8192, 39), (1536, 6144, 4096, 39), (288, 6144, 4096, 7), (384, 6144, 2048, 38), (1700, 1280, 8192, 38),
+    (303, 1696, 6400, 9), (241, 2560, 5120, 7),                 # up to 288 tiles of 64 x 32 stay
+    (2852, 11960, 256, 39), (2873, 10896, 384, 39),             # the narrow wide tile where the costs do not reach
+    (467, 23432, 384, 3), (419, 16728, 384, 39), (977, 11720, 512, 39), (453, 16672, 512, 39), (674, 16088, 768, 39),   # a full third round of short K loops, a nearly empty one, K 768
+    (66, 27848, 384, 38), (66, 28240, 256, 3),                  # K groups
+    (1065, 13264, 10368, 3), (6553, 2320, 7424, 3), (8474, 1896, 12672, 39), (1572, 9480, 640, 3),   # tall outputs
+])
+def test_scaled_mm_tile_rule(M, N, K, kernel):
+    """The tile above M 64: the table, and the cost of whole rounds where that overrules it."""
+    from vllm_amd._lib import lib
+    assert lib.vllm_amd_scaled_mm_kernel(M, N, K, 0) == kernel
+
+
 def test_scaled_mm_two_slices_rule():
     """Two K slices (1000 + tile) instead of the weight stream where there is a workspace, not instead of small groups of rows."""
     from vllm_amd._lib import lib

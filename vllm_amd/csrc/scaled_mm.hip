@@ -302,6 +302,11 @@ using namespace va;
 // launches (18 weight shapes of K 1024 .. 16384, N 1280 .. 28672, M 65 .. 4096, weights from HBM, each kernel forced; 9 .. 13 % rms).
 // Taken where it is 5 % below the tile that the table below would take.  715 other launches: some 90 of them change, to 0.62 .. 1.00 of
 // the time (128 x 128 -> 256 x 192 0.76 on average, 128 x 64 -> 128 x 128 in one round 0.80, -> 64 x 64 0.83); profiles/gemm_rounds.txt.
+// Outside of those sizes, 390 launches of K 256 .. 896 and of M up to 16384: 256 x 192 instead of 128 x 128 0.88 and 0.72, but not below K 512
+// where the 128 x 128 tiles fill their third round (384 -> 23432 at M 467 13.4 -> 14.3 us), when storing the output is what takes the time;
+// 256 x 192 tiles of tall outputs stay, as a workgroup walks its tiles without rounds (128 x 128 instead: 10368 -> 13264 at M 1065 213.5 ->
+// 171.4, 7424 -> 2320 at M 6553 144 -> 132, but 4992 -> 2080 at M 7476 97 -> 101, 12672 -> 1896 at M 8474 228 -> 244); K groups stay unless 128 x
+// 128 tiles two to a CU are 10 % below (384 -> 27848 at M 66 7.3 -> 7.6).
 constexpr int kWide192 = 39;   // scaled_mm_pp.hip's 256 x 192 tiles
 struct TileCost { int sel, bm, bn; double c, a, b, a_odd, b_odd; };   // a_odd < 0: one workgroup per CU
 constexpr TileCost kTileCost[] = {
@@ -325,17 +330,24 @@ static double tile_cost(const TileCost& t, int M, int N, int K) {
 }
 // sel: what the table takes
 static int scaled_mm_by_rounds(int sel, int M, int N, int K) {
-  double own = 0.0, best = 1e30;
+  if (sel == kWide192 && K >= 1024 && M > 7000) return sel;
+  double own = 0.0;
+  for (const TileCost& t : kTileCost)
+    if (t.sel == sel) own = tile_cost(t, M, N, K);
+  double best = 0.95 * own;
   int pick = sel;
-  for (int i = 0; i < (int)(sizeof(kTileCost) / sizeof(kTileCost[0])); ++i) {
-    const double us = tile_cost(kTileCost[i], M, N, K);
-    if (kTileCost[i].sel == sel) own = us;
+  for (const TileCost& t : kTileCost) {
+    const double us = tile_cost(t, M, N, K);
+    bool may = false;
+    if (t.sel == 38) may = true;
+    else if (t.sel == 2 || t.sel == kWide192) may = !(K < 512 && sel == 3 && ceil_div(M, 128) * ceil_div(N, 128) > 614);
+    else if (t.sel == 3) may = sel != 38 || us < 0.9 * own;
     // (64 x 64 instead of 128 x 128 tiles: 0.996 of the time on average, up to 1.10; instead of 64 x 32 ones, of which up to 288 share
     // their CUs: 6400 -> 1696 at M 303, 265 tiles, 14.7 -> 16.7 us, 7936 -> 2176 at M 220, 272 tiles, 18.7 -> 19.6; from 300 on 0.80 .. 0.96)
-    const bool may = i < 4 || (i == 4 && (sel == 5 || sel == 6 || sel == 10 || (sel == 9 && ceil_div(M, 64) * ceil_div(N, 32) > 288)));
-    if (may && us < best) { best = us; pick = kTileCost[i].sel; }
+    else if (t.sel == 7) may = sel == 5 || sel == 6 || sel == 10 || (sel == 9 && ceil_div(M, 64) * ceil_div(N, 32) > 288);
+    if (may && us < best) { best = us; pick = t.sel; }
   }
-  return best < 0.95 * own ? pick : sel;
+  return pick;
 }
 
 // Two K slices of the 64 x 32 tile instead of the weight stream: where the activations that every workgroup of that reads (M x K bytes)
@@ -386,6 +398,15 @@ static int scaled_mm_tile(int M, int N, int K, bool vec16, bool forced, bool may
         break;
       }
     }
+  }
+  // 256 x 192 tiles (scaled_mm_pp.hip, which needs the aligned rows) where they save a round of workgroups: a 192-wide tile costs ~7/8 of
+  // a 256-wide one (it stages 56 instead of 64 KiB per K block), so N 6144 (the fused qkv projection) at M 3072 -- 288 tiles = 2
+  // rounds against 384 narrow ones = 2 x 7/8 -- goes 90.2 -> 78.9 us, at M 4096 / 2048 91.5 / 52.3 -> 89.2 / 50.7 us (profiles/r03_gemm_pp.txt
+  // 13); at K 256, outside of what the costs above were fitted to, 12000 columns at M 2852 39.3 -> 34.8.
+  if (sel == 2 && !forced && splits == 1 && vec16) {
+    const int tm = ceil_div(M, 256);
+    const int r256 = ceil_div(tm * ceil_div(N, 256), 256), r192 = ceil_div(tm * ceil_div(N, 192), 256);
+    if (8 * r256 > 7 * r192) sel = kWide192;
   }
   if (!forced && may_split && splits == 1 && vec16 && M > 64) sel = scaled_mm_by_rounds(sel, M, N, K);
   return sel;
