@@ -446,6 +446,14 @@ int vllm_amd_unified_attention_segments(int num_seqs, int num_heads, int num_kv_
                                         int head_size, int max_seqlen_q, int max_seqlen_k,
                                         int num_tokens, int has_alibi);
 
+/* The order in which a launch of the 256-row prefill kernel (128 rows above head size 128) takes the row blocks of a batch that it does not
+ * cut over the keys, as bits: 1 = half blocks from the front and the back of a chunk, 2 = every XCD its share of a head's blocks one by one,
+ * 4 = in the order of their last keys, 8 = the longest sequence's first; 0 = sequence by sequence.  group: q heads per kv head; row_blocks: per
+ * kv head; chunks: sequences that have some, `over` of them over a context at least twice as long, `cached` over any; decodes: sequences
+ * of one token that the same launch takes as decodes.  Host arithmetic only. */
+int vllm_amd_prefill_order(int head_size, int group, int num_kv_heads, int num_seqs, int row_blocks, int chunks, int over, int cached,
+                           int decodes, int window, int max_seq_len);
+
 /* ------------------------------------------------------------------------- */
 /* Peer-to-peer all-reduce over xGMI                         */
 /* ------------------------------------------------------------------------- */

@@ -147,6 +147,28 @@ def test_scaled_mm_two_slices_rule():
     assert k(100, 512, 12288, 1) == 3711 and k(0, 512, 1024, 1) == k(8, 512, 128, 1) == k(8, 516, 1024, 1) == 0
 
 
+PAIRS, SHARES, BY_END, LONGEST = 1, 2, 4, 8
+
+
+def _order(group, heads, blocks, chunks=1, over=0, cached=0, head=128, seqs=None, decodes=0, window=0, max_len=8192):
+    from vllm_amd._lib import lib
+    return lib.vllm_amd_prefill_order(head, group, heads, chunks + decodes if seqs is None else seqs, blocks, chunks, over, cached, decodes, window, max_len)
+
+
+def test_prefill_order_shares():
+    """1, 2 or 4 kv heads: shares per XCD in more than one round of row blocks or of a single chunk, not in one of several, and not under a
+    window of less than 512 and a fifth of the keys."""
+    assert _order(8, 1, 256) == PAIRS and _order(8, 1, 257) == SHARES and _order(4, 4, 64) == PAIRS and _order(4, 4, 65) == SHARES
+    for one in (dict(head=256), dict(group=12), dict(window=4000), dict(decodes=20)):       # what keeps a round from being paired
+        args = {"group": 8, "heads": 2, "blocks": 128, "chunks": 2, **one}
+        assert _order(**args) & SHARES == 0 and _order(**{**args, "blocks": 129}) & SHARES == SHARES, one
+        assert _order(**{**args, "chunks": 1}) == (0 if "window" in one else SHARES), one
+    assert _order(8, 1, 400, window=512) == SHARES and _order(8, 1, 400, window=511) == 0
+    assert _order(8, 1, 400, window=300, max_len=1500) == SHARES and _order(8, 1, 400, window=300, max_len=1501) == 0
+    assert _order(8, 8, 400) == 0 and _order(8, 3, 400) == 0
+    assert _order(8, 1, 400, chunks=3, over=1) == SHARES | BY_END and _order(8, 1, 400, chunks=3, over=2) == 0
+
+
 def test_shard_helpers():
     from vllm_amd.distributed import shard_kv_heads, shard_range
     assert shard_range(8192, 8, 3) == (3072, 4096)

@@ -46,6 +46,7 @@ SIGNATURES = {
     "vllm_amd_scaled_mm": [
         _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i64, _i64, _i, _i, _i, _vp],
     "vllm_amd_scaled_mm_kernel": [_i, _i, _i, _i],
+    "vllm_amd_prefill_order": [_i] * 11,
     "vllm_amd_set_workspace": [_vp, _i64, _vp],
     "vllm_amd_scaled_mm_static": [
         _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i64, _i64, _i, _i, _i, _i, _vp],

@@ -940,7 +940,7 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
       f.kc_block_bytes = p.kc_block_bytes; f.kc_slot_bytes = p.kc_page_bytes; f.kc_head_bytes = p.kc_head_bytes;
       f.vc_block_bytes = p.vc_block_bytes; f.vc_slot_bytes = p.vc_page_bytes; f.vc_head_bytes = p.vc_head_bytes;
       f.sm_scale = p.sm_scale;
-      f.window = p.sliding_window; f.softcap = p.softcap;
+      f.window = p.sliding_window; f.softcap = p.softcap; f.max_k = max_k;
       f.prefix = 0; f.k_new = f.v_new = nullptr; f.k_stride_t = f.k_stride_h = f.v_stride_t = f.v_stride_h = 0;
       f.blocks_per_seq = 0;
       f.decode_segments = apart ? u.num_segments : 1;

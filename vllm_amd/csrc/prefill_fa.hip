@@ -133,7 +133,9 @@ int launch_unified_fa(const FaParams& given, int dtype, bool fp8, hipStream_t st
   const unsigned gx = p.blocks_per_seq > 0 ? (unsigned)(p.blocks_per_seq * p.num_seqs) : (unsigned)(p.num_tokens / tpb + p.num_seqs);
   const unsigned gy = (unsigned)(p.pack > 1 ? p.num_kv_heads : p.num_heads);
   const unsigned slots = p.num_segments > 1 ? (unsigned)p.seg_slots : 0u;
-  const unsigned per = gy == 1 || gy == 2 || gy == 4 ? 8 / gy : 1;   // (fa_find)
+  p.halves = 128 % p.pack == 0;
+  p.shares = fa_shares((int)gy, p.window, p.max_k);
+  const unsigned per = p.shares ? p.shares : 1;   // (fa_find)
   const dim3 grid(((gx > slots ? gx : slots) + per - 1) / per * per, gy);
   int npairs = 0, sub_shift = 0, order = 0;
   if (u != nullptr) {
@@ -193,6 +195,19 @@ int launch_unified_fa(const FaParams& given, int dtype, bool fp8, hipStream_t st
 }
 
 }  // namespace va
+
+// The order of a launch's row blocks: no device, no launch.
+extern "C" int vllm_amd_prefill_order(int head_size, int group, int num_kv_heads, int num_seqs, int row_blocks, int chunks, int over, int cached,
+                                      int decodes, int window, int max_seq_len) {
+  if (group < 1 || num_kv_heads < 1) return 0;
+  const int bm = head_size > 128 ? 128 : 256, pack = group > 1 && group <= 16 ? group : 1, gy = pack > 1 ? num_kv_heads : num_kv_heads * group;
+  const bool most = 2 * over >= chunks, halves = 128 % pack == 0, pairs = va::fa_pairs(bm, halves, gy, row_blocks, decodes, window);
+  const bool few = va::fa_few(va::fa_shares(gy, window, max_seq_len), gy, row_blocks, chunks, pairs, most, window);
+  const int order = (pairs ? 1 : 0) | (few ? 2 : 0);
+  if (pairs || num_seqs > 64 || chunks < 2 || !(few || gy % 8 == 0)) return order;
+  if (halves && (few || (!most && va::fa_by_end(bm, gy, row_blocks, chunks, cached > 0)))) return order | 4;
+  return order | (most && decodes == 0 ? 8 : 0);
+}
 
 #ifdef VA_PROBES
 extern "C" int vllm_amd_probe_fa_stamps(unsigned long long* dst, int nwg) {

@@ -172,13 +172,17 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
   // of one length leave the decodes to the end (2000 over 1500 among 63 of up to 4096 keys 143 -> 152 us, 2048 fresh among 48 of 2000
   // 69 -> 81); up to that, 8 / 1 heads, 5000 fresh among 40 of 1000 138 -> 109, 2 x 3000 among 20 of 3000 87 -> 71.
   const int decodes = !MIXED ? 0 : p.num_seqs > 64 ? p.num_seqs : (int)__popcll(__ballot(my.qlen == 1));
-  at.pair = !SPLIT && BM == 256 && p.window == 0 && 128 % p.pack == 0 && (total + decodes) * gy <= 256;
+  at.pair = !SPLIT && fa_pairs(BM, p.halves, gy, total, decodes, p.window);
   // 1, 2 or 4 heads, several rounds: every XCD takes its share of a head's blocks one by one.  In runs the long ones meet on the
-  // first XCDs (8 / 1 heads, 10000 fresh tokens 483 -> 277 us, 3 x 5000 231 -> 155; 16 / 4, 6000 229 -> 184).
-  const bool few = !SPLIT && !at.pair && !over && (gy == 1 || gy == 2 || gy == 4);
+  // first XCDs (8 / 1 heads, 10000 fresh tokens 483 -> 277 us, 3 x 5000 231 -> 155; 16 / 4, 6000 229 -> 184; head 256 8 / 2, 4460 + 3411
+  // tokens 608 -> 453; window 7792 of 13000 914 -> 545).  Not in one round of several chunks, where blocks do not wait for each other and a run's share their
+  // keys: 2 % on average over 50 steps that are not paired (head size 256, windows, groups that do not divide 128, beside decodes; 16 / 4, head 256,
+  // 14 chunks of 61 .. 98 28.9 us in shares, 27.6 in runs); those of one chunk differ most in length, and shares spread them (6 / 1 heads, 9061
+  // fresh 251 in runs, 237 in shares).
+  const bool few = !SPLIT && fa_few(p.shares, gy, total, (int)__popcll(chunks), at.pair, over, p.window);
   int gs;
   if (few) {
-    const int per = 8 / gy, xcd = hw % 8;
+    const int per = p.shares, xcd = hw % 8;
     at.y = xcd / per;
     gs = hw / 8 * per + xcd % per;
     if (gs >= work) return at;
@@ -204,9 +208,8 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
       // 600 .. 1000 over 500 .. 1000 141 -> 143, 16 x 180 .. 300 over 750 .. 1500 134 -> 143, 19 x 138 .. 230 fresh, 520 blocks, 43 -> 46,
       // 8 x 403 .. 671 over 198 .. 395, 568 blocks, 86 -> 91, 20 x 56 .. 93 fresh, 280 blocks, 26.4 -> 28.5).  And two prompts without a
       // context at any length (3600 + 6000 429 -> 420, 3001 + 5003 317 -> 312; three of 3000 194 : 195, two of 4000 over 1500 331 -> 340).
-      const int n = (int)__popcll(chunks);
-      const bool in_order = BM == 128 || (total * gy <= 512 ? n <= 16 : n == 2 && __ballot(my.blocks > 0 && my.len > my.qlen) == 0);
-      if (128 % p.pack == 0 && (few || (!over && in_order))) {
+      const bool cached = __ballot(my.blocks > 0 && my.len > my.qlen) != 0;
+      if (p.halves && (few || (!over && fa_by_end(BM, gy, total, (int)__popcll(chunks), cached)))) {
         const int sh = __builtin_ctz(tpb), ctx = my.len - my.qlen;
         const int top = wave_max_i(my.blocks > 0 ? ctx + (my.blocks << sh) : 0), low = -wave_max_i(my.blocks > 0 ? -ctx : -top);
         const int step = ((top - low) >> 6) + 1;
@@ -319,7 +322,7 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   const int tok_base = blk * tpb;
   // The rows of this wave: those of its half of the workgroup (waves 0-3 and 4-7, where the group divides into 128 rows) from row
   // hrow0 and token htok on
-  const bool halves = NW == 8 && 128 % pack == 0;
+  const bool halves = NW == 8 && p.halves;
   const int htpb = halves ? tpb / 2 : tpb, hrow0 = halves && wave >= 4 ? 128 : 0;
   int htok = tok_base + hrow0 / pack, new_end = min(tok_base + tpb, qlen);
   if (at.pair) {
@@ -830,7 +833,10 @@ __device__ __forceinline__ void fa_body(const FaParams& p, uint8_t* lds, int hw,
   auto tile_loop = [&](int t_begin, int t_end, auto mode_c, auto vt_c, auto fast_c) __attribute__((always_inline)) {
     constexpr int MODE = decltype(mode_c)::value;
     t_end = min(t_end, t1);
-    for (int t = max(t_begin, t0); t < t_end; ++t) {
+    // (The place of the loop in the instruction cache's lines is worth up to 1.5 %, with the same instructions: one at the front of a line
+    // and its successors behind it measured best of eight places.  Left to what stands in front, any change there moves it.)
+    [[clang::code_align(64)]] for (int t = max(t_begin, t0); t < t_end; ++t) {
+      asm volatile("s_nop 0");
       if (stage_first) stage(t, fast_c, vt_c);
       FA_T(1);
       if constexpr (MODE < 2) {
