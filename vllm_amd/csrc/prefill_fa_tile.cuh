@@ -158,12 +158,25 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
   Seq my = seq_at(lane);                                    // the first 64 sequences stay in registers
   int incl = wave_scan(my.blocks);
   int here = __builtin_amdgcn_readlane(incl, 63), total = here;
-  for (int i = 64; i < p.num_seqs; i += 64) total += __builtin_amdgcn_readlane(wave_scan(seq_at(i + lane).blocks), 63);
+  const unsigned long long chunks = __ballot(my.blocks > 0);
+  int nchunks = 0, nover = 0;   // sequences with row blocks, those of them over contexts at least twice as long
+  if constexpr (!SPLIT) {
+    nchunks = (int)__popcll(chunks);
+    nover = (int)__popcll(__ballot(my.blocks > 0 && my.len >= 3 * my.qlen));
+  }
+  for (int i = 64; i < p.num_seqs; i += 64) {
+    const Seq q = seq_at(i + lane);
+    total += __builtin_amdgcn_readlane(wave_scan(q.blocks), 63);
+    if constexpr (!SPLIT) {
+      nchunks += (int)__popcll(__ballot(q.blocks > 0));
+      nover += (int)__popcll(__ballot(q.blocks > 0 && q.len >= 3 * q.qlen));
+    }
+  }
   if (total == 0) return at;
   const int work = SPLIT ? max(total, min(p.seg_slots, total * nseg)) : total;   // per head
   // Most chunks are short ones over contexts at least twice as long: a sequence's blocks read the same keys, and belong together.
-  const unsigned long long chunks = __ballot(my.blocks > 0);
-  const bool over = !SPLIT && 2 * __popcll(__ballot(my.blocks > 0 && my.len >= 3 * my.qlen)) >= __popcll(chunks);
+  // (Of all sequences: an engine's decodes come first, and of the first 64 alone none may be a chunk.)
+  const bool over = !SPLIT && 2 * nover >= nchunks;
   // One round of workgroups ends with its longest one, and under the causal mask the rows of a block differ in length by up to the
   // chunk: each takes four waves' rows from the front of the chunk and four from its back, which all add up to the same.
   // (A SIMD's second wave is done early; the first one then walks on alone at 1.2 us a tile, two take 1.9.)
@@ -179,7 +192,7 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
   // keys: 2 % on average over 50 steps that are not paired (head size 256, windows, groups that do not divide 128, beside decodes; 16 / 4, head 256,
   // 14 chunks of 61 .. 98 28.9 us in shares, 27.6 in runs); those of one chunk differ most in length, and shares spread them (6 / 1 heads, 9061
   // fresh 251 in runs, 237 in shares).
-  const bool few = !SPLIT && fa_few(p.shares, gy, total, (int)__popcll(chunks), at.pair, over, p.window);
+  const bool few = !SPLIT && fa_few(p.shares, gy, total, nchunks, at.pair, over, p.window);
   int gs;
   if (few) {
     const int per = p.shares, xcd = hw % 8;
@@ -199,7 +212,7 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
     at.seq_len = __builtin_amdgcn_readlane(my.len, l);
   };
   if constexpr (!SPLIT) {
-    if (!at.pair && p.num_seqs <= 64 && (few || gy % 8 == 0) && __popcll(chunks) > 1) {
+    if (!at.pair && p.num_seqs <= 64 && (few || gy % 8 == 0) && nchunks > 1) {
       // Several chunks: an XCD's workgroups start in this order, and what it ends on should be short.  The row blocks in the order of
       // their last keys, those with most of them first, in 64 steps of the range: lane l counts the blocks of its step and the ones
       // before it.  Up to two rounds and 16 chunks; above that, and over long contexts, the blocks of a sequence stay together at head size
@@ -209,7 +222,7 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
       // 8 x 403 .. 671 over 198 .. 395, 568 blocks, 86 -> 91, 20 x 56 .. 93 fresh, 280 blocks, 26.4 -> 28.5).  And two prompts without a
       // context at any length (3600 + 6000 429 -> 420, 3001 + 5003 317 -> 312; three of 3000 194 : 195, two of 4000 over 1500 331 -> 340).
       const bool cached = __ballot(my.blocks > 0 && my.len > my.qlen) != 0;
-      if (p.halves && (few || (!over && fa_by_end(BM, gy, total, (int)__popcll(chunks), cached)))) {
+      if (p.halves && (few || (!over && fa_by_end(BM, gy, total, nchunks, cached)))) {
         const int sh = __builtin_ctz(tpb), ctx = my.len - my.qlen;
         const int top = wave_max_i(my.blocks > 0 ? ctx + (my.blocks << sh) : 0), low = -wave_max_i(my.blocks > 0 ? -ctx : -top);
         const int step = ((top - low) >> 6) + 1;
