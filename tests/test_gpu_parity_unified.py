@@ -897,3 +897,21 @@ def test_unified_shares_behind_decodes():
     few, many = step(40), step(80)
     us(few), us(many)
     assert us(many) < 1.25 * us(few)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,seqs", [
+    ((64, 32), [(400, 400), (350, 350), (300, 300), (290, 290), (280, 280), (401, 401)]),            # six of two q heads: 560 blocks
+    ((32, 32), [(256 + 20 * i, 256 + 20 * i) for i in range(8)] + [(1, 1)]),                          # nine of one: 544 blocks
+    ((128, 32), [(400, 400), (430, 430), (300, 300)]),                                                # three of four: 576
+    ((128, 32), [(400, 401), (430, 430), (300, 300)]),                                                # one of them over a context: by sequence
+])
+def test_unified_row_blocks_of_more_rounds_by_last_keys(oracle, force_fa, fp8, heads, seqs):
+    """More than two rounds of row blocks without a context, by their last keys where few chunks share an XCD."""
+    from vllm_amd import _lib
+    c = make_unified_case(seqs, heads[0], heads[1], 128, 16, torch.bfloat16, fp8=fp8, seed=len(seqs), kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        run(oracle, c, torch.bfloat16, fp8=fp8)
+    finally:
+        _lib.set_tuning("pf_segs", 0)

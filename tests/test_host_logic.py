@@ -169,6 +169,20 @@ def test_prefill_order_shares():
     assert _order(8, 1, 400, chunks=3, over=1) == SHARES | BY_END and _order(8, 1, 400, chunks=3, over=2) == 0
 
 
+def test_prefill_order_by_last_keys():
+    """Several chunks in the order of their last keys: by the query tokens that share a key on an XCD, 32 x tokens per row block / chunks."""
+    for group, two_rounds, more in ((4, 16, 3), (8, 8, 1), (2, 16, 6), (1, 16, 12), (16, 4, 0)):
+        heads = 8 if group > 1 else 32
+        for blocks, most in ((512 // heads, two_rounds), (512 // heads + 1, more), (2048 // heads, more), (2048 // heads + 1, 0)):
+            for chunks in range(2, 20):
+                assert _order(group, heads, blocks, chunks=chunks) == (BY_END if chunks <= most else 0), (group, blocks, chunks)
+    assert _order(4, 8, 64, chunks=3, cached=3) == BY_END and _order(4, 8, 65, chunks=3, cached=1) == 0           # over a context
+    assert _order(4, 8, 64, chunks=4, over=1) == BY_END and _order(4, 8, 64, chunks=4, over=2) == LONGEST
+    assert _order(4, 8, 64, chunks=4, over=2, decodes=1) == 0 and _order(12, 8, 64, chunks=2) == 0                # a group that does not divide 128
+    assert _order(2, 8, 600, chunks=30, head=256) == BY_END and _order(4, 8, 64, chunks=2, seqs=65) == 0
+    assert _order(4, 8, 32, chunks=4) == PAIRS
+
+
 def test_shard_helpers():
     from vllm_amd.distributed import shard_kv_heads, shard_range
     assert shard_range(8192, 8, 3) == (3072, 4096)

@@ -52,10 +52,11 @@ __host__ __device__ inline bool fa_pairs(int bm, int halves, int gy, int blocks,
 __host__ __device__ inline bool fa_few(int shares, int gy, int blocks, int chunks, bool pairs, bool over, int window) {
   return shares && !pairs && !over && (blocks * gy > 256 || (chunks == 1 && window == 0));
 }
-// several chunks, of which not most are short ones over long contexts: the row blocks in the order of their last keys.  cached: some
-// chunk has a context
-__host__ __device__ inline bool fa_by_end(int bm, int gy, int blocks, int chunks, bool cached) {
-  return bm == 128 || (blocks * gy <= 512 ? chunks <= 16 : chunks == 2 && !cached);
+// several chunks, of which not most are short ones over long contexts: the row blocks in the order of their last keys.  The more chunks
+// there are, the fewer of an XCD's 32 CUs read the keys of any of them at a time: 32 tpb / chunks query tokens do.  cached: some chunk has a
+// context
+__host__ __device__ inline bool fa_by_end(int bm, int tpb, int gy, int blocks, int chunks, bool cached) {
+  return bm == 128 || (blocks * gy <= 512 ? chunks <= 16 && 4 * chunks <= tpb : blocks * gy <= 2048 && 20 * chunks <= tpb && !cached);
 }
 // Under a window much shorter than the sequences their row blocks are of one length, and a run of them reads the same keys: in shares
 // every XCD would (us, runs / shares, 32 / 4 heads, window 201 of 7000 keys 65 / 77, 16 / 2, 263 of 17800 93 / 104, 91 of 600 39 / 43).  From

@@ -205,7 +205,7 @@ extern "C" int vllm_amd_prefill_order(int head_size, int group, int num_kv_heads
   const bool few = va::fa_few(va::fa_shares(gy, window, max_seq_len), gy, row_blocks, chunks, pairs, most, window);
   const int order = (pairs ? 1 : 0) | (few ? 2 : 0);
   if (pairs || num_seqs > 64 || chunks < 2 || !(few || gy % 8 == 0)) return order;
-  if (halves && (few || (!most && va::fa_by_end(bm, gy, row_blocks, chunks, cached > 0)))) return order | 4;
+  if (halves && (few || (!most && va::fa_by_end(bm, bm / pack, gy, row_blocks, chunks, cached > 0)))) return order | 4;
   return order | (most && decodes == 0 ? 8 : 0);
 }
 

@@ -215,14 +215,18 @@ __device__ __forceinline__ FaAt fa_find(const FaParams& p, int lane, int hw, int
     if (!at.pair && p.num_seqs <= 64 && (few || gy % 8 == 0) && nchunks > 1) {
       // Several chunks: an XCD's workgroups start in this order, and what it ends on should be short.  The row blocks in the order of
       // their last keys, those with most of them first, in 64 steps of the range: lane l counts the blocks of its step and the ones
-      // before it.  Up to two rounds and 16 chunks; above that, and over long contexts, the blocks of a sequence stay together at head size
-      // 128, whose tiles take too little time for keys from farther than the L2 (us: 8 x 300 .. 500 over 250 .. 500 70 -> 66, 5 x 540 ..
-      // 900 fresh 61 -> 57, head 256 5 x 550 .. 917 fresh 76 -> 68, 3 x 1200 .. 2000 143 -> 132; but 19 x 745 .. 1242 fresh 284 -> 292, 6 x
-      // 600 .. 1000 over 500 .. 1000 141 -> 143, 16 x 180 .. 300 over 750 .. 1500 134 -> 143, 19 x 138 .. 230 fresh, 520 blocks, 43 -> 46,
-      // 8 x 403 .. 671 over 198 .. 395, 568 blocks, 86 -> 91, 20 x 56 .. 93 fresh, 280 blocks, 26.4 -> 28.5).  And two prompts without a
-      // context at any length (3600 + 6000 429 -> 420, 3001 + 5003 317 -> 312; three of 3000 194 : 195, two of 4000 over 1500 331 -> 340).
+      // before it.  What that costs are the keys: row blocks of other chunks run at the same time, and each chunk's keys are read for fewer
+      // query tokens at once, 32 tpb / chunks of them on an XCD (us: 8 x 300 .. 500 over 250 .. 500, 256 tokens, 70 -> 66, 5 x 540 .. 900 fresh 61
+      // -> 57, 16 / 8 heads 12 x 133 .. 587 96 -> 80; but 64 / 8 13 x 95 .. 154 fresh, 79 tokens, 35.0 -> 36.3).  By the last
+      // keys / by sequence, up to two rounds 135 steps of 160 tokens and more 0.946 (three more than 2 % slower), 28 of 128 .. 159 0.979 (three, by up to
+      // 3 %; 13 x 202 .. 336 fresh 42.5 -> 44.3), 16 of fewer 0.996 (five, by up to 5 %).  In more rounds what a launch ends on matters less, and the
+      // blocks wait for keys that have left the L2: without a context 92 steps below 520 tokens 1.029 (by up to 12 %), 108 from 640 on, up to eight
+      // rounds, 0.972 (four) -- three prompts for a group of 4 q heads, six for one of 2, twelve without (32 / 32, 3605 + 3260 309 -> 282, 16 / 8, 6 x
+      // 735 .. 2825 181 -> 173, 32 / 8, 2606 + 2515 + 1572 168 -> 164, 3001 + 5003 317 -> 312) --, beyond eight rounds 0.992 of 11.  Over
+      // contexts, whose keys every block reads, 0.997 of 80.  Above head size 128 a tile takes long enough for keys from anywhere (5 x 550 .. 917 fresh
+      // 76 -> 68, 3 x 1200 .. 2000 143 -> 132).
       const bool cached = __ballot(my.blocks > 0 && my.len > my.qlen) != 0;
-      if (p.halves && (few || (!over && fa_by_end(BM, gy, total, nchunks, cached)))) {
+      if (p.halves && (few || (!over && fa_by_end(BM, tpb, gy, total, nchunks, cached)))) {
         const int sh = __builtin_ctz(tpb), ctx = my.len - my.qlen;
         const int top = wave_max_i(my.blocks > 0 ? ctx + (my.blocks << sh) : 0), low = -wave_max_i(my.blocks > 0 ? -ctx : -top);
         const int step = ((top - low) >> 6) + 1;
