@@ -915,3 +915,37 @@ def test_unified_row_blocks_of_more_rounds_by_last_keys(oracle, force_fa, fp8, h
         run(oracle, c, torch.bfloat16, fp8=fp8)
     finally:
         _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,D", [((8, 2), 64), ((16, 8), 256), ((4, 4), 128)])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_unified_few_sequences_long_decodes(oracle, heads, D, fp8, softcap):
+    """Fewer than 16 sequences with a decode of 3100 keys: in a launch of their own where the chunks' kernel takes none along, and as row
+    blocks where a key is 1024 bytes; every token written once."""
+    from vllm_amd import _lib
+    c = make_unified_case([(1, 3100), (300, 310), (1, 1), (2, 900)], heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=D + 1, kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        run(oracle, c, torch.bfloat16, fp8=fp8, softcap=softcap)
+    finally:
+        _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("seqs", [
+    [(1, 1100), (150, 400), (1, 7), (170, 170), (1, 900), (163, 300), (1, 1030)],        # the decodes start behind 192 of 256 row blocks
+    [(150, 400), (170, 180), (163, 600), (160, 160), (2, 700)],                          # none
+])
+def test_unified_decodes_between_row_blocks(oracle, force_fa, fp8, seqs):
+    """Decodes behind the first 192 workgroup ids, row blocks on both sides of them: with a group of 16 q heads 16 tokens are a row
+    block, and 8 kv heads make 240 of them."""
+    from vllm_amd import _lib
+    c = make_unified_case(seqs, 128, 8, 128, 16, torch.bfloat16, fp8=fp8, seed=len(seqs), kv_scale=0.5)
+    _lib.set_tuning("pf_segs", 1)
+    try:
+        before = _mixed_launches()
+        run(oracle, c, torch.bfloat16, fp8=fp8, view=lambda t: t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3))
+        assert _mixed_launches() - before == 1
+    finally:
+        _lib.set_tuning("pf_segs", 0)

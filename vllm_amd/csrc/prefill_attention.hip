@@ -912,8 +912,12 @@ static int launch_unified(PrefillParams p, int head_size, int block_size, int ma
                             u.hp == 1 && p.softcap == 0.f && p.sliding_window == 0 && unified_decode_pairs(u) <= 512;
     // In a launch of their own: always with 16 sequences and more; below that where the tile kernel would walk many more keys for one of
     // them than for a chunk (us, head 64, 32 / 8, 2 x 1500 over 500 among 5 of 8000 213 -> 95, 2000 among 3 of 4000 105 -> 76; head 256,
-    // 16 / 8, 312 -> 168, 164 -> 132), and not split (the segments spread the walk).
-    const bool apart = beside && !one_launch && (mixed || (plan.nseg <= 1 && max_q >= 256 && max_k >= 2048));
+    // 16 / 8, fp8 312 -> 168, 164 -> 132), and not split (the segments spread the walk).  Those keys may be a chunk's own context, and the launch in
+    // front then costs what it takes: head 64 from 3072 keys on (5 chunks over up to 1824 among decodes of 377, 598 and 1113 116 -> 127, 6 among one
+    // of 1684 71 -> 82); 1024 bytes a key, which a workgroup of the decode kernel walks no faster, from 6144 on (head 256 over a 16-bit cache, 6 x
+    // 720 .. 1462 among decodes of 2066, 3103, 3657 and 4334 179 -> 260, ten such steps 1.21; among one of 6542 223 -> 192).
+    const int far = head_size <= 64 ? 3072 : 2 * head_size * (FP8 ? 1 : 2) >= 1024 ? 6144 : 2048;
+    const bool apart = beside && !one_launch && (mixed || (plan.nseg <= 1 && max_q >= 256 && max_k >= far));
     // Beside chunks in segments, few decodes are cut like a batch of their own, and the chunks' merge takes theirs along (a merge of
     // their own is 2 us where they turn out short).  us, 8 / 1 heads, 500 among 20 of 8000 69 -> 35, 3 x 1000 among 30 of 10605 127 -> 72,
     // 16-bit 1000 over 2000 among 40 of 4000 76 -> 53, 600 over 1000 among 16 of 5105 76 -> 39; 500 over 8000 among 30 of 200, short

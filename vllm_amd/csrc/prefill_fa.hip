@@ -145,10 +145,12 @@ int launch_unified_fa(const FaParams& given, int dtype, bool fp8, hipStream_t st
       for (order = 1; order < 30 && u->max_seq_len > 0 && (u->max_seq_len >> order) != 0;) ++order;
   }
   const unsigned nfa = (grid.x * grid.y + 7) / 8 * 8;   // (the ids behind them go round-robin over the XCDs too)
-  // Fewer than 16 sequences have a decode with at least twice the longest chunk's keys here, if any: not behind all row blocks but
-  // behind the 24 of every XCD that start first (us, 32 / 8 heads, 2 x 1500 over 500 among 5 of 8000 99 -> 78, 3 x 1200 among one of
-  // 16000 127 -> 98, 2 x 4000 among 10 of 10000 252 -> 233; 16-bit 126 -> 88, 181 -> 155, 291 -> 238).  With more sequences the longest
-  // may be a chunk's context, and what starts late a row block: 64 / 8, 3 x 540 over 4000 among 40 of 2566 183 -> 200.
+  // Fewer than 16 sequences have keys of at least twice the longest chunk's tokens here.  They may be a decode's: those do not come behind all
+  // row blocks but behind the 24 of every XCD that start first (us, 32 / 8 heads, 2 x 1500 over 500 among 5 of 8000 99 -> 78, 3 x 1200 among one
+  // of 16000 127 -> 98, 2 x 4000 among 10 of 10000 252 -> 233; 16-bit 126 -> 88, 181 -> 155, 291 -> 238).  They may as well be a chunk's own
+  // context, and then the workgroups that find no decode keep a few row blocks waiting: 0.2 % on average, up to 2 us (64 / 8, 14 x 62 .. 130 over
+  // 256 .. 678 54.0 -> 56.5); behind all row blocks that was no less.  With more sequences the longest may be a chunk's context, and what
+  // starts late a row block: 64 / 8, 3 x 540 over 4000 among 40 of 2566 183 -> 200.
   const int first = nfa < 8 * 24 ? (int)nfa : 8 * 24, early = p.num_seqs < 16 ? npairs / 8 * 8 : 0;
 #define FA_MIXED(T_, F_)                                                                                                  \
   hipLaunchKernelGGL((fa::fa_mixed_kernel<T_, F_>), dim3(nfa + (unsigned)npairs), dim3(512), 0, st, p, *u, (int)grid.x, \
