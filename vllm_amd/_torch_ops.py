@@ -114,7 +114,6 @@ silu_and_mul_quant = torch.ops._C.silu_and_mul_quant
 compute_slot_mapping = torch.ops._vllm_amd_C.compute_slot_mapping
 #: dynamic activation quantisation + cutlass_scaled_mm; decode in the form that paged_attention_v2's plan has; the attention calls
 #: behind attention/ops
-fp8_linear = torch.ops._vllm_amd_C.fp8_linear.default
 fp8_linear_new = torch.ops._vllm_amd_C.fp8_linear_new.default
 paged_attention_decode = torch.ops._vllm_amd_C.paged_attention_decode.default
 unified_attention = torch.ops._vllm_amd_C.unified_attention.default

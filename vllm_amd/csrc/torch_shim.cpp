@@ -706,6 +706,7 @@ void register_all() {
   x.op("paged_attention_decode",
        "paged_attention_decode(Tensor! out, Tensor query, Tensor key_cache, Tensor value_cache," PA_TAIL,
        &paged_attention_decode);
+  // (with the caller's output; the Python functions take the one below)
   x.op("fp8_linear",
        "fp8_linear(Tensor! out, Tensor input, Tensor weight, Tensor weight_scale, Tensor? scale_ub, Tensor? bias,"
        " bool per_token) -> ()",
