@@ -574,7 +574,8 @@ int vllm_amd_ar_free_shared(void* ptr);
 /* ------------------------------------------------------------------------- */
 int vllm_amd_set_tuning(const char* key, int value);
 /* current value of "pa_balance" / "mm_kernel" / "mm_splitk" (the torch layer asks before it allocates); "pf_mixed_launches": how many
- * mixed unified_attention steps went out as one launch so far, in this process */
+ * mixed unified_attention steps went out as one launch so far, in this process, "pf_cut_launches": in how many the merge of a chunk's key
+ * segments took cut decodes along */
 int vllm_amd_get_tuning(const char* key, int* value);
 
 #ifdef __cplusplus

@@ -486,11 +486,11 @@ def test_unified_mixed_one_launch(oracle, force_fa, heads, D, fp8, n, mode):
             _lib.set_tuning("pa_order", 1)
 
 
-def _mixed_launches():
+def _mixed_launches(key=b"pf_mixed_launches"):
     import ctypes
     from vllm_amd import _lib
     n = ctypes.c_int()
-    _lib.check(_lib.lib.vllm_amd_get_tuning(b"pf_mixed_launches", ctypes.byref(n)))
+    _lib.check(_lib.lib.vllm_amd_get_tuning(key, ctypes.byref(n)))
     return n.value
 
 
@@ -949,3 +949,18 @@ def test_unified_decodes_between_row_blocks(oracle, force_fa, fp8, seqs):
         assert _mixed_launches() - before == 1
     finally:
         _lib.set_tuning("pf_segs", 0)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("heads,D,decodes,most,cut", [
+    ((8, 1), 128, 15, 2200, 1), ((16, 2), 64, 15, 2200, 1), ((8, 2), 256, 15, 2200, 1), ((24, 1), 80, 15, 2200, 1),
+    ((8, 1), 128, 63, 2200, 0),       # 65 (sequence, kv head) pairs
+    ((8, 1), 128, 15, 1900, 0),       # fewer than 2048 keys
+])
+def test_unified_decodes_cut_beside_segments_taken(oracle, heads, D, decodes, most, cut, fp8):
+    """The same, with a look at whether the chunk's merge took the decodes along."""
+    seqs = [(40, most)] + [(1, (1, 63, 64, 65, 128, 129, 900, most - 100, 1025)[i % 9]) for i in range(decodes)] + [(9, 30)]
+    c = make_unified_case(seqs, heads[0], heads[1], D, 16, torch.bfloat16, fp8=fp8, seed=D, kv_scale=0.5)
+    before = _mixed_launches(b"pf_cut_launches")
+    run(oracle, c, torch.bfloat16, fp8=fp8)
+    assert _mixed_launches(b"pf_cut_launches") - before == cut

@@ -40,7 +40,7 @@ extern int g_uni_decode;
 extern int g_pf_fa;
 extern int g_pf_segs;
 extern int g_pf_mixed;
-extern std::atomic<int> g_pf_mixed_launches;   // prefill_fa.hip
+extern std::atomic<int> g_pf_mixed_launches, g_pf_cut_launches;   // prefill_fa.hip
 extern int g_pf_fa_stagger;
 
 template <typename cache_t> struct CacheTraits;
@@ -732,5 +732,6 @@ extern "C" int vllm_amd_get_tuning(const char* key, int* value) {
   if (strcmp(key, "mm_kernel") == 0) { *value = g_mm_kernel; return VLLM_AMD_OK; }
   if (strcmp(key, "mm_splitk") == 0) { *value = g_mm_splitk; return VLLM_AMD_OK; }
   if (strcmp(key, "pf_mixed_launches") == 0) { *value = g_pf_mixed_launches.load(std::memory_order_relaxed); return VLLM_AMD_OK; }
+  if (strcmp(key, "pf_cut_launches") == 0) { *value = g_pf_cut_launches.load(std::memory_order_relaxed); return VLLM_AMD_OK; }
   VA_REQUIRE(false, VLLM_AMD_EINVAL, "get_tuning: unknown key %s", key);
 }

@@ -126,6 +126,7 @@ __global__ __launch_bounds__(256) void fa_reduce_kernel(const FaParams p) {
 
 int g_pf_fa_stagger = 1;   // tuning "pf_fa_stagger": 0 = all eight waves stage at the bottom of the interval
 std::atomic<int> g_pf_mixed_launches{0};   // get_tuning "pf_mixed_launches"
+std::atomic<int> g_pf_cut_launches{0};     // get_tuning "pf_cut_launches": merges that took cut decodes along
 int launch_unified_fa(const FaParams& given, int dtype, bool fp8, hipStream_t st, const UniDecodeParams* u) {
   FaParams p = given;
   const bool wide = p.head_size > 128;                 // 128-row workgroups of four waves
@@ -179,6 +180,7 @@ int launch_unified_fa(const FaParams& given, int dtype, bool fp8, hipStream_t st
   else if (dtype == VLLM_AMD_BF16) { if (fp8) FA_LAUNCH(bf16_t, true); else FA_LAUNCH(bf16_t, false); }
   else { if (fp8) FA_LAUNCH(f16_t, true); else FA_LAUNCH(f16_t, false); }
   if (p.num_segments > 1) {
+    if (p.decode_segments > 1) g_pf_cut_launches.fetch_add(1, std::memory_order_relaxed);
     const dim3 rgrid((unsigned)(((int64_t)p.num_tokens * p.num_heads + 3) / 4));
 #define FA_REDUCE(T_)                                                                          \
   do {                                                                                         \
